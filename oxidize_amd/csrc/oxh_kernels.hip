@@ -2704,8 +2704,8 @@ extern "C" int oxh_moe_route(const float *d_logits, size_t n_tok, size_t n_exper
     if (top_k == 0 || top_k > OXH_MOE_MAX_TOPK || top_k > n_expert)
         return arg_fail("oxh_moe_route: top_k must be 1..8 and at most n_expert");
     if (n_tok > 4096) return arg_fail("oxh_moe_route: at most 4096 tokens per call");
-    /* a wave per token in the first phase, per expert in the second: up to 16 waves */
-    const size_t waves = n_tok > n_expert ? n_tok : n_expert;
+    /* a lane per token: one wave up to 64 tokens, whose barriers then cost nothing, up to 16 waves */
+    const size_t waves = (n_tok + 63u) / 64u;
     const uint32_t threads = 64u * (uint32_t)(waves > 16 ? 16 : waves);
     hipLaunchKernelGGL(k_moe_route, dim3(1), dim3(threads), 0, pick_stream(stream),
                        d_logits, (uint32_t)n_tok, (uint32_t)n_expert, (uint32_t)top_k, renorm, d_ids, d_weights,

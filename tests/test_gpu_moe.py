@@ -103,6 +103,30 @@ def test_route_ties_follow_the_swapping_selection(oxh):
     assert np.allclose(d[1].download(np.float32, n).reshape(n_tok, k), want_w, rtol=2e-6)
 
 
+@pytest.mark.parametrize("n_tok,n_exp,k", [(64, 8, 2), (65, 8, 2), (128, 64, 8), (129, 64, 8), (1024, 8, 1), (1025, 7, 3)])
+def test_route_at_the_edges_of_its_batches(oxh, n_tok, n_exp, k):
+    """A lane per token, batches of what LDS holds (1024 tokens, 128 at 64 experts), runs of 64 pairs per wave;
+    infinite and NaN logits lose or win as in the reference's scan."""
+    o = oxlibs.oracle()
+    logits = synth.normal(n_tok * n_exp, seed=n_tok, stream=77).reshape(n_tok, n_exp)
+    logits[::7, n_exp // 2] = -np.inf
+    logits[3::11, 0] = np.nan
+    logits[5::13, n_exp - 1] = np.nan
+    want = np.zeros((n_tok, k), np.int32)
+    want_w = np.zeros((n_tok, k), np.float32)
+    o.oxo_moe_route(logits.ctypes.data, n_tok, n_exp, k, 1, want.ctypes.data, want_w.ctypes.data)
+    n = n_tok * k
+    d_l = mv.DeviceBuffer.from_host(logits)
+    d = [mv.DeviceBuffer(4 * max(n, n_exp + 1)) for _ in range(6)]
+    mv.moe_route(d_l.ptr, n_tok, n_exp, k, 1, *[b.ptr for b in d])
+    mv.sync()
+    ids = d[0].download(np.int32, n).reshape(n_tok, k)
+    assert np.array_equal(ids, want)
+    assert np.allclose(d[1].download(np.float32, n).reshape(n_tok, k), want_w, rtol=2e-6, atol=1e-30, equal_nan=True)
+    for got, expect, size in zip(d[2:], group(ids, n_exp), (n_exp, n_exp + 1, n, n)):
+        assert np.array_equal(got.download(np.uint32, size), expect)
+
+
 def dot_fn(qt):
     o = oxlibs.oracle()
     if qt == Q6K:
