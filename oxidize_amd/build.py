@@ -33,7 +33,7 @@ def _run(cmd):
     return proc.stdout
 
 
-HIP_UNITS = ("oxh_kernels", "oxh_plan")
+HIP_UNITS = ("oxh_kernels", "oxh_plan", "oxh_experts")
 
 
 def exported_names():

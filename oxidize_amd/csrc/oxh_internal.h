@@ -38,6 +38,14 @@ int oxh_internal_multi_create(const struct OxhPlanOp *ops, size_t n_ops, void **
 int oxh_internal_multi_launch(void *handle, void *stream);
 void oxh_internal_multi_info(const void *handle, size_t *n_items, size_t *workgroups, size_t *lds_bytes);
 int oxh_internal_multi_destroy(void *handle);
+/* Expert matmuls over many tokens per expert (oxh_experts.hip); both return a hipError_t.  `file_type` is
+ * the weights' type without the tile-major mark, `pairs` the (token, expert) pairs in all, `max_tokens` the
+ * most one expert can get; counts and offsets are in device memory.  The caller has checked the sizes. */
+int oxh_internal_experts_init(void);
+int oxh_internal_experts_long(uint32_t file_type, int tile_major, const void *const *d_w, float *const *d_out,
+                              size_t n_mat, size_t n_expert, size_t rows, size_t cols, const void *d_acts,
+                              size_t out_stride, const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs,
+                              size_t max_tokens, void *stream);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
 int oxh_internal_copy16(void *dst, const void *src, size_t bytes, void *stream);
 /* Wait for a stream by polling it `spins` times before blocking. */

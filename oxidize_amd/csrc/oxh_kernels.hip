@@ -937,12 +937,10 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mmq_q6_k_split<2, true, 2>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q45_k_split<false, 2, 2>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q45_k_split<true, 2, 2>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k_experts<1, 1, 4, 2>)) != hipSuccess) return e;
+    if ((e = raise_lds_ceiling(k_mmq_q6_k_experts<2>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q4_k_segments<1, 1, 8, 3>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<1, 1, 8, false, 3>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k_experts<4, 1, 8, 1>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<4, 1, 8, false, 1>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<4, 1, 8, true, 1>)) != hipSuccess) return e;
+    if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<8, false, 3>)) != hipSuccess) return e;
+    if ((e = (hipError_t)oxh_internal_experts_init()) != hipSuccess) return e;
     return hipSuccess;
 }
 
@@ -2714,24 +2712,20 @@ extern "C" int oxh_moe_route(const float *d_logits, size_t n_tok, size_t n_exper
     return OXH_OK;
 }
 
-/* one launch of the MFMA tile kernel over all experts, activation runs from device memory */
-/* one or more launches of the MFMA tile kernel over all experts, activation runs from device memory.
- * `pairs` = (token, expert) pairs in all; from about two dozen per expert on average on, the 128-row x 64-token tile
- * (eight waves) re-streams an expert's weights four times less often than the 64 x 16 one. */
-template <int TC, int WAVES>
+/* one or more launches of the sixteen-token MFMA tile kernel over all experts, activation runs from device memory */
+template <int WAVES>
 static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *const *d_out, size_t n_mat,
                                 size_t n_expert, size_t rows, size_t cols, const void *d_acts, size_t out_stride,
                                 const uint32_t *d_counts, const uint32_t *d_offsets, size_t max_tokens, void *stream)
 {
-    /* sixteen-token tiles take the token tile from the grid's second dimension: as many as an expert that
-     * every token chose would need */
-    const uint32_t ny = TC == 1 ? (uint32_t)((max_tokens + 15u) / 16u ? (max_tokens + 15u) / 16u : 1u) : 1u;
+    /* the token tile is the grid's second dimension: as many as an expert that every token chose would need */
+    const uint32_t ny = max_tokens ? (uint32_t)((max_tokens + 15u) / 16u) : 1u;
     if (ny > 65535u) return arg_fail("moe: too many tokens for the sixteen-token tile");
     const uint32_t tile_major = is_t16(qtype) ? 1u : 0u;
     qtype = t16_base(qtype);
-    typedef MmqGeom<TC, 1, WAVES> G;
-    typedef Mmq6Geom<TC, 1, WAVES> G6;
-    typedef MmqGeom<TC, 1, WAVES, true> G5;
+    typedef MmqGeom<1, 1, WAVES> G;
+    typedef Mmq6Geom<1, 1, WAVES> G6;
+    typedef MmqGeom<1, 1, WAVES, true> G5;
     static_assert(G6::ROWS == G::ROWS && G5::ROWS == G::ROWS, "row tiling is shared by all formats");
     const size_t blocks = cols / OXH_QK_K;
     if (blocks * 292u * 256u > 0xFFFFFFFFull) return arg_fail("moe: cols too large");
@@ -2761,19 +2755,19 @@ static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *c
             }
         t.n = n;
         for (uint32_t i = 1; i < 4 && i < n; i++) t.bound[i - 1] = t.s[i].wg_begin;
-        /* super-blocks per stage: one in the large tile (no LDS to spare), two in the 64-row tile when the
-         * launch is small, three in the 128-row one (Q4_K only) */
-        if constexpr (TC == 1 && WAVES == 8) {
+        /* super-blocks per stage: two in the 64-row tile when the launch is small, three in the 128-row one
+         * (Q4_K only) */
+        if constexpr (WAVES == 8) {
             if (!is_q4k(qtype)) return arg_fail("moe: the 128-row small tile exists for Q4_K only");
-            OXH_EXP_LAUNCH((k_mmq_q45_k_experts<1, 1, 8, false, 3>), G, 3, tile_major);
-        } else if (TC == 1 && mmq_deep_stages(wg)) {
-            if (qtype == OXH_Q6_K) OXH_EXP_LAUNCH((k_mmq_q6_k_experts<TC, 1, WAVES, 2>), G6, 2);
-            else if (is_q5k(qtype)) OXH_EXP_LAUNCH((k_mmq_q45_k_experts<TC, 1, WAVES, true, 2>), G5, 2, tile_major);
-            else OXH_EXP_LAUNCH((k_mmq_q45_k_experts<TC, 1, WAVES, false, 2>), G, 2, tile_major);
+            OXH_EXP_LAUNCH((k_mmq_q45_k_experts<8, false, 3>), G, 3, tile_major);
+        } else if (mmq_deep_stages(wg)) {
+            if (qtype == OXH_Q6_K) OXH_EXP_LAUNCH((k_mmq_q6_k_experts<2>), G6, 2);
+            else if (is_q5k(qtype)) OXH_EXP_LAUNCH((k_mmq_q45_k_experts<4, true, 2>), G5, 2, tile_major);
+            else OXH_EXP_LAUNCH((k_mmq_q45_k_experts<4, false, 2>), G, 2, tile_major);
         } else {
-            if (qtype == OXH_Q6_K) OXH_EXP_LAUNCH((k_mmq_q6_k_experts<TC, 1, WAVES, 1>), G6, 1);
-            else if (is_q5k(qtype)) OXH_EXP_LAUNCH((k_mmq_q45_k_experts<TC, 1, WAVES, true, 1>), G5, 1, tile_major);
-            else OXH_EXP_LAUNCH((k_mmq_q45_k_experts<TC, 1, WAVES, false, 1>), G, 1, tile_major);
+            if (qtype == OXH_Q6_K) OXH_EXP_LAUNCH((k_mmq_q6_k_experts<1>), G6, 1);
+            else if (is_q5k(qtype)) OXH_EXP_LAUNCH((k_mmq_q45_k_experts<4, true, 1>), G5, 1, tile_major);
+            else OXH_EXP_LAUNCH((k_mmq_q45_k_experts<4, false, 1>), G, 1, tile_major);
         }
     }
 #undef OXH_EXP_LAUNCH
@@ -2786,12 +2780,27 @@ static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *
                           const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs, size_t max_tokens,
                           void *stream)
 {
-    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);     /* 0 = never */
     const size_t avg_tokens = pairs / n_expert;
     const uint32_t file_type = t16_base(qtype);
-    if (big_from && avg_tokens >= big_from)
-        return launch_experts_tiled<4, 8>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
-                                          d_counts, d_offsets, max_tokens, stream);
+    const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
+    /* Many tokens per expert (two dozen on average): tiles that read an expert's weights once for 64 or 144 of its
+     * tokens (oxh_experts.hip), unless there are too few of them and of tokens: under 64 tokens per expert a launch
+     * that does not give nearly every CU a 128 x 64 tile runs faster on many 64 x 16 ones (4 experts, top 1, 1024 x
+     * 2048, 200 tokens: 37 against 40 us a layer; 8 experts, top 2, 100 tokens: 45 against 40).  From ten tokens
+     * per expert on when the 64 x 16 tiles are eight to a CU and more, whose second pass over the weights then
+     * costs more than it hides (Mixtral-shaped, 64 tokens: 278 against 232 us).  OXH_MOE_BIG_TILE_FROM overrides
+     * the average to start from, 0 = never. */
+    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);
+    const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
+    const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
+    if (big_from && ((avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) ||
+                     (avg_tokens >= 10 && big_from <= 24 && small_tiles >= 8 * cus))) {
+        if (cols / OXH_QK_K * 292u * 256u > 0xFFFFFFFFull) return arg_fail("moe: cols too large");
+        const int e = oxh_internal_experts_long(file_type, is_t16(qtype), d_w, d_out, n_mat, n_expert, rows, cols, d_acts,
+                                                out_stride, d_counts, d_offsets, pairs, max_tokens, pick_stream(stream));
+        if (e) return hip_fail((hipError_t)e, "expert launch");
+        return OXH_OK;
+    }
     /* few rows per expert (a down projection): the 64-row tile gives at most two workgroups per CU; Q4_K
      * can take 128 rows on eight waves with three super-blocks per stage instead, half as much again in
      * flight (OXH_MOE_WIDE_SMALL=1).  Off by default: launched continuously, Mixtral's down projections at
@@ -2799,13 +2808,12 @@ static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *
      * the wider tile only won when the launches were timed right after an idle period).  Workgroups of
      * experts without a token leave at once, so what counts is the experts that can have one. */
     static const uint32_t wide = env_u32("OXH_MOE_WIDE_SMALL", 0, 0, 1);
-    const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
     const size_t live = pairs < n_expert ? (pairs ? pairs : 1) : n_expert;
     if (wide && is_q4k(file_type) && n_mat * n_expert * ((rows + 63) / 64) <= 2u * cus &&
         n_mat * live * ((rows + 127) / 128) >= cus - cus / 8)
-        return launch_experts_tiled<1, 8>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
+        return launch_experts_tiled<8>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
                                           d_counts, d_offsets, max_tokens, stream);
-    return launch_experts_tiled<1, 4>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
+    return launch_experts_tiled<4>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
                                       d_counts, d_offsets, max_tokens, stream);
 }
 
