@@ -383,7 +383,9 @@ int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
  * on a device of n_cu compute units: the largest of 256 x 128 (128 x 128 for
  * Q5_K, Q6_K and widened Q2_K), 64 x 128 (Q6_K only), 128 x 64, 64 x 32, 64 x 16
  * that still gives nearly every compute unit a workgroup; 128 x 64 always for
- * the 32-value formats.  Pure host arithmetic (no device needed); OXH_DECLINED
+ * the 32-value formats.  (Q6_K and widened Q2_K launches of more than 32
+ * activations weigh the tiles' measured times on top of that and may run on
+ * another of these tiles than the one reported; the results are the same bits.)  Pure host arithmetic (no device needed); OXH_DECLINED
  * for a type without a matrix-core kernel.
  * The reference has no counterpart: its batch kernel takes four activations
  * per weight row regardless of the shape (oxk.c:787-836). */

@@ -46,6 +46,11 @@ int oxh_internal_experts_long(uint32_t file_type, int tile_major, const void *co
                               size_t n_mat, size_t n_expert, size_t rows, size_t cols, const void *d_acts,
                               size_t out_stride, const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs,
                               size_t max_tokens, void *stream);
+/* Q6_K (or widened Q2_K) prefill in 64 x 128 tiles whose weight operands the workgroup builds once
+ * (oxh_mmq6.hip); both return a hipError_t.  Arguments checked by the caller. */
+int oxh_internal_mmq6_init(void);
+int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
+                             float *d_out, size_t out_stride, void *stream);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
 int oxh_internal_copy16(void *dst, const void *src, size_t bytes, void *stream);
 /* Wait for a stream by polling it `spins` times before blocking. */

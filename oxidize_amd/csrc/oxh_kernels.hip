@@ -911,11 +911,7 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mmq_q5_k<8, 1, 8, true>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q5_k<4, 1, 8, true>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q6_k<8, 1, 8>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k<4, 1, 8>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k<8, 1, 4>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k<8, 1, 4, true>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q6_k<8, 1, 8, true>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q6_k<4, 1, 8, true>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 0>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 1>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 2>)) != hipSuccess) return e;
@@ -941,6 +937,7 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mmq_q4_k_segments<1, 1, 8, 3>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<8, false, 3>)) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_experts_init()) != hipSuccess) return e;
+    if ((e = (hipError_t)oxh_internal_mmq6_init()) != hipSuccess) return e;
     return hipSuccess;
 }
 
@@ -2204,10 +2201,9 @@ static void mmq6_launch(const void *d_w, size_t rows, size_t blocks, const void 
 
 /* Which tile a matrix-core launch runs on: the largest one that still gives (nearly) every compute
  * unit a workgroup.  1: 256 x 128 (rows x tokens; 128 x 128 for the types with one row chunk per wave:
- * Q5_K, Q6_K, widened Q2_K), 2: 128 x 64, 3: 64 x 32, 4: 64 x 16, 5: 64 x 128 on four waves, which only the
- * Q6_K tile code has, for matrices with too few rows to fill the device with 128 x 128 tiles (the scaled
- * weight operands a wave builds are then still reused by 128 tokens: 4096 x 14336 x 512 takes 144 us
- * against 167 us on 128 x 64 tiles).  Pure arithmetic: OXH_MMQ_SHAPE = 1..5 overrides it at launch. */
+ * Q5_K, Q6_K, widened Q2_K), 2: 128 x 64, 3: 64 x 32, 4: 64 x 16, 5: 64 x 128, which only
+ * Q6_K and widened Q2_K have; their launches of more than 32 activations go by mmq6_tile_shape() instead, and
+ * this rule is what oxh_mmq_tile() reports for them.  Pure arithmetic: OXH_MMQ_SHAPE = 1..5 overrides it at launch. */
 static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
 {
     const size_t need = cus - cus / 8;
@@ -2226,6 +2222,30 @@ static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
     if (((rows + 255) / 256) * ((n_vec + 127) / 128) >= need) return 1;
     if (((rows + 127) / 128) * ((n_vec + 63) / 64) >= need) return 2;
     return few_tiles ? 4 : 3;
+}
+
+/* Which tile a Q6_K (or widened Q2_K) launch of more than 32 activations runs on, by what it is expected to
+ * take.  The unit is a super-block of a full 64 x 128 tile (1.8 us), in which a matrix of 56 super-blocks
+ * measured: 64 x 128 tiles whose operands the workgroup builds once, one to a CU, 0.375 + 0.078 a token chunk
+ * for every round of tiles (75 us at 5 chunks, 91 at 7, 101 at 8); 128 x 128 tiles, one to a CU, 1.6 a round
+ * (161 us); 64 x 32 tiles, three to a CU, 0.75 up to a tile per CU (76 us), 0.95 just above (95 at 448
+ * tiles of 256 CUs), then by their number (122 at 704, 171 at 1024, 242 at 1536), and a sixth less for
+ * widened Q2_K, whose operands take little building (77 at 448, 104 at 704).  (The 128 x 64 tile took 126 us
+ * where the 64 x 128 one takes 91 and is gone.) */
+static int mmq6_tile_shape(size_t rows, size_t n_vec, size_t cus, bool widened_q2)
+{
+    if (n_vec <= 32 || ((rows + 63) / 64) * ((n_vec + 15) / 16) <= cus) return mmq_tile_shape(OXH_Q6_K, rows, n_vec, cus);
+    const size_t tok_tiles = (n_vec + 127) / 128, chunks = ((n_vec + 15) / 16 + tok_tiles - 1) / tok_tiles;
+    const size_t t5 = ((rows + 63) / 64) * tok_tiles, t1 = ((rows + 127) / 128) * tok_tiles;
+    const double per_cu = (double)(((rows + 63) / 64) * ((n_vec + 31) / 32)) / (double)cus;
+    const double c5 = (double)((t5 + cus - 1) / cus) * (0.375 + 0.078 * (double)chunks);
+    const double c1 = (double)((t1 + cus - 1) / cus) * 1.6;
+    double c3 = 0.15 + 0.385 * per_cu;
+    if (c3 < 0.75) c3 = 0.75;
+    if (per_cu > 1.0 && c3 < 0.95) c3 = 0.95;
+    if (widened_q2) c3 *= 0.84;
+    if (c1 < c5 && c1 < c3) return 1;
+    return c5 < c3 ? 5 : 3;
 }
 
 /* the 32-value formats with a matrix-core kernel, as its LEG parameter; -1 for everything else */
@@ -2433,7 +2453,9 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
         return arg_fail("oxh_mmq: cols too large");
     static int forced = -1;
     if (forced < 0) forced = (int)env_u32("OXH_MMQ_SHAPE", 0, 0, 5);
-    int shape = forced ? forced : mmq_tile_shape(qtype, rows, n_vec, (size_t)(g_n_cu > 0 ? g_n_cu : 256));
+    const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
+    int shape = forced ? forced : qtype == OXH_Q6_K || wide2 ? mmq6_tile_shape(rows, n_vec, cus, wide2)
+                                                             : mmq_tile_shape(qtype, rows, n_vec, cus);
     if (qtype == OXH_Q6_K || is_q5k(qtype) || wide2) {
         if (is_q5k(qtype)) {
             if (shape == 5) shape = 2;
@@ -2446,18 +2468,20 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
             HIP_TRY(hipGetLastError());
             return OXH_OK;
         }
+        if (shape == 5 || shape == 2) {
+            const int e = oxh_internal_mmq6_shared(wide2, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride,
+                                                   pick_stream(stream));
+            if (e) return hip_fail((hipError_t)e, "oxh_mmq");
+            return OXH_OK;
+        }
         if (wide2) {
-            if (shape == 5)      mmq6_launch<8, 1, 4, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
-            else if (shape == 1) mmq6_launch<8, 1, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
-            else if (shape == 2) mmq6_launch<4, 1, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
+            if (shape == 1)      mmq6_launch<8, 1, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             else if (shape == 3) mmq6_launch<2, 1, 4, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             else                 mmq6_launch<1, 1, 4, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             HIP_TRY(hipGetLastError());
             return OXH_OK;
         }
-        if (shape == 5)      mmq6_launch<8, 1, 4>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
-        else if (shape == 1) mmq6_launch<8, 1, 8>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
-        else if (shape == 2) mmq6_launch<4, 1, 8>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
+        if (shape == 1)      mmq6_launch<8, 1, 8>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
         else if (shape == 3) mmq6_launch<2, 1, 4>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
         else                 mmq6_launch<1, 1, 4>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
         HIP_TRY(hipGetLastError());

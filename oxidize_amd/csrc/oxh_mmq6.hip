@@ -1,0 +1,305 @@
+/* oxh_mmq6.hip — the prefill matmul of Q6_K (and widened Q2_K) weights in tiles
+ * whose weight operands are built once per workgroup.
+ *
+ * Arithmetic, operand roles and the activations' LDS image are those of
+ * mmq6_tile() (mmq_tiles.inc; oxidize-c/src/compute/oxk.c:913-964): a 210-byte
+ * block becomes two int8 operand planes, (code - 32) * scale = 256 * hi + lo, and
+ * the f32 step is the reference's per super-block.
+ *
+ * Why another tile.  A wave of mmq6_tile() builds the planes of its own 16 rows,
+ * some 200 vector instructions per super-block, against 20 per 16 x 16 chunk of
+ * results: with 128 tokens to a tile that is as much as the results themselves,
+ * with 32 four times as much, and a matrix of 4096 rows under a few hundred
+ * tokens has only enough tiles of the small kinds to fill the device.  Here a
+ * workgroup covers 64 rows x 128 tokens with eight waves, four row chunks x two
+ * token halves; all 512 threads build the next super-block's planes, each
+ * thread an eighth of one row's block straight from its global loads (no trip of
+ * the raw block through LDS), and both waves of a row chunk read them back as
+ * MFMA operands.  Per wave that is half the build of a 64 x 128 tile on four waves at
+ * twice the waves per SIMD.  The build of super-block b + 1 is spread between
+ * the chunks of super-block b, where the matrix cores cover it; one barrier per
+ * super-block. */
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "oxhip.h"
+#include "oxh_internal.h"
+#include "oxh_device.inc"
+#include "mmq_tiles.inc"
+
+struct Q6sGeom {
+    static constexpr uint32_t ROWS = 64u, TOK = 128u;
+    /* one stage: token values [token][slot] x 16 B, token scales, the two planes [row][slot] x 16 B with the
+     * activations' slot swizzle, d (and dmin) per row */
+    static constexpr uint32_t D_OFF = TOK * 256u;
+    static constexpr uint32_t LO_OFF = D_OFF + TOK * 4u;
+    static constexpr uint32_t HI_OFF = LO_OFF + ROWS * 256u;
+    static constexpr uint32_t DW_OFF = HI_OFF + ROWS * 256u;
+    static constexpr uint32_t STAGE_BYTES = DW_OFF + ROWS * 8u;
+    static constexpr uint32_t LDS_BYTES = 2u * STAGE_BYTES;
+};
+
+/* an eighth of a block: 16 bytes of ql (two groups' low bits), the 16 bytes of qh that belong to them, the
+ * two group scales, and the block's d */
+struct Q6sRaw {
+    U32x4u2 ql, qh;
+    uint32_t sc0, sc1, d, dmin;
+};
+
+/* dword k of the planes of the group in the low (HIGH: high) nibbles */
+template <bool Q2, bool HIGH>
+__device__ __forceinline__ void q6s_dword(uint32_t ql, uint32_t qh, uint32_t sc, uint32_t rot, uint32_t &lo, uint32_t &hi)
+{
+    const uint32_t c = ((HIGH ? ql >> 4 : ql) & 0x0F0F0F0Fu) | (__builtin_amdgcn_alignbit(qh, qh, rot) & 0x30303030u);
+    if (Q2) {
+        lo = c;
+        hi = sc;                    /* the group's minimum in every byte, set up by the caller */
+        return;
+    }
+    const short scs = (short)sc, m32 = (short)(128 - 32 * (int)(short)sc);
+    const v2i16 sc2 = { scs, scs }, off2 = { m32, m32 };
+    const v2i16 ce = __builtin_bit_cast(v2i16, __builtin_amdgcn_perm(c, c, 0x0C020C00u));
+    const v2i16 co = __builtin_bit_cast(v2i16, __builtin_amdgcn_perm(c, c, 0x0C030C01u));
+    const uint32_t ue = __builtin_bit_cast(uint32_t, (v2i16)(ce * sc2 + off2));
+    const uint32_t uo = __builtin_bit_cast(uint32_t, (v2i16)(co * sc2 + off2));
+    lo = __builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u;
+    hi = __builtin_amdgcn_perm(uo, ue, 0x07030501u);
+}
+
+/* A wave's N chunks of 16 tokens, the first of them chunk c_first of the tile, over all super-blocks; results
+ * of tokens below toks_end are its to store.  The waves of a workgroup may run it for different N: each passes the same number of barriers. */
+template <int N, bool Q2>
+__device__ __forceinline__ void
+q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, const uint8_t *__restrict__ a_base,
+         uint32_t toks_here, float *__restrict__ out_base, size_t out_stride, uint32_t c_first, uint32_t toks_end)
+{
+    typedef Q6sGeom G;
+    extern __shared__ __attribute__((aligned(16))) uint8_t mmq_lds[];
+    const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t *)mmq_lds;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r16 = lane & 15u, kq = lane >> 4;
+    const uint32_t act_stride = B * 292u;
+
+    /* activations: 64-lane load wave + 8 * i covers tokens 4 * (wave + 8 * i) .. +3, as in mmq6_tile() */
+    uint32_t q_off[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+        const uint32_t t = 4u * (wave + 8u * i) + (lane >> 4);
+        q_off[i] = min(t, toks_here - 1u) * act_stride + 4u + 16u * ((lane & 15u) ^ (t & 15u));
+    }
+    /* this thread's eighth u = 4n + 2h + lh of row tid / 8: ql piece u, qh piece 2n + lh, groups 8n + 2h + lh
+     * (low nibbles) and four further on (high nibbles) */
+    const uint32_t b_row = tid >> 3, u = tid & 7u;
+    const uint32_t grp = 8u * (u >> 2) + (u & 3u);
+    const uint32_t w_off = min(b_row, rows_here - 1u) * (B * 210u);
+    const uint32_t ql_off = w_off + 16u * u, qh_off = w_off + 128u + 32u * (u >> 2) + 16u * (u & 1u);
+    const uint32_t sc_off = w_off + 192u + (Q2 ? grp >> 1 : grp), sc_step = Q2 ? 2u : 4u;
+    const uint32_t rot0 = ((u & 2u) - 4u) & 31u, rot1 = u & 2u;      /* bits 2h, 2h + 1 (2h + 4, 2h + 5) to 4, 5 */
+    const uint32_t pl_wr = G::LO_OFF + b_row * 256u + ((grp ^ (b_row & 15u)) * 16u);     /* ^ 64: four groups on */
+    const uint32_t a_d_off = min(tid & (G::TOK - 1u), toks_here - 1u) * act_stride;
+
+    auto request = [&](uint32_t blk, uint32_t buf) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++)
+            mmq_dma16(a_base + (size_t)blk * 292u, q_off[i], lds_base + buf * G::STAGE_BYTES + (wave + 8u * i) * 1024u);
+    };
+    auto load_raw = [&](uint32_t blk) -> Q6sRaw {
+        const uint8_t *wb = w_base + (size_t)blk * 210u;
+        Q6sRaw r;
+        r.ql = *reinterpret_cast<const U32x4u2 *>(wb + ql_off);
+        r.qh = *reinterpret_cast<const U32x4u2 *>(wb + qh_off);
+        r.sc0 = wb[sc_off];
+        r.sc1 = wb[sc_off + sc_step];
+        r.d = *reinterpret_cast<const uint16_t *>(wb + w_off + 208u);
+        r.dmin = Q2 ? *reinterpret_cast<const uint16_t *>(wb + w_off + 200u) : 0u;
+        return r;
+    };
+    auto load_dq = [&](uint32_t blk) -> uint32_t {
+        return *reinterpret_cast<const uint32_t *>(a_base + (size_t)blk * 292u + a_d_off);
+    };
+    /* a group's scale as the dword builder takes it */
+    auto scale_of = [&](uint32_t byte) -> uint32_t {
+        return Q2 ? ((byte >> (4u * (grp & 1u))) & 15u) * 0x01010101u : (uint32_t)(int)(int8_t)byte;
+    };
+    u32x4 p_lo[2], p_hi[2];
+    auto build_dword = [&](const Q6sRaw &r, int k) {
+        const uint32_t ql[4] = { r.ql.x, r.ql.y, r.ql.z, r.ql.w }, qh[4] = { r.qh.x, r.qh.y, r.qh.z, r.qh.w };
+        uint32_t lo, hi;
+        q6s_dword<Q2, false>(ql[k], qh[k], scale_of(r.sc0), rot0, lo, hi);
+        p_lo[0][k] = lo;
+        p_hi[0][k] = hi;
+        q6s_dword<Q2, true>(ql[k], qh[k], scale_of(r.sc1), rot1, lo, hi);
+        p_lo[1][k] = lo;
+        p_hi[1][k] = hi;
+    };
+    auto store_planes = [&](const Q6sRaw &r, uint32_t dq, uint32_t buf) {
+        uint8_t *st = mmq_lds + buf * G::STAGE_BYTES;
+        *reinterpret_cast<u32x4 *>(st + pl_wr) = p_lo[0];
+        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 64u)) = p_lo[1];
+        *reinterpret_cast<u32x4 *>(st + pl_wr + (G::HI_OFF - G::LO_OFF)) = p_hi[0];
+        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 64u) + (G::HI_OFF - G::LO_OFF)) = p_hi[1];
+        /* the eight threads of a row, and the four of a token, store the same values: no branch in the loop */
+        float *dw = reinterpret_cast<float *>(st + G::DW_OFF) + 2u * b_row;
+        dw[0] = half_to_float_hw(r.d);
+        if (Q2) dw[1] = half_to_float_hw(r.dmin);
+        *reinterpret_cast<uint32_t *>(st + G::D_OFF + 4u * (tid & (G::TOK - 1u))) = dq;
+    };
+
+    v4f acc[N];
+#pragma unroll
+    for (int c = 0; c < N; c++) acc[c] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
+
+    const uint32_t a_rd = r16 * 256u + ((kq ^ r16) * 16u);                          /* ^ 64 * gp */
+    const uint32_t p_rd = G::LO_OFF + (wave & 3u) * 4096u + a_rd;
+    const uint32_t dw_rd = G::DW_OFF + ((wave & 3u) * 16u + r16) * 8u;
+    const uint32_t dq_rd = G::D_OFF + 16u * kq + 64u * c_first;
+
+    /* the first super-block, and the raw blocks of the second */
+    {
+        const Q6sRaw r = load_raw(0);
+        const uint32_t dq = load_dq(0);
+        request(0, 0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) build_dword(r, k);
+        store_planes(r, dq, 0);
+    }
+    Q6sRaw next = load_raw(min(1u, B - 1u));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        /* the LDS-bound loads, which the compiler does not count */
+    __syncthreads();
+
+    for (uint32_t b = 0; b < B; b++) {
+        const uint32_t buf = b & 1u;
+        const uint8_t *st = mmq_lds + buf * G::STAGE_BYTES;
+        request(min(b + 1u, B - 1u), buf ^ 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        v4i dl[4], dh[4];
+#pragma unroll
+        for (int gp = 0; gp < 4; gp++) {
+            dl[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * (uint32_t)gp)));
+            dh[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * (uint32_t)gp)) + (G::HI_OFF - G::LO_OFF));
+        }
+        const float2 dwm = *reinterpret_cast<const float2 *>(st + dw_rd);
+        /* Chunk by chunk: the operands of chunk c + 1 are on their way, and the f32 step of chunk c - 1 and a share
+         * of the next super-block's planes go between the MFMAs of chunk c.  The order is pinned: left to the
+         * compiler the raw blocks are requested behind the last chunk, so that every super-block ends with a
+         * trip to memory, and all requests in one burst at the top stall the waves at their next load
+         * (4096 x 14336, 512 tokens: 115 and 123 us against 101). */
+        Q6sRaw after;
+        uint32_t dq_next = 0;
+        v4i an[4], lo_p = { 0, 0, 0, 0 }, hi_p = { 0, 0, 0, 0 };
+        float4 dq_p = { 0.0f, 0.0f, 0.0f, 0.0f };
+        auto read_a = [&](int c) {
+#pragma unroll
+            for (int gp = 0; gp < 4; gp++)
+                an[gp] = *reinterpret_cast<const v4i *>(st + (a_rd ^ (64u * (uint32_t)gp)) + 4096u * (c_first + (uint32_t)c));
+        };
+        read_a(0);
+#pragma unroll
+        for (int c = 0; c <= N; c++) {
+            v4i lo = { 0, 0, 0, 0 }, hi = { 0, 0, 0, 0 };
+            float4 dq4 = { 0.0f, 0.0f, 0.0f, 0.0f };
+            if (c < N) {
+                const v4i a[4] = { an[0], an[1], an[2], an[3] };
+                if (c + 1 < N) read_a(c + 1);
+                dq4 = *reinterpret_cast<const float4 *>(st + dq_rd + 64u * (uint32_t)c);
+#pragma unroll
+                for (int gp = 0; gp < 4; gp++) {
+                    lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[gp], dl[gp], lo, 0, 0, 0);
+                    hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[gp], dh[gp], hi, 0, 0, 0);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (k * N / 4 == c) build_dword(next, k);
+            }
+            if (c > 0) {
+                const float dqs[4] = { dq_p.x, dq_p.y, dq_p.z, dq_p.w };
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (Q2) {
+                        const float pos = dwm.x * (float)lo_p[i], neg = dwm.y * (float)hi_p[i];
+                        acc[c - 1][i] += dqs[i] * (pos - neg);
+                    } else {
+                        const int isum = lo_p[i] + 256 * hi_p[i];
+                        const float t = dwm.x * dqs[i];
+                        acc[c - 1][i] += t * (float)isum;
+                    }
+                }
+            }
+            lo_p = lo;
+            hi_p = hi;
+            dq_p = dq4;
+            if (c == 0) {
+                after = load_raw(min(b + 2u, B - 1u));
+                dq_next = load_dq(min(b + 1u, B - 1u));
+            }
+            if (c < N) {
+#pragma unroll
+                for (int g = 0; g < 8; g++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);        /* an MFMA */
+                    __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);        /* vector instructions */
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        store_planes(next, dq_next, buf ^ 1u);
+        next = after;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+
+    const uint32_t row = (wave & 3u) * 16u + r16;
+    if (row < rows_here) {
+#pragma unroll
+        for (int c = 0; c < N; c++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t tok = 16u * (c_first + (uint32_t)c) + 4u * kq + (uint32_t)i;
+                if (tok < toks_end) out_base[(size_t)tok * out_stride + row] = acc[c][i];
+            }
+    }
+}
+
+/* grid (row tiles, token tiles); the token chunks are dealt evenly to the token tiles, and a tile's to its
+ * two halves: both waves of a SIMD belong to one tile, so what counts is the chunks of the two together. */
+template <bool Q2>
+__global__ __launch_bounds__(512, 2) void
+k_mmq_q6_k_shared(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t *__restrict__ acts,
+                  uint32_t n_vec, float *__restrict__ out, size_t out_stride)
+{
+    const uint32_t row0 = blockIdx.x * Q6sGeom::ROWS;
+    const uint32_t chunks = (n_vec + 15u) >> 4;
+    const uint32_t c0 = blockIdx.y * chunks / gridDim.y, nc = (blockIdx.y + 1u) * chunks / gridDim.y - c0;
+    const uint32_t tok0 = 16u * c0, here = min(n_vec - tok0, 16u * nc);
+    const uint8_t *wb = w + (size_t)row0 * B * 210u, *ab = acts + (size_t)tok0 * B * 292u;
+    float *ob = out + (size_t)tok0 * out_stride + row0;
+    const uint32_t first_half = (nc + 1u) >> 1;
+    const bool upper = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0u;
+    const uint32_t mine = upper ? nc - first_half : first_half, at = upper ? first_half : 0u;
+    const uint32_t end = upper ? here : min(here, 16u * first_half);
+    if (mine == 4u) q6s_walk<4, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
+    else if (mine == 3u) q6s_walk<3, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
+    else q6s_walk<2, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
+}
+
+extern "C" int oxh_internal_mmq6_init(void)
+{
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_mmq_q6_k_shared<false>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_mmq_q6_k_shared<true>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return (int)e;
+}
+
+/* see oxh_internal.h */
+extern "C" int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts,
+                                        size_t n_vec, float *d_out, size_t out_stride, void *stream)
+{
+    typedef Q6sGeom G;
+    const dim3 grid((uint32_t)((rows + G::ROWS - 1) / G::ROWS), (uint32_t)((n_vec + G::TOK - 1) / G::TOK));
+    auto kernel = widened_q2 ? k_mmq_q6_k_shared<true> : k_mmq_q6_k_shared<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(512), G::LDS_BYTES, (hipStream_t)stream, (const uint8_t *)d_w, (uint32_t)rows,
+                       (uint32_t)blocks, (const uint8_t *)d_acts, (uint32_t)n_vec, d_out, out_stride);
+    return (int)hipGetLastError();
+}

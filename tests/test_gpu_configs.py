@@ -188,6 +188,15 @@ def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
     assert np.array_equal(bits(got), bits(out[:, :rows]))
 
 
+@pytest.mark.parametrize("rows,cols,n_vec", [(4095, 512, 333), (4100, 768, 129), (14300, 256, 40), (14337, 512, 66),
+                                             (7000, 256, 128), (2049, 1024, 400)])
+def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec):
+    """64 x 128 tiles whose operands the workgroup builds once: 7, 5 (4 and 5), 3, 5, 8 and 7 (6) chunks of tokens to a
+    tile, dealt to its two halves; one to four super-blocks; ragged rows and tokens.  Same checks as above."""
+    test_mmq_tile_variants_ragged(oxh, Q6K, rows, cols, n_vec)
+
+
+
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
 def test_small_batch_launch_on_128_row_tiles(oxh, qtype):
     """Five activations over 30000 rows: 469 tiles of 64 rows would be fewer than two per CU on a 256-CU

@@ -339,6 +339,27 @@ def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec):
         mv.gemv_segments(mv.Q2_K_WIDE, seg, cols, d_a.ptr, 1, rows)
 
 
+@pytest.mark.parametrize("rows,cols,n_vec", [(4099, 512, 130), (3600, 256, 333), (14300, 768, 40)])
+def test_q2k_wide_tiles_with_shared_operands(oxh, rows, cols, n_vec):
+    """The 64 x 128 tiles whose operands the workgroup builds once, on widened raw random blocks, against the
+    64 x 16 tiles (the test above holds those to the oracle) sixteen activations at a time: the same bits."""
+    rng = np.random.default_rng(rows)
+    w = rng.integers(0, 256, rows * (cols // 256) * 84, dtype=np.uint8).reshape(-1, 84)
+    w[:, 81] &= 0x3B
+    w[:, 83] &= 0x3B
+    d_w = mv.DeviceBuffer.from_host(w.reshape(-1))
+    d_wide = mv.DeviceBuffer(rows * (cols // 256) * 210)
+    mv.q2_k_widen(d_w.ptr, rows, cols, d_wide.ptr)
+    nact = mv.act_bytes(Q2K, cols)
+    d_x = mv.DeviceBuffer.from_host(synth.normal(n_vec * cols, seed=6, stream=n_vec))
+    d_a, d_o1, d_o2 = mv.DeviceBuffer(n_vec * nact), mv.DeviceBuffer(n_vec * rows * 4), mv.DeviceBuffer(n_vec * rows * 4)
+    mv.quantize(Q2K, d_x.ptr, cols, n_vec, cols, d_a.ptr)
+    mv.mmq(mv.Q2_K_WIDE, d_wide.ptr, rows, cols, d_a.ptr, n_vec, d_o1.ptr, rows)
+    for v in range(0, n_vec, 16):
+        mv.mmq(mv.Q2_K_WIDE, d_wide.ptr, rows, cols, d_a.ptr + v * nact, min(16, n_vec - v), d_o2.ptr + 4 * v * rows, rows)
+    assert np.array_equal(d_o1.download(np.uint32, n_vec * rows), d_o2.download(np.uint32, n_vec * rows))
+
+
 @pytest.mark.parametrize("qt,rows,cols,n_vec", [(Q3K, 300, 2048, 9), (Q3KS, 65, 256, 16), (Q3KL, 1, 512, 33),
                                                 (Q3K, 1000, 4096, 100), (Q3K, 4096, 4096, 512),
                                                 (Q2K, 300, 2048, 9), (Q2K, 65, 256, 16), (Q2K, 1, 512, 33),
