@@ -51,6 +51,13 @@ int oxh_internal_experts_long(uint32_t file_type, int tile_major, const void *co
 int oxh_internal_mmq6_init(void);
 int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
                              float *d_out, size_t out_stride, void *stream);
+/* K-quant matrices under at most 64 activations, a 16-row group to a workgroup (oxh_batch.hip); init and launch
+ * return a hipError_t, `takes` whether a launch of these sizes belongs there.  fmt: 0 Q4_K, 1 Q5_K, 2 Q6_K,
+ * 3 widened Q2_K.  Arguments checked by the caller. */
+int oxh_internal_batch_init(void);
+int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec);
+int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
+                           size_t out_stride, void *stream);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
 int oxh_internal_copy16(void *dst, const void *src, size_t bytes, void *stream);
 /* Wait for a stream by polling it `spins` times before blocking. */

@@ -938,6 +938,7 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<8, false, 3>)) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_experts_init()) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_mmq6_init()) != hipSuccess) return e;
+    if ((e = (hipError_t)oxh_internal_batch_init()) != hipSuccess) return e;
     return hipSuccess;
 }
 
@@ -2289,6 +2290,20 @@ extern "C" int oxh_mmq(uint32_t qtype, const void *d_w, size_t rows, size_t cols
     return mmq_run(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, false, stream);
 }
 
+/* OXH_MMQ_SHAPE: the tile every matrix-core launch of a K-quant runs on (mmq_tile_shape), 0 = by the rules */
+static int mmq_forced_shape(void)
+{
+    static int forced = -1;
+    if (forced < 0) forced = (int)env_u32("OXH_MMQ_SHAPE", 0, 0, 5);
+    return forced;
+}
+
+/* the small-batch kernel's name for a K-quant */
+static int mmq_batch_fmt(uint32_t qtype)
+{
+    return is_q4k(qtype) ? 0 : is_q5k(qtype) ? 1 : qtype == OXH_Q2_K_WIDE ? 3 : 2;
+}
+
 /* Few tiles and many super-blocks: a tile's columns go to several workgroups (k_mmq_*_split) */
 static bool mmq_split_plan(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride, size_t cus,
                            uint32_t *b_per_slice, uint32_t *slices, size_t *ws_bytes, uint32_t *tile_tokens = nullptr)
@@ -2350,6 +2365,9 @@ extern "C" int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_
     qtype = canon_qtype(qtype);
     const uint32_t B = (uint32_t)(cols / OXH_QK_K);
     if ((size_t)B * 292u * 256u > 0xFFFFFFFFull) return arg_fail("oxh_mmq_split: cols too large");
+    /* most of what used to be split runs on a workgroup per 16 rows now, which needs no workspace */
+    if (!mmq_forced_shape() && oxh_internal_mmq_batch_takes(mmq_batch_fmt(qtype), rows, B, n_vec))
+        return mmq_run(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, false, stream);
     const dim3 grid((uint32_t)((rows + 63) / 64), (uint32_t)((n_vec + tile_tok - 1) / tile_tok), slices), block(4 * 64);
     const size_t split_stride = n_vec * out_stride;
     hipStream_t st = pick_stream(stream);
@@ -2451,8 +2469,13 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
     /* the kernel addresses a workgroup's rows and tokens with 32-bit lane offsets */
     if (blocks * 292u * 256u > 0xFFFFFFFFull)
         return arg_fail("oxh_mmq: cols too large");
-    static int forced = -1;
-    if (forced < 0) forced = (int)env_u32("OXH_MMQ_SHAPE", 0, 0, 5);
+    const int forced = mmq_forced_shape();
+    const int batch_fmt = mmq_batch_fmt(qtype);
+    if (!forced && oxh_internal_mmq_batch_takes(batch_fmt, rows, blocks, n_vec)) {
+        const int e = oxh_internal_mmq_batch(batch_fmt, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, pick_stream(stream));
+        if (e) return hip_fail((hipError_t)e, "oxh_mmq");
+        return OXH_OK;
+    }
     const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
     int shape = forced ? forced : qtype == OXH_Q6_K || wide2 ? mmq6_tile_shape(rows, n_vec, cus, wide2)
                                                              : mmq_tile_shape(qtype, rows, n_vec, cus);

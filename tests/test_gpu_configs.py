@@ -188,6 +188,34 @@ def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
     assert np.array_equal(bits(got), bits(out[:, :rows]))
 
 
+@pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("rows,cols,n_vec", [(16, 256, 1), (17, 512, 16), (1100, 25600, 3), (4099, 4096, 15), (250, 2048, 64),
+                                             (700, 768, 33), (1500, 14336, 17)])
+def test_small_batches_on_a_workgroup_per_16_rows(oxh, qtype, rows, cols, n_vec):
+    """The kernel whose waves share the super-blocks of 16 rows and sum the terms from LDS: one super-block and
+    more waves than super-blocks, 100 of them (what LDS holds), uneven rounds, two workgroups to a CU, one and two
+    16-token chunks, two token tiles, ragged rows and tokens, a padded output.  Against the dot-instruction kernel on
+    the same device data, and three activations against the oracle."""
+    w = synth.weights(qtype, rows, cols, seed=7, stream=rows)
+    xs = synth.normal(n_vec * cols, seed=7, stream=n_vec).reshape(n_vec, cols)
+    d_w, d_x = mv.DeviceBuffer.from_host(w), mv.DeviceBuffer.from_host(xs)
+    nact, stride = mv.act_bytes(qtype, cols), rows + 5
+    d_a, d_o = mv.DeviceBuffer(n_vec * nact), mv.DeviceBuffer(n_vec * stride * 4)
+    d_o.upload(np.full(n_vec * stride, -7.25, np.float32))
+    mv.quantize(qtype, d_x.ptr, cols, n_vec, cols, d_a.ptr)
+    mv.mmq(qtype, d_w.ptr, rows, cols, d_a.ptr, n_vec, d_o.ptr, stride)
+    out = d_o.download(np.float32, n_vec * stride).reshape(n_vec, stride)
+    assert np.all(out[:, rows:] == -7.25)
+    d_o2 = mv.DeviceBuffer(2 * rows * 4)
+    for v in range(0, n_vec, 2):
+        m = min(2, n_vec - v)
+        mv.gemv_segments(qtype, mv.make_segments([(d_w.ptr, d_o2.ptr, rows, v)]), cols, d_a.ptr, m, rows)
+        assert np.array_equal(d_o2.download(np.uint32, m * rows).reshape(m, rows), bits(out[v:v + m, :rows])), v
+    for v in sorted({0, n_vec // 2, n_vec - 1}):
+        want, _ = oracle_matvec(qtype, w, rows, cols, np.ascontiguousarray(xs[v]))
+        assert np.array_equal(bits(out[v, :rows]), bits(want)), v
+
+
 @pytest.mark.parametrize("rows,cols,n_vec", [(4095, 512, 333), (4100, 768, 129), (14300, 256, 40), (14337, 512, 66),
                                              (7000, 256, 128), (2049, 1024, 400)])
 def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec):
