@@ -188,6 +188,27 @@ def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
     assert np.array_equal(bits(got), bits(out[:, :rows]))
 
 
+@pytest.mark.parametrize("rows,cols,n_vec,pad", [(1001, 4096, 1300, 0), (1001, 1024, 1300, 7), (263, 1024, 1024, 0),
+                                                 (14336, 512, 19, 3)])
+def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, pad):
+    """Inputs and outputs above 1 MiB travel in 1 MiB chunks through four slots: more chunks than slots, fewer, chunk
+    boundaries inside a vector, a last chunk that is no multiple of 16 bytes, an output just above 1 MiB, padded
+    strides whose padding stays as it was.  Against calls of eight vectors, which do not go through the ring."""
+    w = synth.weights(Q4K, rows, cols, seed=9, stream=rows)
+    rb = synth.row_bytes(Q4K, cols)
+    xs = np.full((n_vec, cols + pad), 3.5, np.float32)
+    xs[:, :cols] = synth.normal(n_vec * cols, seed=9, stream=n_vec).reshape(n_vec, cols)
+    temp, scratch = np.zeros(cols, np.float32), np.zeros(mv.batch_scratch_bytes(cols), np.uint8)
+    out = np.full((n_vec, rows + pad), -7.25, np.float32)
+    mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, xs, cols + pad, out, rows + pad, n_vec, temp, scratch)
+    assert np.all(out[:, rows:] == -7.25)
+    for v in list(range(0, n_vec, 8 * 9)) + [n_vec - 8]:
+        part, x8 = np.zeros((8, rows), np.float32), np.ascontiguousarray(xs[v:v + 8, :cols])
+        m = x8.shape[0]
+        mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, x8, cols, part, rows, m, temp, scratch)
+        assert np.array_equal(bits(part[:m]), bits(out[v:v + m, :rows])), v
+
+
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
 @pytest.mark.parametrize("rows,cols,n_vec", [(16, 256, 1), (17, 512, 16), (1100, 25600, 3), (4099, 4096, 15), (250, 2048, 64),
                                              (700, 768, 33), (1500, 14336, 17)])
