@@ -139,13 +139,13 @@ extern "C" int oxh_internal_experts_long(uint32_t file_type, int tile_major, con
     /* Which tile.  Up to 64 tokens per expert the 128 x 64 one, two to a CU, holds them all (Mixtral-shaped, Q4_K,
      * 50 tokens per expert: 303 us a layer against 335 on 128 x 144 tiles and 369 on 256 x 144); above, a tile
      * that holds 144 saves building an expert's operands again (8 x 128 tokens: 573 us against 655), of 256 rows
-     * (Q4_K; a little under two of the other kind) or of 128, whichever takes fewer rounds of the CUs, as long as
+     * (Q4_K; one takes as long as 1.75 of the other kind: the layer of 4 x 250 tokens 518 us against 547) or of 128, whichever takes fewer rounds of the CUs, as long as
      * there is one for nearly every CU. */
     const size_t avg = pairs / n_expert, tok_tiles = n_expert * ((avg + 143) / 144);
     const size_t mid = n_mat * ((rows + 127) / 128) * tok_tiles, large = n_mat * ((rows + 255) / 256) * tok_tiles;
     int shape = 3;
     if (avg > 64 && mid >= cus - cus / 8)
-        shape = fmt == EXP_Q4 && 1.85 * (double)((large + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 1 : 2;
+        shape = fmt == EXP_Q4 && 1.75 * (double)((large + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 1 : 2;
 #define OXH_LONG(FMT, TC, RC, GEOM)                                                                            \
     do {                                                                                                       \
         a.row_tiles = (uint32_t)((rows + GEOM::ROWS - 1) / GEOM::ROWS);                                        \

@@ -2892,7 +2892,7 @@ static int moe_ffn_run(const OxhMoe *m, const MoeLayout &l, const float *d_logit
     if ((rc = launch_experts(m->qtype_down, w_dn, o_dn, 1, m->n_expert, m->hidden, m->ffn, ws + l.act_h,
                              m->hidden, counts, offsets, pairs, n_tok, stream))) return rc;
     /* 6. combine in ascending expert order */
-    hipLaunchKernelGGL(k_moe_combine, dim3((uint32_t)((m->hidden + 255u) / 256u), (uint32_t)n_tok), dim3(256), 0,
+    hipLaunchKernelGGL(k_moe_combine, dim3((uint32_t)((m->hidden + 1023u) / 1024u), (uint32_t)n_tok), dim3(256), 0,
                        pick_stream(stream), (const float *)y, m->hidden, (const int32_t *)ids, (const float *)wts,
                        (const uint32_t *)slot_pos, (uint32_t)m->top_k, (uint32_t)m->hidden, d_out, out_stride);
     HIP_TRY(hipGetLastError());
