@@ -809,7 +809,8 @@ static int reserve(DevBuf *b, size_t bytes)
         b->bytes = 0;
         if (rc) return rc;
     }
-    size_t want = bytes < (1u << 20) ? (1u << 20) : bytes + bytes / 4;
+    /* whole 16-byte units: oxh_internal_copy16 moves align16(bytes) of what was reserved */
+    size_t want = align16(bytes < (1u << 20) ? (1u << 20) : bytes + bytes / 4);
     rc = oxh_malloc(&b->p, want);
     if (rc) return rc;
     b->bytes = want;
