@@ -941,9 +941,9 @@ def q80_batch_probe(mv, synth):
 
 
 def split_probe(mv, synth):
-    """For `rocprofv3 --kernel-trace --stats` runs on the small-batch launches whose tiles share their
-    columns between workgroups: a 4096 x 14336 Q6_K matrix under 16 activations, twelve launches of
-    oxh_mmq and twelve of oxh_mmq_split over six copies of the weights in turn.  Prints nothing."""
+    """For `rocprofv3 --kernel-trace --stats` runs on small-batch launches over few rows and many
+    columns: a 4096 x 14336 Q6_K matrix under 16 activations, twelve launches of oxh_mmq and twelve of
+    oxh_mmq_split over six copies of the weights in turn.  Prints nothing."""
     Q6K = 16
     rows, cols, n_vec = 4096, 14336, 16
     w = synth.weights(Q6K, rows, cols, seed=0, stream=12)

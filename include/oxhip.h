@@ -372,7 +372,8 @@ int oxh_mmq_ex(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
  * single workgroup adds them in, so the same bits.  oxh_mmq_split_workspace returns the bytes needed, or 0
  * for a launch that would not be split (types other than Q4_K, Q5_K, Q6_K and OXH_Q2_K_WIDE, more tiles,
  * fewer than eight super-blocks, more than 64 activations); oxh_mmq_split with a smaller workspace, or
- * none, is oxh_mmq.
+ * none, is oxh_mmq.  Most launches of these sizes run on a kernel that shares the columns between the waves of
+ * one workgroup instead, with or without a workspace; the split is what it leaves.
  * The reference has no counterpart (its batch kernel gives every worker whole rows, oxk.c:787-836). */
 size_t oxh_mmq_split_workspace(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride);
 int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
@@ -384,9 +385,10 @@ int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
  * Q5_K, Q6_K and widened Q2_K), 64 x 128 (Q6_K only), 128 x 64, 64 x 32, 64 x 16
  * that still gives nearly every compute unit a workgroup; 128 x 64 always for
  * the 32-value formats.  (Q6_K and widened Q2_K launches of more than 32
- * activations weigh the tiles' measured times on top of that and may run on
- * another of these tiles than the one reported; the results are the same bits.)  Pure host arithmetic (no device needed); OXH_DECLINED
- * for a type without a matrix-core kernel.
+ * activations weigh the tiles' measured times on top of that, and K-quant launches
+ * of up to 64 may go to a kernel with a workgroup per 16 rows: a launch may run on
+ * another tile than the one reported; the results are the same bits.)  Pure host
+ * arithmetic (no device needed); OXH_DECLINED for a type without a matrix-core kernel.
  * The reference has no counterpart: its batch kernel takes four activations
  * per weight row regardless of the shape (oxk.c:787-836). */
 int oxh_mmq_tile(uint32_t qtype, size_t rows, size_t n_vec, size_t n_cu, uint32_t *tile_rows,
