@@ -332,8 +332,8 @@ static uint32_t bat_need(int fmt, uint32_t ch, uint32_t B, uint32_t waves)
  *   16 activations, 4096 x 14336 18 / 26 (Q6_K), 13.6 / 20 (Q4_K); 14336 x 4096 14.6 / 16.7, 20.7 / 24.1; 8192 x 4096
  *   9.4 / 16.2, 12.6 / 22.9.  Not where few rows meet many columns (500 x 14336: 16.1 / 12.6, Q6_K): a workgroup
  *   per 16 rows then leaves most CUs without one (Q5_K, the most bytes, from half the CUs on: 1500 x 14336 14.4 /
- *   13.1).  Nor above some four workgroups to a CU, where the tiles have enough of them too and stage a
- *   token's values for four times the rows (28672 x 4096 23 / 20, 60000 x 4096 42 / 30).
+ *   13.1; Q6_K from 5/16 of them: 1131 x 14080 16.2 / 15.6).  Nor above some
+ *   four workgroups to a CU, where the tiles have enough of them too and stage a token's values for four times the rows (28672 x 4096 23 / 20, 60000 x 4096 42 / 30).
  *   17-32 activations cost a wave twice the LDS and time per weight, so the tiles, which read a row's weights for all
  *   of them once, win as soon as they fill the device: 4096 x 4096 10 / 16, 8192 x 4096 15.6 / 16.7 but 14336 x
  *   4096 28 / 20; the Q6_K tiles, slower at building operands, later (8192 x 4096 18.8 / 23.5, 8192 x 14336 59 / 66).
@@ -346,8 +346,9 @@ extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks,
     if (n_vec > 64 || blocks > 128) return 0;
     const uint32_t ch = n_vec <= 16 ? 1 : 2;
     if (bat_need(fmt, ch, (uint32_t)blocks, 4) > BAT_LDS) return 0;
-    if (n_vec <= 16) return groups <= 4 * cus && (blocks <= 16 || groups >= (fmt == BAT_Q5 ? cus / 2 : cus / 4));
     const bool two_planes = fmt == BAT_Q6;
+    if (n_vec <= 16)
+        return groups <= 4 * cus && (blocks <= 16 || groups >= (fmt == BAT_Q5 ? cus / 2 : two_planes ? 5 * cus / 16 : cus / 4));
     if (n_vec <= 32) return groups <= (two_planes ? 2 * cus : cus + cus / 4);
     if (blocks > 32) return 2 * groups <= (two_planes ? cus : cus / 2);
     return 2 * groups <= (two_planes ? 2 * cus : cus);
