@@ -2230,8 +2230,9 @@ static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
  * measured: 64 x 128 tiles whose operands the workgroup builds once, one to a CU, 0.375 + 0.078 a token chunk
  * for every round of tiles (75 us at 5 chunks, 91 at 7, 101 at 8); 128 x 128 tiles, one to a CU, 1.6 a round
  * (161 us); 64 x 32 tiles, three to a CU, 0.75 up to a tile per CU (76 us), 0.95 just above (95 at 448
- * tiles of 256 CUs), then by their number (122 at 704, 171 at 1024, 242 at 1536), and a sixth less for
- * widened Q2_K, whose operands take little building (77 at 448, 104 at 704).  (The 128 x 64 tile took 126 us
+ * tiles of 256 CUs), then by their number (122 at 704, 171 at 1024, 242 at 1536).  Widened Q2_K, whose
+ * operands take little building, saves 0.18 on the 64 x 32 tiles whatever their number (77 us at 448, 104 at 704; 2064
+ * tiles of 20 super-blocks 111) and takes 1.48 a round of 128 x 128 ones (106 us for two of 20).  (The 128 x 64 tile took 126 us
  * where the 64 x 128 one takes 91 and is gone.) */
 static int mmq6_tile_shape(size_t rows, size_t n_vec, size_t cus, bool widened_q2)
 {
@@ -2240,11 +2241,11 @@ static int mmq6_tile_shape(size_t rows, size_t n_vec, size_t cus, bool widened_q
     const size_t t5 = ((rows + 63) / 64) * tok_tiles, t1 = ((rows + 127) / 128) * tok_tiles;
     const double per_cu = (double)(((rows + 63) / 64) * ((n_vec + 31) / 32)) / (double)cus;
     const double c5 = (double)((t5 + cus - 1) / cus) * (0.375 + 0.078 * (double)chunks);
-    const double c1 = (double)((t1 + cus - 1) / cus) * 1.6;
+    const double c1 = (double)((t1 + cus - 1) / cus) * (widened_q2 ? 1.48 : 1.6);
     double c3 = 0.15 + 0.385 * per_cu;
     if (c3 < 0.75) c3 = 0.75;
     if (per_cu > 1.0 && c3 < 0.95) c3 = 0.95;
-    if (widened_q2) c3 *= 0.84;
+    if (widened_q2) c3 -= c3 < 0.95 ? 0.12 : 0.18;
     if (c1 < c5 && c1 < c3) return 1;
     return c5 < c3 ? 5 : 3;
 }
