@@ -269,7 +269,10 @@ k_mmq_q6_k_shared(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, cons
 {
     const uint32_t row0 = blockIdx.x * Q6sGeom::ROWS;
     const uint32_t chunks = (n_vec + 15u) >> 4;
-    const uint32_t c0 = blockIdx.y * chunks / gridDim.y, nc = (blockIdx.y + 1u) * chunks / gridDim.y - c0;
+    /* the first `over` tiles get a chunk more; no product here passes the number of chunks (y * chunks would
+     * leave 32 bits at three million activations) */
+    const uint32_t each = chunks / gridDim.y, over = chunks - each * gridDim.y;
+    const uint32_t c0 = blockIdx.y * each + min(blockIdx.y, over), nc = each + (blockIdx.y < over ? 1u : 0u);
     const uint32_t tok0 = 16u * c0, here = min(n_vec - tok0, 16u * nc);
     const uint8_t *wb = w + (size_t)row0 * B * 210u, *ab = acts + (size_t)tok0 * B * 292u;
     float *ob = out + (size_t)tok0 * out_stride + row0;

@@ -246,6 +246,29 @@ def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec):
 
 
 
+def test_q6_k_tiles_with_shared_operands_over_three_million_activations(oxh):
+    """The token tiles' share of the 16-token chunks in 32 bits: 23 438 tiles times 187 500 chunks is past 2^32.
+    A thousand activations, repeated: every repetition has the bits of the first, which the oracle holds."""
+    rows, cols, unit, reps = 16, 256, 1000, 3000
+    w = synth.weights(Q6K, rows, cols, seed=51, stream=1)
+    xs = synth.normal(unit * cols, seed=51, stream=2).reshape(unit, cols)
+    d_w, d_x = mv.DeviceBuffer.from_host(w), mv.DeviceBuffer.from_host(xs)
+    nact = mv.act_bytes(Q6K, cols)
+    d_a, d_o = mv.DeviceBuffer(unit * reps * nact), mv.DeviceBuffer(unit * reps * rows * 4)
+    mv.quantize(Q6K, d_x.ptr, cols, unit, cols, d_a.ptr)
+    have = unit * nact
+    while have < d_a.nbytes:
+        n = min(have, d_a.nbytes - have)
+        mv.copy_d2d(d_a.ptr + have, d_a.ptr, n)
+        have += n
+    mv.mmq(Q6K, d_w.ptr, rows, cols, d_a.ptr, unit * reps, d_o.ptr, rows)
+    out = d_o.download(np.uint32, unit * reps * rows).reshape(reps, unit * rows)
+    assert (out == out[0]).all()
+    for v in (0, unit // 2, unit - 1):
+        want, _ = oracle_matvec(Q6K, w, rows, cols, np.ascontiguousarray(xs[v]))
+        assert np.array_equal(out[0].reshape(unit, rows)[v], bits(want)), v
+
+
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
 def test_small_batch_launch_on_128_row_tiles(oxh, qtype):
     """Five activations over 30000 rows: 469 tiles of 64 rows would be fewer than two per CU on a 256-CU
