@@ -66,8 +66,20 @@ __device__ __forceinline__ void q6s_dword(uint32_t ql, uint32_t qh, uint32_t sc,
     hi = __builtin_amdgcn_perm(uo, ue, 0x07030501u);
 }
 
+/* The workgroup's barrier where its waves stand in different instantiations of q6s_walk().  __syncthreads() asks
+ * every thread to reach the same call; s_barrier, which it becomes, is defined per wave: a wave waits until every
+ * wave of its workgroup has executed one, wherever it stands in the program.  So the instruction itself, between
+ * the fences __syncthreads() puts around it: LDS written before is seen after. */
+__device__ __forceinline__ void q6s_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 /* A wave's N chunks of 16 tokens, the first of them chunk c_first of the tile, over all super-blocks; results
- * of tokens below toks_end are its to store.  The waves of a workgroup may run it for different N: each passes the same number of barriers. */
+ * of tokens below toks_end are its to store.  The waves of a workgroup may run it for different N: each executes
+ * 1 + B barriers, whatever N is. */
 template <int N, bool Q2>
 __device__ __forceinline__ void
 q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, const uint8_t *__restrict__ a_base,
@@ -166,7 +178,7 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
     }
     Q6sRaw next = load_raw(min(1u, B - 1u));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        /* the LDS-bound loads, which the compiler does not count */
-    __syncthreads();
+    q6s_barrier();
 
     for (uint32_t b = 0; b < B; b++) {
         const uint32_t buf = b & 1u;
@@ -245,7 +257,7 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
         store_planes(next, dq_next, buf ^ 1u);
         next = after;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        q6s_barrier();
     }
 
     const uint32_t row = (wave & 3u) * 16u + r16;
