@@ -380,14 +380,15 @@ int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
                   const void *d_acts, size_t n_vec, float *d_out, size_t out_stride,
                   void *d_workspace, size_t workspace_bytes, void *stream);
 
-/* The tile (weight rows x activations per workgroup) oxh_mmq picks for a launch
- * on a device of n_cu compute units: the largest of 256 x 128 (128 x 128 for
+/* The tile (weight rows x activations per workgroup) that the rule on sizes names for
+ * a launch on a device of n_cu compute units: the largest of 256 x 128 (128 x 128 for
  * Q5_K, Q6_K and widened Q2_K), 64 x 128 (Q6_K only), 128 x 64, 64 x 32, 64 x 16
  * that still gives nearly every compute unit a workgroup; 128 x 64 always for
- * the 32-value formats.  (Q6_K and widened Q2_K launches of more than 32
- * activations weigh the tiles' measured times on top of that, and K-quant launches
- * of up to 64 may go to a kernel with a workgroup per 16 rows: a launch may run on
- * another tile than the one reported; the results are the same bits.)  Pure host
+ * the 32-value formats.  Q4_K and Q5_K launches of more than 64 activations and the
+ * 32-value formats run on that tile.  Others may run on another one, with the same
+ * bits: Q6_K and widened Q2_K weigh the tiles' measured times on top, and K-quant
+ * launches of up to 64 activations may go to a kernel with a workgroup per 16 rows
+ * (oxh_lab()->mmq_kernel says what a launch runs on).  Pure host
  * arithmetic (no device needed); OXH_DECLINED for a type without a matrix-core kernel.
  * The reference has no counterpart: its batch kernel takes four activations
  * per weight row regardless of the shape (oxk.c:787-836). */

@@ -50,6 +50,20 @@ typedef struct OxhLab {
      * :932-954, :234-237, which the reference's API does not expose. */
     int (*subblock_sums)(uint32_t qtype, const void *d_w, size_t rows, size_t cols, const void *d_act,
                          int32_t *d_sums, void *stream);
+    /* Which kernel a matrix-core launch of these sizes runs on, on a device of
+     * n_cu compute units and with ws_bytes of workspace (oxh_mmq_split; 0 is
+     * oxh_mmq): what the launch itself asks, as host arithmetic.  out: the
+     * kernel (0 tiles, 1 Q6_K tiles whose operands a workgroup builds once,
+     * 2 a workgroup per 16 rows whose waves share the columns, 3 tiles whose
+     * columns several workgroups share), rows and tokens of a workgroup, and
+     * for kernel 2 its waves.  OXH_DECLINED for a type without such a kernel. */
+    int (*mmq_kernel)(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t n_cu, size_t ws_bytes,
+                      uint32_t out[4]);
+    /* The same for one expert launch of oxh_moe_ffn: n_mat matrices of `rows`
+     * rows per expert (gate and up 2, down 1) under `pairs` (token, expert)
+     * pairs in all; tile: rows and tokens of a workgroup. */
+    int (*experts_tile)(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu,
+                        uint32_t tile[2]);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

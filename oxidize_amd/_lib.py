@@ -56,7 +56,9 @@ class OxhLab(ctypes.Structure):
                 ("moe_workspace_parts", ctypes.CFUNCTYPE(I, ctypes.POINTER(OxhMoe), Z, ctypes.POINTER(Z * 12))),
                 ("read_probe", ctypes.CFUNCTYPE(I, V, Z, V, V)),
                 ("mfma_probe", ctypes.CFUNCTYPE(I, I, I, ctypes.POINTER(ctypes.c_double))),
-                ("subblock_sums", ctypes.CFUNCTYPE(I, U32, V, Z, Z, V, V, V))]
+                ("subblock_sums", ctypes.CFUNCTYPE(I, U32, V, Z, Z, V, V, V)),
+                ("mmq_kernel", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 4))),
+                ("experts_tile", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 2)))]
 
 
 # name -> (restype, argtypes); every symbol include/oxhip.h and include/oxhip_lab.h declare

@@ -339,9 +339,8 @@ static uint32_t bat_need(int fmt, uint32_t ch, uint32_t B, uint32_t waves)
  *   4096 28 / 20; the Q6_K tiles, slower at building operands, later (8192 x 4096 18.8 / 23.5, 8192 x 14336 59 / 66).
  *   33-64 are two such halves: 1500 x 4096 9.9 / 13.9, 1500 x 14336 23.6 / 21.9, 4096 x 4096 16.2 / 16.8, 8192 x 4096
  *   28.8 / 19.3; Q6_K 1500 x 14336 30 / 30, 4096 x 4096 18 / 23, 8192 x 4096 35 / 27. */
-extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec)
+extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus)
 {
-    const size_t cus = (size_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
     const size_t groups = (rows + 15) / 16;
     if (n_vec > 64 || blocks > 128) return 0;
     const uint32_t ch = n_vec <= 16 ? 1 : 2;
@@ -354,6 +353,20 @@ extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks,
     return 2 * groups <= (two_planes ? 2 * cus : cus);
 }
 
+/* Two workgroups of four waves to a CU where there are that many and LDS holds them: while one sums, the other
+ * streams (8192 x 4096, 16 activations: 9.4 us against 11.0 with one of eight).  Otherwise as many waves as LDS
+ * holds, as evenly used as the super-blocks allow. */
+extern "C" uint32_t oxh_internal_mmq_batch_waves(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus)
+{
+    const uint32_t B = (uint32_t)blocks, ch = n_vec <= 16 ? 1 : 2;
+    const size_t groups = (rows + 15) / 16 * ((n_vec + 16 * ch - 1) / (16 * ch));
+    uint32_t waves = 4;
+    if (groups <= cus || 2u * bat_need(fmt, ch, B, 4) > BAT_LDS)
+        while (waves < 16u && bat_need(fmt, ch, B, waves + 1u) <= BAT_LDS) waves++;
+    const uint32_t rounds = (B + waves - 1u) / waves;
+    return (B + rounds - 1u) / rounds;
+}
+
 /* see oxh_internal.h */
 extern "C" int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
                                       float *d_out, size_t out_stride, void *stream)
@@ -361,14 +374,7 @@ extern "C" int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, siz
     const uint32_t B = (uint32_t)blocks, ch = n_vec <= 16 ? 1 : 2;
     const size_t cus = (size_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
     const dim3 grid((uint32_t)((rows + 15) / 16), (uint32_t)((n_vec + 16 * ch - 1) / (16 * ch)));
-    /* Two workgroups of four waves to a CU where there are that many and LDS holds them: while one sums, the other
-     * streams (8192 x 4096, 16 activations: 9.4 us against 11.0 with one of eight).  Otherwise as many waves as LDS
-     * holds, as evenly used as the super-blocks allow. */
-    uint32_t waves = 4;
-    if ((size_t)grid.x * grid.y <= cus || 2u * bat_need(fmt, ch, B, 4) > BAT_LDS)
-        while (waves < 16u && bat_need(fmt, ch, B, waves + 1u) <= BAT_LDS) waves++;
-    const uint32_t rounds = (B + waves - 1u) / waves;
-    waves = (B + rounds - 1u) / rounds;
+    const uint32_t waves = oxh_internal_mmq_batch_waves(fmt, rows, blocks, n_vec, cus);
     const uint32_t lds = bat_need(fmt, ch, B, waves);
 #define OXH_BATCH(FMT, CH)                                                                                           \
     hipLaunchKernelGGL((k_mmq_batch<FMT, CH>), grid, dim3(64u * waves), lds, (hipStream_t)stream, (const uint8_t *)d_w, \

@@ -110,13 +110,40 @@ extern "C" int oxh_internal_experts_init(void)
     return 0;
 }
 
+/* Which tile.  Up to 64 tokens per expert the 128 x 64 one, two to a CU, holds them all (Mixtral-shaped, Q4_K,
+ * 50 tokens per expert: 303 us a layer against 335 on 128 x 144 tiles and 369 on 256 x 144); above, a tile
+ * that holds 144 saves building an expert's operands again (8 x 128 tokens: 573 us against 655), of 256 rows
+ * (Q4_K; one takes as long as 1.75 of the other kind: the layer of 4 x 250 tokens 518 us against 547) or of 128,
+ * whichever takes fewer rounds of the CUs, as long as there is one for nearly every CU. */
+static int long_shape(int fmt, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
+{
+    const size_t avg = pairs / n_expert, tok_tiles = n_expert * ((avg + 143) / 144);
+    const size_t mid = n_mat * ((rows + 127) / 128) * tok_tiles, large = n_mat * ((rows + 255) / 256) * tok_tiles;
+    if (avg <= 64 || mid < cus - cus / 8) return 3;
+    return fmt == EXP_Q4 && 1.75 * (double)((large + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 1 : 2;
+}
+
+static int long_fmt(uint32_t file_type)
+{
+    return file_type == OXH_Q6_K ? EXP_Q6 : file_type == OXH_Q5_K_M || file_type == OXH_Q5_K_S ? EXP_Q5 : EXP_Q4;
+}
+
+/* see oxh_internal.h */
+extern "C" void oxh_internal_experts_long_tile(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs,
+                                               size_t cus, uint32_t tile[2])
+{
+    const int shape = long_shape(long_fmt(file_type), n_mat, n_expert, rows, pairs, cus);
+    tile[0] = shape == 1 ? 256u : 128u;
+    tile[1] = shape == 3 ? 64u : 144u;
+}
+
 /* see oxh_internal.h */
 extern "C" int oxh_internal_experts_long(uint32_t file_type, int tile_major, const void *const *d_w, float *const *d_out,
                                          size_t n_mat, size_t n_expert, size_t rows, size_t cols, const void *d_acts,
                                          size_t out_stride, const uint32_t *d_counts, const uint32_t *d_offsets,
                                          size_t pairs, size_t max_tokens, void *stream)
 {
-    const int fmt = file_type == OXH_Q6_K ? EXP_Q6 : file_type == OXH_Q5_K_M || file_type == OXH_Q5_K_S ? EXP_Q5 : EXP_Q4;
+    const int fmt = long_fmt(file_type);
     const size_t cus = (size_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
     ExpertArgs a;
     for (int i = 0; i < 2; i++) {
@@ -136,16 +163,7 @@ extern "C" int oxh_internal_experts_long(uint32_t file_type, int tile_major, con
         const size_t by_pairs = (pairs + n_expert * (tok - 1)) / tok, by_tokens = n_expert * ((max_tokens + tok - 1) / tok);
         return by_pairs < by_tokens ? by_pairs : by_tokens;
     };
-    /* Which tile.  Up to 64 tokens per expert the 128 x 64 one, two to a CU, holds them all (Mixtral-shaped, Q4_K,
-     * 50 tokens per expert: 303 us a layer against 335 on 128 x 144 tiles and 369 on 256 x 144); above, a tile
-     * that holds 144 saves building an expert's operands again (8 x 128 tokens: 573 us against 655), of 256 rows
-     * (Q4_K; one takes as long as 1.75 of the other kind: the layer of 4 x 250 tokens 518 us against 547) or of 128, whichever takes fewer rounds of the CUs, as long as
-     * there is one for nearly every CU. */
-    const size_t avg = pairs / n_expert, tok_tiles = n_expert * ((avg + 143) / 144);
-    const size_t mid = n_mat * ((rows + 127) / 128) * tok_tiles, large = n_mat * ((rows + 255) / 256) * tok_tiles;
-    int shape = 3;
-    if (avg > 64 && mid >= cus - cus / 8)
-        shape = fmt == EXP_Q4 && 1.75 * (double)((large + cus - 1) / cus) <= (double)((mid + cus - 1) / cus) ? 1 : 2;
+    const int shape = long_shape(fmt, n_mat, n_expert, rows, pairs, cus);
 #define OXH_LONG(FMT, TC, RC, GEOM)                                                                            \
     do {                                                                                                       \
         a.row_tiles = (uint32_t)((rows + GEOM::ROWS - 1) / GEOM::ROWS);                                        \

@@ -46,16 +46,20 @@ int oxh_internal_experts_long(uint32_t file_type, int tile_major, const void *co
                               size_t n_mat, size_t n_expert, size_t rows, size_t cols, const void *d_acts,
                               size_t out_stride, const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs,
                               size_t max_tokens, void *stream);
+/* the tile (rows, tokens) such a launch runs on; host arithmetic */
+void oxh_internal_experts_long_tile(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus,
+                                    uint32_t tile[2]);
 /* Q6_K (or widened Q2_K) prefill in 64 x 128 tiles whose weight operands the workgroup builds once
  * (oxh_mmq6.hip); both return a hipError_t.  Arguments checked by the caller. */
 int oxh_internal_mmq6_init(void);
 int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
                              float *d_out, size_t out_stride, void *stream);
 /* K-quant matrices under at most 64 activations, a 16-row group to a workgroup (oxh_batch.hip); init and launch
- * return a hipError_t, `takes` whether a launch of these sizes belongs there.  fmt: 0 Q4_K, 1 Q5_K, 2 Q6_K,
- * 3 widened Q2_K.  Arguments checked by the caller. */
+ * return a hipError_t, `takes` whether a launch of these sizes belongs there, `waves` the waves of its workgroups.
+ * fmt: 0 Q4_K, 1 Q5_K, 2 Q6_K, 3 widened Q2_K.  Arguments checked by the caller. */
 int oxh_internal_batch_init(void);
-int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec);
+int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
+uint32_t oxh_internal_mmq_batch_waves(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
 int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
                            size_t out_stride, void *stream);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
@@ -72,6 +76,8 @@ int oxh_debug_plan_phantom(struct OxhPlan *plan, int on);
 int oxh_debug_moe_workspace_parts(const struct OxhMoe *m, size_t n_tok, size_t parts[12]);
 int oxh_debug_read_probe(const void *d_buf, size_t bytes, uint32_t *d_sink, void *stream);
 int oxh_debug_mfma_probe(int valu_per_mfma, int waves_per_simd, double *pops);
+int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t n_cu, size_t ws_bytes, uint32_t out[4]);
+int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu, uint32_t tile[2]);
 int oxh_debug_subblock_sums(uint32_t qtype, const void *d_w, size_t rows, size_t cols, const void *d_act,
                             int32_t *d_sums, void *stream);
 

@@ -2342,6 +2342,70 @@ static bool mmq_split_plan(uint32_t qtype, size_t rows, size_t cols, size_t n_ve
     return true;
 }
 
+/* The kernel a K-quant launch of these sizes runs on, with `ws_bytes` of workspace (0: oxh_mmq). */
+enum { MMQ_TILES = 0, MMQ_SHARED = 1, MMQ_BATCH = 2, MMQ_SPLIT = 3 };
+struct MmqRoute {
+    int kernel, shape;                          /* shape: of MMQ_TILES, as mmq_tile_shape() numbers them */
+    uint32_t tile_rows, tile_tokens;
+    uint32_t per, slices;                       /* MMQ_SPLIT: super-blocks per slice, slices */
+};
+
+static MmqRoute mmq_route(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride, size_t ws_bytes,
+                          size_t cus)
+{
+    MmqRoute r = { MMQ_TILES, 0, 64u, 16u, 0u, 0u };
+    const bool q6 = qtype == OXH_Q6_K || qtype == OXH_Q2_K_WIDE, q5 = is_q5k(qtype);
+    const int forced = mmq_forced_shape();
+    uint32_t tile_tok = 16;
+    size_t need = 0;
+    const bool planned = ws_bytes && mmq_split_plan(qtype, rows, cols, n_vec, out_stride, cus, &r.per, &r.slices, &need,
+                                                    &tile_tok) && ws_bytes >= need;
+    if (!forced && oxh_internal_mmq_batch_takes(mmq_batch_fmt(qtype), rows, cols / OXH_QK_K, n_vec, cus)) {
+        r.kernel = MMQ_BATCH;
+        r.tile_rows = 16u;
+        r.tile_tokens = n_vec <= 16 ? 16u : 32u;
+        return r;
+    }
+    if (planned) {
+        r.kernel = MMQ_SPLIT;
+        r.tile_tokens = tile_tok;
+        return r;
+    }
+    r.shape = forced ? forced : q6 ? mmq6_tile_shape(rows, n_vec, cus, qtype == OXH_Q2_K_WIDE)
+                                   : mmq_tile_shape(qtype, rows, n_vec, cus);
+    if (!q6 && r.shape == 5) r.shape = 2;       /* the tile only Q6_K and widened Q2_K have ... */
+    if (q6 && r.shape == 2) r.shape = 5;        /* ... in place of this one */
+    if (r.shape == 5) r.kernel = MMQ_SHARED;
+    static const uint32_t tr[6] = { 0, 256, 128, 64, 64, 64 }, tt[6] = { 0, 128, 64, 32, 16, 128 };
+    r.tile_rows = r.shape == 1 && (q6 || q5) ? 128u : tr[r.shape];
+    r.tile_tokens = tt[r.shape];
+    return r;
+}
+
+extern "C" int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t n_cu, size_t ws_bytes,
+                                    uint32_t out[4])
+{
+    if (!out || !rows || !n_vec || !n_cu) return arg_fail("oxh_debug_mmq_kernel: NULL or empty");
+    out[3] = 0;
+    if (mmq80_leg(canon_qtype(qtype)) >= 0 && oxh_act_kind(qtype, cols) == 1) {
+        out[0] = MMQ_TILES;
+        out[1] = MQT_WAVES * 16u;
+        out[2] = MQT_TOK;
+        return OXH_OK;
+    }
+    const bool wide2 = qtype == OXH_Q2_K_WIDE;
+    if ((!is_q4k(qtype) && !is_q5k(qtype) && qtype != OXH_Q6_K && !wide2) ||
+        oxh_act_kind(wide2 ? OXH_Q2_K : qtype, cols) != 2)
+        return OXH_DECLINED;
+    const MmqRoute r = mmq_route(qtype, rows, cols, n_vec, rows, ws_bytes, n_cu);
+    out[0] = (uint32_t)r.kernel;
+    out[1] = r.tile_rows;
+    out[2] = r.tile_tokens;
+    if (r.kernel == MMQ_BATCH)
+        out[3] = oxh_internal_mmq_batch_waves(mmq_batch_fmt(qtype), rows, cols / OXH_QK_K, n_vec, n_cu);
+    return OXH_OK;
+}
+
 extern "C" size_t oxh_mmq_split_workspace(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride)
 {
     size_t bytes = 0;
@@ -2355,10 +2419,9 @@ extern "C" int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_
 {
     int rc = ensure_init();
     if (rc) return rc;
-    uint32_t per = 0, slices = 0, tile_tok = 16;
     size_t need = 0;
     const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
-    if (!mmq_split_plan(qtype, rows, cols, n_vec, out_stride, cus, &per, &slices, &need, &tile_tok) || !d_workspace ||
+    if (!mmq_split_plan(qtype, rows, cols, n_vec, out_stride, cus, nullptr, nullptr, &need) || !d_workspace ||
         workspace_bytes < need)
         return mmq_run(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, false, stream);
     if (!d_w || !d_acts || !d_out) return arg_fail("oxh_mmq_split: NULL pointer");
@@ -2366,9 +2429,9 @@ extern "C" int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_
     qtype = canon_qtype(qtype);
     const uint32_t B = (uint32_t)(cols / OXH_QK_K);
     if ((size_t)B * 292u * 256u > 0xFFFFFFFFull) return arg_fail("oxh_mmq_split: cols too large");
-    /* most of what used to be split runs on a workgroup per 16 rows now, which needs no workspace */
-    if (!mmq_forced_shape() && oxh_internal_mmq_batch_takes(mmq_batch_fmt(qtype), rows, B, n_vec))
-        return mmq_run(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, false, stream);
+    const MmqRoute route = mmq_route(qtype, rows, cols, n_vec, out_stride, workspace_bytes, cus);
+    if (route.kernel != MMQ_SPLIT) return mmq_run(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, false, stream);
+    const uint32_t per = route.per, slices = route.slices, tile_tok = route.tile_tokens;
     const dim3 grid((uint32_t)((rows + 63) / 64), (uint32_t)((n_vec + tile_tok - 1) / tile_tok), slices), block(4 * 64);
     const size_t split_stride = n_vec * out_stride;
     hipStream_t st = pick_stream(stream);
@@ -2470,19 +2533,21 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
     /* the kernel addresses a workgroup's rows and tokens with 32-bit lane offsets */
     if (blocks * 292u * 256u > 0xFFFFFFFFull)
         return arg_fail("oxh_mmq: cols too large");
-    const int forced = mmq_forced_shape();
-    const int batch_fmt = mmq_batch_fmt(qtype);
-    if (!forced && oxh_internal_mmq_batch_takes(batch_fmt, rows, blocks, n_vec)) {
-        const int e = oxh_internal_mmq_batch(batch_fmt, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, pick_stream(stream));
+    const MmqRoute route = mmq_route(qtype, rows, cols, n_vec, out_stride, 0, (size_t)(g_n_cu > 0 ? g_n_cu : 256));
+    const int shape = route.shape;
+    if (route.kernel == MMQ_BATCH) {
+        const int e = oxh_internal_mmq_batch(mmq_batch_fmt(qtype), d_w, rows, blocks, d_acts, n_vec, d_out, out_stride,
+                                             pick_stream(stream));
         if (e) return hip_fail((hipError_t)e, "oxh_mmq");
         return OXH_OK;
     }
-    const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
-    int shape = forced ? forced : qtype == OXH_Q6_K || wide2 ? mmq6_tile_shape(rows, n_vec, cus, wide2)
-                                                             : mmq_tile_shape(qtype, rows, n_vec, cus);
+    if (route.kernel == MMQ_SHARED) {
+        const int e = oxh_internal_mmq6_shared(wide2, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, pick_stream(stream));
+        if (e) return hip_fail((hipError_t)e, "oxh_mmq");
+        return OXH_OK;
+    }
     if (qtype == OXH_Q6_K || is_q5k(qtype) || wide2) {
         if (is_q5k(qtype)) {
-            if (shape == 5) shape = 2;
             if (shape == 1 && relaxed)      mmq5_launch<8, 1, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             else if (shape == 2 && relaxed) mmq5_launch<4, 1, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             else if (shape == 1) mmq5_launch<8, 1, 8>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
@@ -2490,12 +2555,6 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
             else if (shape == 3) mmq5_launch<2, 1, 4>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             else                 mmq5_launch<1, 1, 4>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
             HIP_TRY(hipGetLastError());
-            return OXH_OK;
-        }
-        if (shape == 5 || shape == 2) {
-            const int e = oxh_internal_mmq6_shared(wide2, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride,
-                                                   pick_stream(stream));
-            if (e) return hip_fail((hipError_t)e, "oxh_mmq");
             return OXH_OK;
         }
         if (wide2) {
@@ -2511,7 +2570,6 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
         HIP_TRY(hipGetLastError());
         return OXH_OK;
     }
-    if (shape == 5) shape = 2;
     /* the relaxed f32 step exists for the two prefill tiles; smaller launches are bound by the weight
      * stream and keep the exact one */
     if (shape == 1 && relaxed)      mmq_launch<8, 2, 8, true>(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, stream);
@@ -2823,46 +2881,72 @@ static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *c
     return OXH_OK;
 }
 
+/* Many tokens per expert (two dozen on average): tiles that read an expert's weights once for 64 or 144 of its
+ * tokens (oxh_experts.hip), unless there are too few of them and of tokens: under 64 tokens per expert a launch
+ * that does not give nearly every CU a 128 x 64 tile runs faster on many 64 x 16 ones (4 experts, top 1, 1024 x
+ * 2048, 200 tokens: 37 against 40 us a layer; 8 experts, top 2, 100 tokens: 45 against 40).  From ten tokens
+ * per expert on when the 64 x 16 tiles are eight to a CU and more, whose second pass over the weights then
+ * costs more than it hides (Mixtral-shaped, 64 tokens: 278 against 232 us).  OXH_MOE_BIG_TILE_FROM overrides
+ * the average to start from, 0 = never. */
+static bool experts_long(size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
+{
+    const size_t avg_tokens = pairs / n_expert;
+    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);
+    const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
+    const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
+    return big_from && ((avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) ||
+                        (avg_tokens >= 10 && big_from <= 24 && small_tiles >= 8 * cus));
+}
+
+/* few rows per expert (a down projection): the 64-row tile gives at most two workgroups per CU; Q4_K
+ * can take 128 rows on eight waves with three super-blocks per stage instead, half as much again in
+ * flight (OXH_MOE_WIDE_SMALL=1).  Off by default: launched continuously, Mixtral's down projections at
+ * 16 tokens run faster on the 64-row tiles with two super-blocks per stage (the layer 163 against 169 us;
+ * the wider tile only won when the launches were timed right after an idle period).  Workgroups of
+ * experts without a token leave at once, so what counts is the experts that can have one. */
+static bool experts_wide_small(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
+{
+    static const uint32_t wide = env_u32("OXH_MOE_WIDE_SMALL", 0, 0, 1);
+    const size_t live = pairs < n_expert ? (pairs ? pairs : 1) : n_expert;
+    return wide && is_q4k(file_type) && n_mat * n_expert * ((rows + 63) / 64) <= 2u * cus &&
+           n_mat * live * ((rows + 127) / 128) >= cus - cus / 8;
+}
+
+/* the tile (rows, tokens) of one expert launch of oxh_moe_ffn: 64 x 16 or 128 x 16, or one of oxh_experts.hip */
+extern "C" int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu,
+                                      uint32_t tile[2])
+{
+    if (!tile || !n_mat || !n_expert || !rows || !n_cu) return arg_fail("oxh_debug_experts_tile: NULL or empty");
+    const uint32_t file_type = t16_base(qtype);
+    if (!is_q4k(file_type) && !is_q5k(file_type) && file_type != OXH_Q6_K) return OXH_DECLINED;
+    if (experts_long(n_mat, n_expert, rows, pairs, n_cu)) {
+        oxh_internal_experts_long_tile(file_type, n_mat, n_expert, rows, pairs, n_cu, tile);
+        return OXH_OK;
+    }
+    tile[0] = experts_wide_small(file_type, n_mat, n_expert, rows, pairs, n_cu) ? 128u : 64u;
+    tile[1] = 16u;
+    return OXH_OK;
+}
+
 static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *d_out, size_t n_mat,
                           size_t n_expert, size_t rows, size_t cols, const void *d_acts, size_t out_stride,
                           const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs, size_t max_tokens,
                           void *stream)
 {
-    const size_t avg_tokens = pairs / n_expert;
     const uint32_t file_type = t16_base(qtype);
     const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
-    /* Many tokens per expert (two dozen on average): tiles that read an expert's weights once for 64 or 144 of its
-     * tokens (oxh_experts.hip), unless there are too few of them and of tokens: under 64 tokens per expert a launch
-     * that does not give nearly every CU a 128 x 64 tile runs faster on many 64 x 16 ones (4 experts, top 1, 1024 x
-     * 2048, 200 tokens: 37 against 40 us a layer; 8 experts, top 2, 100 tokens: 45 against 40).  From ten tokens
-     * per expert on when the 64 x 16 tiles are eight to a CU and more, whose second pass over the weights then
-     * costs more than it hides (Mixtral-shaped, 64 tokens: 278 against 232 us).  OXH_MOE_BIG_TILE_FROM overrides
-     * the average to start from, 0 = never. */
-    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);
-    const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
-    const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
-    if (big_from && ((avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) ||
-                     (avg_tokens >= 10 && big_from <= 24 && small_tiles >= 8 * cus))) {
+    if (experts_long(n_mat, n_expert, rows, pairs, cus)) {
         if (cols / OXH_QK_K * 292u * 256u > 0xFFFFFFFFull) return arg_fail("moe: cols too large");
         const int e = oxh_internal_experts_long(file_type, is_t16(qtype), d_w, d_out, n_mat, n_expert, rows, cols, d_acts,
                                                 out_stride, d_counts, d_offsets, pairs, max_tokens, pick_stream(stream));
         if (e) return hip_fail((hipError_t)e, "expert launch");
         return OXH_OK;
     }
-    /* few rows per expert (a down projection): the 64-row tile gives at most two workgroups per CU; Q4_K
-     * can take 128 rows on eight waves with three super-blocks per stage instead, half as much again in
-     * flight (OXH_MOE_WIDE_SMALL=1).  Off by default: launched continuously, Mixtral's down projections at
-     * 16 tokens run faster on the 64-row tiles with two super-blocks per stage (the layer 163 against 169 us;
-     * the wider tile only won when the launches were timed right after an idle period).  Workgroups of
-     * experts without a token leave at once, so what counts is the experts that can have one. */
-    static const uint32_t wide = env_u32("OXH_MOE_WIDE_SMALL", 0, 0, 1);
-    const size_t live = pairs < n_expert ? (pairs ? pairs : 1) : n_expert;
-    if (wide && is_q4k(file_type) && n_mat * n_expert * ((rows + 63) / 64) <= 2u * cus &&
-        n_mat * live * ((rows + 127) / 128) >= cus - cus / 8)
+    if (experts_wide_small(file_type, n_mat, n_expert, rows, pairs, cus))
         return launch_experts_tiled<8>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
-                                          d_counts, d_offsets, max_tokens, stream);
+                                       d_counts, d_offsets, max_tokens, stream);
     return launch_experts_tiled<4>(qtype, d_w, d_out, n_mat, n_expert, rows, cols, d_acts, out_stride,
-                                      d_counts, d_offsets, max_tokens, stream);
+                                   d_counts, d_offsets, max_tokens, stream);
 }
 
 /* the six launches of a layer over a workspace laid out by moe_layout(); arguments already checked */
@@ -3239,7 +3323,8 @@ extern "C" int oxh_mem_info(size_t *free_bytes, size_t *total_bytes)
 extern "C" const OxhLab *oxh_lab(void)
 {
     static const OxhLab lab = { oxh_debug_plan_stamps, oxh_debug_plan_phantom, oxh_debug_moe_workspace_parts,
-                                oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums };
+                                oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums,
+                                oxh_debug_mmq_kernel, oxh_debug_experts_tile };
     return &lab;
 }
 

@@ -198,10 +198,27 @@ def mmq_split(qtype, d_w, rows, cols, d_acts, n_vec, d_out, out_stride, d_ws, ws
 
 
 def mmq_tile(qtype, rows, n_vec, n_cu):
-    """(rows, tokens) of the workgroup tile oxh_mmq would take; host arithmetic only."""
+    """(rows, tokens) of the tile the rule on sizes names (mmq_kernel tells what a launch runs on); host arithmetic."""
     r, t = ctypes.c_uint32(0), ctypes.c_uint32(0)
     check(lib().oxh_mmq_tile(qtype, rows, n_vec, n_cu, ctypes.byref(r), ctypes.byref(t)))
     return r.value, t.value
+
+
+def mmq_kernel(qtype, rows, cols, n_vec, n_cu=256, ws_bytes=0):
+    """(kernel, tile rows, tile tokens, waves) a matrix-core launch runs on (include/oxhip_lab.h); host arithmetic."""
+    out = (ctypes.c_uint32 * 4)()
+    check(_lib.lab().mmq_kernel(qtype, rows, cols, n_vec, n_cu, ws_bytes, ctypes.byref(out)))
+    return tuple(out)
+
+
+MMQ_TILES, MMQ_SHARED, MMQ_BATCH, MMQ_SPLIT = range(4)
+
+
+def experts_tile(qtype, n_mat, n_expert, rows, pairs, n_cu=256):
+    """(rows, tokens) of the tile an expert launch runs on (include/oxhip_lab.h); host arithmetic."""
+    out = (ctypes.c_uint32 * 2)()
+    check(_lib.lab().experts_tile(qtype, n_mat, n_expert, rows, pairs, n_cu, ctypes.byref(out)))
+    return tuple(out)
 
 
 def get_rows(qtype, d_w, rows, cols, d_ids, n_ids, d_out, out_stride, stream=None):

@@ -270,6 +270,36 @@ def test_mmq_tile_choice_is_host_arithmetic():
     assert lib.oxh_mmq_tile(Q4K, 4096, 512, 256, None, None) == 0
 
 
+def test_which_kernel_a_matrix_core_launch_runs_on_is_host_arithmetic():
+    """oxh_lab()->mmq_kernel and ->experts_tile answer with what the launches themselves ask, also where oxh_mmq_tile
+    names another tile: Q6_K prompts, small batches with and without a workspace, expert layers."""
+    from oxidize_amd import matvec as mv
+    Q4K, Q5K, Q6K, Q80, WIDE2, T16 = 13, 15, 16, 7, 0x1008, 0x100A
+    k = mv.mmq_kernel
+    assert k(Q4K, 14336, 4096, 512)[:3] == (mv.MMQ_TILES, 256, 128)
+    assert k(Q5K, 28672, 4096, 512)[:3] == (mv.MMQ_TILES, 128, 128)
+    assert k(Q5K, 3600, 512, 500)[:3] == (mv.MMQ_TILES, 128, 64)
+    assert k(Q6K, 4096, 14336, 333)[:3] == (mv.MMQ_SHARED, 64, 128)
+    assert k(WIDE2, 4096, 14336, 512)[:3] == (mv.MMQ_SHARED, 64, 128)
+    assert k(Q80, 4096, 4096, 512)[:3] == (mv.MMQ_TILES, 128, 64)
+    kernel, rows, tokens, waves = k(Q6K, 4096, 14336, 16)           # one 16-row group per CU, columns shared in LDS
+    assert (kernel, rows, tokens) == (mv.MMQ_BATCH, 16, 16) and 4 <= waves <= 16
+    assert k(Q4K, 4096, 4096, 24)[:3] == (mv.MMQ_BATCH, 16, 32)
+    assert k(Q4K, 32, 14336, 16, ws_bytes=1 << 30)[0] == mv.MMQ_SPLIT      # few rows, many columns, room for the terms
+    assert k(Q4K, 32, 14336, 16, ws_bytes=0)[0] == mv.MMQ_TILES
+    assert k(Q4K, 28672, 4096, 16) == (mv.MMQ_TILES, 64, 16, 0)
+    for qtype, cols in ((25, 4096), (Q4K, 300)):
+        out = (ctypes.c_uint32 * 4)()
+        assert _lib.lab().mmq_kernel(qtype, 4096, cols, 16, 256, 0, ctypes.byref(out)) == _lib.DECLINED
+    t = mv.experts_tile
+    assert t(Q4K, 2, 8, 14336, 32) == t(T16, 2, 8, 14336, 32) == (64, 16)
+    assert t(Q4K, 2, 8, 14336, 8 * 50) == (128, 64)
+    assert t(Q4K, 2, 8, 14336, 8 * 128) == (256, 144)
+    assert t(Q6K, 2, 8, 14336, 8 * 128) == (128, 144)
+    out = (ctypes.c_uint32 * 2)()
+    assert _lib.lab().experts_tile(Q80, 2, 8, 14336, 32, 256, ctypes.byref(out)) == _lib.DECLINED
+
+
 def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
     """The ctypes structures of the bindings against the C compiler's view of include/oxhip.h: size and
     the offset of every field (a field added to the header and not to the bindings would shift what
