@@ -327,30 +327,69 @@ static uint32_t bat_need(int fmt, uint32_t ch, uint32_t B, uint32_t waves)
 
 #define BAT_LDS (160u * 1024u)
 
-/* The rule, from every size measured (us with the quantiser's launch in front, this kernel against the tiles and
- * the split tiles):
- *   16 activations, 4096 x 14336 18 / 26 (Q6_K), 13.6 / 20 (Q4_K); 14336 x 4096 14.6 / 16.7, 20.7 / 24.1; 8192 x 4096
- *   9.4 / 16.2, 12.6 / 22.9.  Not where few rows meet many columns (500 x 14336: 16.1 / 12.6, Q6_K): a workgroup
- *   per 16 rows then leaves most CUs without one (Q5_K, the most bytes, from half the CUs on: 1500 x 14336 14.4 /
- *   13.1; Q6_K from 5/16 of them: 1131 x 14080 16.2 / 15.6).  Nor above some
- *   four workgroups to a CU, where the tiles have enough of them too and stage a token's values for four times the rows (28672 x 4096 23 / 20, 60000 x 4096 42 / 30).
- *   17-32 activations cost a wave twice the LDS and time per weight, so the tiles, which read a row's weights for all
- *   of them once, win as soon as they fill the device: 4096 x 4096 10 / 16, 8192 x 4096 15.6 / 16.7 but 14336 x
- *   4096 28 / 20; the Q6_K tiles, slower at building operands, later (8192 x 4096 18.8 / 23.5, 8192 x 14336 59 / 66).
- *   33-64 are two such halves: 1500 x 4096 9.9 / 13.9, 1500 x 14336 23.6 / 21.9, 4096 x 4096 16.2 / 16.8, 8192 x 4096
- *   28.8 / 19.3; Q6_K 1500 x 14336 30 / 30, 4096 x 4096 18 / 23, 8192 x 4096 35 / 27. */
-extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus)
+/* The rule: against the tiles (oxh_mmq; oxh_mmq_split without a workspace), and where a workspace is at hand against
+ * the split tiles as well.  Measured on 256 CUs over 29 row counts of 16 to 28672, 28 widths of 1 to 128 super-blocks
+ * and 1 to 64 activations, all four formats, matmul launch alone, weights from several copies in turn; us, this
+ * kernel / the other.  `grid` counts workgroups: 16-row groups times token tiles.
+ *
+ * Against the tiles:
+ *   One super-block leaves the waves nothing to share: 4.8 / 4.0 at 17-64 activations, whatever the rows.
+ *   Up to 16 activations this kernel wins up to two workgroups to a CU (Q4_K, 16 activations: 8192 x 4096 8.4 / 15.1,
+ *   4096 x 14336 14.4 / 46.8), to three with five super-blocks or more (12288 x 1024, four: 6.7 / 6.1).  Above, the tiles have enough
+ *   workgroups too and stage a token's values for four times the rows: Q4_K and widened Q2_K still win from 12 to
+ *   28 super-blocks (14336 x 4096 12.6 / 15.1 at one activation; 14336 x 9216, 16 activations, 37.8 / 34.6) and beyond
+ *   with at most eight activations (Q4_K 14336 x 14336 39.5 / 49.3 at five, but 94 / 85 at 95 super-blocks) or, Q2_K,
+ *   from 56 on (69 / 72); Q5_K does not (42.9 / 36.0 at 36); Q6_K, whose tiles build operands longest, always does
+ *   from eight on (five: 10.4 / 9.5).
+ *   Above 16 activations a wave takes twice the LDS and time per weight: past a workgroup per CU not with fewer than
+ *   12 super-blocks (Q6_K: eight; 5120 x 1024 7.6 / 6.5), and not beyond some fill of the device (14336 x 4096
+ *   23.7 / 21.4).  LDS holds the terms of 36, 34, 38 super-blocks there (Q4_K, Q5_K, the others).
+ * Against the split tiles, whose time grows with the terms they move (super-blocks x rows x activations), where this
+ * kernel's grows with its rounds (super-blocks over the waves that LDS has room for) and jumps when the grid passes the
+ * CUs: up to a number of super-blocks that is linear in the grid and in the part of its 16 (32) tokens a token tile has.
+ *   Q4_K, 16 activations: 4096 x 14336 14.4 / 20.5; one: 16 x 9216 7.5 / 6.8, 1024 x 24320 18.9 / 14.2, 5120 x 24320
+ *   47 / 29; 24: 512 x 8192 12.6 / 8.5, 5120 x 8704 24.9 / 19.1. */
+struct SplitLine { double at0, slope, per_share, most; };
+
+static bool beats_split(int fmt, size_t groups, size_t blocks, size_t n_vec, size_t cus)
+{
+    /* [up to 16 activations, more][Q4_K, Q5_K, 210-byte blocks][grid up to a workgroup per CU, larger] */
+    static const SplitLine lines[2][3][2] = {
+        { { { 31, 84, 91, 80 }, { -5, 31, 19, 80 } }, { { 23, 59, 23, 72 }, { -23, 45, 0, 64 } }, { { 20, 116, 11, 72 }, { 10, 17, 0, 80 } } },
+        { { { 7, 35, 61, 40 }, { 18, 0, 0, 18 } }, { { -17, 91, 75, 40 }, { -27, 43, 5, 40 } }, { { -1, 107, 24, 40 }, { -20, 36, 9, 40 } } } };
+    const int kind = fmt == BAT_Q4 ? 0 : fmt == BAT_Q5 ? 1 : 2;
+    const size_t tok = n_vec <= 16 ? 16 : 32, tiles = (n_vec + tok - 1) / tok, grid = groups * tiles;
+    if (grid <= cus && blocks <= 15) return true;           /* 200 x 3840, 17-64 activations: 7.2 / 8.3 */
+    if (kind == 2 && tok == 16) {
+        /* at ten waves at most, 32 super-blocks take four rounds as 40 do: 512 x 8192 11.1 / 10.0 */
+        if (16 * grid < 5 * cus && blocks > 28) return false;
+        if (grid <= cus ? 8 * grid >= 5 * cus : 4 * grid >= 7 * cus) return true;
+    }
+    const SplitLine &l = lines[tok == 16 ? 0 : 1][kind][grid > cus ? 1 : 0];
+    const double share = (double)n_vec / (double)(tok * tiles);
+    const double line = l.at0 + (l.slope + l.per_share * share) * (double)grid / (double)cus;
+    return (double)blocks <= (line < l.most ? line : l.most);
+}
+
+extern "C" int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus, int split)
 {
     const size_t groups = (rows + 15) / 16;
-    if (n_vec > 64 || blocks > 128) return 0;
+    if (n_vec > 64 || blocks < 2 || blocks > 128) return 0;
     const uint32_t ch = n_vec <= 16 ? 1 : 2;
     if (bat_need(fmt, ch, (uint32_t)blocks, 4) > BAT_LDS) return 0;
+    if (split && !beats_split(fmt, groups, blocks, n_vec, cus)) return 0;
     const bool two_planes = fmt == BAT_Q6;
-    if (n_vec <= 16)
-        return groups <= 4 * cus && (blocks <= 16 || groups >= (fmt == BAT_Q5 ? cus / 2 : two_planes ? 5 * cus / 16 : cus / 4));
+    if (n_vec <= 16) {
+        if (groups <= 2 * cus) return 1;
+        if (groups <= 3 * cus) return blocks >= 5;
+        if (groups > 4 * cus || fmt == BAT_Q5) return 0;
+        if (two_planes) return blocks >= 8;
+        return blocks >= 12 && (blocks <= 28 || (fmt == BAT_Q4 ? n_vec <= 8 && blocks <= 80 : n_vec <= 8 || blocks >= 56));
+    }
+    const size_t grid = groups * ((n_vec + 31) / 32);
+    if (grid > cus && blocks < (two_planes ? 8u : 12u)) return 0;
     if (n_vec <= 32) return groups <= (two_planes ? 2 * cus : cus + cus / 4);
-    if (blocks > 32) return 2 * groups <= (two_planes ? cus : cus / 2);
-    return 2 * groups <= (two_planes ? 2 * cus : cus);
+    return grid <= (two_planes ? 2 * cus : cus);
 }
 
 /* Two workgroups of four waves to a CU where there are that many and LDS holds them: while one sums, the other

@@ -55,10 +55,11 @@ int oxh_internal_mmq6_init(void);
 int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
                              float *d_out, size_t out_stride, void *stream);
 /* K-quant matrices under at most 64 activations, a 16-row group to a workgroup (oxh_batch.hip); init and launch
- * return a hipError_t, `takes` whether a launch of these sizes belongs there, `waves` the waves of its workgroups.
+ * return a hipError_t, `takes` whether a launch of these sizes belongs there (split: and could run as tiles that share
+ * their columns through a workspace instead), `waves` the waves of its workgroups.
  * fmt: 0 Q4_K, 1 Q5_K, 2 Q6_K, 3 widened Q2_K.  Arguments checked by the caller. */
 int oxh_internal_batch_init(void);
-int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
+int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus, int split);
 uint32_t oxh_internal_mmq_batch_waves(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
 int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
                            size_t out_stride, void *stream);

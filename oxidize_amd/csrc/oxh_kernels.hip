@@ -2360,7 +2360,7 @@ static MmqRoute mmq_route(uint32_t qtype, size_t rows, size_t cols, size_t n_vec
     size_t need = 0;
     const bool planned = ws_bytes && mmq_split_plan(qtype, rows, cols, n_vec, out_stride, cus, &r.per, &r.slices, &need,
                                                     &tile_tok) && ws_bytes >= need;
-    if (!forced && oxh_internal_mmq_batch_takes(mmq_batch_fmt(qtype), rows, cols / OXH_QK_K, n_vec, cus)) {
+    if (!forced && oxh_internal_mmq_batch_takes(mmq_batch_fmt(qtype), rows, cols / OXH_QK_K, n_vec, cus, planned)) {
         r.kernel = MMQ_BATCH;
         r.tile_rows = 16u;
         r.tile_tokens = n_vec <= 16 ? 16u : 32u;

@@ -286,7 +286,7 @@ def test_which_kernel_a_matrix_core_launch_runs_on_is_host_arithmetic():
     assert (kernel, rows, tokens) == (mv.MMQ_BATCH, 16, 16) and 4 <= waves <= 16
     assert k(Q4K, 4096, 4096, 24)[:3] == (mv.MMQ_BATCH, 16, 32)
     assert k(Q4K, 32, 14336, 16, ws_bytes=1 << 30)[0] == mv.MMQ_SPLIT      # few rows, many columns, room for the terms
-    assert k(Q4K, 32, 14336, 16, ws_bytes=0)[0] == mv.MMQ_TILES
+    assert k(Q4K, 32, 14336, 16, ws_bytes=0)[:3] == (mv.MMQ_BATCH, 16, 16)
     assert k(Q4K, 28672, 4096, 16) == (mv.MMQ_TILES, 64, 16, 0)
     for qtype, cols in ((25, 4096), (Q4K, 300)):
         out = (ctypes.c_uint32 * 4)()
@@ -298,6 +298,27 @@ def test_which_kernel_a_matrix_core_launch_runs_on_is_host_arithmetic():
     assert t(Q6K, 2, 8, 14336, 8 * 128) == (128, 144)
     out = (ctypes.c_uint32 * 2)()
     assert _lib.lab().experts_tile(Q80, 2, 8, 14336, 32, 256, ctypes.byref(out)) == _lib.DECLINED
+
+
+def test_small_batches_go_where_they_measured_fastest():
+    """Sizes at which the workgroups of 16 rows measured slower than the tiles, or than tiles that share their columns
+    through a workspace (one super-block; grids a little past the CUs; few rows under many super-blocks; few
+    super-blocks under more than 16 activations), and sizes at which they measured faster, on 256 compute units."""
+    from oxidize_amd import matvec as mv
+    Q4K, Q5K, Q6K, WIDE2, ROOM = 13, 15, 16, 0x1008, 1 << 40
+    slower = [(Q4K, 4096, 256, 24, 0), (Q6K, 64, 256, 64, 0), (Q4K, 16384, 1024, 16, 0), (Q4K, 16384, 1024, 1, 0),
+              (Q5K, 14336, 9216, 16, 0), (Q4K, 14336, 24320, 16, 0), (WIDE2, 14336, 8192, 16, 0), (Q6K, 5120, 1024, 17, 0),
+              (Q4K, 5120, 1024, 32, 0), (WIDE2, 5120, 2048, 24, 0), (Q4K, 5120, 24320, 1, ROOM), (Q4K, 1024, 24320, 1, ROOM),
+              (Q5K, 5120, 14336, 16, ROOM), (Q6K, 1024, 24320, 5, ROOM), (Q4K, 500, 8192, 24, ROOM),
+              (Q6K, 500, 8192, 33, ROOM), (Q4K, 5120, 8704, 24, ROOM), (Q6K, 500, 8192, 16, ROOM), (Q5K, 16, 9216, 16, ROOM)]
+    for case in slower:
+        qtype, rows, cols, n_vec, ws = case
+        assert mv.mmq_kernel(qtype, rows, cols, n_vec, 256, ws)[0] != mv.MMQ_BATCH, case
+    for case in [(Q6K, 4096, 14336, 16, ROOM), (Q6K, 4096, 14336, 16, 0), (Q4K, 4096, 4096, 24, ROOM), (Q4K, 8192, 4096, 16, 0),
+                 (Q4K, 5120, 24320, 16, 0), (Q4K, 14336, 4096, 16, 0), (Q6K, 14336, 4096, 16, 0), (Q5K, 4096, 4096, 9, ROOM),
+                 (Q6K, 5120, 2048, 32, 0), (Q4K, 1500, 4096, 64, ROOM), (WIDE2, 4096, 14336, 16, ROOM), (Q4K, 16, 2560, 1, 0)]:
+        qtype, rows, cols, n_vec, ws = case
+        assert mv.mmq_kernel(qtype, rows, cols, n_vec, 256, ws)[0] == mv.MMQ_BATCH, case
 
 
 def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
