@@ -2226,27 +2226,41 @@ static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
 }
 
 /* Which tile a Q6_K (or widened Q2_K) launch of more than 32 activations runs on, by what it is expected to
- * take.  The unit is a super-block of a full 64 x 128 tile (1.8 us), in which a matrix of 56 super-blocks
- * measured: 64 x 128 tiles whose operands the workgroup builds once, one to a CU, 0.375 + 0.078 a token chunk
- * for every round of tiles (75 us at 5 chunks, 91 at 7, 101 at 8); 128 x 128 tiles, one to a CU, 1.6 a round
- * (161 us); 64 x 32 tiles, three to a CU, 0.75 up to a tile per CU (76 us), 0.95 just above (95 at 448
- * tiles of 256 CUs), then by their number (122 at 704, 171 at 1024, 242 at 1536).  Widened Q2_K, whose
- * operands take little building, saves 0.18 on the 64 x 32 tiles whatever their number (77 us at 448, 104 at 704; 2064
- * tiles of 20 super-blocks 111) and takes 1.48 a round of 128 x 128 ones (106 us for two of 20).  (The 128 x 64 tile took 126 us
- * where the 64 x 128 one takes 91 and is gone.) */
-static int mmq6_tile_shape(size_t rows, size_t n_vec, size_t cus, bool widened_q2)
+ * take.  The unit is 1.8 us a super-block; measured on 256 CUs at 1 to 97 super-blocks, 64 to 16384 rows and 33 to
+ * 1024 activations, every tile forced in turn, weights from one copy and from several (medians, Q6_K):
+ *   64 x 128 tiles whose operands the workgroup builds once, one to a CU: 0.69 a round up to five token chunks, 0.76,
+ *     0.80, 0.87 with six to eight; a further round costs 1.16 of the first (two rounds of seven chunks 1.74, four
+ *     3.61), the workgroups of a CU no longer starting together;
+ *   128 x 128 tiles, one to a CU: 1.48, two rounds 3.13;
+ *   64 x 32 tiles, three to a CU: 0.70 up to one a CU, 0.95 up to two, 1.2 up to three, then 0.35 each more (1.70, 2.05).
+ * A tile of 128 tokens starts 0.6 us later than one of 32, and 0.2 us in every further round: 1216 x 512 under 585
+ * activations 8.2 us against 7.5.
+ * Widened Q2_K builds its operands in fewer instructions: 0.64 to 0.86 and 1.17; 1.40, 2.99; 0.59, 0.78, 1.0, then
+ * 1.5 and 0.30 each.
+ * Where two tiles are within some 8 % the weights' way in decides, and the order for weights that come from memory was
+ * taken (Q2_K 7433 x 22528 under 78 activations: 136 us on 64 x 128 tiles against 124 on 64 x 32 ones, 10112 x 1792
+ * under 79, which stays in a cache, 13.1 against 15.6; Q6_K 7736 x 17664 under 42: 97 against 105). */
+static int mmq6_tile_shape(size_t rows, size_t blocks, size_t n_vec, size_t cus, bool widened_q2)
 {
-    if (n_vec <= 32 || ((rows + 63) / 64) * ((n_vec + 15) / 16) <= cus) return mmq_tile_shape(OXH_Q6_K, rows, n_vec, cus);
+    const size_t row_tiles = (rows + 63) / 64;
+    if (n_vec <= 32 || row_tiles * ((n_vec + 15) / 16) <= cus) return mmq_tile_shape(OXH_Q6_K, rows, n_vec, cus);
     const size_t tok_tiles = (n_vec + 127) / 128, chunks = ((n_vec + 15) / 16 + tok_tiles - 1) / tok_tiles;
-    const size_t t5 = ((rows + 63) / 64) * tok_tiles, t1 = ((rows + 127) / 128) * tok_tiles;
-    const double per_cu = (double)(((rows + 63) / 64) * ((n_vec + 31) / 32)) / (double)cus;
-    const double c5 = (double)((t5 + cus - 1) / cus) * (0.375 + 0.078 * (double)chunks);
-    const double c1 = (double)((t1 + cus - 1) / cus) * (widened_q2 ? 1.48 : 1.6);
-    double c3 = 0.15 + 0.385 * per_cu;
-    if (c3 < 0.75) c3 = 0.75;
-    if (per_cu > 1.0 && c3 < 0.95) c3 = 0.95;
-    if (widened_q2) c3 -= c3 < 0.95 ? 0.12 : 0.18;
-    if (c1 < c5 && c1 < c3) return 1;
+    const double r5 = (double)((row_tiles * tok_tiles + cus - 1) / cus);
+    const double r1 = (double)(((rows + 127) / 128 * tok_tiles + cus - 1) / cus);
+    const size_t n3 = (row_tiles * ((n_vec + 31) / 32) + cus - 1) / cus;
+    const double fill = (double)(chunks < 4 ? 4 : chunks);
+    double c1, c3, c5;
+    if (widened_q2) {
+        const double few[3] = { 0.59, blocks < 20 ? 0.67 : 0.65, 0.95 };
+        c5 = (0.34 + 0.064 * fill) * (r5 + 0.17 * (r5 - 1.0));
+        c1 = 1.40 * (r1 + 0.13 * (r1 - 1.0));
+        c3 = n3 <= 3 ? few[n3 - 1] : 0.33 + 0.30 * (double)n3;
+    } else {
+        c5 = (0.43 + 0.054 * fill) * (r5 + 0.16 * (r5 - 1.0)) + (0.25 + 0.1 * r5) / (double)blocks;
+        c1 = 1.48 * (r1 + 0.11 * (r1 - 1.0)) + (0.25 + 0.1 * r1) / (double)blocks;
+        c3 = n3 <= 3 ? 0.45 + 0.25 * (double)n3 : 0.32 + 0.35 * (double)n3;
+    }
+    if (c1 <= c5 && c1 < c3) return 1;
     return c5 < c3 ? 5 : 3;
 }
 
@@ -2371,7 +2385,7 @@ static MmqRoute mmq_route(uint32_t qtype, size_t rows, size_t cols, size_t n_vec
         r.tile_tokens = tile_tok;
         return r;
     }
-    r.shape = forced ? forced : q6 ? mmq6_tile_shape(rows, n_vec, cus, qtype == OXH_Q2_K_WIDE)
+    r.shape = forced ? forced : q6 ? mmq6_tile_shape(rows, cols / OXH_QK_K, n_vec, cus, qtype == OXH_Q2_K_WIDE)
                                    : mmq_tile_shape(qtype, rows, n_vec, cus);
     if (!q6 && r.shape == 5) r.shape = 2;       /* the tile only Q6_K and widened Q2_K have ... */
     if (q6 && r.shape == 2) r.shape = 5;        /* ... in place of this one */

@@ -321,6 +321,23 @@ def test_small_batches_go_where_they_measured_fastest():
         assert mv.mmq_kernel(qtype, rows, cols, n_vec, 256, ws)[0] == mv.MMQ_BATCH, case
 
 
+def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
+    """Q6_K and widened Q2_K above the small batches, on 256 compute units: sizes at which the 64 x 128 tiles measured
+    slower than the 64 x 32 or the 128 x 128 ones (few chunks on a part of the device, two rounds against one), and
+    sizes at which they measured faster."""
+    from oxidize_amd import matvec as mv
+    Q6K, WIDE2 = 16, 0x1008
+    for qtype, rows, cols, n_vec, tile in (
+            (Q6K, 14336, 14336, 144, (128, 128)), (Q6K, 16384, 8192, 160, (128, 128)), (Q6K, 1216, 512, 585, (64, 32)),
+            (Q6K, 6144, 256, 40, (64, 32)), (Q6K, 14336, 256, 129, (128, 128)), (WIDE2, 7168, 14336, 48, (64, 32)),
+            (WIDE2, 6144, 5120, 33, (64, 32)), (WIDE2, 8192, 14336, 40, (64, 32)), (WIDE2, 8192, 256, 48, (64, 32)),
+            (WIDE2, 8192, 14336, 96, (64, 32)), (Q6K, 4096, 14336, 333, (64, 128)), (Q6K, 4096, 14336, 512, (64, 128)),
+            (Q6K, 8192, 4096, 129, (64, 128)), (Q6K, 14336, 4096, 512, (128, 128)), (WIDE2, 4096, 14336, 512, (64, 128)),
+            (WIDE2, 10240, 5120, 64, (64, 128)), (Q6K, 7736, 17664, 42, (64, 128)), (WIDE2, 8180, 5120, 75, (64, 32)),
+            (Q6K, 10240, 14336, 64, (64, 128))):
+        assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile, (qtype, rows, cols, n_vec)
+
+
 def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
     """The ctypes structures of the bindings against the C compiler's view of include/oxhip.h: size and
     the offset of every field (a field added to the header and not to the bindings would shift what
