@@ -355,7 +355,7 @@ static bool beats_split(int fmt, size_t groups, size_t blocks, size_t n_vec, siz
 {
     /* [up to 16 activations, more][Q4_K, Q5_K, 210-byte blocks][grid up to a workgroup per CU, larger] */
     static const SplitLine lines[2][3][2] = {
-        { { { 31, 84, 91, 80 }, { -5, 31, 19, 80 } }, { { 23, 59, 23, 72 }, { -23, 45, 0, 64 } }, { { 20, 116, 11, 72 }, { 10, 17, 0, 80 } } },
+        { { { 31, 84, 91, 80 }, { -5, 31, 19, 80 } }, { { 23, 59, 23, 76 }, { -23, 45, 0, 64 } }, { { 20, 116, 11, 80 }, { 12, 17, 0, 80 } } },
         { { { 7, 35, 61, 40 }, { 18, 0, 0, 18 } }, { { -17, 91, 75, 40 }, { -27, 43, 5, 40 } }, { { -1, 107, 24, 40 }, { -20, 36, 9, 40 } } } };
     const int kind = fmt == BAT_Q4 ? 0 : fmt == BAT_Q5 ? 1 : 2;
     const size_t tok = n_vec <= 16 ? 16 : 32, tiles = (n_vec + tok - 1) / tok, grid = groups * tiles;
@@ -363,7 +363,7 @@ static bool beats_split(int fmt, size_t groups, size_t blocks, size_t n_vec, siz
     if (kind == 2 && tok == 16) {
         /* at ten waves at most, 32 super-blocks take four rounds as 40 do: 512 x 8192 11.1 / 10.0 */
         if (16 * grid < 5 * cus && blocks > 28) return false;
-        if (grid <= cus ? 8 * grid >= 5 * cus : 4 * grid >= 7 * cus) return true;
+        if (grid <= cus ? 8 * grid >= 5 * cus : 16 * grid >= 25 * cus) return true;
     }
     const SplitLine &l = lines[tok == 16 ? 0 : 1][kind][grid > cus ? 1 : 0];
     const double share = (double)n_vec / (double)(tok * tiles);
