@@ -2895,21 +2895,36 @@ static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *c
     return OXH_OK;
 }
 
-/* Many tokens per expert (two dozen on average): tiles that read an expert's weights once for 64 or 144 of its
- * tokens (oxh_experts.hip), unless there are too few of them and of tokens: under 64 tokens per expert a launch
- * that does not give nearly every CU a 128 x 64 tile runs faster on many 64 x 16 ones (4 experts, top 1, 1024 x
- * 2048, 200 tokens: 37 against 40 us a layer; 8 experts, top 2, 100 tokens: 45 against 40).  From ten tokens
- * per expert on when the 64 x 16 tiles are eight to a CU and more, whose second pass over the weights then
- * costs more than it hides (Mixtral-shaped, 64 tokens: 278 against 232 us).  OXH_MOE_BIG_TILE_FROM overrides
- * the average to start from, 0 = never. */
-static bool experts_long(size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
+/* Many tokens per expert: tiles that read an expert's weights once for 64 or 144 of its tokens (oxh_experts.hip)
+ * instead of 64 x 16 ones.  From a layer-by-layer timing of both (8 shapes from 1024 x 512 to 7168 x 2048 and 4096 x
+ * 14336, 2 to 32 experts, 8 to 128 tokens per expert on average; us a layer, long tiles for that launch / small ones):
+ *   two dozen tokens and a 128 x 64 tile for nearly every CU, or more than 64 tokens: always;
+ *   with fewer tiles than that many 64 x 16 ones fill the device better (4 experts, top 1, 1024 x 2048, Q4_K, 50 tokens
+ *   40 / 37), until there are two (Q5_K: two and a half) of those to a CU and 32 (Q5_K: 40) tokens, for the types
+ *   that take long to build operands, which a small tile does for 16 tokens only (4 experts of 4096 x 14336, Q6_K, down,
+ *   48 tokens 293 / 336);
+ *   fewer tokens, where the 64 x 16 tiles are eight to a CU and read the weights a second time for every expert with
+ *   more than sixteen: from 12 on Q4_K (8 experts of 4096 x 14336, 16 tokens 232 / 278; ten 195 / 177), from 14 on Q6_K,
+ *   from 18 on Q5_K with four 128 x 64 tiles to a CU (14 tokens 332 / 281, 20 tokens of four experts 202 / 188); from ten
+ *   on all of them where the small tiles need a second launch, having room for 32 matrices in one (60 experts, top 4,
+ *   1024 x 2048, 13 tokens 206 / 248).
+ * OXH_MOE_BIG_TILE_FROM overrides the two dozen, 0 = never. */
+static bool experts_long(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
 {
     const size_t avg_tokens = pairs / n_expert;
     static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);
     const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
     const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
-    return big_from && ((avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) ||
-                        (avg_tokens >= 10 && big_from <= 24 && small_tiles >= 8 * cus));
+    if (!big_from) return false;
+    if (avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) return true;
+    if (big_from > 24) return false;
+    if (n_mat * n_expert > OXH_MAX_SEGS && avg_tokens >= 10 && small_tiles >= 8 * cus) return true;
+    if (is_q5k(file_type))
+        return (avg_tokens >= 40 && 2 * small_tiles >= 5 * cus) ||
+               (avg_tokens >= 18 && small_tiles >= 8 * cus && wide_tiles >= 4 * cus);
+    if (file_type == OXH_Q6_K)
+        return (avg_tokens >= 32 && small_tiles >= 2 * cus) || (avg_tokens >= 14 && small_tiles >= 8 * cus);
+    return avg_tokens >= 12 && small_tiles >= 8 * cus;
 }
 
 /* few rows per expert (a down projection): the 64-row tile gives at most two workgroups per CU; Q4_K
@@ -2933,7 +2948,7 @@ extern "C" int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_exp
     if (!tile || !n_mat || !n_expert || !rows || !n_cu) return arg_fail("oxh_debug_experts_tile: NULL or empty");
     const uint32_t file_type = t16_base(qtype);
     if (!is_q4k(file_type) && !is_q5k(file_type) && file_type != OXH_Q6_K) return OXH_DECLINED;
-    if (experts_long(n_mat, n_expert, rows, pairs, n_cu)) {
+    if (experts_long(file_type, n_mat, n_expert, rows, pairs, n_cu)) {
         oxh_internal_experts_long_tile(file_type, n_mat, n_expert, rows, pairs, n_cu, tile);
         return OXH_OK;
     }
@@ -2949,7 +2964,7 @@ static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *
 {
     const uint32_t file_type = t16_base(qtype);
     const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
-    if (experts_long(n_mat, n_expert, rows, pairs, cus)) {
+    if (experts_long(file_type, n_mat, n_expert, rows, pairs, cus)) {
         if (cols / OXH_QK_K * 292u * 256u > 0xFFFFFFFFull) return arg_fail("moe: cols too large");
         const int e = oxh_internal_experts_long(file_type, is_t16(qtype), d_w, d_out, n_mat, n_expert, rows, cols, d_acts,
                                                 out_stride, d_counts, d_offsets, pairs, max_tokens, pick_stream(stream));

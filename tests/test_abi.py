@@ -338,6 +338,20 @@ def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
         assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile, (qtype, rows, cols, n_vec)
 
 
+def test_expert_launches_go_to_the_tile_that_measured_fastest():
+    """Expert launches on 256 compute units: Q5_K and Q6_K keep the 64 x 16 tiles up to more tokens per expert than Q4_K
+    while those are many, and leave them earlier where there are two or three to a unit."""
+    from oxidize_amd import matvec as mv
+    Q4K, Q5K, Q6K, T5 = 13, 15, 16, 0x100B
+    for qtype, n_mat, n_expert, rows, tokens, small in (
+            (Q5K, 2, 8, 14336, 12, True), (T5, 2, 8, 14336, 16, True), (Q6K, 2, 8, 14336, 12, True), (Q5K, 2, 16, 5632, 12, True),
+            (Q4K, 2, 8, 14336, 10, True), (Q5K, 2, 4, 14336, 20, True), (Q5K, 1, 4, 4096, 48, False), (Q6K, 1, 4, 4096, 48, False),
+            (Q6K, 2, 4, 2048, 48, False), (Q5K, 2, 8, 14336, 20, False), (Q6K, 2, 8, 14336, 16, False),
+            (Q4K, 2, 8, 14336, 16, False), (Q4K, 1, 4, 4096, 48, True), (Q4K, 2, 4, 2048, 50, True), (Q6K, 1, 4, 1024, 48, True),
+            (Q6K, 2, 60, 2048, 13, False), (Q5K, 2, 32, 2048, 16, False), (Q5K, 2, 16, 2048, 16, True)):
+        assert (mv.experts_tile(qtype, n_mat, n_expert, rows, n_expert * tokens) == (64, 16)) == small, (qtype, rows, tokens)
+
+
 def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
     """The ctypes structures of the bindings against the C compiler's view of include/oxhip.h: size and
     the offset of every field (a field added to the header and not to the bindings would shift what
