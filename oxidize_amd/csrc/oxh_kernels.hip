@@ -2908,16 +2908,16 @@ static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *c
  *   from 18 on Q5_K with four 128 x 64 tiles to a CU (14 tokens 332 / 281, 20 tokens of four experts 202 / 188); from ten
  *   on all of them where the small tiles need a second launch, having room for 32 matrices in one (60 experts, top 4,
  *   1024 x 2048, 13 tokens 206 / 248).
- * OXH_MOE_BIG_TILE_FROM overrides the two dozen, 0 = never. */
+ * OXH_MOE_BIG_TILE_FROM takes all this back: the long tiles from that many tokens per expert on, whatever the sizes, 0 =
+ * never. */
 static bool experts_long(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
 {
     const size_t avg_tokens = pairs / n_expert;
-    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", 24, 0, 4096);
+    static const uint32_t by_rule = 0xFFFFFFFFu, big_from = env_u32("OXH_MOE_BIG_TILE_FROM", by_rule, 0, 4096);
     const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
     const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
-    if (!big_from) return false;
-    if (avg_tokens >= big_from && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) return true;
-    if (big_from > 24) return false;
+    if (big_from != by_rule) return big_from && avg_tokens >= big_from;
+    if (avg_tokens >= 24 && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) return true;
     if (n_mat * n_expert > OXH_MAX_SEGS && avg_tokens >= 10 && small_tiles >= 8 * cus) return true;
     if (is_q5k(file_type))
         return (avg_tokens >= 40 && 2 * small_tiles >= 5 * cus) ||

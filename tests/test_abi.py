@@ -8,6 +8,7 @@ import os
 import re
 
 import numpy as np
+import pytest
 
 import oxlibs
 from oxidize_amd import _lib, synth
@@ -273,7 +274,6 @@ def test_mmq_tile_choice_is_host_arithmetic():
 def test_which_kernel_a_matrix_core_launch_runs_on_is_host_arithmetic():
     """oxh_lab()->mmq_kernel and ->experts_tile answer with what the launches themselves ask, also where oxh_mmq_tile
     names another tile: Q6_K prompts, small batches with and without a workspace, expert layers."""
-    from oxidize_amd import matvec as mv
     Q4K, Q5K, Q6K, Q80, WIDE2, T16 = 13, 15, 16, 7, 0x1008, 0x100A
     k = mv.mmq_kernel
     assert k(Q4K, 14336, 4096, 512)[:3] == (mv.MMQ_TILES, 256, 128)
@@ -304,7 +304,6 @@ def test_small_batches_go_where_they_measured_fastest():
     """Sizes at which the workgroups of 16 rows measured slower than the tiles, or than tiles that share their columns
     through a workspace (one super-block; grids a little past the CUs; few rows under many super-blocks; few
     super-blocks under more than 16 activations), and sizes at which they measured faster, on 256 compute units."""
-    from oxidize_amd import matvec as mv
     Q4K, Q5K, Q6K, WIDE2, ROOM = 13, 15, 16, 0x1008, 1 << 40
     slower = [(Q4K, 4096, 256, 24, 0), (Q6K, 64, 256, 64, 0), (Q4K, 16384, 1024, 16, 0), (Q4K, 16384, 1024, 1, 0),
               (Q5K, 14336, 9216, 16, 0), (Q4K, 14336, 24320, 16, 0), (WIDE2, 14336, 8192, 16, 0), (Q6K, 5120, 1024, 17, 0),
@@ -325,7 +324,6 @@ def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
     """Q6_K and widened Q2_K above the small batches, on 256 compute units: sizes at which the 64 x 128 tiles measured
     slower than the 64 x 32 or the 128 x 128 ones (few chunks on a part of the device, two rounds against one), and
     sizes at which they measured faster."""
-    from oxidize_amd import matvec as mv
     Q6K, WIDE2 = 16, 0x1008
     for qtype, rows, cols, n_vec, tile in (
             (Q6K, 14336, 14336, 144, (128, 128)), (Q6K, 16384, 8192, 160, (128, 128)), (Q6K, 1216, 512, 585, (64, 32)),
@@ -341,7 +339,6 @@ def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
 def test_expert_launches_go_to_the_tile_that_measured_fastest():
     """Expert launches on 256 compute units: Q5_K and Q6_K keep the 64 x 16 tiles up to more tokens per expert than Q4_K
     while those are many, and leave them earlier where there are two or three to a unit."""
-    from oxidize_amd import matvec as mv
     Q4K, Q5K, Q6K, T5 = 13, 15, 16, 0x100B
     for qtype, n_mat, n_expert, rows, tokens, small in (
             (Q5K, 2, 8, 14336, 12, True), (T5, 2, 8, 14336, 16, True), (Q6K, 2, 8, 14336, 12, True), (Q5K, 2, 16, 5632, 12, True),
@@ -350,6 +347,22 @@ def test_expert_launches_go_to_the_tile_that_measured_fastest():
             (Q4K, 2, 8, 14336, 16, False), (Q4K, 1, 4, 4096, 48, True), (Q4K, 2, 4, 2048, 50, True), (Q6K, 1, 4, 1024, 48, True),
             (Q6K, 2, 60, 2048, 13, False), (Q5K, 2, 32, 2048, 16, False), (Q5K, 2, 16, 2048, 16, True)):
         assert (mv.experts_tile(qtype, n_mat, n_expert, rows, n_expert * tokens) == (64, 16)) == small, (qtype, rows, tokens)
+
+
+@pytest.mark.parametrize("value,from_tokens", [("8", 8), ("24", 24), ("100", 100), ("0", None)])
+def test_the_tokens_per_expert_to_start_the_long_tiles_from_can_be_set(value, from_tokens):
+    """OXH_MOE_BIG_TILE_FROM, read once per process: that average and nothing else decides, also for launches of few
+    tiles, to which the rule on sizes gives the 64 x 16 ones."""
+    import subprocess
+    import sys
+    code = ("from oxidize_amd import matvec as mv\n"
+            "for rows in (256, 14336):\n"
+            "    print(' '.join(str(mv.experts_tile(13, 2, 4, rows, 4 * t)[1]) for t in (1, 7, 8, 23, 24, 99, 100, 300)))\n")
+    env = dict(os.environ, OXH_MOE_BIG_TILE_FROM=value)
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, check=True, capture_output=True, text=True).stdout
+    for line in out.splitlines():
+        for tokens, tile in zip((1, 7, 8, 23, 24, 99, 100, 300), line.split()):
+            assert (int(tile) > 16) == (from_tokens is not None and tokens >= from_tokens), (value, tokens, tile)
 
 
 def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
