@@ -64,6 +64,9 @@ typedef struct OxhLab {
      * pairs in all; tile: rows and tokens of a workgroup. */
     int (*experts_tile)(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu,
                         uint32_t tile[2]);
+    /* Chunks that host batches have moved through the library's own
+     * page-locked slots so far, both ways together. */
+    size_t (*host_ring_chunks)(void);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

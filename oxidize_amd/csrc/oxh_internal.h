@@ -63,6 +63,10 @@ int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_v
 uint32_t oxh_internal_mmq_batch_waves(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
 int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
                            size_t out_stride, void *stream);
+/* Whether the runtime knows all of this memory (page-locked, managed or on the device) and so copies it without a
+ * detour through staging of its own. */
+int oxh_internal_runtime_memory(const void *p, size_t bytes);
+size_t oxh_debug_host_ring_chunks(void);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
 int oxh_internal_copy16(void *dst, const void *src, size_t bytes, void *stream);
 /* Wait for a stream by polling it `spins` times before blocking. */

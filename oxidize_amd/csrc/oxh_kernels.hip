@@ -3118,6 +3118,22 @@ extern "C" int oxh_free(void *d_ptr)
     return OXH_OK;
 }
 
+/* see oxh_internal.h; a range that is one allocation, or a part of one: its two ends tell */
+extern "C" int oxh_internal_runtime_memory(const void *p, size_t bytes)
+{
+    if (!p || !bytes) return 0;
+    const uint8_t *ends[2] = { (const uint8_t *)p, (const uint8_t *)p + bytes - 1 };
+    for (const uint8_t *at : ends) {
+        hipPointerAttribute_t attr;
+        if (hipPointerGetAttributes(&attr, at) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        if (attr.type == hipMemoryTypeUnregistered) return 0;
+    }
+    return 1;
+}
+
 extern "C" int oxh_memcpy_h2d(void *d_dst, const void *h_src, size_t bytes, void *stream)
 {
     int rc = ensure_init();
@@ -3353,7 +3369,7 @@ extern "C" const OxhLab *oxh_lab(void)
 {
     static const OxhLab lab = { oxh_debug_plan_stamps, oxh_debug_plan_phantom, oxh_debug_moe_workspace_parts,
                                 oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums,
-                                oxh_debug_mmq_kernel, oxh_debug_experts_tile };
+                                oxh_debug_mmq_kernel, oxh_debug_experts_tile, oxh_debug_host_ring_chunks };
     return &lab;
 }
 

@@ -209,6 +209,46 @@ def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, p
         assert np.array_equal(bits(part[:m]), bits(out[v:v + m, :rows])), v
 
 
+@pytest.mark.parametrize("pad", [0, 5])
+@pytest.mark.parametrize("pinned_in,pinned_out", [(False, True), (True, False), (True, True)])
+def test_host_batches_from_and_to_page_locked_memory_are_copied_in_place(oxh, pinned_in, pinned_out, pad):
+    """A caller's page-locked inputs and outputs (oxh_host_alloc) above 1 MiB are one copy by the runtime each, not
+    chunks through the library's own slots, which cost such a caller half again the time; bits and padding as from
+    ordinary memory."""
+    rows, cols, n_vec = 1200, 1024, 300
+    w = synth.weights(Q4K, rows, cols, seed=19, stream=rows)
+    rb = synth.row_bytes(Q4K, cols)
+
+    def host(shape, pinned, fill):
+        n = int(np.prod(shape))
+        p = ctypes.c_void_p()
+        if pinned:
+            mv.check(mv.lib().oxh_host_alloc(ctypes.byref(p), n * 4))
+            locked.append(p)
+            a = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (n,)).reshape(shape)
+        else:
+            a = np.empty(shape, np.float32)
+        a[...] = fill
+        return a
+
+    locked, results = [], []
+    x = synth.normal(n_vec * cols, seed=19, stream=n_vec).reshape(n_vec, cols)
+    temp, scratch = np.zeros(cols, np.float32), np.zeros(mv.batch_scratch_bytes(cols), np.uint8)
+    chunks = mv._lib.lab().host_ring_chunks
+    for pin, pout in ((False, False), (pinned_in, pinned_out)):
+        xs = host((n_vec, cols + pad), pin, 3.5)
+        xs[:, :cols] = x
+        out = host((n_vec, rows + pad), pout, -7.25)
+        before = chunks()
+        mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, xs, cols + pad, out, rows + pad, n_vec, temp, scratch)
+        assert chunks() - before == (0 if pin else 2) + (0 if pout else 2)      # 1.2 and 1.4 MB in chunks of 1 MiB
+        assert np.all(out[:, rows:] == -7.25)
+        results.append(out[:, :rows].copy())
+    assert np.array_equal(bits(results[0]), bits(results[1]))
+    for p in locked:
+        mv.lib().oxh_host_free(p)
+
+
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
 @pytest.mark.parametrize("rows,cols,n_vec", [(16, 256, 1), (17, 512, 16), (1100, 25600, 3), (4099, 4096, 15), (250, 2048, 64),
                                              (700, 768, 33), (1500, 14336, 17)])
