@@ -699,13 +699,15 @@ static int reserve_host(HostBuf *b, size_t bytes)
     return OXH_OK;
 }
 
-/* Batches beyond HOST_DIRECT_MAX go through a ring of page-locked slots, a chunk at a time: a kernel moves one chunk
- * between its slot and the device while the processor copies another between its slot and the caller's (pageable)
- * memory.  Handing the runtime the pageable pointer takes both one after the other: 207 us for 3.7 MB out and 1.6 ms
- * for 28 MB, where the bus alone needs 72 and 500 us and the copy out of memory the device has just written 110 us
- * and 0.9 ms.  A whole call: 14336 x 4096 Q4_K x 64 vectors 290 -> 200 us, 14336 x 2048 Q6_K x 512 1.88 -> 1.22 ms.
- * Memory the runtime knows (page-locked by oxh_host_alloc, say) stays with the runtime's copies, which then are one DMA
- * in place: 14336 x 2048 x 512 with page-locked outputs 0.74 ms, through the ring 1.24.
+/* Outputs beyond HOST_DIRECT_MAX, and inputs beyond it whose vectors are padded apart, go through a ring of page-locked
+ * slots, a chunk at a time: a kernel moves one chunk between its slot and the device while the processor copies another
+ * between its slot and the caller's (pageable) memory.  Handing the runtime the pageable pointer takes both one after the
+ * other: 207 us for 3.7 MB out and 1.6 ms for 28 MB, where the bus alone needs 72 and 500 us and the copy out of memory
+ * the device has just written 110 us and 0.9 ms; its copies of padded vectors go row by row (4 MiB in 2.5 ms, through the ring
+ * 0.17).  A whole call: 14336 x 4096 Q4_K x 64 vectors 290 -> 200 us, 14336 x 2048 Q6_K x 512 1.88 -> 1.25 ms.
+ * Not contiguous inputs: the runtime overlaps the two copies itself on the way in, and the ring is 4 to 12 % slower
+ * (2 MiB 112 against 104 us a call, 16 MiB 573 against 527).  Nor memory the runtime knows (page-locked by oxh_host_alloc,
+ * say), whose copy is one DMA in place: 14336 x 2048 x 512 with page-locked outputs 0.74 ms, through the ring 1.24.
  * Chunks of 1 MiB: half of that 205 us and 1.29 ms (a chunk costs some 15 us of launch and wait), twice 222 us and
  * 1.19 ms; with the DMA engines instead of the kernel 222 us and 1.18 ms. */
 #define RING_SLOTS 4u
@@ -766,6 +768,7 @@ static int ring_push(uint8_t *d, const void *user, size_t width, size_t stride, 
 static int ring_pull(void *user, const uint8_t *d, size_t width, size_t stride, size_t total)
 {
     int rc;
+    if (stride == width) width = stride = total;            /* one run: a copy per chunk, not one per vector */
     const size_t chunks = (total + RING_CHUNK - 1) / RING_CHUNK;
     for (size_t k = 0; k < chunks + RING_SLOTS; k++) {
         if (k >= RING_SLOTS) {                  /* chunk k - RING_SLOTS has its slot until here */
@@ -1202,7 +1205,7 @@ static int mv_batch(uint32_t qtype, const uint8_t *data, size_t rows,
         for (size_t v = 0; v < n_vec; v++)
             memcpy((float *)g_hin.p + v * cols, inputs + v * in_stride, cols * sizeof(float));
         rc = push_input(packed_in);
-    } else if (!oxh_internal_runtime_memory(inputs, (in_span + cols) * sizeof(float)) && ring_ready())
+    } else if (in_stride != cols && !oxh_internal_runtime_memory(inputs, (in_span + cols) * sizeof(float)) && ring_ready())
         rc = ring_push((uint8_t *)g_dx.p, inputs, cols * sizeof(float), in_stride * sizeof(float), packed_in);
     else if (in_stride == cols)
         rc = oxh_memcpy_h2d(g_dx.p, inputs, packed_in, NULL);

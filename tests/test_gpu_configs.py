@@ -191,8 +191,8 @@ def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
 @pytest.mark.parametrize("rows,cols,n_vec,pad", [(1001, 4096, 1300, 0), (1001, 1024, 1300, 7), (263, 1024, 1024, 0),
                                                  (14336, 512, 19, 3)])
 def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, pad):
-    """Inputs and outputs above 1 MiB travel in 1 MiB chunks through four slots: more chunks than slots, fewer, chunk
-    boundaries inside a vector, a last chunk that is no multiple of 16 bytes, an output just above 1 MiB, padded
+    """Outputs above 1 MiB, and padded inputs, travel in 1 MiB chunks through four slots: more chunks than slots, fewer,
+    chunk boundaries inside a vector, a last chunk that is no multiple of 16 bytes, an output just above 1 MiB, padded
     strides whose padding stays as it was.  Against calls of eight vectors, which do not go through the ring."""
     w = synth.weights(Q4K, rows, cols, seed=9, stream=rows)
     rb = synth.row_bytes(Q4K, cols)
@@ -213,8 +213,8 @@ def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, p
 @pytest.mark.parametrize("pinned_in,pinned_out", [(False, True), (True, False), (True, True)])
 def test_host_batches_from_and_to_page_locked_memory_are_copied_in_place(oxh, pinned_in, pinned_out, pad):
     """A caller's page-locked inputs and outputs (oxh_host_alloc) above 1 MiB are one copy by the runtime each, not
-    chunks through the library's own slots, which cost such a caller half again the time; bits and padding as from
-    ordinary memory."""
+    chunks through the library's own slots, which cost such a caller half again the time; nor do contiguous inputs in
+    ordinary memory, whose copy the runtime overlaps itself.  Bits and padding as from ordinary memory."""
     rows, cols, n_vec = 1200, 1024, 300
     w = synth.weights(Q4K, rows, cols, seed=19, stream=rows)
     rb = synth.row_bytes(Q4K, cols)
@@ -241,7 +241,8 @@ def test_host_batches_from_and_to_page_locked_memory_are_copied_in_place(oxh, pi
         out = host((n_vec, rows + pad), pout, -7.25)
         before = chunks()
         mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, xs, cols + pad, out, rows + pad, n_vec, temp, scratch)
-        assert chunks() - before == (0 if pin else 2) + (0 if pout else 2)      # 1.2 and 1.4 MB in chunks of 1 MiB
+        # 1.2 MB in where the vectors are padded apart, 1.4 MB out, in chunks of 1 MiB
+        assert chunks() - before == (0 if pin or not pad else 2) + (0 if pout else 2)
         assert np.all(out[:, rows:] == -7.25)
         results.append(out[:, :rows].copy())
     assert np.array_equal(bits(results[0]), bits(results[1]))
