@@ -369,11 +369,11 @@ int oxh_mmq_ex(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
  * with fewer than half a 64 x 16 tile per compute unit the launch is paced by that walk.  Here several
  * workgroups share a tile's columns, every super-block's terms go to a workspace of
  * cols/256 x n_vec x out_stride floats and a second launch adds them up in block order: the order the
- * single workgroup adds them in, so the same bits.  oxh_mmq_split_workspace returns the bytes needed, or 0
- * for a launch that would not be split (types other than Q4_K, Q5_K, Q6_K and OXH_Q2_K_WIDE, more tiles,
- * fewer than eight super-blocks, more than 64 activations); oxh_mmq_split with a smaller workspace, or
- * none, is oxh_mmq.  Most launches of these sizes run on a kernel that shares the columns between the waves of
- * one workgroup instead, with or without a workspace; the split is what it leaves.
+ * single workgroup adds them in, so the same bits.  oxh_mmq_split_workspace returns the bytes of all of a
+ * launch's terms, or 0 for a launch that is never split (types other than Q4_K, Q5_K, Q6_K and OXH_Q2_K_WIDE, more
+ * tiles, fewer than eight super-blocks, more than 64 activations); oxh_mmq_split with a smaller workspace, or
+ * none, is oxh_mmq.  Where a kernel that shares the columns between the waves of one workgroup measured faster the
+ * launch runs on that and leaves the workspace alone: the answer is an upper bound (oxh_lab()->mmq_kernel tells).
  * The reference has no counterpart (its batch kernel gives every worker whole rows, oxk.c:787-836). */
 size_t oxh_mmq_split_workspace(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride);
 int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,

@@ -1221,13 +1221,15 @@ static int mv_batch(uint32_t qtype, const uint8_t *data, size_t rows,
      * walks the batch in GEMV-sized slices (every output is the same dot either way). */
     const bool kq456 = qtype == OXH_Q4_K_S || qtype == OXH_Q4_K_M || qtype == OXH_Q5_K_S || qtype == OXH_Q5_K_M ||
                        qtype == OXH_Q6_K;
-    /* few rows, many columns, seven activations or more: the tiles' columns shared between workgroups
-     * (up to six the dot kernels are as fast: 4096 x 14336 Q6_K 24.7 us at six, 43 at eight, 28 split) */
-    const size_t split_ws = (kq456 && n_vec >= mmq_split_min_nv()) ? oxh_mmq_split_workspace(qtype, rows, cols, n_vec, rows) : 0;
-    if (split_ws) {
-        if ((rc = reserve(&g_dsplit, split_ws))) return rc;
+    /* Few rows, many columns, seven activations or more: a row's columns shared between the waves of a workgroup, or a
+     * tile's between workgroups, which takes a workspace (4096 x 14336 Q6_K, eight: the dot kernels 43 us, the former 18.
+     * Up to six the dot kernels stay, 24.7 us at six.) */
+    if (kq456 && n_vec >= mmq_split_min_nv() && oxh_mmq_split_workspace(qtype, rows, cols, n_vec, rows)) {
+        const size_t ws = oxh_internal_mmq_split_use(qtype, rows, cols, n_vec, rows);
+        if (ws && (rc = reserve(&g_dsplit, ws))) return rc;
         if ((rc = quantize(kind, d_x, cols, n_vec, cols, g_dact.p))) return rc;
-        if ((rc = oxh_mmq_split(qtype, d_w, rows, cols, g_dact.p, n_vec, d_out, rows, g_dsplit.p, g_dsplit.bytes, NULL)))
+        if ((rc = oxh_mmq_split(qtype, d_w, rows, cols, g_dact.p, n_vec, d_out, rows, ws ? g_dsplit.p : NULL,
+                                ws ? g_dsplit.bytes : 0, NULL)))
             return rc;
     } else if (n_vec > 8 && kq456) {
         if ((rc = quantize(kind, d_x, cols, n_vec, cols, g_dact.p))) return rc;
@@ -1246,7 +1248,7 @@ static int mv_batch(uint32_t qtype, const uint8_t *data, size_t rows,
             return rc;
         if ((rc = quantize(kind, d_x, cols, n_vec, cols, g_dact.p))) return rc;
         const uint32_t as = qtype == OXH_Q2_K ? OXH_Q2_K_WIDE : OXH_Q6_K;
-        const size_t ws = n_vec >= mmq_split_min_nv() ? oxh_mmq_split_workspace(as, rows, cols, n_vec, rows) : 0;
+        const size_t ws = n_vec >= mmq_split_min_nv() ? oxh_internal_mmq_split_use(as, rows, cols, n_vec, rows) : 0;
         if (ws && (rc = reserve(&g_dsplit, ws))) return rc;
         /* without a workspace this is oxh_mmq */
         if ((rc = oxh_mmq_split(as, d_prep, rows, cols, g_dact.p, n_vec, d_out, rows, ws ? g_dsplit.p : NULL,

@@ -67,6 +67,9 @@ int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks,
  * detour through staging of its own. */
 int oxh_internal_runtime_memory(const void *p, size_t bytes);
 size_t oxh_debug_host_ring_chunks(void);
+/* Bytes of workspace an oxh_mmq_split launch of these sizes makes use of: what oxh_mmq_split_workspace says, or 0
+ * where the launch runs on a kernel that needs none. */
+size_t oxh_internal_mmq_split_use(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride);
 /* 16-byte-granular copy by a kernel (either side may be page-locked host memory). */
 int oxh_internal_copy16(void *dst, const void *src, size_t bytes, void *stream);
 /* Wait for a stream by polling it `spins` times before blocking. */

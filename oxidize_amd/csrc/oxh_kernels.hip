@@ -2427,6 +2427,15 @@ extern "C" size_t oxh_mmq_split_workspace(uint32_t qtype, size_t rows, size_t co
     return mmq_split_plan(qtype, rows, cols, n_vec, out_stride, cus, nullptr, nullptr, &bytes) ? bytes : 0;
 }
 
+/* see oxh_internal.h */
+extern "C" size_t oxh_internal_mmq_split_use(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t out_stride)
+{
+    const size_t bytes = oxh_mmq_split_workspace(qtype, rows, cols, n_vec, out_stride);
+    if (!bytes) return 0;
+    const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
+    return mmq_route(canon_qtype(qtype), rows, cols, n_vec, out_stride, bytes, cus).kernel == MMQ_SPLIT ? bytes : 0;
+}
+
 extern "C" int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols, const void *d_acts,
                              size_t n_vec, float *d_out, size_t out_stride, void *d_workspace, size_t workspace_bytes,
                              void *stream)

@@ -310,6 +310,40 @@ def test_q6_k_tiles_with_shared_operands_over_three_million_activations(oxh):
         assert np.array_equal(out[0].reshape(unit, rows)[v], bits(want)), v
 
 
+@pytest.mark.parametrize("qtype,rows,cols,n_vec", [(Q4K, 2048, 8192, 32), (8, 2048, 8192, 32)])
+def test_host_batches_reserve_a_workspace_only_for_launches_that_use_it(oxh, qtype, rows, cols, n_vec):
+    """A host batch that oxh_mmq_split_workspace names a size for, on the kernel that needs none of it: device memory
+    grows by the matrix (Q2_K: and its widened copy) and the vectors, not by the terms.  In a process of its own, whose
+    buffers nothing else has made."""
+    import subprocess
+    import sys
+    run = {8: mv.Q2_K_WIDE}.get(qtype, qtype)
+    terms = mv.mmq_split_workspace(run, rows, cols, n_vec, rows)
+    assert terms >= 4 << 20 and mv.mmq_kernel(run, rows, cols, n_vec, mv.device_info()["n_cu"], terms)[0] == mv.MMQ_BATCH
+    code = """
+import ctypes, numpy as np
+from oxidize_amd import matvec as mv, synth
+def batch(rows, cols, n):
+    w = synth.weights({q}, rows, cols, seed=1, stream=rows)
+    x, o = np.ones((n, cols), np.float32), np.zeros((n, rows), np.float32)
+    mv.matvec_quantized_batch({q}, w, rows, cols, synth.row_bytes({q}, cols), x, cols, o, rows, n, np.zeros(cols, np.float32),
+                              np.zeros(mv.batch_scratch_bytes(cols), np.uint8))
+def free():
+    f, t = ctypes.c_size_t(), ctypes.c_size_t()
+    mv.check(mv.lib().oxh_mem_info(ctypes.byref(f), ctypes.byref(t)))
+    return f.value
+batch(512, 2560, 32)
+before = free()
+batch({rows}, {cols}, {n})
+print(before - free())
+""".format(q=qtype, rows=rows, cols=cols, n=n_vec)
+    used = int(subprocess.run([sys.executable, "-c", code], cwd=oxlibs.ROOT, check=True, capture_output=True, text=True,
+                              timeout=100).stdout)
+    matrices = rows * (synth.row_bytes(qtype, cols) + (cols // 256 * 210 if run != qtype else 0))
+    vectors = n_vec * (cols + rows) * 4 + n_vec * mv.act_bytes(qtype, cols)
+    assert used < matrices + 2 * vectors + (6 << 20) <= matrices + 2 * vectors + 5 * terms // 4, (used, matrices, vectors, terms)
+
+
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
 def test_small_batch_launch_on_128_row_tiles(oxh, qtype):
     """Five activations over 30000 rows: 469 tiles of 64 rows would be fewer than two per CU on a 256-CU
