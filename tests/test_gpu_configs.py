@@ -189,7 +189,7 @@ def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
 
 
 @pytest.mark.parametrize("rows,cols,n_vec,pad", [(1001, 4096, 1300, 0), (1001, 1024, 1300, 7), (263, 1024, 1024, 0),
-                                                 (14336, 512, 19, 3)])
+                                                 (14336, 512, 19, 3), (1001, 256, 1301, 0), (1001, 1024, 1301, 7)])
 def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, pad):
     """Outputs above 1 MiB, and padded inputs, travel in 1 MiB chunks through four slots: more chunks than slots, fewer,
     chunk boundaries inside a vector, a last chunk that is no multiple of 16 bytes, an output just above 1 MiB, padded
@@ -251,13 +251,23 @@ def test_host_batches_from_and_to_page_locked_memory_are_copied_in_place(oxh, pi
 
 
 @pytest.mark.parametrize("qtype", [Q4K, Q5K, Q6K])
-@pytest.mark.parametrize("rows,cols,n_vec", [(16, 256, 1), (17, 512, 16), (1100, 25600, 3), (4099, 4096, 15), (250, 2048, 64),
-                                             (700, 768, 33), (1500, 14336, 17)])
-def test_small_batches_on_a_workgroup_per_16_rows(oxh, qtype, rows, cols, n_vec):
-    """The kernel whose waves share the super-blocks of 16 rows and sum the terms from LDS: one super-block and
-    more waves than super-blocks, 100 of them (what LDS holds), uneven rounds, two workgroups to a CU, one and two
-    16-token chunks, two token tiles, ragged rows and tokens, a padded output.  Against the dot-instruction kernel on
-    the same device data, and three activations against the oracle."""
+@pytest.mark.parametrize("rows,cols,n_vec,waves", [
+    (17, 512, 16, 2),           # fewer super-blocks than waves
+    (2100, 24320, 3, 0),        # 95 super-blocks, nearly all that LDS holds the terms of
+    (1100, 25600, 3, None),     # 100: more than it holds for Q5_K
+    (4099, 4096, 15, 4),        # two workgroups to a CU
+    (250, 2048, 64, 4),         # two chunks of tokens, two token tiles
+    (700, 768, 33, 3),
+    (3000, 2304, 17, 5),        # nine super-blocks: the last round is not full
+    (700, 8704, 40, 4),         # 34, what LDS holds for all types with two chunks; the last round is not full
+    (16, 256, 1, None), (1500, 14336, 17, None)])       # one super-block; more than fit: on the tiles
+def test_small_batches_on_a_workgroup_per_16_rows(oxh, qtype, rows, cols, n_vec, waves):
+    """The kernel whose waves share the super-blocks of 16 rows and sum the terms from LDS, and sizes just outside what
+    it takes; ragged rows and tokens, a padded output.  `waves`: of its workgroups on 256 compute units (0: by type).
+    Against the dot-instruction kernel on the same device data, and three activations against the oracle."""
+    if waves is not None and mv.device_info()["n_cu"] == 256:
+        kernel, _, _, got = mv.mmq_kernel(qtype, rows, cols, n_vec)
+        assert kernel == mv.MMQ_BATCH and got == (waves or got)
     w = synth.weights(qtype, rows, cols, seed=7, stream=rows)
     xs = synth.normal(n_vec * cols, seed=7, stream=n_vec).reshape(n_vec, cols)
     d_w, d_x = mv.DeviceBuffer.from_host(w), mv.DeviceBuffer.from_host(xs)
@@ -278,11 +288,16 @@ def test_small_batches_on_a_workgroup_per_16_rows(oxh, qtype, rows, cols, n_vec)
         assert np.array_equal(bits(out[v, :rows]), bits(want)), v
 
 
-@pytest.mark.parametrize("rows,cols,n_vec", [(4095, 512, 333), (4100, 768, 129), (14300, 256, 40), (14337, 512, 66),
-                                             (7000, 256, 128), (2049, 1024, 400)])
-def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec):
-    """64 x 128 tiles whose operands the workgroup builds once: 7, 5 (4 and 5), 3, 5, 8 and 7 (6) chunks of tokens to a
-    tile, dealt to its two halves; one to four super-blocks; ragged rows and tokens.  Same checks as above."""
+@pytest.mark.parametrize("rows,cols,n_vec,tile", [(4095, 512, 333, (64, 128)), (4100, 768, 129, (64, 128)), (14337, 512, 66, (64, 128)),
+                                                  (8200, 768, 128, (64, 128)), (2049, 1024, 400, (64, 128)), (10300, 768, 90, (64, 128)),
+                                                  (8200, 512, 33, (64, 128)), (16300, 512, 50, (64, 128)), (14300, 256, 40, (64, 32)),
+                                                  (7000, 256, 128, (64, 32)), (8300, 512, 256, (128, 128))])
+def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec, tile):
+    """64 x 128 tiles whose operands the workgroup builds once: 7, 5 and 4, 5, 8, 7 and 6, 6, 3 and 4 chunks of tokens to a
+    tile, dealt to its two halves; two to four super-blocks; ragged rows and tokens; and sizes beside them that the other
+    two tiles take.  Same checks as above."""
+    if mv.device_info()["n_cu"] == 256:
+        assert mv.mmq_kernel(Q6K, rows, cols, n_vec)[:3] == ((mv.MMQ_SHARED if tile == (64, 128) else mv.MMQ_TILES,) + tile)
     test_mmq_tile_variants_ragged(oxh, Q6K, rows, cols, n_vec)
 
 
@@ -444,11 +459,18 @@ def test_mmq_relaxed_mode_is_opt_in_and_within_tolerance(oxh, qtype, rows, cols,
 @pytest.mark.parametrize("qt", [13, 15, 16])
 @pytest.mark.parametrize("rows,cols,n_vec", [(4096, 14336, 16), (1000, 4096, 5), (70, 2048, 40), (64, 8192, 64),
                                              (3000, 2304, 17), (1, 14336, 1), (33, 5120, 3), (257, 7168, 31),
-                                             (100, 5376, 9), (2049, 6400, 18), (4000, 14336, 45), (4096, 4096, 24)])
+                                             (100, 5376, 9), (2049, 6400, 18), (4000, 14336, 45), (4096, 4096, 24),
+                                             (40, 14336, 5), (500, 8192, 20), (130, 24576, 64), (2500, 14336, 20)])
 def test_mmq_with_a_tile_s_columns_shared_between_workgroups(oxh, qt, rows, cols, n_vec):
     """oxh_mmq_split: every super-block's terms go to a workspace and are added in block order by a second
-    launch: bit for bit what oxh_mmq gives, padding between rows and out_stride untouched, and without a
-    workspace (or for a launch that would not be split) it is oxh_mmq."""
+    launch: bit for bit what oxh_mmq gives on its kernels (the tiles or a workgroup per 16 rows), padding between rows and
+    out_stride untouched, and without a workspace, or where a workgroup per 16 rows is as fast, it is oxh_mmq."""
+    if mv.device_info()["n_cu"] == 256:
+        kernel = mv.mmq_kernel(qt, rows, cols, n_vec, ws_bytes=1 << 40)[0]
+        split = (rows, cols) in ((64, 8192), (1, 14336), (257, 7168), (4000, 14336), (40, 14336), (500, 8192), (130, 24576),
+                                 (2500, 14336))
+        assert kernel == (mv.MMQ_SPLIT if split else mv.MMQ_BATCH)
+        assert mv.mmq_kernel(qt, rows, cols, n_vec, ws_bytes=0)[0] in (mv.MMQ_BATCH, mv.MMQ_TILES)
     out_stride = rows + 3
     w = mv.DeviceBuffer.from_host(synth.weights(qt, rows, cols, seed=rows, stream=qt))
     x = mv.DeviceBuffer.from_host(synth.normal(n_vec * cols, seed=n_vec, stream=qt))

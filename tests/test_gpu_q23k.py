@@ -290,28 +290,31 @@ def test_q2k_widened_bytes(oxh):
         mv.q2_k_widen(d_w.ptr, 1, 200, d_o.ptr)
 
 
-@pytest.mark.parametrize("n_vec", [1, 16, 17, 40, 130])
-def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec):
+@pytest.mark.parametrize("n_vec,cols", [(1, 1024), (16, 1024), (17, 1024), (40, 1024), (130, 1024), (16, 256), (17, 256), (40, 256)])
+def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec, cols):
     """oxh_mmq on widened raw random Q2_K blocks (every scale, minimum and code value, arbitrary f16 d and
-    dmin as far as they are finite) against the oracle's Q2_K dot of the original blocks, bit for bit,
-    through every tile shape."""
-    rows, cols = 203, 1024
+    dmin as far as they are finite) against the oracle's Q2_K dot of the original blocks, bit for bit: four
+    super-blocks up to 64 activations on a workgroup per 16 rows, one super-block and more activations on the 64 x 16 tiles."""
+    rows, B = 203, cols // 256
+    if mv.device_info()["n_cu"] == 256:
+        kernel = mv.mmq_kernel(mv.Q2_K_WIDE, rows, cols, n_vec)
+        assert kernel[:3] == ((mv.MMQ_BATCH, 16, 16 if n_vec <= 16 else 32) if B == 4 and n_vec <= 64 else (mv.MMQ_TILES, 64, 16))
     rng = np.random.default_rng(n_vec)
-    w = rng.integers(0, 256, rows * 4 * 84, dtype=np.uint8).reshape(-1, 84)
+    w = rng.integers(0, 256, rows * B * 84, dtype=np.uint8).reshape(-1, 84)
     w[:, 81] &= 0x3B          # |d|, |dmin| below 2: finite, products stay finite
     w[:, 83] &= 0x3B
     w = w.reshape(-1)
     x = synth.normal(n_vec * cols, seed=5, stream=n_vec)
     o = oxlibs.oracle()
-    act = np.zeros(n_vec * 4 * 292, np.uint8)
+    act = np.zeros(n_vec * B * 292, np.uint8)
     for v in range(n_vec):
-        o.oxo_quantize_q8_k(x[v * cols:].ctypes.data, cols, act[v * 4 * 292:].ctypes.data)
+        o.oxo_quantize_q8_k(x[v * cols:].ctypes.data, cols, act[v * B * 292:].ctypes.data)
     want = np.zeros((n_vec, rows), np.float32)
     for v in range(n_vec):
         for r in range(rows):
-            want[v, r] = o.oxo_dot_q2_k_q8_k(w[r * 4 * 84:].ctypes.data, 4, act[v * 4 * 292:].ctypes.data, None)
+            want[v, r] = o.oxo_dot_q2_k_q8_k(w[r * B * 84:].ctypes.data, B, act[v * B * 292:].ctypes.data, None)
     d_w = mv.DeviceBuffer.from_host(w)
-    d_wide = mv.DeviceBuffer(rows * 4 * 210)
+    d_wide = mv.DeviceBuffer(rows * B * 210)
     mv.q2_k_widen(d_w.ptr, rows, cols, d_wide.ptr)
     d_a = mv.DeviceBuffer.from_host(act)
     d_o = mv.DeviceBuffer(n_vec * rows * 4)
@@ -320,15 +323,19 @@ def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec):
     assert np.array_equal(bits(got), bits(want))
     # the widened blocks with a tile's columns shared between workgroups (four super-blocks are too few
     # to split: a wider matrix of the same blocks against the unsplit launch)
-    wide_rows = rows // 14
-    need = mv.mmq_split_workspace(mv.Q2_K_WIDE, wide_rows, 14 * cols, n_vec, wide_rows)
+    times = 56 // B
+    wide_rows = rows // times
+    need = mv.mmq_split_workspace(mv.Q2_K_WIDE, wide_rows, times * cols, n_vec, wide_rows)
     if n_vec <= 64:
         assert need == 56 * n_vec * wide_rows * 4
-        d_a14 = mv.DeviceBuffer.from_host(np.tile(act.reshape(n_vec, -1), (1, 14)).reshape(-1))
+        if mv.device_info()["n_cu"] == 256:
+            assert mv.mmq_kernel(mv.Q2_K_WIDE, wide_rows, times * cols, n_vec, ws_bytes=need)[0] == mv.MMQ_SPLIT
+            assert mv.mmq_kernel(mv.Q2_K_WIDE, wide_rows, times * cols, n_vec)[0] != mv.MMQ_SPLIT
+        d_a14 = mv.DeviceBuffer.from_host(np.tile(act.reshape(n_vec, -1), (1, times)).reshape(-1))
         d_ws = mv.DeviceBuffer(need)
         d_o1, d_o2 = mv.DeviceBuffer(n_vec * wide_rows * 4), mv.DeviceBuffer(n_vec * wide_rows * 4)
-        mv.mmq(mv.Q2_K_WIDE, d_wide.ptr, wide_rows, 14 * cols, d_a14.ptr, n_vec, d_o1.ptr, wide_rows)
-        mv.mmq_split(mv.Q2_K_WIDE, d_wide.ptr, wide_rows, 14 * cols, d_a14.ptr, n_vec, d_o2.ptr, wide_rows,
+        mv.mmq(mv.Q2_K_WIDE, d_wide.ptr, wide_rows, times * cols, d_a14.ptr, n_vec, d_o1.ptr, wide_rows)
+        mv.mmq_split(mv.Q2_K_WIDE, d_wide.ptr, wide_rows, times * cols, d_a14.ptr, n_vec, d_o2.ptr, wide_rows,
                      d_ws.ptr, need)
         assert np.array_equal(d_o1.download(np.uint32, n_vec * wide_rows), d_o2.download(np.uint32, n_vec * wide_rows))
     else:
@@ -339,10 +346,14 @@ def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec):
         mv.gemv_segments(mv.Q2_K_WIDE, seg, cols, d_a.ptr, 1, rows)
 
 
-@pytest.mark.parametrize("rows,cols,n_vec", [(4099, 512, 130), (3600, 256, 333), (14300, 768, 40)])
-def test_q2k_wide_tiles_with_shared_operands(oxh, rows, cols, n_vec):
-    """The 64 x 128 tiles whose operands the workgroup builds once, on widened raw random blocks, against the
-    64 x 16 tiles (the test above holds those to the oracle) sixteen activations at a time: the same bits."""
+@pytest.mark.parametrize("rows,cols,n_vec,tile", [(4099, 512, 130, (64, 128)), (3600, 256, 333, (64, 128)), (14300, 768, 40, (64, 128)),
+                                                  (8200, 768, 128, (64, 128)), (2049, 1280, 390, (64, 32)), (8300, 512, 256, (128, 128))])
+def test_q2k_wide_tiles_with_shared_operands(oxh, rows, cols, n_vec, tile):
+    """The 64 x 128 tiles whose operands the workgroup builds once, and the two tiles beside them, on widened raw random
+    blocks, against the kernels of sixteen activations (the test above holds both of those to the oracle) sixteen
+    at a time: the same bits."""
+    if mv.device_info()["n_cu"] == 256:
+        assert mv.mmq_kernel(mv.Q2_K_WIDE, rows, cols, n_vec)[1:3] == tile
     rng = np.random.default_rng(rows)
     w = rng.integers(0, 256, rows * (cols // 256) * 84, dtype=np.uint8).reshape(-1, 84)
     w[:, 81] &= 0x3B

@@ -121,9 +121,22 @@ def test_several_segments_with_their_own_counts(oxh):
     assert np.array_equal(bits(o2.download(np.float32, n_act * rows)), bits(o1.download(np.float32, n_act * rows)))
 
 
-@pytest.mark.parametrize("qt_gu,qt_dn,n_tok", [(Q4K, Q4K, 16), (Q5K, Q4K, 5), (Q4K, Q6K, 9), (Q4K, Q4K, 200)])
-def test_expert_layer_bits_equal_the_file_layout(oxh, qt_gu, qt_dn, n_tok):
-    n_expert, top_k, hidden, ffn = 8, 2, 512, 1280
+@pytest.mark.parametrize("qt_gu,qt_dn,n_tok,hidden,ffn,tiles", [
+    (Q4K, Q4K, 16, 512, 1280, ((64, 16), (64, 16))), (Q5K, Q4K, 5, 512, 1280, ((64, 16), (64, 16))),
+    (Q4K, Q6K, 9, 512, 1280, ((64, 16), (64, 16))), (Q4K, Q4K, 200, 512, 1280, ((64, 16), (64, 16))),
+    (Q4K, Q4K, 560, 256, 3584, ((256, 144), (128, 64))),        # an expert's second and third tile, ragged chunks
+    (Q4K, Q4K, 577, 256, 2048, ((128, 144), (128, 64))),
+    (Q5K, Q5K, 300, 256, 3584, ((128, 144), (128, 64))),
+    (Q4K, Q4K, 130, 3584, 512, ((64, 16), (128, 64))), (Q5K, Q5K, 1100, 2048, 512, ((128, 64), (128, 144)))])
+def test_expert_layer_bits_equal_the_file_layout(oxh, qt_gu, qt_dn, n_tok, hidden, ffn, tiles):
+    """The layer over tile-major experts and over the same ones in the file's layout, which test_gpu_moe.py holds to
+    the oracle, on every tile that takes tile-major weights (256 rows are two 16-row groups to a wave); from 300 tokens
+    on the routing is skewed: one popular expert, one without a token."""
+    n_expert, top_k = 8, 2
+    if mv.device_info()["n_cu"] == 256:
+        pairs = n_tok * top_k
+        assert (mv.experts_tile(T16[qt_gu], 2, n_expert, ffn, pairs),
+                mv.experts_tile(T16.get(qt_dn, qt_dn), 1, n_expert, hidden, pairs)) == tiles
     wg = synth.weights(qt_gu, n_expert * ffn, hidden, seed=44, stream=1)
     wu = synth.weights(qt_gu, n_expert * ffn, hidden, seed=44, stream=2)
     wd = synth.weights(qt_dn, n_expert * hidden, ffn, seed=44, stream=3)
@@ -133,7 +146,10 @@ def test_expert_layer_bits_equal_the_file_layout(oxh, qt_gu, qt_dn, n_tok):
         d_d, t_d = tiled_copy(qt_dn, wd, n_expert * hidden, ffn)
     else:
         d_d = t_d = mv.DeviceBuffer.from_host(wd)
-    logits = synth.normal(n_tok * n_expert, seed=44, stream=4)
+    logits = synth.normal(n_tok * n_expert, seed=44, stream=4).reshape(n_tok, n_expert)
+    if n_tok >= 300:
+        logits[:, 2] += 1.0
+        logits[:, 5] = -40.0
     x = synth.normal(n_tok * hidden, seed=44, stream=5)
     d_l, d_x = mv.DeviceBuffer.from_host(logits), mv.DeviceBuffer.from_host(x)
     y1, y2 = mv.DeviceBuffer(n_tok * hidden * 4), mv.DeviceBuffer(n_tok * hidden * 4)
