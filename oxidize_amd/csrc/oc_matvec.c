@@ -768,7 +768,9 @@ static int ring_push(uint8_t *d, const void *user, size_t width, size_t stride, 
 static int ring_pull(void *user, const uint8_t *d, size_t width, size_t stride, size_t total)
 {
     int rc;
-    if (stride == width) width = stride = total;            /* one run: a copy per chunk, not one per vector */
+    /* one run: in pieces of 64 KiB, whatever the vectors' length (short vectors cost a call each, and a whole
+     * chunk at once the processor writes past its caches: 64 x 14336 outputs 196 -> 229 us a call) */
+    if (stride == width) width = stride = (size_t)1 << 16;
     const size_t chunks = (total + RING_CHUNK - 1) / RING_CHUNK;
     for (size_t k = 0; k < chunks + RING_SLOTS; k++) {
         if (k >= RING_SLOTS) {                  /* chunk k - RING_SLOTS has its slot until here */
