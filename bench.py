@@ -357,8 +357,8 @@ def secondary_figures(mv, synth):
     from oxidize_amd import _lib
     _lib.check(_lib.lib().oxh_weight_clear())
     out["host_pointer_api_us_per_call"] = host_api
-    # small batches over the decode matrices with few rows: the dot kernels (up to eight activations), one
-    # workgroup per 64 x 16 tile (oxh_mmq), and the tiles' columns shared between workgroups (oxh_mmq_split)
+    # small batches over the decode matrices with few rows: the dot kernels (up to eight activations) and the
+    # matrix-core launch without and with a workspace (oxh_mmq, oxh_mmq_split), with the kernel each runs on
     small = {}
     for name, qt, r_, c_ in (("q6_k_4096x14336", Q6K, 4096, 14336), ("q4_k_4096x4096", Q4K, 4096, 4096)):
         w = synth.weights(qt, r_, c_, seed=0, stream=12)
@@ -386,11 +386,14 @@ def secondary_figures(mv, synth):
                 state["i"] += 1
                 mv.mmq_split(qt, copies[state["i"] % 6].ptr, r_, c_, d_a.ptr, nv, d_o.ptr, r_, d_ws.ptr, need)
 
-            row = {"one_workgroup_per_tile_us": round(timed(run_tiles, 24, mv), 1)}
+            kernels = ("tiles", "tiles", "workgroup_per_16_rows", "columns_shared_between_workgroups")
+            row = {"mmq_us": round(timed(run_tiles, 24, mv), 1),
+                   "mmq_kernel": kernels[mv.mmq_kernel(qt, r_, c_, nv, mv.device_info()["n_cu"])[0]]}
             if nv <= 8:
                 row["dot_kernel_us"] = round(timed(run_dot, 24, mv), 1)
             if need:
-                row["columns_shared_us"] = round(timed(run_split, 24, mv), 1)
+                row["mmq_with_workspace_us"] = round(timed(run_split, 24, mv), 1)
+                row["mmq_with_workspace_kernel"] = kernels[mv.mmq_kernel(qt, r_, c_, nv, mv.device_info()["n_cu"], need)[0]]
             per["batch%d" % nv] = row
             for b_ in (d_x, d_a, d_o, d_ws):
                 b_.free()
@@ -943,7 +946,7 @@ def q80_batch_probe(mv, synth):
 def split_probe(mv, synth):
     """For `rocprofv3 --kernel-trace --stats` runs on small-batch launches over few rows and many
     columns: a 4096 x 14336 Q6_K matrix under 16 activations, twelve launches of oxh_mmq and twelve of
-    oxh_mmq_split over six copies of the weights in turn.  Prints nothing."""
+    oxh_mmq_split (the same kernel at this size) over six copies of the weights in turn.  Prints nothing."""
     Q6K = 16
     rows, cols, n_vec = 4096, 14336, 16
     w = synth.weights(Q6K, rows, cols, seed=0, stream=12)
