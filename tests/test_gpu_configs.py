@@ -140,29 +140,35 @@ def test_config3_mmq_prefill_512_tokens(oxh, rows):
         assert np.array_equal(bits(got), bits(out[v0:v0 + 2]))
 
 
-@pytest.mark.parametrize("qtype,rows,cols,n_vec", [
-    (Q4K, 7165, 512, 507),      # 256x128 tiles would be 28 x 4 workgroups: 128x64 tiles, 56 x 8
-    (Q4K, 14329, 256, 500),     # 256x128 tiles: 56 x 4 = 224 workgroups
-    (Q4K, 4100, 512, 40),       # too few workgroups for either: 64x32 tiles, 65 x 2
-    (Q6K, 7165, 512, 507),      # Q6_K: 128x128 tiles, 56 x 4
-    (Q6K, 3600, 256, 500),      # Q6_K: 64x128 tiles on four waves, 57 x 4
-    (Q6K, 14250, 256, 100),     # Q6_K: 128x64 tiles, 112 x 2 (223 tiles of 64x128 would leave CUs idle)
-    (Q6K, 4100, 512, 40),       # Q6_K: 64x32 tiles
-    (Q5K, 7165, 512, 507),      # Q5_K: 128x128 tiles, 56 x 4
-    (Q5K, 3600, 256, 500),      # Q5_K: 128x64 tiles, 29 x 8
-    (Q5K, 4100, 512, 40),       # Q5_K: 64x32 tiles
+@pytest.mark.parametrize("qtype,rows,cols,n_vec,tile", [
+    (Q4K, 7165, 512, 507, (128, 64)),       # 256x128 tiles would be 28 x 4 workgroups: 128x64 tiles, 56 x 8
+    (Q4K, 14329, 256, 500, (256, 128)),     # 56 x 4 = 224 workgroups
+    (Q4K, 7000, 512, 40, (64, 32)),         # too few workgroups for either: 110 x 2
+    (Q4K, 4100, 512, 40, (64, 16)),         # 65 x 3 of the smallest leave no CU with two
+    (Q6K, 7165, 512, 507, (128, 128)),
+    (Q6K, 3600, 256, 500, (64, 128)),       # operands built once per workgroup, 57 x 4
+    (Q6K, 14250, 256, 100, (64, 128)),
+    (Q6K, 7000, 256, 40, (64, 32)),
+    (Q6K, 4100, 512, 40, (64, 16)),
+    (Q5K, 7165, 512, 507, (128, 128)),
+    (Q5K, 3600, 256, 500, (128, 64)),       # 29 x 8
+    (Q5K, 7000, 512, 40, (64, 32)),
+    (Q5K, 4100, 512, 40, (64, 16)),
 ])
-def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec):
-    """The MFMA kernel comes in several tile shapes (256x128, 128x64, 64x32,
+def test_mmq_tile_variants_ragged(oxh, qtype, rows, cols, n_vec, tile):
+    """The MFMA kernel comes in several tile shapes (256x128, 128x128, 128x64, 64x32,
     64x16 rows x tokens, and 64x128 for Q6_K), picked from the launch size;
-    these cases select all but 64x16 on a 256-CU device and leave the last row tile and the last
-    token tile partly filled.  Every output is checked against the
-    dot-instruction GEMV kernel on the same device data (two activations per
-    launch: three or more would run on the matrix cores too), and a sample of
-    tokens against the oracle."""
-    info = mv.device_info()
-    if info["n_cu"] != 256:
+    these cases select each of them on a 256-CU device and leave the last row tile and the last
+    token tile partly filled."""
+    if mv.device_info()["n_cu"] != 256:
         pytest.skip("tile choice is tied to 256 compute units")
+    assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile
+    check_mmq(qtype, rows, cols, n_vec)
+
+
+def check_mmq(qtype, rows, cols, n_vec):
+    """Every output of an oxh_mmq launch against the dot-instruction GEMV kernel on the same device data (two
+    activations per launch: three or more would run on the matrix cores too), and a sample of tokens against the oracle."""
     w = synth.weights(qtype, rows, cols, seed=5, stream=rows)
     xs = synth.normal(n_vec * cols, seed=5, stream=n_vec).reshape(n_vec, cols)
     d_w = mv.DeviceBuffer.from_host(w)
@@ -298,7 +304,7 @@ def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec, tile):
     two tiles take.  Same checks as above."""
     if mv.device_info()["n_cu"] == 256:
         assert mv.mmq_kernel(Q6K, rows, cols, n_vec)[:3] == ((mv.MMQ_SHARED if tile == (64, 128) else mv.MMQ_TILES,) + tile)
-    test_mmq_tile_variants_ragged(oxh, Q6K, rows, cols, n_vec)
+    check_mmq(Q6K, rows, cols, n_vec)
 
 
 
@@ -504,8 +510,8 @@ def test_mmq_with_a_tile_s_columns_shared_between_workgroups(oxh, qt, rows, cols
 @pytest.mark.parametrize("qt", [13, 15, 16, 10, 8])
 @pytest.mark.parametrize("rows,cols,n_vec", [(300, 5120, 9), (1000, 4096, 7), (130, 14336, 33)])
 def test_batch_entry_point_over_few_rows_and_many_columns(oxh, qt, rows, cols, n_vec):
-    """oc_matvec_quantized_batch over shapes whose tiles share their columns between workgroups (seven
-    vectors or more of a K-quant; Q2_K and Q3_K from nine on, through their rewritten forms): padded
+    """oc_matvec_quantized_batch over shapes whose columns are shared between the waves of a workgroup (the first two) or
+    between workgroups (seven vectors or more of a K-quant; Q2_K and Q3_K from nine on, through their rewritten forms): padded
     strides, every output with the oracle's bits, nothing written between rows and out_stride."""
     assert mv.mmq_split_workspace(16 if qt in (10, 8) else qt, rows, cols, n_vec, rows) > 0
     rb = synth.row_bytes(qt, cols)

@@ -262,25 +262,30 @@ def test_layer_top1_and_all_experts(oxh):
 
 @pytest.mark.parametrize("qt_gu,qt_dn", [(Q4K, Q6K), (Q5K, Q4K), (Q6K, Q5K)])
 def test_layer_with_prefill_sized_token_counts(oxh, qt_gu, qt_dn):
-    """150 pairs per expert on average: the expert launches take the 128-row x 64-token tile and walk
-    three token tiles per expert, the popular expert more."""
+    """150 pairs per expert on average and too few rows for the 144-token tiles: the expert launches take the 128-row x
+    64-token one, three token tiles per expert, the popular expert more."""
+    if mv.device_info()["n_cu"] == 256:
+        assert mv.experts_tile(qt_gu, 2, 4, 768, 600) == mv.experts_tile(qt_dn, 1, 4, 512, 600) == (128, 64)
     check_layer(qt_gu, qt_dn, 4, 2, 512, 768, 300, seed=21, sample=lambda n, offsets: sorted(
         set(int(v) for v in offsets[:-1] if v < n) | set(int(v) - 1 for v in offsets[1:] if v > 0) |
         set(range(0, n, 37))))
 
 
-@pytest.mark.parametrize("qt_gu,qt_dn,n_exp,k,hidden,ffn,n_tok", [
-    (Q4K, Q4K, 8, 2, 256, 3584, 560),       # 256 x 144 tiles: 14 x 2 of each expert's 140 tokens and their second tiles
-    (Q4K, Q6K, 8, 2, 256, 2048, 577),    # 128 x 144: one round of them
-    (Q5K, Q4K, 8, 2, 256, 3584, 300),       # 128 x 144, Q5_K, 75 tokens each
-    (Q6K, Q5K, 8, 2, 256, 3584, 581),       # 128 x 144, Q6_K, ragged counts above 144
-    (Q4K, Q5K, 8, 2, 3584, 512, 130),       # 128 x 64 tiles: experts below and just above 32, one with more than 64
-    (Q6K, Q6K, 16, 1, 1792, 512, 400),         # 128 x 64, Q6_K
+@pytest.mark.parametrize("qt_gu,qt_dn,n_exp,k,hidden,ffn,n_tok,tiles", [
+    (Q4K, Q4K, 8, 2, 256, 3584, 560, ((256, 144), (128, 64))),  # 14 x 2 of each expert's 140 tokens and their second tiles
+    (Q4K, Q6K, 8, 2, 256, 2048, 577, ((128, 144), (128, 64))),  # one round of them
+    (Q5K, Q4K, 8, 2, 256, 3584, 300, ((128, 144), (128, 64))),  # Q5_K, 75 tokens each
+    (Q6K, Q5K, 8, 2, 256, 3584, 581, ((128, 144), (128, 64))),  # Q6_K, ragged counts above 144
+    (Q4K, Q5K, 8, 2, 3584, 512, 130, ((64, 16), (128, 64))),    # experts below and just above 32, one with more than 64
+    (Q6K, Q6K, 16, 1, 1792, 512, 400, ((64, 16), (128, 64))),
 ])
-def test_layer_on_the_tiles_for_many_tokens(oxh, qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok):
+def test_layer_on_the_tiles_for_many_tokens(oxh, qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok, tiles):
     """The kernels that deal an expert's 16-token chunks evenly to its tiles: every tile size of every type, with
     counts that leave tiles of any number of chunks and a last chunk of any number of tokens, an expert without a
     token and a popular one with several tiles.  Pairs at both ends of every expert's run and of its chunks."""
+    if mv.device_info()["n_cu"] == 256:
+        pairs = n_tok * k
+        assert (mv.experts_tile(qt_gu, 2, n_exp, ffn, pairs), mv.experts_tile(qt_dn, 1, n_exp, hidden, pairs)) == tiles
     check_layer(qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok, seed=41 + n_tok, sample=lambda n, offsets: sorted(
         set(int(v) for v in offsets[:-1] if v < n) | set(int(v) - 1 for v in offsets[1:] if v > 0) |
         set(int(offsets[0]) + 16 * i for i in range(n // 16) if int(offsets[0]) + 16 * i < n) | set(range(0, n, 61))))
