@@ -33,7 +33,7 @@ def _run(cmd):
     return proc.stdout
 
 
-HIP_UNITS = ("oxh_kernels", "oxh_plan", "oxh_experts", "oxh_mmq6", "oxh_batch")
+HIP_UNITS = ("oxh_kernels", "oxh_plan", "oxh_experts", "oxh_mmq6", "oxh_mmq32", "oxh_batch")
 
 
 def exported_names():

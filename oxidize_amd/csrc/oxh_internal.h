@@ -54,6 +54,14 @@ void oxh_internal_experts_long_tile(uint32_t file_type, size_t n_mat, size_t n_e
 int oxh_internal_mmq6_init(void);
 int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
                              float *d_out, size_t out_stride, void *stream);
+/* The 32-value formats under a batch, in tiles of 64 or 128 rows x 64 tokens (oxh_mmq32.hip); init and launch return a
+ * hipError_t.  leg: 0 Q8_0, 1 Q4_0, 2 Q4_1, 3 Q5_0, 4 Q5_1, 5 AL5_XS; `fits`: whether the grid holds the launch's tiles,
+ * `tile`: their rows and tokens.  Arguments checked by the caller. */
+int oxh_internal_mmq32_init(void);
+int oxh_internal_mmq32_fits(size_t rows, size_t n_vec);
+void oxh_internal_mmq32_tile(size_t rows, size_t n_vec, size_t cus, uint32_t tile[2]);
+int oxh_internal_mmq32(int leg, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
+                       size_t out_stride, size_t cus, void *stream);
 /* K-quant matrices under at most 64 activations, a 16-row group to a workgroup (oxh_batch.hip); init and launch
  * return a hipError_t, `takes` whether a launch of these sizes belongs there (split: and could run as tiles that share
  * their columns through a workspace instead), `waves` the waves of its workgroups.

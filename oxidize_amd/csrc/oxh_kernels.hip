@@ -918,12 +918,6 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 3>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 4>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mfma_q8_0_segments<4, 5>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<0>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<1>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<2>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<3>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<4>)) != hipSuccess) return e;
-    if ((e = raise_lds_ceiling(k_mmq_q80<5>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q6_k_segments<1, 1, 4, 2>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q6_k_split<2>)) != hipSuccess) return e;
     if ((e = raise_lds_ceiling(k_mmq_q6_k_split<2, true>)) != hipSuccess) return e;
@@ -938,6 +932,7 @@ static hipError_t raise_all_lds_ceilings(void)
     if ((e = raise_lds_ceiling(k_mmq_q45_k_experts<8, false, 3>)) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_experts_init()) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_mmq6_init()) != hipSuccess) return e;
+    if ((e = (hipError_t)oxh_internal_mmq32_init()) != hipSuccess) return e;
     if ((e = (hipError_t)oxh_internal_batch_init()) != hipSuccess) return e;
     return hipSuccess;
 }
@@ -2282,8 +2277,8 @@ extern "C" int oxh_mmq_tile(uint32_t qtype, size_t rows, size_t n_vec, size_t n_
                             uint32_t *tile_tokens)
 {
     if (mmq80_leg(canon_qtype(qtype)) >= 0 && rows && n_vec && n_cu) {       /* one tile for these */
-        if (tile_rows) *tile_rows = MQT_WAVES * 16u;
-        if (tile_tokens) *tile_tokens = MQT_TOK;
+        if (tile_rows) *tile_rows = 128u;
+        if (tile_tokens) *tile_tokens = 64u;
         return OXH_OK;
     }
     const bool one_chunk = qtype == OXH_Q6_K || is_q5k(qtype) || qtype == OXH_Q2_K_WIDE;
@@ -2403,8 +2398,7 @@ extern "C" int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, si
     out[3] = 0;
     if (mmq80_leg(canon_qtype(qtype)) >= 0 && oxh_act_kind(qtype, cols) == 1) {
         out[0] = MMQ_TILES;
-        out[1] = MQT_WAVES * 16u;
-        out[2] = MQT_TOK;
+        oxh_internal_mmq32_tile(rows, n_vec, n_cu, out + 1);
         return OXH_OK;
     }
     const bool wide2 = qtype == OXH_Q2_K_WIDE;
@@ -2522,25 +2516,9 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
             snprintf(g_err, sizeof g_err, "oxh_mmq: rows of qtype %u with cols %zu are shorter than 16 bytes", qtype, cols);
             return OXH_DECLINED;
         }
-        const uint32_t n_rt = (uint32_t)((rows + MQT_WAVES * 16u - 1u) / (MQT_WAVES * 16u));
-        const uint32_t n_tt = (uint32_t)((n_vec + MQT_TOK - 1u) / MQT_TOK);
-        const uint64_t wgs = (uint64_t)((n_rt + 7u) / 8u) * 8u * n_tt;
-        if (wgs > 0x7FFFFFFFull) return arg_fail("oxh_mmq: too many tiles");
-        hipStream_t st = pick_stream(stream);
-#define OXH_MQT(LEG) hipLaunchKernelGGL((k_mmq_q80<LEG>), dim3((uint32_t)wgs), dim3(MQT_WAVES * 64u),          \
-                                        MqtGeom<LEG>::LDS_BYTES, st, (const uint8_t *)d_w, (uint32_t)rows,     \
-                                        (uint32_t)blocks32, (const uint8_t *)d_acts, (uint32_t)n_vec, d_out,   \
-                                        out_stride, n_rt, n_tt)
-        switch (leg) {
-        case 1:  OXH_MQT(1); break;
-        case 2:  OXH_MQT(2); break;
-        case 3:  OXH_MQT(3); break;
-        case 4:  OXH_MQT(4); break;
-        case 5:  OXH_MQT(5); break;
-        default: OXH_MQT(0); break;
-        }
-#undef OXH_MQT
-        HIP_TRY(hipGetLastError());
+        if (!oxh_internal_mmq32_fits(rows, n_vec)) return arg_fail("oxh_mmq: too many tiles");
+        HIP_TRY((hipError_t)oxh_internal_mmq32(leg, d_w, rows, blocks32, d_acts, n_vec, d_out, out_stride,
+                                               (size_t)(g_n_cu > 0 ? g_n_cu : 256), pick_stream(stream)));
         return OXH_OK;
     }
     const bool wide2 = qtype == OXH_Q2_K_WIDE;

@@ -1,0 +1,361 @@
+/* oxh_mmq32.hip — the prefill matmul of the six 32-value formats (Q8_0, Q4_0, Q4_1, Q5_0, Q5_1, AL5_XS).
+ *
+ * Arithmetic.  Per (row, token, block) the reference adds (dw*dq)*(float)isum, for the _1 formats plus
+ * (mw*dq)*(float)qsum, block after block (oxk.c:88-241).  A block is the K of one v_mfma_i32_16x16x32_i8; the
+ * float step is the reference's, in its order, so every result has the single-vector dot's bits.  Codes with an
+ * offset are staged as the signed values code - offset, so four formats share Q8_0's step exactly.
+ *
+ * What bounds it.  The float step: four vector instructions per result and block (seven for the _1 formats) beside a
+ * 256th of an MFMA, 64 cycles of a SIMD's issue port per 16 x 16 tile against the MFMA's 16 (4096 x 4096 x 512: some
+ * 30 us of it).  So everything else has to stay off that port: a block is fetched and taken apart ONCE per
+ * workgroup, by a lane that owns it (eight lanes along a row's consecutive blocks, so that a wave's load touches some
+ * 24 cache lines and not 64), and goes to LDS as MFMA operands, int8 values and f32 scales; the inner loop issues
+ * MFMAs, the float step and nothing else but LDS reads, eleven of 16 bytes per eight tiles.  Of a wave's 310 vector
+ * instructions per step of eight blocks 256 are the float step.
+ *
+ * Shape.  A wave computes 16 rows x 32 tokens; eight waves, 64 rows x 64 tokens, to a workgroup and two workgroups to
+ * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues a vector
+ * instruction every eight cycles at best.  Steps of eight blocks, two stages in LDS, one
+ * barrier per step; the next step's blocks go to LDS in the middle of a step and the ones after it are requested
+ * then.  Q8_0 4096 x 4096 x 512 takes 41 us (128 x 64 tiles whose waves kept raw blocks in regions of their own, one
+ * workgroup to a CU: 69; 128 x 64 on eight waves of 32 x 32: 42.5, and 162 us at 14336 rows where this takes 136). */
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "oxhip.h"
+#include "oxh_internal.h"
+#include "oxh_device.inc"
+#include "blocks32.inc"
+#include "mmq_tiles.inc"
+
+template <int LEG, bool WIDE> struct Mmq32Geom {
+    static constexpr bool HAS_M = LEG == 2 || LEG == 4;
+    static constexpr uint32_t BB = LEG == 0 ? 34u : LegGeom<LEG ? LEG : 1>::BYTES;
+    static constexpr uint32_t RW = WIDE ? 8 : 4, TW = 2, RC = 1, TC = 2;   /* waves, 16-chunks of a wave */
+    static constexpr uint32_t KP = 4, KB = 2u * KP;    /* pairs of blocks, blocks to a step */
+    static constexpr uint32_t ROWS = RW * RC * 16u, TOK = TW * TC * 16u, THREADS = RW * TW * 64u;
+    /* A stage.  Values: [pair][row or token][16-byte slot]: slot s of row r holds values 8k .. 8k+7 of the pair's
+     * two blocks, k = s ^ mmq32_swizzle(r); a pair is skewed by a slot row.  Scales of rows [block][row], of tokens [four blocks][token][4]. */
+    static constexpr uint32_t W_PAIR = ROWS * 64u, A_PAIR = TOK * 64u;
+    /* the skew spreads the eight blocks' scales over the banks; with the minimums too there is no room for it */
+    static constexpr uint32_t D_PITCH = ROWS + (HAS_M ? 0u : 8u);
+    static constexpr uint32_t A_OFF = KP * W_PAIR;
+    static constexpr uint32_t DW_OFF = A_OFF + KP * A_PAIR;
+    static constexpr uint32_t DQ_OFF = DW_OFF + KB * D_PITCH * 4u;
+    static constexpr uint32_t MW_OFF = DQ_OFF + KB * TOK * 4u;
+    static constexpr uint32_t QS_OFF = MW_OFF + (HAS_M ? KB * D_PITCH * 4u : 0u);
+    static constexpr uint32_t STAGE_BYTES = QS_OFF + (HAS_M ? KB * TOK * 4u : 0u);
+    static constexpr uint32_t LDS_BYTES = 2u * STAGE_BYTES;
+    static constexpr uint32_t W_UNITS = ROWS * KB / THREADS, A_UNITS = (TOK * KB + THREADS - 1u) / THREADS;      /* blocks a thread stages */
+    static_assert(W_UNITS * THREADS == ROWS * KB && TOK * KB % (THREADS < TOK * KB ? THREADS : TOK * KB) == 0u && KP % 2u == 0u, "staging");
+    static_assert((WIDE ? 1u : 2u) * LDS_BYTES <= 160u * 1024u, "workgroups to a CU");
+};
+
+/* Rows lie 64 bytes apart: eight aligned rows' slots of one k fall on the eight 16-byte pieces of 128 bytes, sixteen
+ * rows' on the sixteen of 256. */
+__device__ __forceinline__ uint32_t mmq32_swizzle(uint32_t row) { return ((row >> 1) & 3u) ^ ((row >> 3) & 1u); }
+
+template <int LEG> struct Mmq32Raw { LegRegs r; };
+template <> struct Mmq32Raw<0> { Q80Regs r; };
+
+template <int LEG, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 1024 : 512, 4) void
+k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t *__restrict__ acts, uint32_t nv,
+         float *__restrict__ out, size_t out_stride, uint32_t n_row_tiles, uint32_t n_tok_tiles)
+{
+    typedef Mmq32Geom<LEG, WIDE> G;
+    constexpr bool HAS_M = G::HAS_M;
+    constexpr int RC = (int)G::RC, TC = (int)G::TC, KP = (int)G::KP;
+    extern __shared__ __attribute__((aligned(16))) uint8_t mmq_lds[];
+    /* workgroups whose numbers are equal modulo 8 share an XCD and its L2: the token tiles of a row tile get such
+     * numbers, so a row tile's weights come from HBM once */
+    const uint32_t place = blockIdx.x >> 3;
+    const uint32_t row_tile = (place / n_tok_tiles) * 8u + (blockIdx.x & 7u), tok_tile = place % n_tok_tiles;
+    if (row_tile >= n_row_tiles) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r16 = lane & 15u, kq = lane >> 4;
+    const uint32_t row_first = row_tile * G::ROWS, tok_first = tok_tile * G::TOK;
+    const uint32_t rows_here = min(rows - row_first, G::ROWS), toks_here = min(nv - tok_first, G::TOK);
+
+    /* staging: this thread's blocks are block tid % KB of a step, rows (tokens) tid / KB and further ones */
+    const uint32_t s_blk = tid % G::KB, s_row = tid / G::KB;
+    const uint8_t *w_at[G::W_UNITS], *a_at[G::A_UNITS];
+    uint32_t w_dst[G::W_UNITS], a_dst[G::A_UNITS];
+#pragma unroll
+    for (uint32_t i = 0; i < G::W_UNITS; i++) {
+        const uint32_t r = s_row + i * (G::THREADS / G::KB);
+        w_at[i] = w + (size_t)(row_first + min(r, rows_here - 1u)) * B * G::BB;
+        w_dst[i] = (s_blk >> 1) * G::W_PAIR + r * 64u + 16u * (mmq32_swizzle(r) ^ ((s_blk >> 1) & 3u)) + 8u * (s_blk & 1u);      /* ^ 16 k */
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < G::A_UNITS; i++) {
+        const uint32_t t = s_row + i * (G::THREADS / G::KB);
+        a_at[i] = acts + (size_t)(tok_first + min(t, toks_here - 1u)) * B * 34u;
+        a_dst[i] = G::A_OFF + (s_blk >> 1) * G::A_PAIR + t * 64u + 16u * (mmq32_swizzle(t) ^ ((s_blk >> 1) & 3u)) + 8u * (s_blk & 1u);
+    }
+    Mmq32Raw<LEG> w_raw[G::W_UNITS];
+    Q80Regs a_raw[G::A_UNITS];
+    auto load = [&](uint32_t step) {
+        const uint32_t b = min(step * G::KB + s_blk, B - 1u);
+#pragma unroll
+        for (uint32_t i = 0; i < G::W_UNITS; i++) {
+            if constexpr (LEG == 0) q80_load_at(w_raw[i].r, w_at[i] + (size_t)b * G::BB);
+            else leg_load_at<LEG>(w_raw[i].r, w_at[i] + (size_t)b * G::BB);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < G::A_UNITS; i++) q80_load_at(a_raw[i], a_at[i] + (size_t)b * 34u);
+    };
+    /* blocks past the row's end are staged as zeros with zero scales: their term is +0, which changes nothing (a
+     * sum that starts at +0 never becomes -0) */
+    auto put = [&](uint8_t *st, uint32_t dst, const uint32_t q[8], bool live) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4u; k++)
+            *reinterpret_cast<uint2 *>(st + (dst ^ (16u * k))) = live ? make_uint2(q[2 * k], q[2 * k + 1]) : make_uint2(0u, 0u);
+    };
+    auto store = [&](uint32_t step) {
+        uint8_t *st = mmq_lds + (step & 1u) * G::STAGE_BYTES;
+        const bool live = step * G::KB + s_blk < B;
+#pragma unroll
+        for (uint32_t i = 0; i < G::W_UNITS; i++) {
+            const uint32_t r = s_row + i * (G::THREADS / G::KB);
+            uint32_t q[8], d;
+            float m = 0.0f;
+            if constexpr (LEG == 0) {
+                d = q80_unpack(w_raw[i].r, q);
+            } else {
+                uint32_t lo[4], hi[4];
+                d = leg_unpack<LEG>(w_raw[i].r, lo, hi);
+                if (HAS_M) m = half_to_float_hw(w_raw[i].r.hdr >> 16);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    /* code - offset as a signed byte: codes stay below 2 * offset, so no carry leaves a byte */
+                    constexpr uint32_t UP = 0x01010101u * (128u - (uint32_t)LegGeom<LEG>::OFFSET);
+                    q[k] = HAS_M ? lo[k] : (lo[k] + UP) ^ 0x80808080u;
+                    q[4 + k] = HAS_M ? hi[k] : (hi[k] + UP) ^ 0x80808080u;
+                }
+            }
+            put(st, w_dst[i], q, live);
+            reinterpret_cast<float *>(st + G::DW_OFF)[s_blk * G::D_PITCH + r] = live ? half_to_float_hw(d) : 0.0f;
+            if (HAS_M) reinterpret_cast<float *>(st + G::MW_OFF)[s_blk * G::D_PITCH + r] = live ? m : 0.0f;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < G::A_UNITS; i++) {
+            const uint32_t t = s_row + i * (G::THREADS / G::KB);
+            if (WIDE && wave >= G::TOK * G::KB / 64u) break;        /* more threads than token blocks */
+            uint32_t q[8];
+            const uint32_t d = q80_unpack(a_raw[i], q);
+            put(st, a_dst[i], q, live);
+            const uint32_t at = ((s_blk >> 2) * G::TOK + t) * 4u + (s_blk & 3u);
+            reinterpret_cast<float *>(st + G::DQ_OFF)[at] = live ? half_to_float_hw(d) : 0.0f;
+            if (HAS_M) {
+                int qs = 0;
+#pragma unroll
+                for (int k = 0; k < 8; k++) qs = dot4(0x01010101u, q[k], qs);
+                reinterpret_cast<float *>(st + G::QS_OFF)[at] = live ? (float)qs : 0.0f;
+            }
+        }
+    };
+
+    /* a wave's operands of one pair of blocks */
+    struct Frag {
+        u32x4 w[RC], a[TC];
+        v4f dw[2][RC];
+    };
+    const uint32_t rw = wave % G::RW, tw = wave / G::RW;
+    const uint32_t w_row = rw * (16u * G::RC) + r16, a_row = tw * (16u * G::TC) + r16;
+    const uint32_t swz = 16u * (kq ^ mmq32_swizzle(r16));
+    const uint32_t w_rd = w_row * 64u + swz, a_rd = G::A_OFF + a_row * 64u + swz;
+    const uint32_t dw_rd = G::DW_OFF + (rw * (16u * G::RC) + 4u * kq) * 4u;
+    const uint32_t dq_rd = G::DQ_OFF + a_row * 16u;
+    auto fetch = [&](const uint8_t *st, int p) -> Frag {
+        Frag f;
+#pragma unroll
+        for (int rc = 0; rc < RC; rc++) f.w[rc] = *reinterpret_cast<const u32x4 *>(st + (w_rd ^ (16u * ((uint32_t)p & 3u))) + (uint32_t)p * G::W_PAIR + 1024u * (uint32_t)rc);
+#pragma unroll
+        for (int tc = 0; tc < TC; tc++) f.a[tc] = *reinterpret_cast<const u32x4 *>(st + (a_rd ^ (16u * ((uint32_t)p & 3u))) + (uint32_t)p * G::A_PAIR + 1024u * (uint32_t)tc);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int rc = 0; rc < RC; rc++) {
+                const uint32_t at = ((2u * (uint32_t)p + (uint32_t)j) * G::D_PITCH + 16u * (uint32_t)rc) * 4u;
+                f.dw[j][rc] = *reinterpret_cast<const v4f *>(st + dw_rd + at);
+            }
+        return f;
+    };
+    v4f acc[RC][TC];
+#pragma unroll
+    for (int rc = 0; rc < RC; rc++)
+#pragma unroll
+        for (int tc = 0; tc < TC; tc++) acc[rc][tc] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
+    const v4i zero = { 0, 0, 0, 0 };
+    auto block_of = [](const u32x4 &v, int j) -> long {
+        return (long)(((unsigned long)v[2 * j + 1] << 32) | (unsigned long)v[2 * j]);
+    };
+    auto compute = [&](const Frag &f, const uint8_t *st, const v4f dq[TC], const v4f qs[TC], int p) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int bq = 2 * (p & 1) + j;
+            v4i isum[RC][TC];
+            v4f mw[RC];
+#pragma unroll
+            for (int rc = 0; rc < RC; rc++) {
+#pragma unroll
+                for (int tc = 0; tc < TC; tc++)
+                    /* weights first: result i of a lane is row 4 kq + i against token r16 */
+                    isum[rc][tc] = __builtin_amdgcn_mfma_i32_16x16x32_i8(block_of(f.w[rc], j), block_of(f.a[tc], j), zero, 0, 0, 0);
+                if (HAS_M)
+                    mw[rc] = *reinterpret_cast<const v4f *>(st + dw_rd + (G::MW_OFF - G::DW_OFF) +
+                                                            ((2u * (uint32_t)p + (uint32_t)j) * G::D_PITCH + 16u * (uint32_t)rc) * 4u);
+            }
+#pragma unroll
+            for (int rc = 0; rc < RC; rc++)
+#pragma unroll
+                for (int tc = 0; tc < TC; tc++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float t = f.dw[j][rc][i] * dq[tc][bq];
+                        const float up = t * (float)isum[rc][tc][i];
+                        if (HAS_M) {
+                            const float tm = mw[rc][i] * dq[tc][bq];
+                            const float off = tm * qs[tc][bq];
+                            acc[rc][tc][i] += up + off;
+                        } else {
+                            acc[rc][tc][i] += up;
+                        }
+                    }
+        }
+    };
+
+    const uint32_t n_steps = (B + G::KB - 1u) / G::KB;
+    load(0u);
+    store(0u);
+    load(1u < n_steps ? 1u : 0u);
+    __syncthreads();
+    for (uint32_t s = 0; s < n_steps; s++) {
+        const uint8_t *st = mmq_lds + (s & 1u) * G::STAGE_BYTES;
+        const uint32_t nb = min(B - s * G::KB, G::KB);
+        Frag cur = fetch(st, 0);
+#pragma unroll
+        for (int q = 0; q < KP / 2; q++) {
+            if (4u * (uint32_t)q < nb) {
+                v4f dq[TC], qs[TC];
+#pragma unroll
+                for (int tc = 0; tc < TC; tc++) {
+                    dq[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
+                    if (HAS_M) qs[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (G::QS_OFF - G::DQ_OFF) + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
+                }
+                const Frag nxt = fetch(st, 2 * q + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(cur, st, dq, qs, 2 * q);
+                if (q + 1 < KP / 2) cur = fetch(st, 2 * q + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                compute(nxt, st, dq, qs, 2 * q + 1);
+            }
+            if (q == 0 && s + 1u < n_steps) {
+                store(s + 1u);
+                load(min(s + 2u, n_steps - 1u));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+    }
+
+    const bool wide = (out_stride & 3u) == 0u && ((uintptr_t)out & 15u) == 0u;
+#pragma unroll
+    for (int tc = 0; tc < TC; tc++) {
+        const uint32_t tok = a_row + 16u * (uint32_t)tc;
+        if (tok >= toks_here) continue;
+        float *o = out + (size_t)(tok_first + tok) * out_stride + row_first;
+#pragma unroll
+        for (int rc = 0; rc < RC; rc++) {
+            const uint32_t r = rw * (16u * G::RC) + 16u * (uint32_t)rc + 4u * kq;
+            if (wide && r + 4u <= rows_here) {
+                *reinterpret_cast<v4f *>(o + r) = acc[rc][tc];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (r + (uint32_t)i < rows_here) o[r + (uint32_t)i] = acc[rc][tc][i];
+            }
+        }
+    }
+}
+
+template <int LEG> static hipError_t mmq32_raise(void)
+{
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_mmq_32<LEG, false>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_mmq_32<LEG, true>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return e;
+}
+
+extern "C" int oxh_internal_mmq32_init(void)
+{
+    hipError_t e;
+    if ((e = mmq32_raise<0>()) != hipSuccess || (e = mmq32_raise<1>()) != hipSuccess || (e = mmq32_raise<2>()) != hipSuccess ||
+        (e = mmq32_raise<3>()) != hipSuccess || (e = mmq32_raise<4>()) != hipSuccess || (e = mmq32_raise<5>()) != hipSuccess)
+        return (int)e;
+    return (int)hipSuccess;
+}
+
+/* Workgroups: row tiles in runs of eight (one to an XCD) by token tiles. */
+static uint64_t mmq32_tiles(size_t rows, size_t n_vec, uint32_t tile_rows)
+{
+    const uint64_t n_rt = (rows + tile_rows - 1u) / tile_rows, n_tt = (n_vec + 63u) / 64u;
+    return (n_rt + 7u) / 8u * 8u * n_tt;
+}
+
+/* Which tile.  64 x 64, two to a CU, unless there are more of them than CUs and one round of 128 x 64 tiles, a CU's
+ * worth of waves each, holds the launch: then every CU gets the same and the smaller tiles' third more staging shows
+ * (us, 64 / 128 rows: 4096 x 4096 x 512 41.7 / 40.6, 3072 x 2048 x 512 22.7 / 22.1, Q5_1 31.1 / 29.9).  With fewer tiles
+ * a small one alone on its CU is done sooner (2048 x 2048 x 333 14.6 / 21.1), with more their rounds are finer (5120 x
+ * 2048 x 512 33.0 / 41.2, 8192 rows 43.0 / 43.6, 14336 x 4096 x 512 136 / 149). */
+static bool mmq32_wide(size_t rows, size_t n_vec, size_t cus)
+{
+    const uint64_t n_tt = (n_vec + 63u) / 64u;
+    return (rows + 63u) / 64u * n_tt > cus && (rows + 127u) / 128u * n_tt <= cus;
+}
+
+/* see oxh_internal.h */
+extern "C" void oxh_internal_mmq32_tile(size_t rows, size_t n_vec, size_t cus, uint32_t tile[2])
+{
+    tile[0] = mmq32_wide(rows, n_vec, cus) ? Mmq32Geom<0, true>::ROWS : Mmq32Geom<0, false>::ROWS;
+    tile[1] = Mmq32Geom<0, false>::TOK;
+}
+
+extern "C" int oxh_internal_mmq32_fits(size_t rows, size_t n_vec)
+{
+    return mmq32_tiles(rows, n_vec, Mmq32Geom<0, false>::ROWS) <= 0x7FFFFFFFull;
+}
+
+template <int LEG, bool WIDE>
+static void mmq32_launch(const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
+                         size_t out_stride, hipStream_t st)
+{
+    typedef Mmq32Geom<LEG, WIDE> G;
+    const uint32_t n_rt = (uint32_t)((rows + G::ROWS - 1u) / G::ROWS), n_tt = (uint32_t)((n_vec + G::TOK - 1u) / G::TOK);
+    hipLaunchKernelGGL((k_mmq_32<LEG, WIDE>), dim3((uint32_t)mmq32_tiles(rows, n_vec, G::ROWS)), dim3(G::THREADS), G::LDS_BYTES,
+                       st, (const uint8_t *)d_w, (uint32_t)rows, (uint32_t)blocks, (const uint8_t *)d_acts, (uint32_t)n_vec, d_out,
+                       out_stride, n_rt, n_tt);
+}
+
+/* see oxh_internal.h */
+extern "C" int oxh_internal_mmq32(int leg, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
+                                  float *d_out, size_t out_stride, size_t cus, void *stream)
+{
+    hipStream_t st = (hipStream_t)stream;
+    const bool wide = mmq32_wide(rows, n_vec, cus);
+#define OXH_M32(LEG) (wide ? mmq32_launch<LEG, true> : mmq32_launch<LEG, false>)(d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, st)
+    switch (leg) {
+    case 1:  OXH_M32(1); break;
+    case 2:  OXH_M32(2); break;
+    case 3:  OXH_M32(3); break;
+    case 4:  OXH_M32(4); break;
+    case 5:  OXH_M32(5); break;
+    default: OXH_M32(0); break;
+    }
+#undef OXH_M32
+    return (int)hipGetLastError();
+}

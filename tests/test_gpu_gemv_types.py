@@ -492,6 +492,35 @@ def test_token_tiled_kernel_of_the_32_value_formats(oxh, qtype, rows, cols, n_ve
         assert np.array_equal(bits(outs[v, :rows]), bits(want)), v
 
 
+@pytest.mark.parametrize("qtype,rows,cols,n_vec,tile", [
+    (Q80, 2049, 288, 510, (128, 64)),       # 33 x 8 tiles of 64 rows, 17 x 8 of 128: one round of these; 9 blocks, one row over
+    (6, 2150, 544, 449, (128, 64)),         # Q5_1: minimums and sums, sixteen waves; 17 blocks
+    (18, 2112, 96, 512, (128, 64)),         # AL5_XS, 3 blocks: rows of 42 bytes
+    (Q80, 2048, 288, 512, (64, 64)),        # 256 tiles of 64 rows: one to a CU
+    (5, 4161, 256, 513, (64, 64)),          # Q5_0: 33 x 9 tiles of 128 rows would be a second round
+    (4, 63, 224, 127, (64, 64)),            # Q4_1, 7 blocks: half a step and its odd half
+])
+def test_both_tiles_of_the_32_value_formats_under_a_prompt(oxh, qtype, rows, cols, n_vec, tile):
+    """oxh_mmq on tiles of 64 and of 128 rows: bits of the single-vector dots at the tiles' edges, stores of four
+    results at a time (output rows a multiple of four floats apart) and nothing written beside the outputs."""
+    if mv.device_info()["n_cu"] == 256:
+        assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile
+    w = synth.weights(qtype, rows, cols, seed=89, stream=rows + cols)
+    xs = synth.normal(n_vec * cols, seed=89, stream=n_vec).reshape(n_vec, cols)
+    d_w, d_x = mv.DeviceBuffer.from_host(w), mv.DeviceBuffer.from_host(xs)
+    d_a = mv.DeviceBuffer(n_vec * mv.act_bytes(qtype, cols))
+    mv.quantize(qtype, d_x.ptr, cols, n_vec, cols, d_a.ptr)
+    stride = (rows + 7) & ~3
+    d_out = mv.DeviceBuffer.from_host(np.full((n_vec, stride), -7.25, np.float32))
+    mv.mmq(qtype, d_w.ptr, rows, cols, d_a.ptr, n_vec, d_out.ptr, stride)
+    mv.sync()
+    outs = d_out.download(np.float32, n_vec * stride).reshape(n_vec, stride)
+    assert np.all(outs[:, rows:] == -7.25)
+    for v in sorted({0, 15, 16, 31, 32, 63, 64, 65, n_vec // 2, n_vec - 2, n_vec - 1}):
+        want, _ = oracle_matvec(qtype, w, rows, cols, np.ascontiguousarray(xs[v]))
+        assert np.array_equal(bits(outs[v, :rows]), bits(want)), v
+
+
 @pytest.mark.parametrize("qtype,rows,cols,n_vec", [(Q4K, 40, 512, 3), (Q80, 33, 256, 1), (Q6K, 70, 256, 8)])
 def test_a_call_with_more_than_32_segments_runs_as_launches_of_32(oxh, qtype, rows, cols, n_vec):
     """Seventy segments, each its own matrix and run of activations, in one call: the bits of the same
