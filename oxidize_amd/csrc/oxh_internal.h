@@ -53,7 +53,9 @@ void oxh_internal_experts_long_tile(uint32_t file_type, size_t n_mat, size_t n_e
  * (oxh_mmq6.hip); both return a hipError_t.  Arguments checked by the caller. */
 int oxh_internal_mmq6_init(void);
 int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec,
-                             float *d_out, size_t out_stride, void *stream);
+                             float *d_out, size_t out_stride, size_t cus, void *stream);
+/* the token tiles such a launch is cut into; host arithmetic */
+size_t oxh_internal_mmq6_tok_tiles(size_t rows, size_t n_vec, size_t cus);
 /* The 32-value formats under a batch, in tiles of 64 or 128 rows x 64 tokens (oxh_mmq32.hip); init and launch return a
  * hipError_t.  leg: 0 Q8_0, 1 Q4_0, 2 Q4_1, 3 Q5_0, 4 Q5_1, 5 AL5_XS; `fits`: whether the grid holds the launch's tiles,
  * `tile`: their rows and tokens.  Arguments checked by the caller. */

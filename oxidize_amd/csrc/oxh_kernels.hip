@@ -2232,6 +2232,8 @@ static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
  * activations 8.2 us against 7.5.
  * Widened Q2_K builds its operands in fewer instructions: 0.64 to 0.86 and 1.17; 1.40, 2.99; 0.59, 0.78, 1.0, then
  * 1.5 and 0.30 each.
+ * (The first kind has become 3 to 25 % faster since, most with few chunks, now that its waves no longer wait for memory
+ * every super-block and a launch of one round is cut into more tiles; the lines are where they were before.)
  * Where two tiles are within some 8 % the weights' way in decides, and the order for weights that come from memory was
  * taken (Q2_K 7433 x 22528 under 78 activations: 136 us on 64 x 128 tiles against 124 on 64 x 32 ones, 10112 x 1792
  * under 79, which stays in a cache, 13.1 against 15.6; Q6_K 7736 x 17664 under 42: 97 against 105). */
@@ -2543,7 +2545,8 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
         return OXH_OK;
     }
     if (route.kernel == MMQ_SHARED) {
-        const int e = oxh_internal_mmq6_shared(wide2, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride, pick_stream(stream));
+        const int e = oxh_internal_mmq6_shared(wide2, d_w, rows, blocks, d_acts, n_vec, d_out, out_stride,
+                                               (size_t)(g_n_cu > 0 ? g_n_cu : 256), pick_stream(stream));
         if (e) return hip_fail((hipError_t)e, "oxh_mmq");
         return OXH_OK;
     }

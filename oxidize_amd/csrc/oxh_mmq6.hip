@@ -39,11 +39,16 @@ struct Q6sGeom {
     static constexpr uint32_t LDS_BYTES = 2u * STAGE_BYTES;
 };
 
-/* an eighth of a block: 16 bytes of ql (two groups' low bits), the 16 bytes of qh that belong to them, the
- * two group scales, and the block's d */
+/* an eighth of a block: 16 bytes of ql (two groups' low bits), the 16 bytes of qh that belong to them, the eight bytes
+ * their two scales are in (Q2: all sixteen minima), and the dwords d (upper half) and, Q2, dmin (lower half) are in:
+ * dwords and more, because a byte or half word would be widened by an instruction that waits for its load */
+typedef uint32_t u32x4_2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2_2 __attribute__((ext_vector_type(2), aligned(2)));
 struct Q6sRaw {
-    U32x4u2 ql, qh;
-    uint32_t sc0, sc1, d, dmin;
+    u32x4 ql, qh;
+    u32x2 sc;
+    uint32_t d, dmin;
 };
 
 /* dword k of the planes of the group in the low (HIGH: high) nibbles */
@@ -106,9 +111,13 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
     const uint32_t grp = 8u * (u >> 2) + (u & 3u);
     const uint32_t w_off = min(b_row, rows_here - 1u) * (B * 210u);
     const uint32_t ql_off = w_off + 16u * u, qh_off = w_off + 128u + 32u * (u >> 2) + 16u * (u & 1u);
-    const uint32_t sc_off = w_off + 192u + (Q2 ? grp >> 1 : grp), sc_step = Q2 ? 2u : 4u;
+    const uint32_t sc_off = w_off + 192u + (Q2 ? 0u : 8u * (u >> 2));
+    /* where in those eight bytes: group grp and the one four on (Q2: nibbles) */
+    const uint32_t sc_bit = Q2 ? 4u * (grp & 7u) : 8u * (u & 3u);
     const uint32_t rot0 = ((u & 2u) - 4u) & 31u, rot1 = u & 2u;      /* bits 2h, 2h + 1 (2h + 4, 2h + 5) to 4, 5 */
-    const uint32_t pl_wr = G::LO_OFF + b_row * 256u + ((grp ^ (b_row & 15u)) * 16u);     /* ^ 64: four groups on */
+    /* group 8n + 4h + j of a row goes to slot (8h + 4n + j) ^ row: a row's eight threads then write eight different
+     * slots of 128 bytes */
+    const uint32_t pl_wr = G::LO_OFF + b_row * 256u + (((4u * (u >> 2) + (u & 3u)) ^ (b_row & 15u)) * 16u);  /* ^ 128: four groups on */
     const uint32_t a_d_off = min(tid & (G::TOK - 1u), toks_here - 1u) * act_stride;
 
     auto request = [&](uint32_t blk, uint32_t buf) {
@@ -119,42 +128,42 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
     auto load_raw = [&](uint32_t blk) -> Q6sRaw {
         const uint8_t *wb = w_base + (size_t)blk * 210u;
         Q6sRaw r;
-        r.ql = *reinterpret_cast<const U32x4u2 *>(wb + ql_off);
-        r.qh = *reinterpret_cast<const U32x4u2 *>(wb + qh_off);
-        r.sc0 = wb[sc_off];
-        r.sc1 = wb[sc_off + sc_step];
-        r.d = *reinterpret_cast<const uint16_t *>(wb + w_off + 208u);
-        r.dmin = Q2 ? *reinterpret_cast<const uint16_t *>(wb + w_off + 200u) : 0u;
+        r.ql = *reinterpret_cast<const u32x4_2 *>(wb + ql_off);
+        r.qh = *reinterpret_cast<const u32x4_2 *>(wb + qh_off);
+        r.sc = *reinterpret_cast<const u32x2_2 *>(wb + sc_off);
+        r.d = reinterpret_cast<const U32u2 *>(wb + w_off + 206u)->v;
+        r.dmin = Q2 ? reinterpret_cast<const U32u2 *>(wb + w_off + 200u)->v : 0u;
         return r;
     };
     auto load_dq = [&](uint32_t blk) -> uint32_t {
         return *reinterpret_cast<const uint32_t *>(a_base + (size_t)blk * 292u + a_d_off);
     };
-    /* a group's scale as the dword builder takes it */
-    auto scale_of = [&](uint32_t byte) -> uint32_t {
-        return Q2 ? ((byte >> (4u * (grp & 1u))) & 15u) * 0x01010101u : (uint32_t)(int)(int8_t)byte;
+    /* the two groups' scales (Q2: minima, spread over four bytes) as the dword builder takes them.  Q2: groups 8n + j and
+     * 8n + j + 4 are nibbles j and j + 4 of dword n */
+    auto scale_of = [&](const Q6sRaw &r, int second) -> uint32_t {
+        if (Q2) return (((u & 4u ? r.sc[1] : r.sc[0]) >> ((sc_bit + 16u * (uint32_t)second) & 31u)) & 15u) * 0x01010101u;
+        return (uint32_t)__builtin_amdgcn_sbfe((int)r.sc[second], sc_bit, 8u);
     };
     u32x4 p_lo[2], p_hi[2];
     auto build_dword = [&](const Q6sRaw &r, int k) {
-        const uint32_t ql[4] = { r.ql.x, r.ql.y, r.ql.z, r.ql.w }, qh[4] = { r.qh.x, r.qh.y, r.qh.z, r.qh.w };
         uint32_t lo, hi;
-        q6s_dword<Q2, false>(ql[k], qh[k], scale_of(r.sc0), rot0, lo, hi);
+        q6s_dword<Q2, false>(r.ql[k], r.qh[k], scale_of(r, 0), rot0, lo, hi);
         p_lo[0][k] = lo;
         p_hi[0][k] = hi;
-        q6s_dword<Q2, true>(ql[k], qh[k], scale_of(r.sc1), rot1, lo, hi);
+        q6s_dword<Q2, true>(r.ql[k], r.qh[k], scale_of(r, 1), rot1, lo, hi);
         p_lo[1][k] = lo;
         p_hi[1][k] = hi;
     };
-    auto store_planes = [&](const Q6sRaw &r, uint32_t dq, uint32_t buf) {
+    auto store_planes = [&](float d, float dmin, uint32_t dq, uint32_t buf) {
         uint8_t *st = mmq_lds + buf * G::STAGE_BYTES;
         *reinterpret_cast<u32x4 *>(st + pl_wr) = p_lo[0];
-        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 64u)) = p_lo[1];
+        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 128u)) = p_lo[1];
         *reinterpret_cast<u32x4 *>(st + pl_wr + (G::HI_OFF - G::LO_OFF)) = p_hi[0];
-        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 64u) + (G::HI_OFF - G::LO_OFF)) = p_hi[1];
+        *reinterpret_cast<u32x4 *>(st + (pl_wr ^ 128u) + (G::HI_OFF - G::LO_OFF)) = p_hi[1];
         /* the eight threads of a row, and the four of a token, store the same values: no branch in the loop */
         float *dw = reinterpret_cast<float *>(st + G::DW_OFF) + 2u * b_row;
-        dw[0] = half_to_float_hw(r.d);
-        if (Q2) dw[1] = half_to_float_hw(r.dmin);
+        dw[0] = d;
+        if (Q2) dw[1] = dmin;
         *reinterpret_cast<uint32_t *>(st + G::D_OFF + 4u * (tid & (G::TOK - 1u))) = dq;
     };
 
@@ -167,38 +176,48 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
     const uint32_t dw_rd = G::DW_OFF + ((wave & 3u) * 16u + r16) * 8u;
     const uint32_t dq_rd = G::D_OFF + 16u * kq + 64u * c_first;
 
-    /* the first super-block, and the raw blocks of the second */
+    constexpr int RAW_LOADS = Q2 ? 5 : 4;           /* vector loads of one load_raw() */
+    /* Two sets of raw blocks: while super-block b is computed one holds b + 1, complete, and is sent for b + 3 once its
+     * planes are built; the other holds b + 2, still on its way. */
+    Q6sRaw set0, set1;
     {
         const Q6sRaw r = load_raw(0);
         const uint32_t dq = load_dq(0);
         request(0, 0);
 #pragma unroll
         for (int k = 0; k < 4; k++) build_dword(r, k);
-        store_planes(r, dq, 0);
+        store_planes(half_to_float_hw(r.d >> 16), half_to_float_hw(r.dmin & 0xFFFFu), dq, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        set0 = load_raw(min(1u, B - 1u));
+        __builtin_amdgcn_sched_barrier(0);
+        set1 = load_raw(min(2u, B - 1u));
+        __builtin_amdgcn_sched_barrier(0);
+        /* the LDS-bound loads, which the compiler does not count, and set0: all but the last loads */
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(RAW_LOADS) : "memory");
+        q6s_barrier();
     }
-    Q6sRaw next = load_raw(min(1u, B - 1u));
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        /* the LDS-bound loads, which the compiler does not count */
-    q6s_barrier();
 
-    for (uint32_t b = 0; b < B; b++) {
+    auto step = [&](uint32_t b, Q6sRaw &next) {
         const uint32_t buf = b & 1u;
         const uint8_t *st = mmq_lds + buf * G::STAGE_BYTES;
+        /* `next` is complete since the last barrier's wait; said here, before this step's LDS-bound loads are issued,
+         * because the compiler would count those out of its own wait for it and so wait for them too */
+        asm volatile("" : "+v"(next.ql), "+v"(next.qh), "+v"(next.sc), "+v"(next.d), "+v"(next.dmin));
+        __builtin_amdgcn_sched_barrier(0);
         request(min(b + 1u, B - 1u), buf ^ 1u);
+        const uint32_t dq_next = load_dq(min(b + 1u, B - 1u));
         __builtin_amdgcn_sched_barrier(0);
         v4i dl[4], dh[4];
+        auto slot_of = [](int gp) -> uint32_t { return 2u * ((uint32_t)gp & 1u) + ((uint32_t)gp >> 1); };
 #pragma unroll
         for (int gp = 0; gp < 4; gp++) {
-            dl[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * (uint32_t)gp)));
-            dh[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * (uint32_t)gp)) + (G::HI_OFF - G::LO_OFF));
+            dl[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * slot_of(gp))));
+            dh[gp] = *reinterpret_cast<const v4i *>(st + (p_rd ^ (64u * slot_of(gp))) + (G::HI_OFF - G::LO_OFF));
         }
         const float2 dwm = *reinterpret_cast<const float2 *>(st + dw_rd);
         /* Chunk by chunk: the operands of chunk c + 1 are on their way, and the f32 step of chunk c - 1 and a share
-         * of the next super-block's planes go between the MFMAs of chunk c.  The order is pinned: left to the
-         * compiler the raw blocks are requested behind the last chunk, so that every super-block ends with a
-         * trip to memory, and all requests in one burst at the top stall the waves at their next load
-         * (4096 x 14336, 512 tokens: 115 and 123 us against 101). */
-        Q6sRaw after;
-        uint32_t dq_next = 0;
+         * of the next super-block's planes go between the MFMAs of chunk c.  The order is pinned. */
+        float d_next = 0.0f, dmin_next = 0.0f;
         v4i an[4], lo_p = { 0, 0, 0, 0 }, hi_p = { 0, 0, 0, 0 };
         float4 dq_p = { 0.0f, 0.0f, 0.0f, 0.0f };
         auto read_a = [&](int c) {
@@ -241,10 +260,6 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
             lo_p = lo;
             hi_p = hi;
             dq_p = dq4;
-            if (c == 0) {
-                after = load_raw(min(b + 2u, B - 1u));
-                dq_next = load_dq(min(b + 1u, B - 1u));
-            }
             if (c < N) {
 #pragma unroll
                 for (int g = 0; g < 8; g++) {
@@ -253,12 +268,29 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (c == N - 1) {
+                d_next = half_to_float_hw(next.d >> 16);
+                dmin_next = Q2 ? half_to_float_hw(next.dmin & 0xFFFFu) : 0.0f;
+                asm volatile("" : "+v"(d_next), "+v"(dmin_next));      /* out of `next` before it is loaded again */
+                __builtin_amdgcn_sched_barrier(0);
+                next = load_raw(min(b + 3u, B - 1u));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        store_planes(next, dq_next, buf ^ 1u);
-        next = after;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        store_planes(d_next, dmin_next, dq_next, buf ^ 1u);
+        /* loads return in order: this step's LDS-bound ones and the other set are complete when no more than the
+         * raw blocks requested last are missing */
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(RAW_LOADS) : "memory");
         q6s_barrier();
+    };
+    uint32_t b = 0;
+    for (; b + 1u < B; b += 2u) {
+        step(b, set0);
+        step(b + 1u, set1);
     }
+    if (b < B) step(b, set0);
+    /* the last requests, which nobody reads: the workgroup's LDS must be its own until they have landed */
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     const uint32_t row = (wave & 3u) * 16u + r16;
     if (row < rows_here) {
@@ -272,8 +304,8 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
     }
 }
 
-/* grid (row tiles, token tiles); the token chunks are dealt evenly to the token tiles, and a tile's to its
- * two halves: both waves of a SIMD belong to one tile, so what counts is the chunks of the two together. */
+/* grid (row tiles, token tiles); the token chunks are dealt evenly to the token tiles, at least one to each, and a
+ * tile's to its two halves: both waves of a SIMD belong to one tile, so what counts is the chunks of the two together. */
 template <bool Q2>
 __global__ __launch_bounds__(512, 2) void
 k_mmq_q6_k_shared(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t *__restrict__ acts,
@@ -285,6 +317,7 @@ k_mmq_q6_k_shared(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, cons
      * leave 32 bits at three million activations) */
     const uint32_t each = chunks / gridDim.y, over = chunks - each * gridDim.y;
     const uint32_t c0 = blockIdx.y * each + min(blockIdx.y, over), nc = each + (blockIdx.y < over ? 1u : 0u);
+    if (nc == 0u) return;           /* not launched: oxh_internal_mmq6_tok_tiles() is at most the number of chunks */
     const uint32_t tok0 = 16u * c0, here = min(n_vec - tok0, 16u * nc);
     const uint8_t *wb = w + (size_t)row0 * B * 210u, *ab = acts + (size_t)tok0 * B * 292u;
     float *ob = out + (size_t)tok0 * out_stride + row0;
@@ -294,7 +327,8 @@ k_mmq_q6_k_shared(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, cons
     const uint32_t end = upper ? here : min(here, 16u * first_half);
     if (mine == 4u) q6s_walk<4, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
     else if (mine == 3u) q6s_walk<3, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
-    else q6s_walk<2, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
+    else if (mine == 2u) q6s_walk<2, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
+    else q6s_walk<1, Q2>(wb, rows - row0, B, ab, here, ob, out_stride, at, end);
 }
 
 extern "C" int oxh_internal_mmq6_init(void)
@@ -307,12 +341,25 @@ extern "C" int oxh_internal_mmq6_init(void)
     return (int)e;
 }
 
+/* see oxh_internal.h.  At least one tile per eight chunks (what a workgroup has LDS for).  While one round holds the
+ * launch, as many more as CUs are left, down to two chunks a tile: a super-block costs a workgroup about a microsecond
+ * whatever its tokens, and 0.05 of that per chunk on top (4096 x 14336, us by number of tiles: 128 activations
+ * 78 / 62 / 59 on 1 / 2 / 3, 80 66 / 59 / 57, 333 72.2 / 70.7 on 3 / 4).  A second round costs more than it shortens the
+ * first (14336 x 4096 under 160: 43 us on 2 tiles, 58 on 3). */
+extern "C" size_t oxh_internal_mmq6_tok_tiles(size_t rows, size_t n_vec, size_t cus)
+{
+    const size_t row_tiles = (rows + Q6sGeom::ROWS - 1) / Q6sGeom::ROWS, chunks = (n_vec + 15) / 16;
+    const size_t least = (n_vec + Q6sGeom::TOK - 1) / Q6sGeom::TOK, most = (chunks + 1) / 2, room = cus / row_tiles;
+    const size_t more = room < most ? room : most;
+    return more > least ? more : least;
+}
+
 /* see oxh_internal.h */
 extern "C" int oxh_internal_mmq6_shared(int widened_q2, const void *d_w, size_t rows, size_t blocks, const void *d_acts,
-                                        size_t n_vec, float *d_out, size_t out_stride, void *stream)
+                                        size_t n_vec, float *d_out, size_t out_stride, size_t cus, void *stream)
 {
     typedef Q6sGeom G;
-    const dim3 grid((uint32_t)((rows + G::ROWS - 1) / G::ROWS), (uint32_t)((n_vec + G::TOK - 1) / G::TOK));
+    const dim3 grid((uint32_t)((rows + G::ROWS - 1) / G::ROWS), (uint32_t)oxh_internal_mmq6_tok_tiles(rows, n_vec, cus));
     auto kernel = widened_q2 ? k_mmq_q6_k_shared<true> : k_mmq_q6_k_shared<false>;
     hipLaunchKernelGGL(kernel, grid, dim3(512), G::LDS_BYTES, (hipStream_t)stream, (const uint8_t *)d_w, (uint32_t)rows,
                        (uint32_t)blocks, (const uint8_t *)d_acts, (uint32_t)n_vec, d_out, out_stride);

@@ -308,6 +308,16 @@ def test_q6_k_tiles_with_shared_operands(oxh, rows, cols, n_vec, tile):
 
 
 
+@pytest.mark.parametrize("rows,cols,n_vec", [(4031, 2816, 165), (3333, 1280, 145), (6100, 1280, 81), (8200, 1280, 33), (2049, 1792, 400)])
+def test_q6_k_tiles_with_shared_operands_walk_odd_numbers_of_blocks_in_more_tiles(oxh, rows, cols, n_vec):
+    """The same tiles over five, seven and eleven super-blocks (raw blocks are kept in two sets that take turns), cut
+    into more token tiles than the tokens need: chunks 3, 3, 3, 2 and 3, 3, 2, 2 to a tile (halves of 2, 1 and one
+    chunk), 3 and 3, one tile of 3, and seven tiles."""
+    if mv.device_info()["n_cu"] == 256:
+        assert mv.mmq_kernel(Q6K, rows, cols, n_vec)[0] == mv.MMQ_SHARED
+    check_mmq(Q6K, rows, cols, n_vec)
+
+
 def test_q6_k_tiles_with_shared_operands_over_three_million_activations(oxh):
     """The token tiles' share of the 16-token chunks in 32 bits: 23 438 tiles times 187 500 chunks is past 2^32.
     A thousand activations, repeated: every repetition has the bits of the first, which the oracle holds."""
