@@ -42,22 +42,26 @@ k_mmq_experts_long(const ExpertArgs a)
     constexpr uint32_t WB = FMT == EXP_Q4 ? 144u : FMT == EXP_Q5 ? 176u : 210u;
     constexpr uint32_t ROWS = 8u * RC * 16u, TOK = TCMAX * 16u;
     const uint32_t lane = threadIdx.x & 63u;
-    /* a lane per expert: its tiles, their running sum, the expert tile y falls in */
+    /* a lane per expert: its tiles and where they start, the expert tile y falls in.  Workgroups start in the order of
+     * y, so experts whose tiles hold the most chunks come first: with the counts as they fall a launch of little more
+     * than one round ended with a whole tile that started late (8 experts, 1024 pairs, 4096 rows, one expert above 144
+     * tokens: 265 us, 219 in this order; no difference where all fit one round). */
     const uint32_t cnt = lane < a.n_expert ? a.counts[lane] : 0u;
     const uint32_t off = lane < a.n_expert ? a.offsets[lane] : 0u;
     const uint32_t tiles = (cnt + TOK - 1u) / TOK;
-    uint32_t upto = tiles;
-#pragma unroll
-    for (uint32_t d = 1; d < 64u; d <<= 1) {
-        const uint32_t v = __shfl_up(upto, d);
-        if (lane >= d) upto += v;
+    const uint32_t size = tiles ? (((cnt + 15u) >> 4) + tiles - 1u) / tiles : 0u;
+    uint32_t from = 0u;
+    for (uint32_t o = 0; o < a.n_expert; o++) {
+        const uint32_t o_size = (uint32_t)__builtin_amdgcn_readlane((int)size, (int)o);
+        const uint32_t o_tiles = (uint32_t)__builtin_amdgcn_readlane((int)tiles, (int)o);
+        if (o_size > size || (o_size == size && o < lane)) from += o_tiles;
     }
-    const unsigned long long past = __ballot(upto > blockIdx.y);
-    if (past == 0ull) return;
-    const int e = __builtin_ctzll(past);
+    const unsigned long long here_is = __ballot(tiles != 0u && blockIdx.y >= from && blockIdx.y - from < tiles);
+    if (here_is == 0ull) return;
+    const int e = __builtin_ctzll(here_is);
     const uint32_t nv = (uint32_t)__builtin_amdgcn_readlane((int)cnt, e);
     const uint32_t n_tiles = (uint32_t)__builtin_amdgcn_readlane((int)tiles, e);
-    const uint32_t tile = blockIdx.y - ((uint32_t)__builtin_amdgcn_readlane((int)upto, e) - n_tiles);
+    const uint32_t tile = blockIdx.y - (uint32_t)__builtin_amdgcn_readlane((int)from, e);
     const uint32_t chunks = (nv + 15u) >> 4;
     const uint32_t c0 = tile * chunks / n_tiles, nc = (tile + 1u) * chunks / n_tiles - c0;
     const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)off, e) + 16u * c0;
