@@ -842,6 +842,23 @@ static int push_input(size_t bytes)
     return oxh_memcpy_h2d(g_dx.p, g_hin.p, bytes, NULL);
 }
 
+/* `n_vec` vectors of at most HOST_DIRECT_MAX bytes in all through the page-locked image.  From 512 KiB on in two halves: the
+ * device pulls the first one over while the processor copies the second (a launch costs the processor some 4 us, which a
+ * half's trip over the bus is worth from there on: 64 vectors of 4096, 14336 rows of Q4_K, 199 -> 194 us a call). */
+static int push_vectors(const float *inputs, size_t in_stride, size_t cols, size_t n_vec)
+{
+    const size_t width = cols * sizeof(float), half = n_vec * width >= ((size_t)512 << 10) && width % 16u == 0 ? n_vec / 2 : 0;
+    for (size_t v = 0; v < n_vec; v++) {
+        if (half && v == half) {
+            const int rc = oxh_internal_copy16(g_dx.p, g_hin.p, half * width, NULL);
+            if (rc) return rc;
+        }
+        memcpy((float *)g_hin.p + v * cols, inputs + v * in_stride, width);
+    }
+    const size_t at = half * width;
+    return oxh_internal_copy16((uint8_t *)g_dx.p + at, (uint8_t *)g_hin.p + at, align16(n_vec * width - at), NULL);
+}
+
 static bool mul_ok(size_t a, size_t b, size_t *out)
 {
     if (a != 0 && b > SIZE_MAX / a) return false;
@@ -1204,9 +1221,7 @@ static int mv_batch(uint32_t qtype, const uint8_t *data, size_t rows,
     const bool in_direct = packed_in <= HOST_DIRECT_MAX, out_direct = packed_out <= HOST_DIRECT_MAX;
     if (in_direct) {
         if ((rc = reserve_host(&g_hin, packed_in))) return rc;
-        for (size_t v = 0; v < n_vec; v++)
-            memcpy((float *)g_hin.p + v * cols, inputs + v * in_stride, cols * sizeof(float));
-        rc = push_input(packed_in);
+        rc = push_vectors(inputs, in_stride, cols, n_vec);
     } else if (in_stride != cols && !oxh_internal_runtime_memory(inputs, (in_span + cols) * sizeof(float)) && ring_ready())
         rc = ring_push((uint8_t *)g_dx.p, inputs, cols * sizeof(float), in_stride * sizeof(float), packed_in);
     else if (in_stride == cols)

@@ -215,6 +215,25 @@ def test_host_batches_through_the_ring_of_pinned_slots(oxh, rows, cols, n_vec, p
         assert np.array_equal(bits(part[:m]), bits(out[v:v + m, :rows])), v
 
 
+@pytest.mark.parametrize("cols,n_vec,pad", [(1024, 127, 0), (1024, 128, 3), (1024, 129, 0), (2048, 128, 5), (256, 1023, 0)])
+def test_host_batches_whose_inputs_go_over_in_two_halves(oxh, cols, n_vec, pad):
+    """Inputs up to 1 MiB through the page-locked image: below 512 KiB in one piece, from there on in two, an odd number of
+    vectors among them.  Every vector's outputs against calls of eight vectors."""
+    rows = 65
+    w = synth.weights(Q4K, rows, cols, seed=29, stream=cols)
+    rb = synth.row_bytes(Q4K, cols)
+    xs = np.full((n_vec, cols + pad), 3.5, np.float32)
+    xs[:, :cols] = synth.normal(n_vec * cols, seed=29, stream=n_vec).reshape(n_vec, cols)
+    temp, scratch = np.zeros(cols, np.float32), np.zeros(mv.batch_scratch_bytes(cols), np.uint8)
+    out = np.zeros((n_vec, rows), np.float32)
+    mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, xs, cols + pad, out, rows, n_vec, temp, scratch)
+    for v in range(0, n_vec, 8):
+        part, x8 = np.zeros((8, rows), np.float32), np.ascontiguousarray(xs[v:v + 8, :cols])
+        m = x8.shape[0]
+        mv.matvec_quantized_batch(Q4K, w, rows, cols, rb, x8, cols, part, rows, m, temp, scratch)
+        assert np.array_equal(bits(part[:m]), bits(out[v:v + m])), v
+
+
 @pytest.mark.parametrize("pad", [0, 5])
 @pytest.mark.parametrize("pinned_in,pinned_out", [(False, True), (True, False), (True, True)])
 def test_host_batches_from_and_to_page_locked_memory_are_copied_in_place(oxh, pinned_in, pinned_out, pad):
