@@ -49,7 +49,7 @@ template <int FMT, int CH> struct BatGeom {
 /* the parts of a block that lane (r, kq) builds its operands from, out of row r's LDS image */
 template <int FMT> struct BatRaw {
     u32x4 hdr;                  /* Q4/Q5: d, dmin, scales; Q6: the sixteen scales; Q2: minima and dmin */
-    u32x4 v[4];                 /* Q4/Q5: nibbles of the four k steps; Q6/Q2: ql, ql, qh, qh */
+    u32x4 v[4];                 /* Q4/Q5: two pieces of nibbles, two k steps each (mmq_tile()); Q6/Q2: ql, ql, qh, qh */
     u32x4 plane;                /* Q5: fifth bits */
     uint32_t d;                 /* Q6/Q2: f16 d */
 };
@@ -65,7 +65,7 @@ __device__ __forceinline__ BatRaw<FMT> bat_read(const uint8_t *row, uint32_t kq)
         r.hdr = get(0u);
         if (FMT == BAT_Q5) r.plane = get(16u + 16u * (kq & 1u));
 #pragma unroll
-        for (uint32_t gp = 0; gp < 4u; gp++) r.v[gp] = get((FMT == BAT_Q5 ? 48u : 16u) + 32u * gp + 16u * (kq & 1u));
+        for (uint32_t p = 0; p < 2u; p++) r.v[p] = get((FMT == BAT_Q5 ? 48u : 16u) + 16u * kq + 64u * p);
     } else {
 #pragma unroll
         for (uint32_t n = 0; n < 2u; n++) {
@@ -102,16 +102,16 @@ __device__ __forceinline__ BatOps<FMT> bat_build(const BatRaw<FMT> &r, uint32_t 
         o.dmin = half_to_float_hw(r.hdr.x >> 16);
 #pragma unroll
         for (int gp = 0; gp < 4; gp++) {
-            const uint32_t sc = (sc_w[gp >> 1] >> (16u * (uint32_t)(gp & 1) + 8u * half)) & 0xFFu;
+            const uint32_t sc = (sc_w[gp >> 1] >> (16u * half + 8u * (uint32_t)(gp & 1))) & 0xFFu;
             const unsigned short sl = (unsigned short)(sc & 7u), sh = (unsigned short)(sc >> 3), sx = (unsigned short)(2u * sc);
             const v2u16 sl2 = { sl, sl }, sh2 = { sh, sh }, sx2 = { sx, sx };
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const v2u16 p = __builtin_bit_cast(v2u16, (r.v[gp][k] >> (4u * half)) & 0x0F0F0F0Fu);
+                const v2u16 p = __builtin_bit_cast(v2u16, (gp & 1 ? r.v[gp >> 1][k] >> 4 : r.v[gp >> 1][k]) & 0x0F0F0F0Fu);
                 o.lo[gp][k] = __builtin_bit_cast(int, (v2u16)(p * sl2));
                 o.hi[gp][k] = __builtin_bit_cast(int, (v2u16)(p * sh2));
                 if (FMT == BAT_Q5) {
-                    const uint32_t fifth = (r.plane[k] >> (2u * (uint32_t)gp + half)) & 0x01010101u;
+                    const uint32_t fifth = (r.plane[k] >> (4u * (uint32_t)(gp >> 1) + 2u * half + (uint32_t)(gp & 1))) & 0x01010101u;
                     o.x[gp][k] = __builtin_bit_cast(int, (v2u16)(__builtin_bit_cast(v2u16, fifth) * sx2));
                 }
             }
@@ -225,7 +225,9 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
     }
     __syncthreads();
 
-    const uint32_t a_rd = G::A_OFF + r16 * 256u + ((kq ^ r16) * 16u);                 /* ^ 64 * gp */
+    /* the slot of this lane's values of step 0, and what the other steps change in it */
+    const uint32_t a_rd = G::A_OFF + r16 * 256u + (((G::DMA ? 4u * (kq >> 1) + (kq & 1u) : kq) ^ r16) * 16u);
+    auto a_step = [](int gp) -> uint32_t { return G::DMA ? 32u * ((uint32_t)gp & 1u) + 128u * ((uint32_t)gp >> 1) : 64u * (uint32_t)gp; };
     const v4i zero = { 0, 0, 0, 0 };
     const v4f fzero = { 0.0f, 0.0f, 0.0f, 0.0f };
     uint32_t buf = 0;
@@ -253,7 +255,7 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
             v4i lo = zero, hi = zero;
 #pragma unroll
             for (int gp = 0; gp < 4; gp++) {
-                const v4i av = *reinterpret_cast<const v4i *>(my + (a_rd ^ (64u * (uint32_t)gp)) + buf * G::A_BYTES + 4096u * (uint32_t)c);
+                const v4i av = *reinterpret_cast<const v4i *>(my + (a_rd ^ a_step(gp)) + buf * G::A_BYTES + 4096u * (uint32_t)c);
                 lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, o.lo[gp], lo, 0, 0, 0);
                 hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, o.hi[gp], hi, 0, 0, 0);
                 if (FMT == BAT_Q5) hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, o.x[gp], hi, 0, 0, 0);
