@@ -104,8 +104,7 @@ k_quantize_q8_k(const float *__restrict__ x, size_t in_stride, uint32_t blocks_p
     /* max |x| over the block; NaNs never win a '>' comparison in the
      * reference's scan, fmaxf drops them the same way */
     float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+    amax = wave_max(amax);
 
     const float d = amax / 127.0f;
     const float inv = (d != 0.0f) ? 1.0f / d : 0.0f;
@@ -143,8 +142,7 @@ k_quantize_q8_0(const float *__restrict__ x, size_t in_stride, uint32_t blocks_p
         v0 = src[0]; v1 = src[1]; v2 = src[2]; v3 = src[3];
     }
     float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
-#pragma unroll
-    for (int m = 4; m >= 1; m >>= 1) amax = fmaxf(amax, __shfl_xor(amax, m, 64));
+    amax = oct_max(amax);
     const float d = amax / 127.0f;
     const float inv = (d != 0.0f) ? 1.0f / d : 0.0f;
     const int q0 = quantize_one(v0, inv), q1 = quantize_one(v1, inv);
