@@ -55,8 +55,10 @@ typedef struct OxhLab {
      * oxh_mmq): what the launch itself asks, as host arithmetic.  out: the
      * kernel (0 tiles, 1 Q6_K tiles whose operands a workgroup builds once,
      * 2 a workgroup per 16 rows whose waves share the columns, 3 tiles whose
-     * columns several workgroups share), rows and tokens of a workgroup, and
-     * for kernel 2 its waves.  OXH_DECLINED for a type without such a kernel. */
+     * columns several workgroups share), rows and tokens of a workgroup (for
+     * kernel 1 the tokens it has room for), and for kernel 2 its waves, for
+     * kernel 1 the token tiles the launch is cut into.  OXH_DECLINED for a
+     * type without such a kernel. */
     int (*mmq_kernel)(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t n_cu, size_t ws_bytes,
                       uint32_t out[4]);
     /* The same for one expert launch of oxh_moe_ffn: n_mat matrices of `rows`

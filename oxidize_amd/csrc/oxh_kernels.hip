@@ -2218,45 +2218,54 @@ static int mmq_tile_shape(uint32_t qtype, size_t rows, size_t n_vec, size_t cus)
     return few_tiles ? 4 : 3;
 }
 
-/* Which tile a Q6_K (or widened Q2_K) launch of more than 32 activations runs on, by what it is expected to
- * take.  The unit is 1.8 us a super-block; measured on 256 CUs at 1 to 97 super-blocks, 64 to 16384 rows and 33 to
- * 1024 activations, every tile forced in turn, weights from one copy and from several (medians, Q6_K):
- *   64 x 128 tiles whose operands the workgroup builds once, one to a CU: 0.69 a round up to five token chunks, 0.76,
- *     0.80, 0.87 with six to eight; a further round costs 1.16 of the first (two rounds of seven chunks 1.74, four
- *     3.61), the workgroups of a CU no longer starting together;
- *   128 x 128 tiles, one to a CU: 1.48, two rounds 3.13;
- *   64 x 32 tiles, three to a CU: 0.70 up to one a CU, 0.95 up to two, 1.2 up to three, then 0.35 each more (1.70, 2.05).
- * A tile of 128 tokens starts 0.6 us later than one of 32, and 0.2 us in every further round: 1216 x 512 under 585
- * activations 8.2 us against 7.5.
- * Widened Q2_K builds its operands in fewer instructions: 0.64 to 0.86 and 1.17; 1.40, 2.99; 0.59, 0.78, 1.0, then
- * 1.5 and 0.30 each.
- * (The first kind has become 3 to 25 % faster since, most with few chunks, now that its waves no longer wait for memory
- * every super-block and a launch of one round is cut into more tiles; the lines are where they were before.)
- * Where two tiles are within some 8 % the weights' way in decides, and the order for weights that come from memory was
- * taken (Q2_K 7433 x 22528 under 78 activations: 136 us on 64 x 128 tiles against 124 on 64 x 32 ones, 10112 x 1792
- * under 79, which stays in a cache, 13.1 against 15.6; Q6_K 7736 x 17664 under 42: 97 against 105). */
+/* Which tile a Q6_K (or widened Q2_K) launch of more than 32 activations runs on: the one expected to be done first.
+ * What a launch takes, in us, by the tiles n of the busiest CU (for 64 x 128 tiles the ones it is really cut into,
+ * oxh_internal_mmq6_tok_tiles(), and the 16-token chunks of the largest):
+ *   start + tile * n + super-blocks * s(n),   s(n) = few[n - 1] up to three tiles, base + more * n from there.
+ * The constants are the least squares of the logarithms over 1480 random launches with every tile forced in turn, on 256
+ * CUs (1 to 97 super-blocks, 64 to 60000 rows, 33 to 4096 activations; geometric mean of weights that stay in a cache and
+ * weights from memory); s.d. of a time about its line 5 to 10 %.  The tile so chosen is 0.2 % (Q6_K) and 0.4 % (Q2_K) above
+ * the fastest of the four in the geometric mean.  Before, with the line of the 64 x 128 tiles from when each had up to
+ * eight chunks and waited for memory every super-block, and 64 x 16 tiles wherever one a CU held the launch, it was
+ * 3.1 and 3.2 %: the quarter of the launches that changed tile is 10 % faster, single ones up to 31 % faster and up to 10 %
+ * slower (Q6_K 4096 x 14336 under 80 activations 77.7 us on 64 x 32 tiles, 61.3 on 64 x 128 ones, 14336 rows under 144
+ * 155 / 138; widened Q2_K 1766 x 3072 under 183 14.3 / 15.5). */
+struct Mmq6Us {
+    double start, tile, few[3], base, more;
+    double of(size_t n, double blocks) const
+    {
+        return start + tile * (double)n + blocks * (n <= 3 ? few[n - 1] : base + more * (double)n);
+    }
+};
+
 static int mmq6_tile_shape(size_t rows, size_t blocks, size_t n_vec, size_t cus, bool widened_q2)
 {
-    const size_t row_tiles = (rows + 63) / 64;
-    if (n_vec <= 32 || row_tiles * ((n_vec + 15) / 16) <= cus) return mmq_tile_shape(OXH_Q6_K, rows, n_vec, cus);
-    const size_t tok_tiles = (n_vec + 127) / 128, chunks = ((n_vec + 15) / 16 + tok_tiles - 1) / tok_tiles;
-    const double r5 = (double)((row_tiles * tok_tiles + cus - 1) / cus);
-    const double r1 = (double)(((rows + 127) / 128 * tok_tiles + cus - 1) / cus);
-    const size_t n3 = (row_tiles * ((n_vec + 31) / 32) + cus - 1) / cus;
-    const double fill = (double)(chunks < 4 ? 4 : chunks);
-    double c1, c3, c5;
-    if (widened_q2) {
-        const double few[3] = { 0.59, blocks < 20 ? 0.67 : 0.65, 0.95 };
-        c5 = (0.34 + 0.064 * fill) * (r5 + 0.17 * (r5 - 1.0));
-        c1 = 1.40 * (r1 + 0.13 * (r1 - 1.0));
-        c3 = n3 <= 3 ? few[n3 - 1] : 0.33 + 0.30 * (double)n3;
-    } else {
-        c5 = (0.43 + 0.054 * fill) * (r5 + 0.16 * (r5 - 1.0)) + (0.25 + 0.1 * r5) / (double)blocks;
-        c1 = 1.48 * (r1 + 0.11 * (r1 - 1.0)) + (0.25 + 0.1 * r1) / (double)blocks;
-        c3 = n3 <= 3 ? 0.45 + 0.25 * (double)n3 : 0.32 + 0.35 * (double)n3;
-    }
-    if (c1 <= c5 && c1 < c3) return 1;
-    return c5 < c3 ? 5 : 3;
+    if (n_vec <= 32) return mmq_tile_shape(OXH_Q6_K, rows, n_vec, cus);
+    const size_t row_tiles = (rows + 63) / 64, chunks = (n_vec + 15) / 16;
+    const size_t tok_tiles = oxh_internal_mmq6_tok_tiles(rows, n_vec, cus);
+    const double c = (double)((chunks + tok_tiles - 1) / tok_tiles), B = (double)blocks;
+    auto busiest = [cus](size_t tiles) { return (tiles + cus - 1) / cus; };
+    /* 64 x 128 tiles: a round's super-block takes a + b per chunk, less in further rounds, whose tiles start one by one */
+    const double first = widened_q2 ? 0.69 + 0.101 * c : 0.756 + 0.093 * c, next = widened_q2 ? 0.35 + 0.136 * c : 0.505 + 0.119 * c;
+    const Mmq6Us shared = { widened_q2 ? 0.77 : 0.27, widened_q2 ? 3.26 : 3.57, { first, first + next, first + 2.0 * next }, first - next, next };
+    static const Mmq6Us q6[3] = {       /* 128 x 128, 64 x 32, 64 x 16 */
+        { -0.96, 5.11, { 2.61, 5.53, 8.45 }, -0.31, 2.92 },
+        { 1.63, 0.73, { 1.21, 1.72, 2.19 }, 0.26, 0.70 },
+        { 1.69, 0.54, { 1.04, 1.45, 1.89 }, 0.09, 0.565 } };
+    static const Mmq6Us q2[3] = {
+        { -0.73, 4.96, { 2.47, 5.22, 7.98 }, -0.29, 2.76 },
+        { 1.66, 0.79, { 1.03, 1.38, 1.94 }, 0.16, 0.615 },
+        { 1.74, 0.52, { 0.88, 1.23, 1.68 }, 0.11, 0.513 } };
+    const Mmq6Us *own = widened_q2 ? q2 : q6;
+    const double us[4] = { shared.of(busiest(row_tiles * tok_tiles), B),
+                           own[0].of(busiest((rows + 127) / 128 * ((n_vec + 127) / 128)), B),
+                           own[1].of(busiest(row_tiles * ((n_vec + 31) / 32)), B),
+                           own[2].of(busiest(row_tiles * chunks), B) };
+    static const int shape[4] = { 5, 1, 3, 4 };
+    int best = 0;
+    for (int i = 1; i < 4; i++)
+        if (us[i] < us[best]) best = i;
+    return shape[best];
 }
 
 /* the 32-value formats with a matrix-core kernel, as its LEG parameter; -1 for everything else */
@@ -2411,6 +2420,7 @@ extern "C" int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, si
     out[2] = r.tile_tokens;
     if (r.kernel == MMQ_BATCH)
         out[3] = oxh_internal_mmq_batch_waves(mmq_batch_fmt(qtype), rows, cols / OXH_QK_K, n_vec, n_cu);
+    if (r.kernel == MMQ_SHARED) out[3] = (uint32_t)oxh_internal_mmq6_tok_tiles(rows, n_vec, n_cu);
     return OXH_OK;
 }
 

@@ -205,7 +205,7 @@ def mmq_tile(qtype, rows, n_vec, n_cu):
 
 
 def mmq_kernel(qtype, rows, cols, n_vec, n_cu=256, ws_bytes=0):
-    """(kernel, tile rows, tile tokens, waves) a matrix-core launch runs on (include/oxhip_lab.h); host arithmetic."""
+    """(kernel, tile rows, tile tokens, waves or token tiles) a matrix-core launch runs on (include/oxhip_lab.h); host arithmetic."""
     out = (ctypes.c_uint32 * 4)()
     check(_lib.lab().mmq_kernel(qtype, rows, cols, n_vec, n_cu, ws_bytes, ctypes.byref(out)))
     return tuple(out)

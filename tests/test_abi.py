@@ -279,8 +279,10 @@ def test_which_kernel_a_matrix_core_launch_runs_on_is_host_arithmetic():
     assert k(Q4K, 14336, 4096, 512)[:3] == (mv.MMQ_TILES, 256, 128)
     assert k(Q5K, 28672, 4096, 512)[:3] == (mv.MMQ_TILES, 128, 128)
     assert k(Q5K, 3600, 512, 500)[:3] == (mv.MMQ_TILES, 128, 64)
-    assert k(Q6K, 4096, 14336, 333)[:3] == (mv.MMQ_SHARED, 64, 128)
-    assert k(WIDE2, 4096, 14336, 512)[:3] == (mv.MMQ_SHARED, 64, 128)
+    assert k(Q6K, 4096, 14336, 333) == (mv.MMQ_SHARED, 64, 128, 4)          # 21 chunks of 16 tokens in 4 tiles, not 3
+    assert k(Q6K, 4096, 14336, 128) == (mv.MMQ_SHARED, 64, 128, 4)          # two chunks a tile
+    assert k(WIDE2, 4096, 14336, 512) == (mv.MMQ_SHARED, 64, 128, 4)
+    assert k(Q6K, 14336, 14336, 144) == (mv.MMQ_SHARED, 64, 128, 2)         # 224 row tiles: what the tokens need
     assert k(Q80, 4096, 4096, 512)[:3] == (mv.MMQ_TILES, 128, 64)
     kernel, rows, tokens, waves = k(Q6K, 4096, 14336, 16)           # one 16-row group per CU, columns shared in LDS
     assert (kernel, rows, tokens) == (mv.MMQ_BATCH, 16, 16) and 4 <= waves <= 16
@@ -322,17 +324,19 @@ def test_small_batches_go_where_they_measured_fastest():
 
 def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
     """Q6_K and widened Q2_K above the small batches, on 256 compute units: sizes at which the 64 x 128 tiles measured
-    slower than the 64 x 32 or the 128 x 128 ones (few chunks on a part of the device, two rounds against one), and
-    sizes at which they measured faster."""
+    slower than the 64 x 32, the 64 x 16 or the 128 x 128 ones (one super-block, two rounds against one), and sizes at which
+    they measured faster, among them launches of one round, which are cut into more tiles than the tokens need."""
     Q6K, WIDE2 = 16, 0x1008
     for qtype, rows, cols, n_vec, tile in (
-            (Q6K, 14336, 14336, 144, (128, 128)), (Q6K, 16384, 8192, 160, (128, 128)), (Q6K, 1216, 512, 585, (64, 32)),
-            (Q6K, 6144, 256, 40, (64, 32)), (Q6K, 14336, 256, 129, (128, 128)), (WIDE2, 7168, 14336, 48, (64, 32)),
-            (WIDE2, 6144, 5120, 33, (64, 32)), (WIDE2, 8192, 14336, 40, (64, 32)), (WIDE2, 8192, 256, 48, (64, 32)),
-            (WIDE2, 8192, 14336, 96, (64, 32)), (Q6K, 4096, 14336, 333, (64, 128)), (Q6K, 4096, 14336, 512, (64, 128)),
-            (Q6K, 8192, 4096, 129, (64, 128)), (Q6K, 14336, 4096, 512, (128, 128)), (WIDE2, 4096, 14336, 512, (64, 128)),
-            (WIDE2, 10240, 5120, 64, (64, 128)), (Q6K, 7736, 17664, 42, (64, 128)), (WIDE2, 8180, 5120, 75, (64, 32)),
-            (Q6K, 10240, 14336, 64, (64, 128))):
+            (Q6K, 8300, 512, 256, (128, 128)), (Q6K, 4096, 4096, 2048, (128, 128)), (Q6K, 12544, 4096, 4096, (128, 128)),
+            (Q6K, 6144, 256, 40, (64, 32)), (Q6K, 14336, 256, 129, (128, 128)), (WIDE2, 8192, 256, 48, (64, 32)),
+            (WIDE2, 4099, 512, 130, (64, 32)), (Q6K, 414, 1024, 135, (64, 16)), (Q6K, 14336, 4096, 512, (128, 128)),
+            (Q6K, 4096, 14336, 333, (64, 128)), (Q6K, 4096, 14336, 512, (64, 128)), (Q6K, 4096, 14336, 80, (64, 128)),
+            (Q6K, 4096, 14336, 128, (64, 128)), (Q6K, 14336, 14336, 144, (64, 128)), (Q6K, 16384, 8192, 160, (64, 128)),
+            (Q6K, 8192, 4096, 129, (64, 128)), (Q6K, 7736, 17664, 42, (64, 128)), (Q6K, 10240, 14336, 64, (64, 128)),
+            (Q6K, 164, 16640, 448, (64, 128)), (WIDE2, 4096, 14336, 512, (64, 128)), (WIDE2, 4096, 14336, 80, (64, 128)),
+            (WIDE2, 10240, 5120, 64, (64, 128)), (WIDE2, 8180, 5120, 75, (64, 128)), (WIDE2, 7168, 14336, 48, (64, 128)),
+            (WIDE2, 6144, 5120, 33, (64, 128)), (WIDE2, 8192, 14336, 96, (64, 128)), (WIDE2, 2049, 1280, 390, (64, 128))):
         assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile, (qtype, rows, cols, n_vec)
 
 

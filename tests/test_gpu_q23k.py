@@ -346,8 +346,8 @@ def test_q2k_wide_tile_kernel_on_raw_blocks(oxh, n_vec, cols):
         mv.gemv_segments(mv.Q2_K_WIDE, seg, cols, d_a.ptr, 1, rows)
 
 
-@pytest.mark.parametrize("rows,cols,n_vec,tile", [(4099, 512, 130, (64, 128)), (3600, 256, 333, (64, 128)), (14300, 768, 40, (64, 128)),
-                                                  (8200, 768, 128, (64, 128)), (2049, 1280, 390, (64, 32)), (8300, 512, 256, (128, 128)),
+@pytest.mark.parametrize("rows,cols,n_vec,tile", [(4099, 768, 130, (64, 128)), (3600, 256, 333, (64, 128)), (14300, 768, 40, (64, 128)),
+                                                  (8200, 768, 128, (64, 128)), (4099, 512, 130, (64, 32)), (2049, 1280, 390, (64, 128)), (8300, 512, 256, (128, 128)),
                                                   (3333, 1280, 145, (64, 128))])
 def test_q2k_wide_tiles_with_shared_operands(oxh, rows, cols, n_vec, tile):
     """The 64 x 128 tiles whose operands the workgroup builds once, and the two tiles beside them, on widened raw random
