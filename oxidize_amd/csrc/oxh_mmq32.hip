@@ -307,15 +307,20 @@ static uint64_t mmq32_tiles(size_t rows, size_t n_vec, uint32_t tile_rows)
     return (n_rt + 7u) / 8u * 8u * n_tt;
 }
 
-/* Which tile.  64 x 64, two to a CU, unless there are more of them than CUs and one round of 128 x 64 tiles, a CU's
- * worth of waves each, holds the launch: then every CU gets the same and the smaller tiles' third more staging shows
- * (us, 64 / 128 rows: 4096 x 4096 x 512 41.7 / 40.6, 3072 x 2048 x 512 22.7 / 22.1, Q5_1 31.1 / 29.9).  With fewer tiles
- * a small one alone on its CU is done sooner (2048 x 2048 x 333 14.6 / 21.1), with more their rounds are finer (5120 x
- * 2048 x 512 33.0 / 41.2, 8192 rows 43.0 / 43.6, 14336 x 4096 x 512 136 / 149). */
+/* Which tile.  64 x 64, two to a CU, unless some XCD gets more of them than it has CUs and one round of 128 x 64 tiles, a
+ * CU's worth of waves each, holds the launch on every XCD: then every CU gets the same and the smaller tiles' third more
+ * staging shows (us, 64 / 128 rows: 4096 x 4096 x 512 42.7 / 42.2, Q5_1 60.3 / 57.7, 3072 x 2048 x 512 23.3 / 22.3).  With
+ * fewer tiles a small one alone on its CU is done sooner (2048 x 2048 x 333 14.6 / 21.1), with more their rounds are finer
+ * (5120 x 2048 x 512 33.0 / 41.2, 8192 rows 43.0 / 43.6, 14336 x 4096 x 512 136 / 149).  The XCD and not the device is what
+ * fills: the row tiles are dealt to eight of them, and the first gets the odd ones with all their token tiles (4224 x 4096
+ * under 448, 231 tiles of 128 rows, 35 of them on the first XCD's 32 CUs: 44.4 / 74.6; 2100 rows under 960 58.6 / 72.0).
+ * Over 200 random launches near the lines the choice is 0.1 % above the faster tile, at most 5.5 % at 16 us; counted over
+ * the whole device it was 4.3 %, at most 80 %. */
 static bool mmq32_wide(size_t rows, size_t n_vec, size_t cus)
 {
-    const uint64_t n_tt = (n_vec + 63u) / 64u;
-    return (rows + 63u) / 64u * n_tt > cus && (rows + 127u) / 128u * n_tt <= cus;
+    const uint64_t xcd_cus = cus / 8u;
+    auto busiest = [&](uint64_t tile_rows) { return mmq32_tiles(rows, n_vec, (uint32_t)tile_rows) / 8u; };
+    return busiest(64u) > xcd_cus && busiest(128u) <= xcd_cus;
 }
 
 /* see oxh_internal.h */

@@ -340,6 +340,16 @@ def test_q6_k_prompts_go_to_the_tile_that_measured_fastest():
         assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile, (qtype, rows, cols, n_vec)
 
 
+def test_prompts_of_the_32_value_formats_take_the_wide_tile_where_one_round_of_it_holds_on_every_xcd():
+    """The row tiles are dealt to eight XCDs of 32 compute units: what counts is the tiles of the one that gets the most, not
+    those of the device.  Sizes at which both tiles measured, between 231 and 256 tiles of 128 rows in all."""
+    for rows, n_vec, tile in ((4224, 448, (64, 64)), (2100, 960, (64, 64)), (2199, 703, (64, 64)), (4250, 410, (64, 64)),
+                              (2776, 666, (64, 64)), (3551, 542, (64, 64)), (4096, 512, (128, 64)), (3072, 512, (128, 64)),
+                              (1717, 519, (128, 64)), (5354, 165, (128, 64)), (2048, 512, (64, 64)), (14336, 512, (64, 64)),
+                              (8192, 512, (64, 64)), (64, 1024, (64, 64))):
+        assert mv.mmq_kernel(7, rows, 4096, n_vec) == (mv.MMQ_TILES,) + tile + (0,), (rows, n_vec)
+
+
 def test_expert_launches_go_to_the_tile_that_measured_fastest():
     """Expert launches on 256 compute units: Q5_K and Q6_K keep the 64 x 16 tiles up to more tokens per expert than Q4_K
     while those are many, and leave them earlier where there are two or three to a unit."""
