@@ -181,19 +181,23 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
      * planes are built; the other holds b + 2, still on its way. */
     Q6sRaw set0, set1;
     {
+        request(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
         const Q6sRaw r = load_raw(0);
         const uint32_t dq = load_dq(0);
-        request(0, 0);
 #pragma unroll
         for (int k = 0; k < 4; k++) build_dword(r, k);
         store_planes(half_to_float_hw(r.d >> 16), half_to_float_hw(r.dmin & 0xFFFFu), dq, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        /* the LDS-bound loads, which the compiler does not count.  All that is on its way here, and next to nothing to
+         * wait for behind the loads above, which are younger; a count that leaves set0 and set1 out would hold only as
+         * long as the compiler requests both in front of it (it requests set1 behind the barrier) */
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         set0 = load_raw(min(1u, B - 1u));
         __builtin_amdgcn_sched_barrier(0);
         set1 = load_raw(min(2u, B - 1u));
         __builtin_amdgcn_sched_barrier(0);
-        /* the LDS-bound loads, which the compiler does not count, and set0: all but the last loads */
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(RAW_LOADS) : "memory");
         q6s_barrier();
     }
 
@@ -279,7 +283,8 @@ q6s_walk(const uint8_t *__restrict__ w_base, uint32_t rows_here, uint32_t B, con
         }
         store_planes(d_next, dmin_next, dq_next, buf ^ 1u);
         /* loads return in order: this step's LDS-bound ones and the other set are complete when no more than the
-         * raw blocks requested last are missing */
+         * raw blocks requested last are missing.  (dq_next, just stored, is younger than the LDS-bound ones: they are
+         * complete wherever the compiler puts the raw blocks.) */
         asm volatile("s_waitcnt vmcnt(%0)" :: "n"(RAW_LOADS) : "memory");
         q6s_barrier();
     };

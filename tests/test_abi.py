@@ -404,3 +404,44 @@ def test_bindings_lay_the_structs_out_as_the_header_does(tmp_path):
         assert seen[(name, "size")] == ctypes.sizeof(cls), name
         for field, _ in cls._fields_:
             assert seen[(name, field)] == getattr(cls, field).offset, (name, field)
+
+
+def test_shared_operand_tiles_wait_for_their_lds_bound_loads_before_each_barrier(tmp_path):
+    """Loads that go straight to LDS are counted by nobody but the kernel's own waits.  In the compiled 64 x 128 tiles
+    (oxh_mmq6.hip), before every barrier that such loads stand in front of: in the prologue, ahead of all results, a wait for
+    everything on its way, stated in the source, whatever the compiler asks for next; inside the walk a wait (the source's, or
+    the compiler's for a younger load) that leaves out no more loads than were asked for after them."""
+    import subprocess
+    from oxidize_amd import build
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    out = str(tmp_path / "mmq6.s")
+    subprocess.run([build.HIPCC] + build.HIP_FLAGS + ["-I", build.INCLUDE, "-I", build.CSRC, "-S", "--cuda-device-only",
+                   os.path.join(build.CSRC, "oxh_mmq6.hip"), "-o", out], check=True, capture_output=True)
+    prologues = steps = 0
+    lds = own = product = False
+    loads = 0           # vector loads since the last LDS-bound one
+    for line in open(out):
+        word = line.split()
+        if not word or word[0].startswith((".", "_Z")):
+            continue
+        if word[0].startswith("global_load_lds"):
+            lds, waited, loads = True, False, 0
+        elif word[0].startswith("global_load"):
+            loads += 1
+        elif "mfma" in word[0]:
+            product = True
+        elif word[0] == ";;#ASMSTART":
+            own = True
+        elif word[0] == ";;#ASMEND":
+            own = False
+        elif word[0] == "s_waitcnt" and lds and "vmcnt" in line:
+            left = int(re.search(r"vmcnt\((\d+)\)", line).group(1))
+            waited = waited or (left <= loads if product else own and left == 0)
+        elif word[0] == "s_barrier" and lds:
+            assert waited, line
+            prologues, steps = prologues + (not product), steps + product
+            lds = product = False
+        elif word[0] == "s_endpgm":
+            lds = product = False
+    assert prologues == 8 and steps >= 16           # halves of one to four chunks, two formats
