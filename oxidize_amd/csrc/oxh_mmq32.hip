@@ -332,18 +332,30 @@ extern "C" void oxh_internal_mmq32_tile(size_t rows, size_t n_vec, size_t cus, u
 
 extern "C" int oxh_internal_mmq32_fits(size_t rows, size_t n_vec)
 {
-    return mmq32_tiles(rows, n_vec, Mmq32Geom<0, false>::ROWS) <= 0x7FFFFFFFull;
+    return mmq32_tiles(rows, n_vec, Mmq32Geom<0, true>::ROWS) <= 0x7FFFFFFFull;
 }
 
+/* One launch, or several where the grid would reach the 2^32 threads that HIP takes in one dimension (8.4 million tiles:
+ * 513 rows and 33.6 million tokens): row tiles first, then token tiles. */
 template <int LEG, bool WIDE>
 static void mmq32_launch(const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
                          size_t out_stride, hipStream_t st)
 {
     typedef Mmq32Geom<LEG, WIDE> G;
-    const uint32_t n_rt = (uint32_t)((rows + G::ROWS - 1u) / G::ROWS), n_tt = (uint32_t)((n_vec + G::TOK - 1u) / G::TOK);
-    hipLaunchKernelGGL((k_mmq_32<LEG, WIDE>), dim3((uint32_t)mmq32_tiles(rows, n_vec, G::ROWS)), dim3(G::THREADS), G::LDS_BYTES,
-                       st, (const uint8_t *)d_w, (uint32_t)rows, (uint32_t)blocks, (const uint8_t *)d_acts, (uint32_t)n_vec, d_out,
-                       out_stride, n_rt, n_tt);
+    const size_t most = 0xFFFFFFFFull / G::THREADS / 8u * 8u;
+    const size_t rows_each = rows < most * G::ROWS ? rows : most * G::ROWS;
+    for (size_t r0 = 0; r0 < rows; r0 += rows_each) {
+        const size_t r_here = rows - r0 < rows_each ? rows - r0 : rows_each;
+        const uint32_t n_rt = (uint32_t)((r_here + G::ROWS - 1u) / G::ROWS);
+        const size_t toks_each = most / ((n_rt + 7u) / 8u * 8u) * G::TOK;
+        for (size_t t0 = 0; t0 < n_vec; t0 += toks_each) {
+            const size_t t_here = n_vec - t0 < toks_each ? n_vec - t0 : toks_each;
+            hipLaunchKernelGGL((k_mmq_32<LEG, WIDE>), dim3((uint32_t)mmq32_tiles(r_here, t_here, G::ROWS)), dim3(G::THREADS),
+                               G::LDS_BYTES, st, (const uint8_t *)d_w + r0 * blocks * G::BB, (uint32_t)r_here, (uint32_t)blocks,
+                               (const uint8_t *)d_acts + t0 * blocks * 34u, (uint32_t)t_here, d_out + t0 * out_stride + r0,
+                               out_stride, n_rt, (uint32_t)((t_here + G::TOK - 1u) / G::TOK));
+        }
+    }
 }
 
 /* see oxh_internal.h */

@@ -7,6 +7,8 @@ f32 outputs bit-exact for Q4_K and Q6_K; Q8_0 f32 outputs bit-exact against the
 oracle's block-sequential chain and within |a-b| <= 1e-4 + 1e-5*|ref| of the
 compiled reference (whose x86 decode kernel sums the same terms in f32 lanes).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -519,6 +521,37 @@ def test_both_tiles_of_the_32_value_formats_under_a_prompt(oxh, qtype, rows, col
     for v in sorted({0, 15, 16, 31, 32, 63, 64, 65, n_vec // 2, n_vec - 2, n_vec - 1}):
         want, _ = oracle_matvec(qtype, w, rows, cols, np.ascontiguousarray(xs[v]))
         assert np.array_equal(bits(outs[v, :rows]), bits(want)), v
+
+
+def test_the_32_value_formats_under_more_tiles_than_a_grid_holds(oxh):
+    """513 rows are sixteen row tiles with the ones that pad them to whole runs of eight: beyond 33 554 368 activations the
+    tiles' threads pass 2^32 and the call is two launches.  A thousand activations, repeated; the outputs at the start, on
+    both sides of the seam and at the end have the oracle's bits."""
+    rows, cols, unit, seam = 513, 32, 1000, 33554368
+    n_vec = seam + 70
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    mv.check(mv.lib().oxh_mem_info(ctypes.byref(free), ctypes.byref(total)))
+    if free.value < 80 << 30:
+        pytest.skip("needs 70 GB of device memory")
+    w = synth.weights(Q80, rows, cols, seed=90, stream=1)
+    xs = synth.normal(unit * cols, seed=90, stream=2).reshape(unit, cols)
+    want = np.zeros((unit, rows), np.uint32)
+    nact = mv.act_bytes(Q80, cols)
+    d_w, d_x, d_a = mv.DeviceBuffer.from_host(w), mv.DeviceBuffer.from_host(xs), mv.DeviceBuffer(n_vec * nact)
+    mv.quantize(Q80, d_x.ptr, cols, unit, cols, d_a.ptr)
+    have = unit * nact
+    while have < d_a.nbytes:
+        n = min(have, d_a.nbytes - have)
+        mv.copy_d2d(d_a.ptr + have, d_a.ptr, n)
+        have += n
+    d_out = mv.DeviceBuffer(n_vec * rows * 4)
+    mv.mmq(Q80, d_w.ptr, rows, cols, d_a.ptr, n_vec, d_out.ptr, rows)
+    mv.sync()
+    for v in range(unit):
+        want[v] = bits(oracle_matvec(Q80, w, rows, cols, np.ascontiguousarray(xs[v]))[0])
+    for first, count in ((0, unit), (n_vec // 2, 300), (seam - 300, 300 + 70)):
+        got = d_out.download(np.uint32, count * rows, first * rows * 4).reshape(count, rows)
+        assert np.array_equal(got, want[(first + np.arange(count)) % unit]), first
 
 
 @pytest.mark.parametrize("qtype,rows,cols,n_vec", [(Q4K, 40, 512, 3), (Q80, 33, 256, 1), (Q6K, 70, 256, 8)])
