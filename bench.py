@@ -280,7 +280,7 @@ def secondary_figures(mv, synth):
     out["q2k_q3k_prefill_14336x4096x512"] = pre
     for b_ in (d_x, d_a, d_o, d_wide):
         b_.free()
-    # the 32-value formats, 512 activations: 128 x 64 tiles, one 16x16x32 MFMA per block and token chunk
+    # the 32-value formats, 512 activations: 64 x 64 or 128 x 64 tiles, one 16x16x32 MFMA per block and token chunk
     rows, cols, nv = 4096, 4096, 512
     d_x = mv.DeviceBuffer.from_host(synth.normal(nv * cols, seed=0, stream=2009))
     d_a = mv.DeviceBuffer(nv * mv.act_bytes(Q80, cols))

@@ -383,12 +383,12 @@ int oxh_mmq_split(uint32_t qtype, const void *d_w, size_t rows, size_t cols,
 /* The tile (weight rows x activations per workgroup) that the rule on sizes names for
  * a launch on a device of n_cu compute units: the largest of 256 x 128 (128 x 128 for
  * Q5_K, Q6_K and widened Q2_K), 64 x 128 (Q6_K only), 128 x 64, 64 x 32, 64 x 16
- * that still gives nearly every compute unit a workgroup; 128 x 64 always for
- * the 32-value formats.  Q4_K and Q5_K launches of more than 64 activations run on
- * that tile.  Others may run on another one, with the same bits: the 32-value formats
- * in halves of 64 x 64 unless one round of whole ones fits the device best, Q6_K and
- * widened Q2_K weigh the tiles' measured times on top, and K-quant launches of up to
- * 64 activations may go to a kernel with a workgroup per 16 rows
+ * that still gives nearly every compute unit a workgroup; for the 32-value formats
+ * 64 x 64, or 128 x 64 where one round of those fits the device best.  Launches of
+ * the 32-value formats, and Q4_K and Q5_K ones of more than 64 activations, run on
+ * that tile.  Others may run on another one, with the same bits: Q6_K and widened
+ * Q2_K go by the tiles' measured times, and K-quant launches of up to 64
+ * activations may go to a kernel with a workgroup per 16 rows
  * (oxh_lab()->mmq_kernel says what a launch runs on).  Pure host arithmetic (no
  * device needed); OXH_DECLINED for a type without a matrix-core kernel.
  * The reference has no counterpart: its batch kernel takes four activations

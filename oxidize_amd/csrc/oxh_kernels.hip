@@ -2285,9 +2285,11 @@ static int mmq80_leg(uint32_t qtype)
 extern "C" int oxh_mmq_tile(uint32_t qtype, size_t rows, size_t n_vec, size_t n_cu, uint32_t *tile_rows,
                             uint32_t *tile_tokens)
 {
-    if (mmq80_leg(canon_qtype(qtype)) >= 0 && rows && n_vec && n_cu) {       /* one tile for these */
-        if (tile_rows) *tile_rows = 128u;
-        if (tile_tokens) *tile_tokens = 64u;
+    if (mmq80_leg(canon_qtype(qtype)) >= 0 && rows && n_vec && n_cu) {
+        uint32_t tile[2];
+        oxh_internal_mmq32_tile(rows, n_vec, n_cu, tile);
+        if (tile_rows) *tile_rows = tile[0];
+        if (tile_tokens) *tile_tokens = tile[1];
         return OXH_OK;
     }
     const bool one_chunk = qtype == OXH_Q6_K || is_q5k(qtype) || qtype == OXH_Q2_K_WIDE;
@@ -2517,12 +2519,12 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
     if (!d_w || !d_acts || !d_out) return arg_fail("oxh_mmq: NULL pointer");
     const int leg = mmq80_leg(canon_qtype(qtype));
     if (leg >= 0 && oxh_act_kind(qtype, cols) == 1) {
-        /* 32-value blocks against Q8_0 activations: one tile shape, exact f32 step only */
+        /* 32-value blocks against Q8_0 activations: exact f32 step only */
         if (out_stride < rows) return arg_fail("oxh_mmq: out_stride < rows");
         const size_t blocks32 = cols / OXH_QK8_0;
         if (rows > 0x7FFFFFFFull || n_vec > 0x7FFFFFFFull || blocks32 > 0xFFFFFFull)
             return arg_fail("oxh_mmq: dimension too large");
-        if (blocks32 * block_bytes(qtype) < 16u) {
+        if (blocks32 * block_bytes(qtype) < 16u) {      /* a single AL5_XS block: the tiles would take it, the interface does not */
             snprintf(g_err, sizeof g_err, "oxh_mmq: rows of qtype %u with cols %zu are shorter than 16 bytes", qtype, cols);
             return OXH_DECLINED;
         }

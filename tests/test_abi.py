@@ -263,9 +263,13 @@ def test_mmq_tile_choice_is_host_arithmetic():
             for n_vec in (1, 16, 17, 32, 33, 64, 100, 128, 129, 512, 2048):
                 for n_cu in (64, 256, 304):
                     assert tile(qtype, rows, n_vec, n_cu) == (0,) + rule(qtype, rows, n_vec, n_cu)
-    # the 32-value formats have one tile; the codebook formats have no matrix-core kernel
+    # the 32-value formats have two, and run on the one named; the codebook formats have no matrix-core kernel
     for qtype in (Q80, 3, 4, 5, 6, 17, 18, 19, 20):
         assert tile(qtype, 4096, 512) == (0, 128, 64)
+        for rows, n_vec in ((64, 17), (4096, 64), (4096, 512), (4224, 448), (14336, 512), (151936, 2048)):
+            for n_cu in (64, 256, 304):
+                assert tile(qtype, rows, n_vec, n_cu)[1:] == mv.mmq_kernel(qtype, rows, 4096, n_vec, n_cu)[1:3]
+        assert tile(qtype, 14336, 512) == (0, 64, 64)
     assert tile(25, 4096, 512)[0] == _lib.DECLINED
     assert tile(Q4K, 0, 512)[0] == _lib.DECLINED
     assert lib.oxh_mmq_tile(Q4K, 4096, 512, 256, None, None) == 0

@@ -460,19 +460,19 @@ def test_long_batches_of_types_without_a_tile_kernel(oxh, qtype, cols, n_vec):
 
 
 @pytest.mark.parametrize("qtype,rows,cols,n_vec", [
-    (Q80, 70, 896, 600),        # 28 blocks: a full step and a short one; ragged row and token tiles
-    (Q80, 130, 4096, 65),       # a second row tile of two rows, a second token tile of one token
+    (Q80, 70, 896, 600),        # 28 blocks: three full steps and a half; ragged row and token tiles
+    (Q80, 130, 4096, 65),       # a third row tile of two rows, a second token tile of one token
     (Q80, 16, 32, 64),          # one block per row
     (3, 257, 1024, 64),         # Q4_0
     (4, 128, 544, 100),         # Q4_1, 17 blocks: the last step is a single block
     (5, 17, 992, 33),           # Q5_0, 31 blocks: an odd last step
     (6, 300, 2048, 129),        # Q5_1
-    (18, 129, 1056, 70),        # AL5_XS, 33 blocks of 14 bytes: a last step shorter than one 16-byte piece
+    (18, 129, 1056, 70),        # AL5_XS, 33 blocks of 14 bytes: a last step of one, shorter than 16 bytes
     (20, 64, 512, 17),          # AL8: the Q8_0 layout under its own id
 ])
 def test_token_tiled_kernel_of_the_32_value_formats(oxh, qtype, rows, cols, n_vec):
-    """oxh_mmq over the 32-value formats (128 rows x 64 tokens per workgroup, activations staged sixteen
-    blocks at a time): every output is the single-vector dot, bit for bit, and nothing outside the
+    """oxh_mmq over the 32-value formats (64 rows x 64 tokens per workgroup, eight blocks of weights and
+    activations staged at a time): every output is the single-vector dot, bit for bit, and nothing outside the
     rows x n_vec outputs is written."""
     canon = {17: 3, 19: 5, 20: 7}.get(qtype, qtype)
     w = synth.weights(canon, rows, cols, seed=83, stream=rows + cols)
@@ -484,7 +484,7 @@ def test_token_tiled_kernel_of_the_32_value_formats(oxh, qtype, rows, cols, n_ve
     mv.quantize(qtype, d_x.ptr, cols, n_vec, cols, d_a.ptr)
     stride = rows + 3
     d_out = mv.DeviceBuffer.from_host(np.full((n_vec, stride), -7.25, np.float32))
-    assert mv.mmq_tile(qtype, rows, n_vec, 256) == (128, 64)
+    assert mv.mmq_tile(qtype, rows, n_vec, 256) == (64, 64) == mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3]
     mv.mmq(qtype, d_w.ptr, rows, cols, d_a.ptr, n_vec, d_out.ptr, stride)
     mv.sync()
     outs = d_out.download(np.float32, n_vec * stride).reshape(n_vec, stride)
@@ -498,13 +498,17 @@ def test_token_tiled_kernel_of_the_32_value_formats(oxh, qtype, rows, cols, n_ve
     (Q80, 2049, 288, 510, (128, 64)),       # 33 x 8 tiles of 64 rows, 17 x 8 of 128: one round of these; 9 blocks, one row over
     (6, 2150, 544, 449, (128, 64)),         # Q5_1: minimums and sums, sixteen waves; 17 blocks
     (18, 2112, 96, 512, (128, 64)),         # AL5_XS, 3 blocks: rows of 42 bytes
+    (3, 2177, 288, 480, (128, 64)),         # Q4_0: blocks on odd half words; 18 row tiles, three of them on one XCD
+    (4, 2070, 352, 512, (128, 64)),         # Q4_1: minimums and sums on the wide tile; 11 blocks
+    (5, 2300, 416, 430, (128, 64)),         # Q5_0, 13 blocks
     (Q80, 2048, 288, 512, (64, 64)),        # 256 tiles of 64 rows: one to a CU
     (5, 4161, 256, 513, (64, 64)),          # Q5_0: 33 x 9 tiles of 128 rows would be a second round
     (4, 63, 224, 127, (64, 64)),            # Q4_1, 7 blocks: half a step and its odd half
 ])
 def test_both_tiles_of_the_32_value_formats_under_a_prompt(oxh, qtype, rows, cols, n_vec, tile):
     """oxh_mmq on tiles of 64 and of 128 rows: bits of the single-vector dots at the tiles' edges, stores of four
-    results at a time (output rows a multiple of four floats apart) and nothing written beside the outputs."""
+    results at a time (output rows a multiple of four floats apart) and nothing written beside the outputs; the same
+    from a matrix that starts two bytes past a multiple of four."""
     if mv.device_info()["n_cu"] == 256:
         assert mv.mmq_kernel(qtype, rows, cols, n_vec)[1:3] == tile
     w = synth.weights(qtype, rows, cols, seed=89, stream=rows + cols)
@@ -521,6 +525,11 @@ def test_both_tiles_of_the_32_value_formats_under_a_prompt(oxh, qtype, rows, col
     for v in sorted({0, 15, 16, 31, 32, 63, 64, 65, n_vec // 2, n_vec - 2, n_vec - 1}):
         want, _ = oracle_matvec(qtype, w, rows, cols, np.ascontiguousarray(xs[v]))
         assert np.array_equal(bits(outs[v, :rows]), bits(want)), v
+    # the same matrix two bytes into an allocation: every block on the other half word
+    d_w2 = mv.DeviceBuffer(w.nbytes + 2)
+    d_w2.upload(w.view(np.uint8), 2)
+    mv.mmq(qtype, d_w2.ptr + 2, rows, cols, d_a.ptr, n_vec, d_out.ptr, stride)
+    assert np.array_equal(d_out.download(np.uint32, n_vec * stride).reshape(n_vec, stride), bits(outs))
 
 
 def test_the_32_value_formats_under_more_tiles_than_a_grid_holds(oxh):
