@@ -278,6 +278,8 @@ def test_layer_with_prefill_sized_token_counts(oxh, qt_gu, qt_dn):
     (Q6K, Q5K, 8, 2, 256, 3584, 581, ((128, 144), (128, 64))),  # Q6_K, ragged counts above 144
     (Q4K, Q5K, 8, 2, 3584, 512, 130, ((64, 16), (128, 64))),    # experts below and just above 32, one with more than 64
     (Q6K, Q6K, 16, 1, 1792, 512, 400, ((64, 16), (128, 64))),
+    (Q4K, Q5K, 64, 8, 256, 512, 600, ((256, 144), (128, 64))),  # a lane per expert; tiles of 4, 5, 6 and 8 chunks, the popular expert four
+    (Q4K, Q4K, 37, 6, 256, 768, 900, ((256, 144), (128, 64))),  # one or two tiles of 5 to 9 chunks, the popular expert six
 ])
 def test_layer_on_the_tiles_for_many_tokens(oxh, qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok, tiles):
     """The kernels that deal an expert's 16-token chunks evenly to its tiles: every tile size of every type, with
