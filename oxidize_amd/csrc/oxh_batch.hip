@@ -21,9 +21,10 @@
  * twice the lines of loads along a row's bytes: straight into registers 4096 x 14336
  * (Q6_K, 16 activations) took 29.6 us, this way 18.1, quantiser included; the split
  * tiles 26.
- * What bounds it: 48 MB in some 13 us is 3.7 TB/s; the operand build (300 vector
- * instructions per super-block) and the activations, 292 bytes per token and
- * super-block read by every workgroup from the L2 again, come next. */
+ * What bounds it: not settled.  48 MB in some 13 us is 3.7 TB/s; the compiled loop
+ * has 209 vector instructions per super-block and wave (Q6_K, 16 activations), at 4
+ * cycles each 5 us of it; each super-block begins with a wait for loads asked for one
+ * super-block earlier. */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -6,19 +6,22 @@
  * offset are staged as the signed values code - offset, so four formats share Q8_0's step exactly.
  *
  * What bounds it.  The float step: four vector instructions per result and block (seven for the _1 formats) beside a
- * 256th of an MFMA, 64 cycles of a SIMD's issue port per 16 x 16 tile against the MFMA's 16 (4096 x 4096 x 512: some
- * 30 us of it).  So everything else has to stay off that port: a block is fetched and taken apart ONCE per
+ * 256th of an MFMA.  Alone on a SIMD with two or four waves those four (multiply, convert, multiply, add) take 2.6 cycles
+ * each, 41 per 16 x 16 tile, the MFMA 8, both in one loop 55: 4096 x 4096 x 512 would be 23 us of that loop.  So
+ * everything else has to stay off that port: a block is fetched and taken apart ONCE per
  * workgroup, by a lane that owns it (eight lanes along a row's consecutive blocks, so that a wave's load touches some
  * 24 cache lines and not 64), and goes to LDS as MFMA operands, int8 values and f32 scales; the inner loop issues
- * MFMAs, the float step and nothing else but LDS reads, eleven of 16 bytes per eight tiles.  Of a wave's 310 vector
- * instructions per step of eight blocks 256 are the float step.
+ * MFMAs, the float step and nothing else but LDS reads, twelve of 16 bytes per eight tiles (eighteen for the _1
+ * formats).  Of the compiled step of eight blocks' 335 vector instructions (Q8_0; Q4_1 537) 256 (448) are the float step.
  *
  * Shape.  A wave computes 16 rows x 32 tokens; eight waves, 64 rows x 64 tokens, to a workgroup and two workgroups to
- * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues a vector
- * instruction every eight cycles at best.  Steps of eight blocks, two stages in LDS, one
+ * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues dependent
+ * vector instructions 8.3 cycles apart and independent ones 4.7 to 5.4.  Steps of eight blocks, two stages in LDS, one
  * barrier per step; the next step's blocks go to LDS in the middle of a step and the ones after it are requested
  * then.  Q8_0 4096 x 4096 x 512 takes 41 us (128 x 64 tiles whose waves kept raw blocks in regions of their own, one
- * workgroup to a CU: 69; 128 x 64 on eight waves of 32 x 32: 42.5, and 162 us at 14336 rows where this takes 136). */
+ * workgroup to a CU: 69; 128 x 64 on eight waves of 32 x 32: 42.5, and 162 us at 14336 rows where this takes 136).
+ * At the 128 registers that four waves allow, Q4_1's narrow tile spills 12 bytes, its wide one and Q5_1's narrow one 4;
+ * one reload, 8 bytes in Q4_1's narrow tile, is inside the step loop. */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
