@@ -63,12 +63,18 @@ typedef struct OxhLab {
                       uint32_t out[4]);
     /* The same for one expert launch of oxh_moe_ffn: n_mat matrices of `rows`
      * rows per expert (gate and up 2, down 1) under `pairs` (token, expert)
-     * pairs in all; tile: rows and tokens of a workgroup. */
+     * pairs in all; tile: rows and tokens of a workgroup, where the launch is
+     * one of tiles (see experts_batch). */
     int (*experts_tile)(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu,
                         uint32_t tile[2]);
     /* Chunks that host batches have moved through the library's own
      * page-locked slots so far, both ways together. */
     size_t (*host_ring_chunks)(void);
+    /* Whether an expert launch of oxh_moe_ffn over rows x cols matrices gives
+     * every workgroup 16 rows and all their columns (1) or runs on the tile
+     * that experts_tile names (0); n_mat as there. */
+    int (*experts_batch)(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t cols, size_t top_k,
+                         size_t n_tok, size_t n_cu);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

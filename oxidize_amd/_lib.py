@@ -59,7 +59,8 @@ class OxhLab(ctypes.Structure):
                 ("subblock_sums", ctypes.CFUNCTYPE(I, U32, V, Z, Z, V, V, V)),
                 ("mmq_kernel", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 4))),
                 ("experts_tile", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 2))),
-                ("host_ring_chunks", ctypes.CFUNCTYPE(Z))]
+                ("host_ring_chunks", ctypes.CFUNCTYPE(Z)),
+                ("experts_batch", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, Z, Z))]
 
 
 # name -> (restype, argtypes); every symbol include/oxhip.h and include/oxhip_lab.h declare

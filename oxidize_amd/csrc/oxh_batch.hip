@@ -26,6 +26,7 @@
  * cycles each 5 us of it; each super-block begins with a wait for loads asked for one
  * super-block earlier. */
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 #include "oxhip.h"
@@ -157,10 +158,13 @@ template <int FMT, int CH> static inline uint32_t bat_lds_bytes(uint32_t B, uint
     return waves * BatGeom<FMT, CH>::WAVE_BYTES + B * CH * (64u + 1024u);
 }
 
-template <int FMT, int CH>
-__global__ __launch_bounds__(1024, 4) void
-k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t *__restrict__ acts, uint32_t n_vec,
-            float *__restrict__ out, size_t out_stride)
+/* One workgroup's 16 rows under at most CH * 16 activations, all columns.  w0: the first row's blocks; a0: the first
+ * activation; out: &out[first activation][first row].  TM: the tile-major layout, whose 16 blocks of a block index lie
+ * next to each other (whole groups only). */
+template <int FMT, int CH, bool TM>
+__device__ __forceinline__ void
+bat_tile(const uint8_t *__restrict__ w0, uint32_t rows_here, uint32_t B, const uint8_t *__restrict__ a0, uint32_t toks,
+         float *__restrict__ out, size_t out_stride)
 {
     typedef BatGeom<FMT, CH> G;
     extern __shared__ __attribute__((aligned(16))) uint8_t bat_lds[];
@@ -170,10 +174,9 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
     uint8_t *my = bat_lds + wave * G::WAVE_BYTES;
     const uint32_t my_at = (uint32_t)(size_t)(__attribute__((address_space(3))) uint8_t *)bat_lds + wave * G::WAVE_BYTES;
     float *s_dq = reinterpret_cast<float *>(bat_lds + waves * G::WAVE_BYTES), *s_term = s_dq + B * CH * 16u;
-    const uint32_t row0 = blockIdx.x * 16u, tok0 = blockIdx.y * (CH * 16u);
-    const uint32_t rows_here = min(rows - row0, 16u), toks = min(n_vec - tok0, CH * 16u);
     const uint32_t act_stride = B * 292u;
-    const uint8_t *w0 = w + (size_t)row0 * B * G::WB, *a0 = acts + (size_t)tok0 * act_stride;
+    static_assert(!TM || G::DMA, "Q4_K and Q5_K have a tile-major form");
+    constexpr uint32_t W_STEP = TM ? 16u * G::WB : G::WB;                /* from one super-block to the next */
 
     /* loads run along the contiguous bytes of a row's block and of a token's values; rows and tokens past the
      * last are the last again */
@@ -181,7 +184,7 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
 #pragma unroll
     for (uint32_t i = 0; i < G::LOADS; i++) {
         const uint32_t g = min(64u * i + lane, G::PIECES - 1u), r = g / G::WP, part = g - G::WP * r;
-        w_off[i] = min(r, rows_here - 1u) * (B * G::WB) + 16u * part;
+        w_off[i] = TM ? 16u * g : min(r, rows_here - 1u) * (B * G::WB) + 16u * part;
         w_dst[i] = r * G::W_PITCH + 16u * part;
     }
 #pragma unroll
@@ -197,7 +200,7 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
     struct { U32x4u2 q[G::DMA ? 1 : G::LOADS]; uint16_t d; } wr;         /* Q6/Q2: the next block on its way */
     uint2 sums[CH];                                                     /* Q4/Q5: its tokens' sums 4 kq .. + 3 */
     auto request = [&](uint32_t b, uint32_t buf) {
-        const uint8_t *wb = w0 + (size_t)b * G::WB, *ab = a0 + (size_t)b * 292u;
+        const uint8_t *wb = w0 + (size_t)b * W_STEP, *ab = a0 + (size_t)b * 292u;
         if constexpr (G::DMA) {
 #pragma unroll
             for (uint32_t i = 0; i < G::LOADS; i++)
@@ -293,12 +296,61 @@ k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        /* the last request's, which nobody reads */
     __syncthreads();
     for (uint32_t i = tid; i < CH * 256u; i += blockDim.x) {
-        const uint32_t tok = i >> 4, row = row0 + (i & 15u);
+        const uint32_t tok = i >> 4, row = i & 15u;
         float acc = 0.0f;
 #pragma unroll 8
         for (uint32_t b = 0; b < B; b++) acc += s_term[b * CH * 256u + i];
-        if (tok < toks && row < rows) out[(size_t)(tok0 + tok) * out_stride + row] = acc;
+        if (tok < toks && row < rows_here) out[(size_t)tok * out_stride + row] = acc;
     }
+}
+
+template <int FMT, int CH>
+__global__ __launch_bounds__(1024, 4) void
+k_mmq_batch(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t *__restrict__ acts, uint32_t n_vec,
+            float *__restrict__ out, size_t out_stride)
+{
+    const uint32_t row0 = blockIdx.x * 16u, tok0 = blockIdx.y * (CH * 16u);
+    bat_tile<FMT, CH, false>(w + (size_t)row0 * B * BatGeom<FMT, CH>::WB, min(rows - row0, 16u), B,
+                             acts + (size_t)tok0 * B * 292u, min(n_vec - tok0, CH * 16u),
+                             out + (size_t)tok0 * out_stride + row0, out_stride);
+}
+
+/* The same over the experts of a mixture-of-experts layer that got tokens, whose numbers are known on the device only:
+ * grid.x walks the 16-row groups of the launch's one or two matrices, grid.y the (expert, token tile) pairs, expert by
+ * expert.  The grid has as many y as any routing can need; what is beyond the last leaves at once. */
+struct BatExperts {
+    const uint8_t *w[2];
+    float *out[2];
+    uint32_t rows, B, groups, n_expert;
+    const uint8_t *acts;
+    size_t out_stride;
+    const uint32_t *counts, *offsets;
+};
+
+template <int FMT, int CH, bool TM>
+__global__ __launch_bounds__(1024, 4) void
+k_mmq_batch_experts(const BatExperts a)
+{
+    constexpr uint32_t TOK = CH * 16u;
+    const uint32_t lane = threadIdx.x & 63u;
+    /* a lane per expert: its tiles and, by ballots over the bits of their numbers, how many the experts before it have */
+    const uint32_t cnt = lane < a.n_expert ? a.counts[lane] : 0u, off = lane < a.n_expert ? a.offsets[lane] : 0u;
+    const uint32_t tiles = (cnt + TOK - 1u) / TOK;
+    uint32_t from = 0u;
+    for (uint32_t k = 0u; __ballot((tiles >> k) != 0u) != 0ull; k++) {
+        const unsigned long long set = __ballot(((tiles >> k) & 1u) != 0u);
+        from += __builtin_amdgcn_mbcnt_hi((uint32_t)(set >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)set, 0u)) << k;
+    }
+    const unsigned long long mine = __ballot(blockIdx.y >= from && blockIdx.y - from < tiles);
+    if (mine == 0ull) return;
+    const int e = __builtin_ctzll(mine);
+    const uint32_t tok0 = (blockIdx.y - (uint32_t)__builtin_amdgcn_readlane((int)from, e)) * TOK;
+    const uint32_t toks = min((uint32_t)__builtin_amdgcn_readlane((int)cnt, e) - tok0, TOK);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)off, e) + tok0;
+    const uint32_t second = blockIdx.x >= a.groups ? 1u : 0u, row0 = (blockIdx.x - second * a.groups) * 16u;
+    bat_tile<FMT, CH, TM>((second ? a.w[1] : a.w[0]) + ((size_t)e * a.rows + row0) * a.B * BatGeom<FMT, CH>::WB,
+                          min(a.rows - row0, 16u), a.B, a.acts + (size_t)first * a.B * 292u, toks,
+                          (second ? a.out[1] : a.out[0]) + (size_t)first * a.out_stride + row0, a.out_stride);
 }
 
 template <typename K> static hipError_t bat_whole_lds(K kernel)
@@ -317,8 +369,14 @@ extern "C" int oxh_internal_batch_init(void)
     if ((e = bat_whole_lds(k_mmq_batch<BAT_Q6, 1>)) != hipSuccess) return (int)e;
     if ((e = bat_whole_lds(k_mmq_batch<BAT_Q6, 2>)) != hipSuccess) return (int)e;
     if ((e = bat_whole_lds(k_mmq_batch<BAT_Q2W, 1>)) != hipSuccess) return (int)e;
+    if ((e = bat_whole_lds(k_mmq_batch_experts<BAT_Q4, 1, false>)) != hipSuccess) return (int)e;
+    if ((e = bat_whole_lds(k_mmq_batch_experts<BAT_Q4, 1, true>)) != hipSuccess) return (int)e;
+    if ((e = bat_whole_lds(k_mmq_batch_experts<BAT_Q5, 1, false>)) != hipSuccess) return (int)e;
+    if ((e = bat_whole_lds(k_mmq_batch_experts<BAT_Q5, 1, true>)) != hipSuccess) return (int)e;
+    if ((e = bat_whole_lds(k_mmq_batch_experts<BAT_Q6, 1, false>)) != hipSuccess) return (int)e;
     return (int)bat_whole_lds(k_mmq_batch<BAT_Q2W, 2>);
 }
+
 static uint32_t bat_need(int fmt, uint32_t ch, uint32_t B, uint32_t waves)
 {
     switch (fmt) {
@@ -433,5 +491,76 @@ extern "C" int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, siz
     } else {
         OXH_BATCH_F(2)
     }
+    return (int)hipGetLastError();
+}
+
+/* (expert, token tile) pairs any routing can need */
+static size_t exp_slots(size_t n_expert, size_t pairs, size_t max_tokens)
+{
+    const size_t by_pairs = (pairs + n_expert * 15) / 16, each = (max_tokens + 15) / 16;
+    const size_t live = pairs < n_expert ? pairs : n_expert;
+    return live * each < by_pairs ? live * each : by_pairs;
+}
+
+/* Workgroups that find tokens when each token chooses its experts evenly: the experts some token chose, a token tile
+ * each, or where they have more tokens than eight half a tile more than those fill. */
+static double exp_workgroups(size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_tok)
+{
+    const double missed = 1.0 - (double)pairs / (double)n_tok / (double)n_expert;
+    const double hit = (double)n_expert * (1.0 - pow(missed > 0.0 ? missed : 0.0, (double)n_tok));
+    const double filled = 0.5 * hit + (double)pairs / 16.0;
+    return (double)(n_mat * ((rows + 15) / 16)) * (hit > filled ? hit : filled);
+}
+
+/* The rule, against the 64-row tiles of the experts (and the long ones, where those are taken).  From 1300 random layers
+ * (4, 8 and 16 experts, top 1 to 3, 1024 x 768 to 4096 x 14336, 1 to 100 tokens; the layer's time with this kernel for one
+ * of its launches / without): the fewer workgroups a CU gets the more is gained, and more than the tiles' way through
+ * all of a row's super-blocks costs is lost once the device is full of tiles as well, since each of these workgroups
+ * stages the tokens for 16 rows only.  Where LDS holds two workgroups the lines lie at four to a CU (Q4_K, Q5_K) and six
+ * (Q6_K, whose tiles take longest), where it holds one at three and four and a half: one layer in a hundred within them is
+ * slower, by 1 to 4 %.  us a layer, without / with: down of 16 experts 2560 x 6144, Q6_K, 3 tokens 69.6 / 44.3; of four
+ * 1536 x 5120, Q4_K, 36 tokens 38.8 / 31.3; gate and up of 16 of 4096 x 3072, Q4_K, two tokens 50.2 / 40.3; beyond the
+ * lines, down of 8 of 4096 x 14336, Q4_K, 16 tokens 162 / 190. */
+extern "C" int oxh_internal_experts_batch_takes(int fmt, size_t n_mat, size_t n_expert, size_t rows, size_t blocks, size_t pairs,
+                                                size_t n_tok, size_t cus)
+{
+    if (blocks < 2 || blocks > 128 || pairs == 0 || n_tok == 0 || n_expert > 64) return 0;
+    const uint32_t need = bat_need(fmt, 1, (uint32_t)blocks, 4);
+    if (need > BAT_LDS) return 0;
+    const double per_cu = 2u * need > BAT_LDS ? 0.75 : 1.0;
+    return exp_workgroups(n_mat, n_expert, rows, pairs, n_tok) <= per_cu * (fmt == BAT_Q6 ? 6.0 : 4.0) * (double)cus;
+}
+
+/* see oxh_internal.h */
+extern "C" int oxh_internal_experts_batch(int fmt, int tile_major, const void *const *d_w, float *const *d_out, size_t n_mat,
+                                          size_t n_expert, size_t rows, size_t blocks, const void *d_acts, size_t out_stride,
+                                          const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs,
+                                          size_t max_tokens, void *stream)
+{
+    const size_t cus = (size_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
+    BatExperts a;
+    for (int i = 0; i < 2; i++) {
+        a.w[i] = (const uint8_t *)d_w[(size_t)i < n_mat ? i : 0];
+        a.out[i] = d_out[(size_t)i < n_mat ? i : 0];
+    }
+    a.rows = (uint32_t)rows;
+    a.B = (uint32_t)blocks;
+    a.groups = (uint32_t)((rows + 15) / 16);
+    a.n_expert = (uint32_t)n_expert;
+    a.acts = (const uint8_t *)d_acts;
+    a.out_stride = out_stride;
+    a.counts = d_counts;
+    a.offsets = d_offsets;
+    const size_t slots = exp_slots(n_expert, pairs, max_tokens);
+    const dim3 grid((uint32_t)(n_mat * a.groups), (uint32_t)slots);
+    const uint32_t waves = oxh_internal_mmq_batch_waves(fmt, 16 * n_mat * a.groups * slots, blocks, 1, cus);
+    const uint32_t lds = bat_need(fmt, 1, a.B, waves);
+#define OXH_EXPB(FMT, TM) hipLaunchKernelGGL((k_mmq_batch_experts<FMT, 1, TM>), grid, dim3(64u * waves), lds, (hipStream_t)stream, a)
+    if (fmt == BAT_Q6) OXH_EXPB(BAT_Q6, false);
+    else if (fmt == BAT_Q5 && tile_major) OXH_EXPB(BAT_Q5, true);
+    else if (fmt == BAT_Q5) OXH_EXPB(BAT_Q5, false);
+    else if (tile_major) OXH_EXPB(BAT_Q4, true);
+    else OXH_EXPB(BAT_Q4, false);
+#undef OXH_EXPB
     return (int)hipGetLastError();
 }

@@ -73,6 +73,11 @@ int oxh_internal_mmq_batch_takes(int fmt, size_t rows, size_t blocks, size_t n_v
 uint32_t oxh_internal_mmq_batch_waves(int fmt, size_t rows, size_t blocks, size_t n_vec, size_t cus);
 int oxh_internal_mmq_batch(int fmt, const void *d_w, size_t rows, size_t blocks, const void *d_acts, size_t n_vec, float *d_out,
                            size_t out_stride, void *stream);
+int oxh_internal_experts_batch_takes(int fmt, size_t n_mat, size_t n_expert, size_t rows, size_t blocks, size_t pairs,
+                                     size_t n_tok, size_t cus);
+int oxh_internal_experts_batch(int fmt, int tile_major, const void *const *d_w, float *const *d_out, size_t n_mat,
+                               size_t n_expert, size_t rows, size_t blocks, const void *d_acts, size_t out_stride,
+                               const uint32_t *d_counts, const uint32_t *d_offsets, size_t pairs, size_t max_tokens, void *stream);
 /* Whether the runtime knows all of this memory (page-locked, managed or on the device) and so copies it without a
  * detour through staging of its own. */
 int oxh_internal_runtime_memory(const void *p, size_t bytes);
@@ -95,6 +100,8 @@ int oxh_debug_moe_workspace_parts(const struct OxhMoe *m, size_t n_tok, size_t p
 int oxh_debug_read_probe(const void *d_buf, size_t bytes, uint32_t *d_sink, void *stream);
 int oxh_debug_mfma_probe(int valu_per_mfma, int waves_per_simd, double *pops);
 int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, size_t n_vec, size_t n_cu, size_t ws_bytes, uint32_t out[4]);
+int oxh_debug_experts_batch(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t cols, size_t top_k, size_t n_tok,
+                            size_t n_cu);
 int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu, uint32_t tile[2]);
 int oxh_debug_subblock_sums(uint32_t qtype, const void *d_w, size_t rows, size_t cols, const void *d_act,
                             int32_t *d_sums, void *stream);

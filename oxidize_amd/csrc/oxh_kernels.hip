@@ -2910,13 +2910,20 @@ static int launch_experts_tiled(uint32_t qtype, const void *const *d_w, float *c
  *   1024 x 2048, 13 tokens 206 / 248).
  * OXH_MOE_BIG_TILE_FROM takes all this back: the long tiles from that many tokens per expert on, whatever the sizes, 0 =
  * never. */
+#define OXH_BY_RULE 0xFFFFFFFFu
+static uint32_t experts_long_from(void)
+{
+    static const uint32_t big_from = env_u32("OXH_MOE_BIG_TILE_FROM", OXH_BY_RULE, 0, 4096);
+    return big_from;
+}
+
 static bool experts_long(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t cus)
 {
     const size_t avg_tokens = pairs / n_expert;
-    static const uint32_t by_rule = 0xFFFFFFFFu, big_from = env_u32("OXH_MOE_BIG_TILE_FROM", by_rule, 0, 4096);
+    const uint32_t big_from = experts_long_from();
     const size_t wide_tiles = n_mat * ((rows + 127) / 128) * n_expert;
     const size_t small_tiles = n_mat * ((rows + 63) / 64) * pairs / 16;
-    if (big_from != by_rule) return big_from && avg_tokens >= big_from;
+    if (big_from != OXH_BY_RULE) return big_from && avg_tokens >= big_from;
     if (avg_tokens >= 24 && (avg_tokens > 64 || wide_tiles >= cus - cus / 8)) return true;
     if (n_mat * n_expert > OXH_MAX_SEGS && avg_tokens >= 10 && small_tiles >= 8 * cus) return true;
     if (is_q5k(file_type))
@@ -2941,7 +2948,30 @@ static bool experts_wide_small(uint32_t file_type, size_t n_mat, size_t n_expert
            n_mat * live * ((rows + 127) / 128) >= cus - cus / 8;
 }
 
-/* the tile (rows, tokens) of one expert launch of oxh_moe_ffn: 64 x 16 or 128 x 16, or one of oxh_experts.hip */
+static int batch_fmt(uint32_t file_type)
+{
+    return file_type == OXH_Q6_K ? 2 : is_q5k(file_type) ? 1 : 0;
+}
+
+/* a 16-row group to a workgroup whose waves share the columns (oxh_batch.hip), unless one of the two switches above
+ * asks for a tile */
+static bool experts_batch(uint32_t file_type, size_t n_mat, size_t n_expert, size_t rows, size_t blocks, size_t pairs,
+                          size_t n_tok, size_t cus)
+{
+    if (experts_long_from() != OXH_BY_RULE || experts_wide_small(file_type, n_mat, n_expert, rows, pairs, cus)) return false;
+    return oxh_internal_experts_batch_takes(batch_fmt(file_type), n_mat, n_expert, rows, blocks, pairs, n_tok, cus) != 0;
+}
+
+extern "C" int oxh_debug_experts_batch(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t cols, size_t top_k,
+                                       size_t n_tok, size_t n_cu)
+{
+    const uint32_t file_type = t16_base(qtype);
+    if ((!is_q4k(file_type) && !is_q5k(file_type) && file_type != OXH_Q6_K) || !n_mat || !n_expert || !n_cu) return 0;
+    return experts_batch(file_type, n_mat, n_expert, rows, cols / OXH_QK_K, n_tok * top_k, n_tok, n_cu) ? 1 : 0;
+}
+
+/* the tile (rows, tokens) of one expert launch of oxh_moe_ffn that experts_batch does not take: 64 x 16 or 128 x 16, or
+ * one of oxh_experts.hip */
 extern "C" int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu,
                                       uint32_t tile[2])
 {
@@ -2964,6 +2994,13 @@ static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *
 {
     const uint32_t file_type = t16_base(qtype);
     const size_t cus = (size_t)(g_n_cu > 0 ? g_n_cu : 256);
+    if (experts_batch(file_type, n_mat, n_expert, rows, cols / OXH_QK_K, pairs, max_tokens, cus)) {
+        const int e = oxh_internal_experts_batch(batch_fmt(file_type), is_t16(qtype), d_w, d_out, n_mat, n_expert, rows,
+                                                 cols / OXH_QK_K, d_acts, out_stride, d_counts, d_offsets, pairs, max_tokens,
+                                                 pick_stream(stream));
+        if (e) return hip_fail((hipError_t)e, "expert launch");
+        return OXH_OK;
+    }
     if (experts_long(file_type, n_mat, n_expert, rows, pairs, cus)) {
         if (cols / OXH_QK_K * 292u * 256u > 0xFFFFFFFFull) return arg_fail("moe: cols too large");
         const int e = oxh_internal_experts_long(file_type, is_t16(qtype), d_w, d_out, n_mat, n_expert, rows, cols, d_acts,
@@ -3369,7 +3406,7 @@ extern "C" const OxhLab *oxh_lab(void)
 {
     static const OxhLab lab = { oxh_debug_plan_stamps, oxh_debug_plan_phantom, oxh_debug_moe_workspace_parts,
                                 oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums,
-                                oxh_debug_mmq_kernel, oxh_debug_experts_tile, oxh_debug_host_ring_chunks };
+                                oxh_debug_mmq_kernel, oxh_debug_experts_tile, oxh_debug_host_ring_chunks, oxh_debug_experts_batch };
     return &lab;
 }
 

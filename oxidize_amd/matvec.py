@@ -221,6 +221,11 @@ def experts_tile(qtype, n_mat, n_expert, rows, pairs, n_cu=256):
     return tuple(out)
 
 
+def experts_batch(qtype, n_mat, n_expert, rows, cols, top_k, n_tok, n_cu=256):
+    """Whether an expert launch gives every workgroup 16 rows and all their columns (include/oxhip_lab.h)."""
+    return bool(_lib.lab().experts_batch(qtype, n_mat, n_expert, rows, cols, top_k, n_tok, n_cu))
+
+
 def get_rows(qtype, d_w, rows, cols, d_ids, n_ids, d_out, out_stride, stream=None):
     check(lib().oxh_get_rows(qtype, ctypes.c_void_p(d_w), rows, cols, ctypes.c_void_p(d_ids), n_ids,
                              ctypes.c_void_p(d_out), out_stride, stream))

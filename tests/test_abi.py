@@ -367,6 +367,26 @@ def test_expert_launches_go_to_the_tile_that_measured_fastest():
         assert (mv.experts_tile(qtype, n_mat, n_expert, rows, n_expert * tokens) == (64, 16)) == small, (qtype, rows, tokens)
 
 
+def test_expert_launches_of_few_workgroups_go_to_those_of_16_rows():
+    """On 256 compute units: up to four (Q6_K six) workgroups of 16 rows to a unit where LDS holds two, three quarters of that
+    where it holds one; never over one super-block, nor against the switch that fixes the tiles."""
+    Q4K, Q5K, Q6K, T16, Q80 = 13, 15, 16, 0x100A, 7
+    b = mv.experts_batch
+    for qtype, n_mat, n_expert, rows, cols, k, n_tok, takes in (
+            (Q4K, 2, 8, 14336, 4096, 2, 16, False), (Q4K, 1, 8, 4096, 14336, 2, 16, False), (Q6K, 1, 16, 2560, 6144, 1, 3, True),
+            (T16, 1, 4, 1536, 5120, 1, 36, True), (T16, 2, 16, 3072, 4096, 1, 2, True), (Q4K, 2, 16, 3072, 4096, 1, 8, False),
+            (Q4K, 1, 4, 4096, 7168, 1, 4, True), (Q5K, 1, 4, 4096, 14336, 3, 4, False), (Q6K, 1, 4, 4096, 14336, 3, 4, True),
+            (Q4K, 1, 4, 4096, 256, 1, 4, False), (Q4K, 1, 8, 1024, 2048, 2, 1024, False), (Q80, 1, 4, 512, 512, 1, 1, False),
+            (Q4K, 1, 4, 512, 129 * 256, 1, 1, False)):
+        assert b(qtype, n_mat, n_expert, rows, cols, k, n_tok) == takes, (qtype, n_mat, n_expert, rows, cols, k, n_tok)
+    import subprocess
+    import sys
+    code = "from oxidize_amd import matvec as mv; print(mv.experts_batch(16, 1, 16, 2560, 6144, 1, 3))"
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=dict(os.environ, OXH_MOE_BIG_TILE_FROM="24"), check=True,
+                         capture_output=True, text=True).stdout
+    assert out.strip() == "False"
+
+
 @pytest.mark.parametrize("value,from_tokens", [("8", 8), ("24", 24), ("100", 100), ("0", None)])
 def test_the_tokens_per_expert_to_start_the_long_tiles_from_can_be_set(value, from_tokens):
     """OXH_MOE_BIG_TILE_FROM, read once per process: that average and nothing else decides, also for launches of few

@@ -302,6 +302,25 @@ def test_layer_whose_down_projection_gives_two_workgroups_per_cu(oxh, qt_gu, qt_
     check_layer(qt_gu, qt_dn, 9, 3, 3584, 512, 9, seed=32, skew=True)
 
 
+@pytest.mark.parametrize("qt_gu,qt_dn,n_exp,k,hidden,ffn,n_tok,by_rows", [
+    (Q4K, Q4K, 4, 2, 512, 768, 1, (True, True)),        # fewer blocks (2, 3) than waves
+    (Q5K, Q6K, 8, 3, 1280, 512, 17, (True, True)),      # an expert with a second tile of one token
+    (Q6K, Q5K, 4, 1, 512, 1280, 33, (True, True)),
+    (Q4K, Q5K, 64, 8, 512, 512, 3, (False, True)),      # a lane per expert, most of them without a token
+    (Q4K, Q4K, 3, 3, 256, 8192, 2, (False, True)),      # one block: tiles; 32 blocks: one workgroup to a CU
+    (Q6K, Q6K, 2, 2, 256, 14336, 16, (False, True)),    # 56 blocks, chunks of sixteen tokens
+    (Q4K, Q4K, 8, 2, 4096, 512, 40, (True, False)),     # down has too many rows for it
+])
+def test_layer_of_few_rows_or_tokens(oxh, qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok, by_rows):
+    """Expert launches that give every workgroup 16 rows and all their columns, at the fewest and the most super-blocks,
+    with one token, token tiles of one and of sixteen tokens, and experts without any."""
+    if mv.device_info()["n_cu"] == 256:
+        assert (mv.experts_batch(qt_gu, 2, n_exp, ffn, hidden, k, n_tok),
+                mv.experts_batch(qt_dn, 1, n_exp, hidden, ffn, k, n_tok)) == by_rows
+    check_layer(qt_gu, qt_dn, n_exp, k, hidden, ffn, n_tok, seed=51 + n_tok, skew=n_exp > k and n_tok > 1, replay=n_tok == 17,
+                sample=lambda n, offsets: sorted(set(int(v) for v in offsets[:-1] if v < n) | {n - 1} | set(range(0, n, 13))))
+
+
 def test_the_128_row_tile_when_switched_on(oxh):
     """OXH_MOE_WIDE_SMALL=1 is read once per process: the layers above, the Mixtral-shaped layer and
     configuration 4's expert launches over host-made lists, in a process of their own with the switch on,
