@@ -77,7 +77,41 @@ static int arg_fail(const char *what)
 
 /* ─── activation quantisers ───────────────────────────────────────────── */
 
-/* One wave per 256-value block; lane l owns values 4l..4l+3.  Two optional
+/* A 256-value block in a wave: lane l owns values 4l..4l+3, and after quantising their codes, the block's scale and (every
+ * fourth lane) the sum of sixteen codes. */
+struct __attribute__((packed, aligned(4))) float4a4 { float x, y, z, w; };
+struct Q8kLane {
+    float4a4 v;
+    uint32_t packed;
+    float d;
+    int sum;
+};
+
+__device__ __forceinline__ void q8k_lane_quantize(Q8kLane &b)
+{
+    /* max |x| over the block; NaNs never win a '>' comparison in the
+     * reference's scan, fmaxf drops them the same way */
+    float amax = fmaxf(fmaxf(fabsf(b.v.x), fabsf(b.v.y)), fmaxf(fabsf(b.v.z), fabsf(b.v.w)));
+    amax = wave_max(amax);
+
+    b.d = amax / 127.0f;
+    const float inv = (b.d != 0.0f) ? 1.0f / b.d : 0.0f;
+    const int q0 = quantize_one(b.v.x, inv), q1 = quantize_one(b.v.y, inv);
+    const int q2 = quantize_one(b.v.z, inv), q3 = quantize_one(b.v.w, inv);
+    b.packed = (uint32_t)(q0 & 255) | ((uint32_t)(q1 & 255) << 8) |
+               ((uint32_t)(q2 & 255) << 16) | ((uint32_t)(q3 & 255) << 24);
+    b.sum = quad_sum(q0 + q1 + q2 + q3);         /* 16 values = one bsum group */
+}
+
+__device__ __forceinline__ void q8k_lane_store(const Q8kLane &b, uint8_t *dst, uint32_t lane)
+{
+    reinterpret_cast<uint32_t *>(dst + 4)[lane] = b.packed;
+    if (lane == 0) *reinterpret_cast<float *>(dst) = b.d;
+    if ((lane & 3u) == 0u)
+        reinterpret_cast<int16_t *>(dst + 260)[lane >> 2] = (int16_t)b.sum;
+}
+
+/* One wave per 256-value block.  Two optional
  * extras for the mixture-of-experts path: `row_index` makes output vector v
  * read input row row_index[v] (the gather of each expert's tokens), and `up`
  * (laid out like x, same row) makes the value quantised silu(x) * up. */
@@ -92,34 +126,16 @@ k_quantize_q8_k(const float *__restrict__ x, size_t in_stride, uint32_t blocks_p
     const uint32_t vec = gb / blocks_per_vec;
     const uint32_t blk = gb - vec * blocks_per_vec;
     const size_t at = (size_t)(row_index ? row_index[vec] : vec) * in_stride + (size_t)blk * 256u + 4u * lane;
-    const float *src = x + at;
-    float v0 = src[0], v1 = src[1], v2 = src[2], v3 = src[3];
+    Q8kLane b;
+    b.v = *reinterpret_cast<const float4a4 *>(x + at);
     if (up) {
-        const float *u = up + at;
-        const float s0 = 1.0f / (1.0f + expf(-v0)), s1 = 1.0f / (1.0f + expf(-v1));
-        const float s2 = 1.0f / (1.0f + expf(-v2)), s3 = 1.0f / (1.0f + expf(-v3));
-        v0 = v0 * s0 * u[0]; v1 = v1 * s1 * u[1]; v2 = v2 * s2 * u[2]; v3 = v3 * s3 * u[3];
+        const float4a4 u = *reinterpret_cast<const float4a4 *>(up + at);
+        const float s0 = 1.0f / (1.0f + expf(-b.v.x)), s1 = 1.0f / (1.0f + expf(-b.v.y));
+        const float s2 = 1.0f / (1.0f + expf(-b.v.z)), s3 = 1.0f / (1.0f + expf(-b.v.w));
+        b.v.x = b.v.x * s0 * u.x; b.v.y = b.v.y * s1 * u.y; b.v.z = b.v.z * s2 * u.z; b.v.w = b.v.w * s3 * u.w;
     }
-
-    /* max |x| over the block; NaNs never win a '>' comparison in the
-     * reference's scan, fmaxf drops them the same way */
-    float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
-    amax = wave_max(amax);
-
-    const float d = amax / 127.0f;
-    const float inv = (d != 0.0f) ? 1.0f / d : 0.0f;
-    const int q0 = quantize_one(v0, inv), q1 = quantize_one(v1, inv);
-    const int q2 = quantize_one(v2, inv), q3 = quantize_one(v3, inv);
-
-    uint8_t *dst = act + (size_t)gb * OXH_Q8_K_BYTES;
-    const uint32_t packed = (uint32_t)(q0 & 255) | ((uint32_t)(q1 & 255) << 8) |
-                            ((uint32_t)(q2 & 255) << 16) | ((uint32_t)(q3 & 255) << 24);
-    reinterpret_cast<uint32_t *>(dst + 4)[lane] = packed;
-    if (lane == 0) *reinterpret_cast<float *>(dst) = d;
-
-    const int s = quad_sum(q0 + q1 + q2 + q3);   /* 16 values = one bsum group */
-    if ((lane & 3u) == 0u)
-        reinterpret_cast<int16_t *>(dst + 260)[lane >> 2] = (int16_t)s;
+    q8k_lane_quantize(b);
+    q8k_lane_store(b, act + (size_t)gb * OXH_Q8_K_BYTES, lane);
 }
 
 /* One wave per 8 blocks of 32 values; lane l owns values 4l..4l+3 of the
@@ -3015,7 +3031,14 @@ static int launch_experts(uint32_t qtype, const void *const *d_w, float *const *
                                    d_counts, d_offsets, max_tokens, stream);
 }
 
-/* the six launches of a layer over a workspace laid out by moe_layout(); arguments already checked */
+/* Routing and quantising in one launch (k_moe_route_quantize), up to as many tokens as a workgroup of four waves routes in
+ * about the time its own values take to arrive: the layer of random shapes in the geometric mean 0.96 of its time with two
+ * launches at 1 to 128 tokens (8 experts, 1024 x 3328, two tokens 27.8 -> 26.0 us), none slower; 0.99 at 129 to 256 with
+ * single ones 2 % slower, and 1.01 with 8 % above (every workgroup then takes the 5 to 8 us that routing takes by itself). */
+#define OXH_ROUTE_QUANT_TOKENS 128u
+static_assert(OXH_ROUTE_QUANT_TOKENS * OXH_MOE_MAX_TOPK <= OXH_ROUTE_QUANT_PAIRS, "the positions kept in LDS");
+
+/* the five or six launches of a layer over a workspace laid out by moe_layout(); arguments already checked */
 static int moe_ffn_run(const OxhMoe *m, const MoeLayout &l, const float *d_logits, const float *d_x, size_t x_stride,
                        size_t n_tok, float *d_out, size_t out_stride, uint8_t *ws, void *stream)
 {
@@ -3028,9 +3051,23 @@ static int moe_ffn_run(const OxhMoe *m, const MoeLayout &l, const float *d_logit
     const size_t pairs = n_tok * m->top_k;
 
     /* 1. route and group; 2. gather + quantise each pair's token */
-    if ((rc = oxh_moe_route(d_logits, n_tok, m->n_expert, m->top_k, m->renorm, ids, wts, counts, offsets, perm,
-                            slot_pos, stream))) return rc;
-    if ((rc = quantize_q8_k_ex(d_x, x_stride, pairs, m->hidden, ws + l.act_x, perm, nullptr, stream))) return rc;
+    if (n_tok <= OXH_ROUTE_QUANT_TOKENS) {
+        const uint32_t blocks = (uint32_t)(m->hidden / OXH_QK_K), units = (uint32_t)n_tok * blocks;
+        const uint32_t waves = 4u;
+#define OXH_ROUTE_QUANT(U)                                                                                              \
+    hipLaunchKernelGGL(k_moe_route_quantize<U>, dim3((units + waves * U - 1u) / (waves * U)), dim3(64u * waves), 0,     \
+                       pick_stream(stream), d_logits, (uint32_t)n_tok, (uint32_t)m->n_expert, (uint32_t)m->top_k,       \
+                       m->renorm, ids, wts, counts, offsets, perm, slot_pos, d_x, x_stride, blocks, ws + l.act_x)
+        if (units > 4u * 512u) OXH_ROUTE_QUANT(8);
+        else if (units > 512u) OXH_ROUTE_QUANT(2);
+        else OXH_ROUTE_QUANT(1);
+#undef OXH_ROUTE_QUANT
+        HIP_TRY(hipGetLastError());
+    } else {
+        if ((rc = oxh_moe_route(d_logits, n_tok, m->n_expert, m->top_k, m->renorm, ids, wts, counts, offsets, perm,
+                                slot_pos, stream))) return rc;
+        if ((rc = quantize_q8_k_ex(d_x, x_stride, pairs, m->hidden, ws + l.act_x, perm, nullptr, stream))) return rc;
+    }
     /* 3. gate and up of every expert over its own pairs */
     const void *w_gu[2] = { m->d_w_gate, m->d_w_up };
     float *o_gu[2] = { gate, up };

@@ -321,6 +321,13 @@ def test_layer_of_few_rows_or_tokens(oxh, qt_gu, qt_dn, n_exp, k, hidden, ffn, n
                 sample=lambda n, offsets: sorted(set(int(v) for v in offsets[:-1] if v < n) | {n - 1} | set(range(0, n, 13))))
 
 
+@pytest.mark.parametrize("n_tok,n_exp,k,hidden", [(127, 8, 2, 256), (128, 64, 8, 1024), (129, 8, 2, 256), (128, 5, 1, 5376)])
+def test_layer_at_the_edge_of_routing_and_quantising_in_one_launch(oxh, n_tok, n_exp, k, hidden):
+    """Up to 128 tokens one launch routes and places the quantised tokens (one, two or eight blocks to a wave); above, two."""
+    check_layer(Q4K, Q4K, n_exp, k, hidden, 256, n_tok, seed=n_tok + n_exp,
+                sample=lambda n, offsets: sorted(set(int(v) for v in offsets[:-1] if v < n) | {n - 1} | set(range(0, n, 29))))
+
+
 def test_the_128_row_tile_when_switched_on(oxh):
     """OXH_MOE_WIDE_SMALL=1 is read once per process: the layers above, the Mixtral-shaped layer and
     configuration 4's expert launches over host-made lists, in a process of their own with the switch on,
