@@ -453,18 +453,20 @@ plan_row_sums(const float *terms, const PWork &k, uint32_t B, uint32_t term_stri
  * wrote come through the caches.
  *
  * The launches (stage_begin / stage_end) give a wave one 256-value unit at a time, lane l holding
- * values 4l .. 4l+3.  Here a block goes to 16 lanes: lane l of a row holds values 16l .. 16l+15 of
- * block 4 * wave + row.  An instruction costs a 1024-thread workgroup sixteen issue slots whatever its
+ * values 4l .. 4l+3.  Here a block goes to 16 lanes: lane l of a row holds values 4l .. 4l+3 of each
+ * quarter of block 4 * wave + row.  A load past the L2s is answered in 64-byte pieces that no cache keeps, so a
+ * row's lanes ask for neighbouring 16 bytes (with values 16l .. 16l+15 per lane each of the four loads touched
+ * every piece of the block: the down projection's 56 KiB were 224 KiB of requests per workgroup; 32-layer chain
+ * 1.244 against 1.223 ms).  An instruction costs a 1024-thread workgroup sixteen issue slots whatever its
  * lanes do, so the quantiser's fixed part (maximum, two divisions, slot arithmetic, stores) is paid once
  * per four blocks instead of once per block, and for 4096 values four waves run it while twelve go on
  * to their weight requests.  The bytes are the launches': a maximum and the integer sums do not depend
  * on the order they are taken in, and the sum of squares is added in the launches' order.  There, lane
  * L of wave W adds up its four squares of units W, W + 16, ... in turn, the wave adds its lanes in
  * four exchange steps (neighbour, pair, eight, sixteen) and combines its four rows as (r0 + r1) + (r2 +
- * r3), and the waves' sums are added the same way.  A lane here holds what four neighbouring lanes
- * hold there: row 4w + r of waves 0..3 stands for wave W = 4w + r, walks W's units, does the first two
- * steps in registers, and the same four exchange instructions then perform the launches' last two steps
- * and the combination of the four rows. */
+ * r3), and the waves' sums are added the same way.  A lane's quarter j here is lane 16j + l
+ * there: row 4w + r of waves 0..3 stands for wave W = 4w + r, walks W's units, and the same exchange steps on
+ * each quarter give the launches' four row sums. */
 struct XStage {
     XRegs x[4], t[4], b[4];
 };
@@ -481,19 +483,19 @@ plan_stage_issue(const OpHead &op, XStage &xs, uint32_t lane, uint32_t wave)
     const CohBuf xc = coh_buf(gptr<const float>(op.x)), ac = coh_buf(gptr<const float>(op.pro_add)), bc = coh_buf(b);
     const uint32_t blk = wave * 4u + (lane >> 4);
     if (blk < op.blocks) {
-        const uint32_t at0 = blk * 256u + 16u * (lane & 15u);
+        const uint32_t at0 = blk * 256u + 4u * (lane & 15u);
 #pragma unroll
-        for (int j = 0; j < 4; j++) xs.x[j] = cload4(xc, (at0 + 4u * (uint32_t)j) * 4u);
+        for (int j = 0; j < 4; j++) xs.x[j] = cload4(xc, (at0 + 64u * (uint32_t)j) * 4u);
         if (pro == GEMV_PRO_ADD_RMSNORM) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) xs.t[j] = cload4(ac, (at0 + 4u * (uint32_t)j) * 4u);
+            for (int j = 0; j < 4; j++) xs.t[j] = cload4(ac, (at0 + 64u * (uint32_t)j) * 4u);
         }
         if (pro == GEMV_PRO_SWIGLU) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) xs.b[j] = cload4(bc, (at0 + 4u * (uint32_t)j) * 4u);
+            for (int j = 0; j < 4; j++) xs.b[j] = cload4(bc, (at0 + 64u * (uint32_t)j) * 4u);
         } else if (pro != GEMV_PRO_NONE) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) xs.b[j] = x_load4(b + at0 + 4u * (uint32_t)j);      /* norm weights: constants */
+            for (int j = 0; j < 4; j++) xs.b[j] = x_load4(b + at0 + 64u * (uint32_t)j);     /* norm weights: constants */
         }
     }
 }
@@ -538,7 +540,7 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
                 for (uint32_t b2 = blk + PLAN_W; b2 < B; b2 += PLAN_W) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        const uint32_t at = b2 * 256u + 16u * l + 4u * (uint32_t)j;
+                        const uint32_t at = b2 * 256u + 4u * l + 64u * (uint32_t)j;
                         XRegs v = cload4(xc, at * 4u);
                         if (add) {
                             const XRegs t = cload4(ac, at * 4u);
@@ -548,11 +550,14 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
                     }
                 }
             }
-            float q = (p[0] + p[1]) + (p[2] + p[3]);
-            q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0xB1, 0xF, 0xF, false));
-            q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x4E, 0xF, 0xF, false));
-            q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x141, 0xF, 0xF, false));
-            q += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q), 0x140, 0xF, 0xF, false));
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                p[j] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p[j]), 0xB1, 0xF, 0xF, false));
+                p[j] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p[j]), 0x4E, 0xF, 0xF, false));
+                p[j] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p[j]), 0x141, 0xF, 0xF, false));
+                p[j] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p[j]), 0x140, 0xF, 0xF, false));
+            }
+            const float q = (p[0] + p[1]) + (p[2] + p[3]);
             if (l == 0u) red[blk] = q;
         }
         __syncthreads();
@@ -565,15 +570,15 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
     const bool has_fout = pro != GEMV_PRO_NONE && storer && op.pro_out != 0u;
     if (blk < B) {
         const CohBuf sout = coh_buf(gptr<float>(op.pro_sum_out)), fout = coh_buf(gptr<float>(op.pro_out));
-        const uint32_t at = blk * 256u + 16u * l;
+        const uint32_t at = blk * 256u + 4u * l;
         XRegs y[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if (has_sout) cstore4(sout, (at + 4u * (uint32_t)j) * 4u, xr[j]);
+            if (has_sout) cstore4(sout, (at + 64u * (uint32_t)j) * 4u, xr[j]);
             y[j] = xr[j];
             if (rms) y[j] = prologue_apply<GEMV_PRO_RMSNORM>(xr[j], xs.b[j], inv);
             else if (pro == GEMV_PRO_SWIGLU) y[j] = prologue_apply<GEMV_PRO_SWIGLU>(xr[j], xs.b[j], inv);
-            if (has_fout) cstore4(fout, (at + 4u * (uint32_t)j) * 4u, y[j]);
+            if (has_fout) cstore4(fout, (at + 64u * (uint32_t)j) * 4u, y[j]);
         }
         float m = fmaxf(fmaxf(fabsf(y[0].v0), fabsf(y[0].v1)), fmaxf(fabsf(y[0].v2), fabsf(y[0].v3)));
 #pragma unroll
@@ -582,31 +587,30 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
         m = dpp_max_step(oct_max(m), 3);                /* over the row's sixteen lanes */
         const float d = m / 127.0f;
         const float invd = (d != 0.0f) ? 1.0f / d : 0.0f;
-        u32x4 packed;
-        uint32_t pk;
-        int s16 = quantize_sum4(y[0], invd, pk); packed.x = pk;
-        s16 += quantize_sum4(y[1], invd, pk); packed.y = pk;
-        s16 += quantize_sum4(y[2], invd, pk); packed.z = pk;
-        s16 += quantize_sum4(y[3], invd, pk); packed.w = pk;
-        /* value dwords 4l .. 4l+3 of a block are neighbours in both staged layouts */
-        *reinterpret_cast<u32x4 *>(reinterpret_cast<uint32_t *>(base) + q8k_slot<Q6>(B, blk, 4u * l)) = packed;
-        if (Q6) {
-            const uint32_t n = l >> 3, k = (l >> 1) & 3u, lh = l & 1u;
-            reinterpret_cast<int32_t *>(base + B * 256u)[(blk * 4u + 2u * n + lh) * 4u + k] = -32 * s16;
-        } else {
-            const int bj = s16 + __builtin_amdgcn_update_dpp(0, s16, 0xB1, 0xF, 0xF, false);
-            if ((l & 1u) == 0u) {
-                const uint32_t j = l >> 1;
-                reinterpret_cast<int16_t *>(base + B * 256u)[(blk * 4u + (j >> 1)) * 2u + (j & 1u)] = (int16_t)bj;
+        uint8_t *const dst = storer && op.act_out ? gptr<uint8_t>(op.act_out) + (size_t)blk * 292u : nullptr;
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; j++) {
+            uint32_t pk;
+            const int s16 = quad_sum(quantize_sum4(y[j], invd, pk));        /* of values 16g .. 16g+15 */
+            const uint32_t g = 4u * j + (l >> 2);
+            reinterpret_cast<uint32_t *>(base)[q8k_slot<Q6>(B, blk, 16u * j + l)] = pk;
+            if (Q6) {
+                const uint32_t n = g >> 3, k = (g >> 1) & 3u, lh = g & 1u;
+                if ((l & 3u) == 0u)
+                    reinterpret_cast<int32_t *>(base + B * 256u)[(blk * 4u + 2u * n + lh) * 4u + k] = -32 * s16;
+            } else {
+                const int bj = s16 + __builtin_amdgcn_update_dpp(0, s16, 0x141, 0xF, 0xF, false);
+                if ((l & 7u) == 0u)
+                    reinterpret_cast<int16_t *>(base + B * 256u)[(blk * 4u + j) * 2u + (l >> 3)] = (int16_t)bj;
+            }
+            if (dst) {
+                reinterpret_cast<uint32_t *>(dst + 4)[16u * j + l] = pk;
+                if ((l & 3u) == 0u) reinterpret_cast<int16_t *>(dst + 260)[g] = (int16_t)s16;
             }
         }
-        if (l == 0u) reinterpret_cast<float *>(base + B * 256u + B * (Q6 ? 64u : 16u))[blk] = d;
-        if (storer && op.act_out) {
-            uint8_t *dst = gptr<uint8_t>(op.act_out) + (size_t)blk * 292u;
-            uint32_t *qs = reinterpret_cast<uint32_t *>(dst + 4) + 4u * l;
-            qs[0] = packed.x; qs[1] = packed.y; qs[2] = packed.z; qs[3] = packed.w;
-            if (l == 0u) *reinterpret_cast<float *>(dst) = d;
-            reinterpret_cast<int16_t *>(dst + 260)[l] = (int16_t)s16;
+        if (l == 0u) {
+            reinterpret_cast<float *>(base + B * 256u + B * (Q6 ? 64u : 16u))[blk] = d;
+            if (dst) *reinterpret_cast<float *>(dst) = d;
         }
     }
     /* the side outputs are acknowledged where the trip that follows the passes begins (k_plan), or after
