@@ -75,6 +75,9 @@ typedef struct OxhLab {
      * that experts_tile names (0); n_mat as there. */
     int (*experts_batch)(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t cols, size_t top_k,
                          size_t n_tok, size_t n_cu);
+    /* Whether the operations of a chained plan hand their results over by
+     * value (1) or wait for whole operations (0). */
+    int (*plan_by_value)(const OxhPlan *plan);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

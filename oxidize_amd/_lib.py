@@ -60,7 +60,8 @@ class OxhLab(ctypes.Structure):
                 ("mmq_kernel", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 4))),
                 ("experts_tile", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 2))),
                 ("host_ring_chunks", ctypes.CFUNCTYPE(Z)),
-                ("experts_batch", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, Z, Z))]
+                ("experts_batch", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, Z, Z)),
+                ("plan_by_value", ctypes.CFUNCTYPE(I, V))]
 
 
 # name -> (restype, argtypes); every symbol include/oxhip.h and include/oxhip_lab.h declare

@@ -35,6 +35,10 @@
  *     works on operation i.  An operation boundary then costs the row sums
  *     and one workgroup barrier; no workgroup reads or quantises a vector that
  *     255 others quantise as well.
+ *   - In most chains a vector an operation hands on is its own announcement (BY_VALUE): it goes through slots that
+ *     hold a word no arithmetic returns until the value arrives, and whoever needs it polls the values themselves.
+ *     That leaves out the acknowledgement of the stores, the counter and the trip for the vector after it
+ *     (SLOT_EMPTY; plans of longer vectors, and those plan_slots turns down, wait for whole operations).
  *   - Every wait is bounded: after `spin_limit` polls a workgroup raises the
  *     plan's error word and leaves, and every other workgroup leaves at its
  *     next wait, so a launch that cannot make progress (not all workgroups
@@ -109,6 +113,7 @@ struct PlanSync {
     uint32_t spin_limit;
     uint64_t *stamps;               /* measurement aid: [op][workgroup][8] clock readings, or NULL */
     uint32_t *host_err;             /* page-locked host word that mirrors go[1], so that the next launch can be refused */
+    uint32_t set_bytes;             /* plans that hand over by value: bytes of one set of slots (two lie side by side) */
 };
 
 #define PLAN_STAMPS 8u
@@ -176,6 +181,8 @@ __device__ __forceinline__ void cstore4(CohBuf b, uint32_t byte_off, const XRegs
     __builtin_amdgcn_raw_buffer_store_b128(v, b, (int)byte_off, 0, OXH_SYSTEM_COHERENT);
 }
 
+template <typename T> __device__ __forceinline__ T *gptr(gaddr v);
+
 /* workgroup barrier that orders LDS only: __syncthreads() may also wait for every
  * global load in flight, and the prefetched weights of the next operation are */
 __device__ __forceinline__ void lds_barrier()
@@ -236,6 +243,18 @@ struct PWork {
 __device__ __forceinline__ uint32_t plan_block_bytes(uint32_t kind)
 {
     return kind >= PLAN_Q6_K ? 210u : kind == PLAN_Q5_K ? 176u : 144u;
+}
+
+/* where this workgroup's rows of an operation are handed over by value, or 0 (PlanSeg::rows_q / rows_rem, which only
+ * k_plan_ext deals by, hold the address) */
+__device__ __forceinline__ gaddr plan_out_slots(const PlanOp *op)
+{
+    const uint32_t wg = blockIdx.x, n = uni(op->n_segs);
+    uint32_t si = 0;
+#pragma unroll
+    for (uint32_t i = 1; i < PLAN_OP_SEGS; i++)
+        if (i < n && wg >= uni(op->s[i].wg_begin)) si = i;
+    return (gaddr)op->s[si].rows_q | ((gaddr)op->s[si].rows_rem << 32);
 }
 
 __device__ __forceinline__ PWork plan_work(const PlanOp *op, uint32_t wave)
@@ -471,33 +490,133 @@ struct XStage {
     XRegs x[4], t[4], b[4];
 };
 
+/* ─── values that carry their own arrival ───
+ *
+ * What a chained operation hands on goes to a slot (and to the caller's vector): until it is there the slot holds
+ * SLOT_EMPTY.  A workgroup that needs the vector reads the slot until nothing in it is empty.  Each result has two
+ * slots, used in turn (by the same result of later layers, or from launch to launch); storing into one empties the
+ * other, which everybody has read by then (plan_slots makes sure).
+ *
+ * Why: waiting for whole operations costs three trips through the fabric one after the other (the stores'
+ * acknowledgement, the counter, the vector), this one.  An operation of at most sixteen blocks takes some 0.8 us less,
+ * a longer one some 0.9 us more (its vector is read over and over by every workgroup while the last ones still
+ * stream their weights).  Chains of layers, both ways (us): 16 of 1024 x 2560 358 / 303, 9 of 2304 x 6144 258 / 233,
+ * 12 of 3072 x 8192 351 / 322, 6 of 4096 x 8192 191 / 182, 32 of 4096 x 14336 1228 / 1211, and 5 of 5120 x 12800,
+ * where every vector is long, 244 / 260: so a plan goes by value if more short operations than long ones wait.
+ * Two kinds of wait in one kernel (the long ones by counter) cost it twenty more scalars kept in vector lanes and were
+ * slower than either; so was the first poll before the first weights (32 layers 1253: the weights then start late). */
+
+#define SLOT_EMPTY 0x7FA5C3E1u      /* a signalling NaN: no arithmetic returns one */
+#define SLOT_X 0x10000u             /* OpHead::wait: which inputs come out of slots */
+#define SLOT_ADD 0x20000u
+#define SLOT_B 0x40000u
+
+__device__ __forceinline__ bool here(const XRegs &v)
+{
+    return __float_as_uint(v.v0) != SLOT_EMPTY && __float_as_uint(v.v1) != SLOT_EMPTY &&
+           __float_as_uint(v.v2) != SLOT_EMPTY && __float_as_uint(v.v3) != SLOT_EMPTY;
+}
+__device__ __forceinline__ uint32_t slot_word(float v)
+{
+    const uint32_t b = __float_as_uint(v);
+    return b == SLOT_EMPTY ? b | 0x00400000u : b;       /* quieted, as its first use would */
+}
+/* whether all of a wave's values have arrived (the time-out test's extra workgroup never does) */
+__device__ __forceinline__ bool plan_there(const PlanSync &sy, uint32_t waits, bool there)
+{
+    return __all(there) && (sy.n_wait <= gridDim.x || (waits & (SLOT_X | SLOT_ADD | SLOT_B)) == 0u);
+}
+/* The table's slot addresses are multiples of four; bit 0 says which of the two sets, bit 1 whether the sets change
+ * places from one launch to the next (par: the launch's parity). */
+__device__ __forceinline__ gaddr slot_at(gaddr a, uint32_t par, uint32_t set_bytes)
+{
+    const uint32_t lo = (uint32_t)a;
+    return (a & ~(gaddr)3u) + (((lo ^ ((lo >> 1) & par)) & 1u) ? set_bytes : 0u);
+}
+
+/* where a prologue's side outputs are handed over by value: the operation's row of the table (NULL: they are not),
+ * this launch's set of slots and the other one, which is emptied for the next launch */
+struct SideSlots {
+    const PlanOp *row;
+    uint32_t par, set_bytes;
+    /* (addresses in vector registers, two words a store: few waves store these, and scalar registers are what every
+     * workgroup is short of) */
+    static __device__ __forceinline__ void two(gaddr to, uint32_t a, uint32_t b)
+    {
+        __hip_atomic_store(gptr<uint64_t>(to), (uint64_t)a | ((uint64_t)b << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __device__ __forceinline__ void store4(gaddr slot, gaddr out, uint32_t byte_off, const XRegs &y) const
+    {
+        if (slot != 0u) {
+            const gaddr to = slot_at(slot, par, set_bytes) + byte_off, other = slot_at(slot ^ 1u, par, set_bytes) + byte_off;
+            two(to, slot_word(y.v0), slot_word(y.v1));
+            two(to + 8u, slot_word(y.v2), slot_word(y.v3));
+            two(other, SLOT_EMPTY, SLOT_EMPTY);
+            two(other + 8u, SLOT_EMPTY, SLOT_EMPTY);
+        }
+        if (out != 0u) {
+            two(out + byte_off, __float_as_uint(y.v0), __float_as_uint(y.v1));
+            two(out + byte_off + 8u, __float_as_uint(y.v2), __float_as_uint(y.v3));
+        }
+    }
+};
+/* after a poll that found something missing: whether to give up */
+__device__ __forceinline__ bool plan_poll_over(const PlanSync &sy, uint32_t spins)
+{
+    const bool over = spins >= sy.spin_limit || ((spins & 63u) == 63u && cload(sy.go + 1) != 0u);
+    if (over && (threadIdx.x & 63u) == 0u) { cstore(sy.go + 1, 1u); cstore(sy.host_err, 1u); }
+    return over;
+}
+
 /* Every vector that may have been written in this launch is read with coherent loads, whether it was
  * or not: choosing the instruction per load at run time gives the compiler two definitions of each
  * register to merge, which it does with a move, and a move waits for the load (and for the weights
  * requested before it). */
-__device__ __forceinline__ void
-plan_stage_issue(const OpHead &op, XStage &xs, uint32_t lane, uint32_t wave)
+template <bool BY_VALUE>
+__device__ __forceinline__ bool
+plan_stage_issue(const PlanSync &sy, const OpHead &op, XStage &xs, uint32_t lane, uint32_t wave)
 {
     const uint32_t pro = op.pro;
     const float *b = gptr<const float>(op.pro_b);
     const CohBuf xc = coh_buf(gptr<const float>(op.x)), ac = coh_buf(gptr<const float>(op.pro_add)), bc = coh_buf(b);
     const uint32_t blk = wave * 4u + (lane >> 4);
-    if (blk < op.blocks) {
-        const uint32_t at0 = blk * 256u + 4u * (lane & 15u);
+    bool ok = true;
+    if (wave * 4u < op.blocks) {
+        /* (lanes of a wave whose last rows lie beyond the vector read its first block) */
+        const uint32_t at0 = (BY_VALUE && blk >= op.blocks ? 0u : blk * 256u) + 4u * (lane & 15u);
+        for (uint32_t spins = 0; BY_VALUE || blk < op.blocks; spins++) {
+            bool there = true;
 #pragma unroll
-        for (int j = 0; j < 4; j++) xs.x[j] = cload4(xc, (at0 + 64u * (uint32_t)j) * 4u);
-        if (pro == GEMV_PRO_ADD_RMSNORM) {
+            for (int j = 0; j < 4; j++) xs.x[j] = cload4(xc, (at0 + 64u * (uint32_t)j) * 4u);
+            if (pro == GEMV_PRO_ADD_RMSNORM) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) xs.t[j] = cload4(ac, (at0 + 64u * (uint32_t)j) * 4u);
+                for (int j = 0; j < 4; j++) xs.t[j] = cload4(ac, (at0 + 64u * (uint32_t)j) * 4u);
+            }
+            if (pro == GEMV_PRO_SWIGLU) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) xs.b[j] = cload4(bc, (at0 + 64u * (uint32_t)j) * 4u);
+            }
+            if (!BY_VALUE) break;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (op.wait & SLOT_X) there = there && here(xs.x[j]);
+                if (op.wait & SLOT_ADD) there = there && here(xs.t[j]);
+                if (op.wait & SLOT_B) there = there && here(xs.b[j]);
+            }
+            if (plan_there(sy, op.wait, there)) break;
+            if (plan_poll_over(sy, spins)) { ok = false; break; }
         }
-        if (pro == GEMV_PRO_SWIGLU) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) xs.b[j] = cload4(bc, (at0 + 64u * (uint32_t)j) * 4u);
-        } else if (pro != GEMV_PRO_NONE) {
+        if (pro == GEMV_PRO_SWIGLU || blk >= op.blocks) { }
+        else if (pro != GEMV_PRO_NONE) {
 #pragma unroll
             for (int j = 0; j < 4; j++) xs.b[j] = x_load4(b + at0 + 64u * (uint32_t)j);     /* norm weights: constants */
         }
+        if (BY_VALUE && blk >= op.blocks) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) xs.x[j] = xs.t[j] = XRegs{ 0.f, 0.f, 0.f, 0.f };
+        }
     }
+    return ok;
 }
 
 __device__ __forceinline__ int quantize_sum4(const XRegs &y, float inv, uint32_t &packed)
@@ -511,8 +630,8 @@ __device__ __forceinline__ int quantize_sum4(const XRegs &y, float inv, uint32_t
 
 template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */>
 __device__ __forceinline__ void
-plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red, bool storer,
-                  uint32_t lane, uint32_t wave)
+plan_stage_finish(const OpHead &op, const SideSlots &slots, const XStage &xs, uint8_t *base, float *red,
+                  bool storer, uint32_t lane, uint32_t wave)
 {
     constexpr bool Q6 = KIND == 1;
     const uint32_t B = op.blocks, pro = op.pro;
@@ -526,30 +645,28 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
     }
     float inv = 1.0f;
     if (rms) {
-        if (wave < PLAN_W / 4u) {
-            /* rows beyond the vector hold zeros, the sums of the launches' idle waves */
-            float p[4];
+        /* Rows beyond the vector hold zeros, the sums of the launches' idle waves.  Vectors of more than sixteen
+         * blocks: the further units of a wave of the launches are other rows here, which pass their lanes' squares on in
+         * the staging area, not written yet (asked for again instead, they were one more trip to memory: five
+         * layers of 5120 x 12800 247 against 244 us). */
+        float p[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                p[j] = xr[j].v0 * xr[j].v0 + xr[j].v1 * xr[j].v1 + xr[j].v2 * xr[j].v2 + xr[j].v3 * xr[j].v3;
-            /* vectors of more than sixteen blocks: the further units of the wave this row stands for,
-             * one round trip each (their values are not kept: the rows that quantise them asked for
-             * them already) */
-            if (B > PLAN_W) {
-                const CohBuf xc = coh_buf(gptr<const float>(op.x)), ac = coh_buf(gptr<const float>(op.pro_add));
-                for (uint32_t b2 = blk + PLAN_W; b2 < B; b2 += PLAN_W) {
+        for (int j = 0; j < 4; j++)
+            p[j] = xr[j].v0 * xr[j].v0 + xr[j].v1 * xr[j].v1 + xr[j].v2 * xr[j].v2 + xr[j].v3 * xr[j].v3;
+        if (B > PLAN_W) {
+            float *const more = reinterpret_cast<float *>(base);
+            if (blk >= PLAN_W && blk < B) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const uint32_t at = b2 * 256u + 4u * l + 64u * (uint32_t)j;
-                        XRegs v = cload4(xc, at * 4u);
-                        if (add) {
-                            const XRegs t = cload4(ac, at * 4u);
-                            v.v0 += t.v0; v.v1 += t.v1; v.v2 += t.v2; v.v3 += t.v3;
-                        }
-                        p[j] += v.v0 * v.v0 + v.v1 * v.v1 + v.v2 * v.v2 + v.v3 * v.v3;
-                    }
-                }
+                for (int j = 0; j < 4; j++) more[(blk - PLAN_W) * 64u + 16u * (uint32_t)j + l] = p[j];
             }
+            lds_barrier();
+            if (wave < PLAN_W / 4u)
+                for (uint32_t b2 = blk; b2 + PLAN_W < B; b2 += PLAN_W) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) p[j] += more[b2 * 64u + 16u * (uint32_t)j + l];
+                }
+        }
+        if (wave < PLAN_W / 4u) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 p[j] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(p[j]), 0xB1, 0xF, 0xF, false));
@@ -566,8 +683,8 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
             inv = 1.0f / sqrtf(tot / (float)(B * 256u) + op.eps);
         }
     }
-    const bool has_sout = add && storer && op.pro_sum_out != 0u;
-    const bool has_fout = pro != GEMV_PRO_NONE && storer && op.pro_out != 0u;
+    const bool has_sout = slots.row == nullptr && add && storer && op.pro_sum_out != 0u;
+    const bool has_fout = slots.row == nullptr && pro != GEMV_PRO_NONE && storer && op.pro_out != 0u;
     if (blk < B) {
         const CohBuf sout = coh_buf(gptr<float>(op.pro_sum_out)), fout = coh_buf(gptr<float>(op.pro_out));
         const uint32_t at = blk * 256u + 4u * l;
@@ -575,10 +692,14 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if (has_sout) cstore4(sout, (at + 64u * (uint32_t)j) * 4u, xr[j]);
+            if (slots.row != nullptr && storer && add)
+                slots.store4(slots.row->xq, slots.row->pro_sum_out, (at + 64u * (uint32_t)j) * 4u, xr[j]);
             y[j] = xr[j];
             if (rms) y[j] = prologue_apply<GEMV_PRO_RMSNORM>(xr[j], xs.b[j], inv);
             else if (pro == GEMV_PRO_SWIGLU) y[j] = prologue_apply<GEMV_PRO_SWIGLU>(xr[j], xs.b[j], inv);
             if (has_fout) cstore4(fout, (at + 64u * (uint32_t)j) * 4u, y[j]);
+            if (slots.row != nullptr && storer && pro != GEMV_PRO_NONE)
+                slots.store4(slots.row->reserved, slots.row->pro_out, (at + 64u * (uint32_t)j) * 4u, y[j]);
         }
         float m = fmaxf(fmaxf(fabsf(y[0].v0), fabsf(y[0].v1)), fmaxf(fabsf(y[0].v2), fabsf(y[0].v3)));
 #pragma unroll
@@ -587,7 +708,8 @@ plan_stage_finish(const OpHead &op, const XStage &xs, uint8_t *base, float *red,
         m = dpp_max_step(oct_max(m), 3);                /* over the row's sixteen lanes */
         const float d = m / 127.0f;
         const float invd = (d != 0.0f) ? 1.0f / d : 0.0f;
-        uint8_t *const dst = storer && op.act_out ? gptr<uint8_t>(op.act_out) + (size_t)blk * 292u : nullptr;
+        const gaddr act_out = !storer ? 0u : slots.row != nullptr ? slots.row->act_out : op.act_out;
+        uint8_t *const dst = act_out != 0u ? gptr<uint8_t>(act_out) + (size_t)blk * 292u : nullptr;
 #pragma unroll
         for (uint32_t j = 0; j < 4u; j++) {
             uint32_t pk;
@@ -630,23 +752,36 @@ struct XUnit {
     XRegs x, t, b;
 };
 
-__device__ __forceinline__ void
-plan_stage_issue_unit(const OpHead &op, XUnit &xu, uint32_t lane, uint32_t wave)
+template <bool BY_VALUE>
+__device__ __forceinline__ bool
+plan_stage_issue_unit(const PlanSync &sy, const OpHead &op, XUnit &xu, uint32_t lane, uint32_t wave)
 {
     const uint32_t pro = op.pro;
+    bool ok = true;
     if (wave < op.blocks) {
         const float *b = gptr<const float>(op.pro_b);
         const uint32_t at = (wave * 256u + 4u * lane) * 4u;
-        xu.x = cload4(coh_buf(gptr<const float>(op.x)), at);
-        if (pro == GEMV_PRO_ADD_RMSNORM) xu.t = cload4(coh_buf(gptr<const float>(op.pro_add)), at);
-        if (pro == GEMV_PRO_SWIGLU) xu.b = cload4(coh_buf(b), at);
-        else if (pro != GEMV_PRO_NONE) xu.b = x_load4(b + wave * 256u + 4u * lane);      /* norm weights: constants */
+        if (BY_VALUE && pro != GEMV_PRO_NONE && pro != GEMV_PRO_SWIGLU) xu.b = x_load4(b + wave * 256u + 4u * lane);
+        for (uint32_t spins = 0;; spins++) {
+            xu.x = cload4(coh_buf(gptr<const float>(op.x)), at);
+            if (pro == GEMV_PRO_ADD_RMSNORM) xu.t = cload4(coh_buf(gptr<const float>(op.pro_add)), at);
+            if (pro == GEMV_PRO_SWIGLU) xu.b = cload4(coh_buf(b), at);
+            else if (!BY_VALUE && pro != GEMV_PRO_NONE) xu.b = x_load4(b + wave * 256u + 4u * lane);      /* norm weights: constants */
+            if (!BY_VALUE) break;
+            bool there = true;
+            if (op.wait & SLOT_X) there = here(xu.x);
+            if (op.wait & SLOT_ADD) there = there && here(xu.t);
+            if (op.wait & SLOT_B) there = there && here(xu.b);
+            if (plan_there(sy, op.wait, there)) break;
+            if (plan_poll_over(sy, spins)) { ok = false; break; }
+        }
     }
+    return ok;
 }
 
 template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */>
 __device__ __forceinline__ void
-plan_stage_finish_unit(const OpHead &op, const XUnit &xu, uint8_t *base, float *red, bool storer,
+plan_stage_finish_unit(const OpHead &op, const SideSlots &slots, const XUnit &xu, uint8_t *base, float *red, bool storer,
                        uint32_t lane, uint32_t wave)
 {
     const uint32_t B = op.blocks, pro = op.pro;
@@ -665,12 +800,15 @@ plan_stage_finish_unit(const OpHead &op, const XUnit &xu, uint8_t *base, float *
     }
     if (wave < B) {
         const uint32_t at = (wave * 256u + 4u * lane) * 4u;
-        if (add && storer && op.pro_sum_out != 0u) cstore4(coh_buf(gptr<float>(op.pro_sum_out)), at, xr);
+        if (slots.row == nullptr && add && storer && op.pro_sum_out != 0u) cstore4(coh_buf(gptr<float>(op.pro_sum_out)), at, xr);
+        if (slots.row != nullptr && add && storer) slots.store4(slots.row->xq, slots.row->pro_sum_out, at, xr);
         XRegs y = xr;
         if (rms) y = prologue_apply<GEMV_PRO_RMSNORM>(xr, xu.b, inv);
         else if (pro == GEMV_PRO_SWIGLU) y = prologue_apply<GEMV_PRO_SWIGLU>(xr, xu.b, inv);
-        if (pro != GEMV_PRO_NONE && storer && op.pro_out != 0u) cstore4(coh_buf(gptr<float>(op.pro_out)), at, y);
-        q8k_x_finish<KIND == 1>(y, B, wave, base, (storer && op.act_out) ? gptr<uint8_t>(op.act_out) : nullptr, lane);
+        if (slots.row == nullptr && pro != GEMV_PRO_NONE && storer && op.pro_out != 0u) cstore4(coh_buf(gptr<float>(op.pro_out)), at, y);
+        if (slots.row != nullptr && pro != GEMV_PRO_NONE && storer) slots.store4(slots.row->reserved, slots.row->pro_out, at, y);
+        const gaddr act_out = !storer ? 0u : slots.row != nullptr ? slots.row->act_out : op.act_out;
+        q8k_x_finish<KIND == 1>(y, B, wave, base, act_out ? gptr<uint8_t>(act_out) : nullptr, lane);
     }
 }
 
@@ -745,7 +883,7 @@ plan_wait(const PlanSync &sy, uint32_t target, int *s_ok, uint32_t lane, uint32_
 
 /* ─── the kernel ──────────────────────────────────────────────────────── */
 
-template <bool HAS_Q5, bool STAMPS = false>
+template <bool HAS_Q5, bool BY_VALUE, bool STAMPS = false>
 __global__ __launch_bounds__(1024) void
 k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const PlanLds ld)
 {
@@ -758,7 +896,10 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
     float *const outs = reinterpret_cast<float *>(lds + ld.outs_off);
     float *const red = reinterpret_cast<float *>(lds + ld.red_off);
     int *const s_ok = reinterpret_cast<int *>(red + 24);      /* the reduction uses slots 0..15 of 32 */
+    int *const s_bad = reinterpret_cast<int *>(red + 25);     /* BY_VALUE: a wave gave up at its polls */
     float *const terms = reinterpret_cast<float *>(lds + ld.terms_off) + (size_t)wave * ld.terms_per_wave;
+    const uint32_t par = uni(base) & 1u;                      /* the counters' step per launch is odd (BY_VALUE) */
+    if (BY_VALUE && threadIdx.x == 0u) *s_bad = 0;
 
     /* The loop is cut between an operation's last pass and its row sums: at that point no load is in
      * flight and no weight or input register holds anything, so nothing but scalars crosses the loop
@@ -787,13 +928,38 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
              * operation: those queue up in the memory pipeline (a compute unit takes in about 12 bytes
              * per cycle), and anything placed after them in program order waits for that queue. */
             plan_row_sums(terms, prev, po.blocks, po.term_stride, outs, ln);
-            /* a prologue's side outputs (stored while staging, by any wave of one workgroup) have to be
+            /* a prologue's side outputs (stored while staging) have to be
              * acknowledged before the workgroup announces the operation: no load is in flight here, so
              * the wait costs nothing unless such a store is still on its way */
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            gaddr slots = 0u;
+            bool bad = false;
+            if (BY_VALUE) {
+                if (wave == 0u) slots = plan_out_slots(&tab[i - 1u]);
+                bad = uni((uint32_t)*s_bad) != 0u;
+            }
             lds_barrier();
             plan_stamp<STAMPS>(sy, i - 1u, 6, ln, wave);
-            if (wave == 0u) {
+            if (bad) return;
+            if (BY_VALUE && wave == 0u) {
+                const CohBuf dst = coh_buf(prev.out + prev.wg_row0);
+                if (slots != 0u) {
+                    const gaddr to = slot_at(slots, par, sy.set_bytes) + prev.wg_row0 * 4u;
+                    const gaddr other = slot_at(slots ^ 1u, par, sy.set_bytes) + prev.wg_row0 * 4u;
+                    for (uint32_t r = ln; r < prev.wg_rows; r += 64u) {
+                        cstore(gptr<uint32_t>(to + r * 4u), slot_word(outs[r]));
+                        cstore_f32(dst, r * 4u, outs[r]);
+                        cstore(gptr<uint32_t>(other + r * 4u), SLOT_EMPTY);
+                    }
+                } else {
+                    for (uint32_t r = ln; r < prev.wg_rows; r += 64u) cstore_f32(dst, r * 4u, outs[r]);
+                }
+                if (i == n_ops) {
+                    const uint32_t now = cload(sy.flags + blockIdx.x);      /* still where it was when the launch began */
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    plan_announce(sy, now + ((n_ops + 1u) | 1u), ln);
+                }
+            } else if (wave == 0u) {
                 const CohBuf dst = coh_buf(prev.out + prev.wg_row0);
                 for (uint32_t r = ln; r < prev.wg_rows; r += 64u) cstore_f32(dst, r * 4u, outs[r]);
                 if (po.signal != 0u || i == n_ops) {
@@ -806,7 +972,7 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
         }
         if (i == n_ops) break;
 
-        const OpHead op = plan_head(&tab[i]);
+        OpHead op = plan_head(&tab[i]);
         uint8_t *act = lds + (size_t)(i & 1u) * ld.act_bytes;
         plan_stamp<STAMPS>(sy, i, 0, ln, wave);
         /* Loads complete in the order a wave issued them, and the compiler waits for ALL of them
@@ -828,10 +994,19 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
         /* what this wave owns of the next operation: scalar arithmetic, done while nothing waits for it */
         PWork nx = cur;
         if (i + 1u < n_ops) nx = plan_work(&tab[i + 1u], wave);
-        if (op.wait == 0u) {
+        bool got = true;
+        if (BY_VALUE) {
+            if (op.wait & SLOT_X) op.x = slot_at(op.x, par, sy.set_bytes);
+            if (op.wait & SLOT_ADD) op.pro_add = slot_at(op.pro_add, par, sy.set_bytes);
+            if (op.wait & SLOT_B) op.pro_b = slot_at(op.pro_b, par, sy.set_bytes);
+            plan_prefetch<HAS_Q5>(cur, A, 0u, ln);
+            if (by_unit) got = plan_stage_issue_unit<true>(sy, op, xu, ln, wave);
+            else         got = plan_stage_issue<true>(sy, op, xs, ln, wave);
+            if (!got) *s_bad = 1;
+        } else if (op.wait == 0u) {
             /* nothing to wait for: the vector goes first and is there in a microsecond */
-            if (by_unit) plan_stage_issue_unit(op, xu, ln, wave);
-            else         plan_stage_issue(op, xs, ln, wave);
+            if (by_unit) plan_stage_issue_unit<false>(sy, op, xu, ln, wave);
+            else         plan_stage_issue<false>(sy, op, xs, ln, wave);
             plan_prefetch<HAS_Q5>(cur, A, 0u, ln);
         } else {
             /* Wave 0 polls, and a poll comes back behind everything the wave asked for before it: its
@@ -843,26 +1018,28 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
              * and up against 1.32 ms.) */
             if (wave != 0u) plan_prefetch<HAS_Q5>(cur, A, 0u, ln);
             if (!plan_wait(sy, base + op.wait, s_ok, ln, wave)) return;
-            if (by_unit) plan_stage_issue_unit(op, xu, ln, wave);
-            else         plan_stage_issue(op, xs, ln, wave);
+            if (by_unit) plan_stage_issue_unit<false>(sy, op, xu, ln, wave);
+            else         plan_stage_issue<false>(sy, op, xs, ln, wave);
             if (wave == 0u) plan_prefetch<HAS_Q5>(cur, A, 0u, ln);
         }
         plan_stamp<STAMPS>(sy, i, 1, ln, wave);
 
-        /* a prologue's side outputs are one workgroup's work, and not workgroup 0's: that one gathers the
-         * counters, and whatever holds it up holds everybody up */
-        const bool storer = blockIdx.x == gridDim.x - 1u;
+        /* a prologue's side outputs: every workgroup has them, and wave w of the w-th workgroup from the end stores its
+         * part (one workgroup storing all of it was late with its rows, and everybody else late with it: 32-layer
+         * chain 1.221 against 1.210 ms, six layers of 4096 x 8192 188 against 182 us) */
+        const bool storer = blockIdx.x + 1u + wave == gridDim.x || (gridDim.x <= wave && blockIdx.x == 0u);
+        const SideSlots slots = { BY_VALUE ? &tab[i] : nullptr, par, sy.set_bytes };
         const uint32_t Bk = op.blocks;
         if (STAMPS && sy.stamps != nullptr) {         /* measurement only: when has the vector arrived? */
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             plan_stamp<STAMPS>(sy, i, 5, ln, wave);
         }
         if (by_unit) {
-            if (op.kind >= PLAN_Q6_K) plan_stage_finish_unit<1>(op, xu, act, red, storer, ln, wave);
-            else                      plan_stage_finish_unit<0>(op, xu, act, red, storer, ln, wave);
+            if (op.kind >= PLAN_Q6_K) plan_stage_finish_unit<1>(op, slots, xu, act, red, storer, ln, wave);
+            else                      plan_stage_finish_unit<0>(op, slots, xu, act, red, storer, ln, wave);
         } else {
-            if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, xs, act, red, storer, ln, wave);
-            else                      plan_stage_finish<0>(op, xs, act, red, storer, ln, wave);
+            if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, slots, xs, act, red, storer, ln, wave);
+            else                      plan_stage_finish<0>(op, slots, xs, act, red, storer, ln, wave);
         }
         plan_prefetch<HAS_Q5>(cur, B, 1u, ln);
         plan_stamp<STAMPS>(sy, i, 2, ln, wave);
@@ -944,9 +1121,9 @@ k_plan_ext(const PlanOp *__restrict__ ins, uint32_t n_ins, const PlanOp *__restr
         XStage xs;
 #pragma unroll
         for (int u = 0; u < 4; u++) xs.x[u] = xs.t[u] = xs.b[u] = XRegs{ 0.f, 0.f, 0.f, 0.f };
-        plan_stage_issue(op, xs, lane, wave);
-        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, xs, lds, red, true, lane, wave);
-        else                      plan_stage_finish<0>(op, xs, lds, red, true, lane, wave);
+        plan_stage_issue<false>(sy, op, xs, lane, wave);
+        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, SideSlots{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
+        else                      plan_stage_finish<0>(op, SideSlots{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
         __syncthreads();
         const uint32_t bytes = plan_image_bytes(op.kind, op.blocks);
         const CohBuf img = coh_buf(gptr<uint8_t>(uni(ins[j].xq)));
@@ -1056,6 +1233,9 @@ struct OxhPlan {
     PlanOp *d_run;                  /* k_plan_ext: the table it walks (d_ops stays the list of inputs) */
     uint32_t n_run;
     void *multi;                    /* a plan over a 32-value format: the table of GEMV launches (oxh_kernels.hip) */
+    bool by_value;                  /* k_plan hands results over by value (plan_slots) */
+    uint8_t *d_slots;               /* two sets of slots, set_bytes each */
+    size_t set_bytes;
     uint32_t *h_err;                /* page-locked: set by the kernel when a wait gave up, read before every launch */
 };
 
@@ -1063,10 +1243,14 @@ static const void *plan_kernel(const OxhPlan *pl)
 {
     /* with clock stamps attached (plans without Q5_K only): the variants that write them */
     if (pl->d_stamps != nullptr && !pl->has_q5)
-        return pl->ext ? reinterpret_cast<const void *>(k_plan_ext<false, true>) : reinterpret_cast<const void *>(k_plan<false, true>);
+        return pl->ext ? reinterpret_cast<const void *>(k_plan_ext<false, true>)
+             : pl->by_value ? reinterpret_cast<const void *>(k_plan<false, true, true>)
+                            : reinterpret_cast<const void *>(k_plan<false, false, true>);
     if (pl->ext)
         return pl->has_q5 ? reinterpret_cast<const void *>(k_plan_ext<true>) : reinterpret_cast<const void *>(k_plan_ext<false>);
-    return pl->has_q5 ? reinterpret_cast<const void *>(k_plan<true>) : reinterpret_cast<const void *>(k_plan<false>);
+    if (pl->by_value)
+        return pl->has_q5 ? reinterpret_cast<const void *>(k_plan<true, true>) : reinterpret_cast<const void *>(k_plan<false, true>);
+    return pl->has_q5 ? reinterpret_cast<const void *>(k_plan<true, false>) : reinterpret_cast<const void *>(k_plan<false, false>);
 }
 
 #define PLAN_TRY(call)                                                                      \
@@ -1129,6 +1313,159 @@ extern "C" int oxh_plan_deal(const size_t *rows, const int *paired, size_t n_seg
     return OXH_OK;
 }
 
+
+/* ─── handing over by value ───
+ *
+ * Every vector a later operation reads goes through slots in which its values are their own announcement (k_plan).
+ * Nothing then holds a workgroup back but the values it reads, so this is for plans in which that is enough: every
+ * input is one result of one earlier operation, whole or a part of it, or nothing in the plan has written it; and
+ * where two operations touch the same memory otherwise (an input written over later, results stored at the same
+ * place) either one wave stores both, in order, or every workgroup is known to have passed the first when the second is
+ * reached.  Any other plan waits for whole operations.
+ *
+ * Known: an operation all of whose results have been read, and which gave every workgroup rows, has been passed by
+ * every workgroup, with all that came before it. */
+struct PlanKnown {
+    size_t *read_by;                /* per operation: the one by which all its results have been read; 0: none, or not every workgroup had rows */
+    /* whether a workgroup that has taken in operation `at`'s inputs knows that all others have finished `op` */
+    bool passed(size_t op, size_t at) const
+    {
+        for (size_t k = op; k < at; k++)
+            if (read_by[k] != 0 && read_by[k] <= at) return true;
+        return false;
+    }
+};
+
+/* two slots used in turn by results of one length that the same workgroups store */
+struct PlanRing {
+    size_t at, bytes, from, to, side, turns, last_op, last_read;
+};
+
+/* the workgroups [from, to) that own a result, or the side outputs' one */
+static void plan_owner(const PlanOp &o, int w, size_t *from, size_t *to)
+{
+    *from = *to = 0;
+    if (w < 3) return;
+    const uint32_t k = (uint32_t)w - 3u;
+    *from = o.s[k].wg_begin;
+    *to = k + 1u < o.n_segs ? o.s[k + 1u].wg_begin : o.n_wg;
+}
+
+/* reads: four spans per operation (x, the prologue's b and addend); writes: eight (its output, its sum, the quantised
+ * blocks, the segments' results).  Returns false, or fills in the slots' offsets (+ 4, with slot_at's bits) and the
+ * operations' masks. */
+static bool plan_slots(PlanOp *h, size_t n_ops, uint32_t grid, const Span *reads, const Span *writes, size_t *set_bytes)
+{
+    struct Use { size_t first, last, at, ring; };
+    Use *use = (Use *)calloc(n_ops * 8, sizeof *use);
+    size_t *src = (size_t *)calloc(n_ops * 4, sizeof *src);
+    PlanRing *ring = (PlanRing *)calloc(n_ops * 8, sizeof *ring);
+    PlanKnown known = { (size_t *)calloc(n_ops, sizeof(size_t)) };
+    bool ok = use && src && ring && known.read_by;
+    for (size_t i = 0; ok && i < n_ops; i++)
+        for (int r = 0; r < 4 && ok; r++) {
+            const Span &rd = reads[i * 4 + r];
+            size_t &from = src[i * 4 + r];
+            for (size_t j = i; j-- > 0 && rd.p && !from && ok;)
+                for (int w = 0; w < 8 && ok; w++) {
+                    const Span &wr = writes[j * 8 + w];
+                    if (!spans_meet(rd, wr)) continue;
+                    /* the latest writer gives all of it, through one span, and not as quantised blocks */
+                    ok = !from && w != 2 && rd.p >= wr.p && rd.p + rd.n <= wr.p + wr.n && (rd.p - wr.p) % 4 == 0 &&
+                         (r != 1 || h[i].pro == GEMV_PRO_SWIGLU);
+                    from = j * 8 + (size_t)w + 1u;
+                }
+            if (ok && from) {
+                Use &u = use[from - 1u];
+                if (!u.first) u.first = i;
+                u.last = i;
+            }
+        }
+    for (size_t k = 0; ok && k < n_ops; k++) {
+        size_t last = 0;
+        bool all = h[k].n_wg == grid;
+        for (uint32_t g = 0; g < h[k].n_segs && all; g++) {
+            size_t first = 0;
+            for (size_t m = k + 1u; m < n_ops && !first; m++)
+                for (int r = 0; r < 4; r++)
+                    if (src[m * 4 + r] == k * 8 + 3u + g + 1u && reads[m * 4 + r].n == writes[k * 8 + 3u + g].n) first = m;
+            all = first != 0;
+            if (first > last) last = first;
+        }
+        known.read_by[k] = all ? last : 0;
+    }
+    for (size_t j = 1; ok && j < n_ops; j++)
+        for (size_t i = 0; i < j && ok; i++)
+            for (int w = 0; w < 8 && ok; w++) {
+                const Span &wj = writes[j * 8 + w];
+                const size_t at = w < 3 ? j - 1u : j;       /* side outputs are stored when part of the inputs has been taken in */
+                for (int r = 0; r < 4 && ok; r++)
+                    if (!src[i * 4 + r] && spans_meet(wj, reads[i * 4 + r])) ok = known.passed(i, at);
+                for (int v = 0; v < 8 && ok; v++) {
+                    const Span &wi = writes[i * 8 + v];
+                    if (!spans_meet(wj, wi)) continue;
+                    size_t f0, t0, f1, t1;
+                    plan_owner(h[i], v, &f0, &t0);
+                    plan_owner(h[j], w, &f1, &t1);
+                    /* one wave stores both, in order: the same rows, or the same part of a prologue's side output (a
+                     * workgroup's stores of operation i are acknowledged before it stores those of i + 1) */
+                    const bool same = wi.p == wj.p && wi.n == wj.n && (w < 3 ? v == w : v >= 3 && f0 == f1 && t0 == t1);
+                    ok = same || known.passed(i + 1u, at);
+                }
+            }
+    /* Slots: a result takes the ring of an earlier one where, when it is stored, everybody has read that one (its slot
+     * is emptied now), and the emptying of its own slot, which was done then, is known to everybody that reads it. */
+    size_t n_rings = 0, bytes = 0;
+    for (size_t i = 0; ok && i < n_ops; i++)
+        for (int w = 0; w < 8; w++) {
+            Use &u = use[i * 8 + w];
+            if (!u.first) continue;
+            size_t from, to, r = 0;
+            plan_owner(h[i], w, &from, &to);
+            const size_t n = writes[i * 8 + w].n, side = w < 3 ? 1u : 0u;
+            for (; r < n_rings; r++) {
+                const PlanRing &g = ring[r];
+                if (g.bytes == n && g.from == from && g.to == to && g.side == side && g.last_op < i && known.passed(g.last_read, i - side) &&
+                    known.passed(g.last_op + 1u, u.first - 1u)) break;
+            }
+            PlanRing &g = ring[r];
+            if (r == n_rings) {
+                g.at = bytes; g.bytes = n; g.from = from; g.to = to; g.side = side; g.turns = 0;
+                bytes += (n + 255u) & ~(size_t)255u;
+                n_rings++;
+            }
+            u.ring = r;
+            u.at = g.at + 4u + (g.turns & 1u);
+            g.turns++;
+            g.last_op = i;
+            g.last_read = u.last;
+        }
+    for (size_t i = 0; ok && i < n_ops * 8; i++)
+        if (use[i].first && (ring[use[i].ring].turns & 1u)) use[i].at += 2u;      /* an odd number of turns: the next launch begins with the other slot */
+    ok = ok && bytes > 0 && bytes < 0x10000000u;
+    /* more short operations than long ones wait for something: see SLOT_EMPTY */
+    size_t n_short = 0, n_long = 0;
+    for (size_t i = 0; ok && i < n_ops; i++)
+        if (src[i * 4] || src[i * 4 + 1] || src[i * 4 + 2]) (h[i].blocks > PLAN_W ? n_long : n_short)++;
+    ok = ok && n_long < n_short;
+    for (size_t i = 0; ok && i < n_ops; i++) {
+        gaddr *const in[3] = { &h[i].x, &h[i].pro_b, &h[i].pro_add };
+        const uint32_t bit[3] = { SLOT_X, SLOT_B, SLOT_ADD };
+        h[i].wait = 0;
+        for (int r = 0; r < 3; r++)
+            if (src[i * 4 + r]) {
+                const size_t w = src[i * 4 + r] - 1u;
+                *in[r] = (gaddr)use[w].at + (gaddr)(reads[i * 4 + r].p - writes[w].p);
+                h[i].wait |= bit[r];
+            }
+        h[i].reserved = (gaddr)use[i * 8 + 0].at;
+        h[i].xq = (gaddr)use[i * 8 + 1].at;
+        for (uint32_t g = 0; g < h[i].n_segs; g++) h[i].s[g].rows_q = (uint32_t)use[i * 8 + 3u + g].at;
+    }
+    *set_bytes = bytes;
+    free(use); free(src); free(ring); free(known.read_by);
+    return ok;
+}
 
 struct PlanLimits { uint32_t max_wg_rows, max_wg_terms, max_cap_terms; };
 
@@ -1321,7 +1658,7 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_plan_create: 1..65535 operations");
     if (oxh_internal_multi_which(ops[0].qtype) >= 0) return plan_create_multi(ops, n_ops, out);
     const uint32_t n_cu = (uint32_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
-    const uint32_t grid = n_cu > PLAN_MAX_WG ? PLAN_MAX_WG : n_cu;
+    uint32_t grid = n_cu > PLAN_MAX_WG ? PLAN_MAX_WG : n_cu;
 
     PlanOp *h = (PlanOp *)calloc(n_ops, sizeof *h);
     Span *reads = (Span *)calloc(n_ops * 4, sizeof *reads), *writes = (Span *)calloc(n_ops * 8, sizeof *writes);
@@ -1435,6 +1772,15 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         d.wait = wait;
         if (wait) { h[wait - 1].signal = 1; n_waits++; }
     }
+    /* no more workgroups than some operation has rows for: the others would only wait along */
+    uint32_t used = 1;
+    for (size_t i = 0; !rc && i < n_ops; i++) used = h[i].n_wg > used ? h[i].n_wg : used;
+    if (n_waits != 0) grid = used;
+    /* OXH_PLAN_BY_VALUE=0 keeps a chain on whole operations */
+    const char *bv = getenv("OXH_PLAN_BY_VALUE");
+    size_t set_bytes = 0;
+    const bool by_value = !rc && n_waits != 0 && n_ops * sizeof(PlanOp) <= 160u * 1024u && !(bv && bv[0] == '0') &&
+                          plan_slots(h, n_ops, grid, reads, writes, &set_bytes);
     free(reads);
     free(writes);
     if (rc) { free(h); return rc; }
@@ -1445,6 +1791,8 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
     pl->grid = grid;
     pl->n_waits = n_waits;
     pl->has_q5 = has_q5;
+    pl->by_value = by_value;
+    pl->set_bytes = by_value ? set_bytes : 0;
     {
         /* OXH_PLAN_PRESTAGE=0 keeps a plan of independent operations on the chained kernel */
         const char *ps = getenv("OXH_PLAN_PRESTAGE");
@@ -1523,7 +1871,23 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
     if (e == hipSuccess && pl->ext) e = hipMalloc((void **)&pl->d_img, img_bytes);
     if (e == hipSuccess && pl->ext) e = hipMalloc((void **)&pl->d_run, n_run * sizeof(PlanOp));
     /* the staged inputs' offsets become addresses */
-    for (size_t i = 0; i < n_ops; i++) h[i].xq = pl->ext ? (gaddr)(uintptr_t)pl->d_img + h[i].xq : 0u;
+    for (size_t i = 0; !by_value && i < n_ops; i++) h[i].xq = pl->ext ? (gaddr)(uintptr_t)pl->d_img + h[i].xq : 0u;
+    /* ... and so do the slots' */
+    if (e == hipSuccess && by_value) e = hipMalloc((void **)&pl->d_slots, 2u * set_bytes);
+    if (e == hipSuccess && by_value) e = hipMemsetD32((hipDeviceptr_t)pl->d_slots, (int)SLOT_EMPTY, 2u * set_bytes / 4u);
+    for (size_t i = 0; by_value && i < n_ops; i++) {
+        const gaddr base = (gaddr)(uintptr_t)pl->d_slots;
+        if (h[i].wait & SLOT_X) h[i].x += base - 4u;
+        if (h[i].wait & SLOT_B) h[i].pro_b += base - 4u;
+        if (h[i].wait & SLOT_ADD) h[i].pro_add += base - 4u;
+        h[i].xq = h[i].xq ? base + h[i].xq - 4u : 0u;
+        h[i].reserved = h[i].reserved ? base + h[i].reserved - 4u : 0u;
+        for (uint32_t k = 0; k < h[i].n_segs; k++) {
+            const gaddr to = h[i].s[k].rows_q ? base + h[i].s[k].rows_q - 4u : 0u;
+            h[i].s[k].rows_q = (uint32_t)to;
+            h[i].s[k].rows_rem = (uint32_t)(to >> 32);
+        }
+    }
     /* the chained kernel reads its deal of rows to workgroups from the segments' xq (plan_work) */
     for (size_t i = 0; !pl->ext && i < n_ops; i++)
         for (uint32_t k = 0; k < h[i].n_segs; k++) {
@@ -1545,6 +1909,7 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         if (pl->d_ops) (void)hipFree(pl->d_ops);
         if (pl->d_run) (void)hipFree(pl->d_run);
         if (pl->d_img) (void)hipFree(pl->d_img);
+        if (pl->d_slots) (void)hipFree(pl->d_slots);
         if (pl->d_sync) (void)hipFree(pl->d_sync);
         if (pl->h_err) (void)hipHostFree(pl->h_err);
         free(pl);
@@ -1582,6 +1947,7 @@ extern "C" int oxh_plan_launch(OxhPlan *pl, void *stream)
     sy.spin_limit = pl->spin_limit;
     sy.stamps = pl->d_stamps;
     sy.host_err = pl->h_err;
+    sy.set_bytes = (uint32_t)pl->set_bytes;
 #define PLAN_LAUNCH(K)                                                                                  \
     hipLaunchKernelGGL(K, dim3(pl->grid), dim3(1024), pl->lds_bytes, st, (const PlanOp *)pl->d_ops,    \
                        pl->n_ops, sy, pl->ld)
@@ -1594,9 +1960,13 @@ extern "C" int oxh_plan_launch(OxhPlan *pl, void *stream)
         else if (pl->has_q5) PLAN_LAUNCH_EXT(k_plan_ext<true>);
         else                 PLAN_LAUNCH_EXT(k_plan_ext<false>);
     } else {
-        if (stamped)         PLAN_LAUNCH((k_plan<false, true>));
-        else if (pl->has_q5) PLAN_LAUNCH(k_plan<true>);
-        else                 PLAN_LAUNCH(k_plan<false>);
+        const bool val = pl->by_value;
+        if (stamped && val)         PLAN_LAUNCH((k_plan<false, true, true>));
+        else if (stamped)           PLAN_LAUNCH((k_plan<false, false, true>));
+        else if (pl->has_q5 && val) PLAN_LAUNCH((k_plan<true, true>));
+        else if (pl->has_q5)        PLAN_LAUNCH((k_plan<true, false>));
+        else if (val)               PLAN_LAUNCH((k_plan<false, true>));
+        else                        PLAN_LAUNCH((k_plan<false, false>));
     }
 #undef PLAN_LAUNCH
 #undef PLAN_LAUNCH_EXT
@@ -1645,6 +2015,11 @@ extern "C" int oxh_debug_plan_phantom(OxhPlan *pl, int on)
     return OXH_OK;
 }
 
+extern "C" int oxh_debug_plan_by_value(const OxhPlan *pl)
+{
+    return pl && pl->by_value ? 1 : 0;
+}
+
 extern "C" int oxh_debug_plan_stamps(OxhPlan *pl, uint64_t *d_stamps)
 {
     if (!pl) return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_debug_plan_stamps: NULL plan");
@@ -1664,6 +2039,7 @@ extern "C" int oxh_plan_status(OxhPlan *pl, void *stream)
     if (go[1] == 0u) return OXH_OK;
     /* a wait ran out: the counters are no longer equal, start them afresh */
     PLAN_TRY(hipMemset(pl->d_sync, 0, (PLAN_COPIES * PLAN_MAX_WG + 8u) * sizeof(uint32_t)));
+    if (pl->by_value) PLAN_TRY(hipMemsetD32((hipDeviceptr_t)pl->d_slots, (int)SLOT_EMPTY, 2u * pl->set_bytes / 4u));
     PLAN_TRY(hipDeviceSynchronize());
     *(volatile uint32_t *)pl->h_err = 0u;
     return oxh_internal_errorf(OXH_ERR_TIMEOUT, "plan: a wait between operations ran out of polls (not every workgroup "
@@ -1678,6 +2054,7 @@ extern "C" int oxh_plan_destroy(OxhPlan *pl)
     if (pl->d_ops) (void)hipFree(pl->d_ops);
     if (pl->d_run) (void)hipFree(pl->d_run);
     if (pl->d_img) (void)hipFree(pl->d_img);
+    if (pl->d_slots) (void)hipFree(pl->d_slots);
     if (pl->d_sync) (void)hipFree(pl->d_sync);
     if (pl->h_err) (void)hipHostFree(pl->h_err);
     free(pl);

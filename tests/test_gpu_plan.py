@@ -246,6 +246,60 @@ def test_clock_stamps_run_the_stamped_kernels_with_the_same_bits(oxh):
     plan.destroy()
 
 
+@pytest.mark.parametrize("hidden,kv,ffn,layers,by_value", [(256, 256, 512, 5, 1), (1024, 256, 2816, 4, 1), (2304, 256, 6144, 3, 1),
+                                                           (4096, 1024, 4352, 2, 1), (4352, 256, 8192, 2, 0)])
+def test_chains_by_value_and_by_whole_operations_are_the_launches(oxh, monkeypatch, hidden, kv, ffn, layers, by_value):
+    """Both hand-overs of a chain, with other inputs before every launch, so that a value left in a slot by an earlier
+    launch or layer would show: fewer rows than workgroups, an odd and an even number of layers, vectors on both
+    sides of sixteen blocks; and values that are NaN, which have to arrive as well."""
+    d = DecodeSet(hidden=hidden, kv=kv, ffn=ffn, layers=layers, seed=5)
+    a, b, c = (DecodeChain(d, seed=5) for _ in range(3))
+    value = mv.Plan(b.plan_ops())
+    monkeypatch.setenv("OXH_PLAN_BY_VALUE", "0")
+    whole = mv.Plan(c.plan_ops())
+    monkeypatch.delenv("OXH_PLAN_BY_VALUE")
+    assert _lib.lab().plan_by_value(value.handle) == by_value and _lib.lab().plan_by_value(whole.handle) == 0
+    for rep in range(6):
+        x = np.array(synth.normal(hidden, seed=rep, stream=77))
+        if rep == 4:
+            x[::97] = np.nan
+        f = synth.normal(hidden, seed=rep, stream=78)
+        for s in (a, b, c):
+            s.x0.upload(x)
+            s.f0.upload(f)
+        a.launch_step()
+        mv.sync()
+        want = chain_state(a)
+        for s, plan in ((b, value), (c, whole)):
+            plan.launch()
+            assert plan.status() == 0
+            got = chain_state(s)
+            for k in ("qkv", "o", "h", "f", "x"):
+                assert np.array_equal(got[k], want[k], equal_nan=True), (rep, k)
+                assert rep == 4 or np.array_equal(bits(got[k]), bits(want[k])), (rep, k)
+    value.destroy()
+    whole.destroy()
+
+
+def test_an_input_made_of_two_results_waits_for_the_whole_operation(oxh):
+    w = [mv.DeviceBuffer.from_host(synth.weights(Q4K, r, 1024, seed=3, stream=i)) for i, r in enumerate((1024, 300, 40))]
+    half = 512 * synth.row_bytes(Q4K, 1024)
+    x, mid, out = mv.DeviceBuffer.from_host(synth.normal(1024, seed=3)), mv.DeviceBuffer(4096), mv.DeviceBuffer(1200)
+    two = mv.make_segments([(w[0].ptr, mid.ptr, 512, 0), (w[0].ptr + half, mid.ptr + 2048, 512, 0)])
+    one = mv.make_segments([(w[1].ptr, out.ptr, 300, 0)])
+    mv.gemv_segments_f32(Q4K, two, 1024, x.ptr, 1024, None, 1, 0)
+    mv.gemv_segments_f32(Q4K, one, 1024, mid.ptr, 1024, None, 1, 0)
+    mv.sync()
+    want = out.download(np.float32, 300)
+    plan = mv.Plan([dict(qtype=Q4K, segs=two, cols=1024, d_x=x.ptr), dict(qtype=Q4K, segs=one, cols=1024, d_x=mid.ptr)])
+    assert plan.info()["n_waits"] == 1 and _lib.lab().plan_by_value(plan.handle) == 0
+    for _ in range(2):
+        plan.launch()
+        assert plan.status() == 0
+        assert np.array_equal(bits(out.download(np.float32, 300)), bits(want))
+    plan.destroy()
+
+
 def test_a_wait_that_cannot_be_satisfied_gives_up(oxh):
     """The waits expect one workgroup more than exist and may poll 300 times: every workgroup must leave,
     the launch must end, the status must say so, and the plan must work again afterwards."""
