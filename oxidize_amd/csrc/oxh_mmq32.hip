@@ -5,14 +5,15 @@
  * float step is the reference's, in its order, so every result has the single-vector dot's bits.  Codes with an
  * offset are staged as the signed values code - offset, so four formats share Q8_0's step exactly.
  *
- * What bounds it.  The float step: four vector instructions per result and block (seven for the _1 formats) beside a
- * 256th of an MFMA.  Alone on a SIMD with two or four waves those four (multiply, convert, multiply, add) take 2.6 cycles
- * each, 41 per 16 x 16 tile, the MFMA 8, both in one loop 55: 4096 x 4096 x 512 would be 23 us of that loop.  So
- * everything else has to stay off that port: a block is fetched and taken apart ONCE per
- * workgroup, by a lane that owns it (eight lanes along a row's consecutive blocks, so that a wave's load touches some
- * 24 cache lines and not 64), and goes to LDS as MFMA operands, int8 values and f32 scales; the inner loop issues
- * MFMAs, the float step and nothing else but LDS reads, twelve of 16 bytes per eight tiles (eighteen for the _1
- * formats).  Of the compiled step of eight blocks' 335 vector instructions (Q8_0; Q4_1 537) 256 (448) are the float step.
+ * What bounds it.  The float step: three vector instructions per result and block (seven for the _1 formats) beside a
+ * 256th of an MFMA, at 2.6 cycles each on a SIMD of two or four waves.  So everything else has to stay off that port: a
+ * block is fetched and taken apart ONCE per workgroup, by a lane that owns it (eight lanes along a row's consecutive
+ * blocks, so that a wave's load touches some 24 cache lines and not 64), and goes to LDS as MFMA operands, int8 values and
+ * scales; the inner loop issues MFMAs, the float step and little else but LDS reads.  The products of the scales come
+ * from the matrix cores as well, four blocks to an instruction (`scales`): one of four vector instructions gone, and
+ * three two-byte reads of LDS per sixteen tiles in the place of six of 16 bytes, on a pipe that was nearly as busy
+ * (quantiser and matmul, us: Q8_0 4096 x 4096 x 512 50.2 -> 48.4, 14336 x 4096 x 256 85.0 -> 81.1, Q4_0 85.1 -> 81.7,
+ * AL5_XS 90.7 -> 87.6).  The _1 formats have two products and no registers for both: theirs stay vector instructions.
  *
  * Shape.  A wave computes 16 rows x 32 tokens; eight waves, 64 rows x 64 tokens, to a workgroup and two workgroups to
  * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues dependent
@@ -40,12 +41,12 @@ template <int LEG, bool WIDE> struct Mmq32Geom {
     /* A stage.  Values: [pair][row or token][16-byte slot]: slot s of row r holds values 8k .. 8k+7 of the pair's
      * two blocks, k = s ^ mmq32_swizzle(r); a pair is skewed by a slot row.  Scales of rows [block][row], of tokens [four blocks][token][4]. */
     static constexpr uint32_t W_PAIR = ROWS * 64u, A_PAIR = TOK * 64u;
-    /* the skew spreads the eight blocks' scales over the banks; with the minimums too there is no room for it */
-    static constexpr uint32_t D_PITCH = ROWS + (HAS_M ? 0u : 8u);
+    static constexpr uint32_t D_PITCH = ROWS;
     static constexpr uint32_t A_OFF = KP * W_PAIR;
     static constexpr uint32_t DW_OFF = A_OFF + KP * A_PAIR;
-    static constexpr uint32_t DQ_OFF = DW_OFF + KB * D_PITCH * 4u;
-    static constexpr uint32_t MW_OFF = DQ_OFF + KB * TOK * 4u;
+    /* without minimums: the halves themselves, [row or token][block] */
+    static constexpr uint32_t DQ_OFF = DW_OFF + (HAS_M ? KB * D_PITCH * 4u : ROWS * KB * 2u);
+    static constexpr uint32_t MW_OFF = DQ_OFF + KB * TOK * (HAS_M ? 4u : 2u);
     static constexpr uint32_t QS_OFF = MW_OFF + (HAS_M ? KB * D_PITCH * 4u : 0u);
     static constexpr uint32_t STAGE_BYTES = QS_OFF + (HAS_M ? KB * TOK * 4u : 0u);
     static constexpr uint32_t LDS_BYTES = 2u * STAGE_BYTES;
@@ -139,7 +140,8 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
                 }
             }
             put(st, w_dst[i], q, live);
-            reinterpret_cast<float *>(st + G::DW_OFF)[s_blk * G::D_PITCH + r] = live ? half_to_float_hw(d) : 0.0f;
+            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DW_OFF)[r * G::KB + s_blk] = live ? (uint16_t)d : (uint16_t)0u;
+            if (HAS_M) reinterpret_cast<float *>(st + G::DW_OFF)[s_blk * G::D_PITCH + r] = live ? half_to_float_hw(d) : 0.0f;
             if (HAS_M) reinterpret_cast<float *>(st + G::MW_OFF)[s_blk * G::D_PITCH + r] = live ? m : 0.0f;
         }
 #pragma unroll
@@ -150,8 +152,9 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
             const uint32_t d = q80_unpack(a_raw[i], q);
             put(st, a_dst[i], q, live);
             const uint32_t at = ((s_blk >> 2) * G::TOK + t) * 4u + (s_blk & 3u);
-            reinterpret_cast<float *>(st + G::DQ_OFF)[at] = live ? half_to_float_hw(d) : 0.0f;
+            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DQ_OFF)[t * G::KB + s_blk] = live ? (uint16_t)d : (uint16_t)0u;
             if (HAS_M) {
+                reinterpret_cast<float *>(st + G::DQ_OFF)[at] = live ? half_to_float_hw(d) : 0.0f;
                 int qs = 0;
 #pragma unroll
                 for (int k = 0; k < 8; k++) qs = dot4(0x01010101u, q[k], qs);
@@ -163,7 +166,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     /* a wave's operands of one pair of blocks */
     struct Frag {
         u32x4 w[RC], a[TC];
-        v4f dw[2][RC];
+        v4f dw[HAS_M ? 2 : 1][RC];
     };
     const uint32_t rw = wave % G::RW, tw = wave / G::RW;
     const uint32_t w_row = rw * (16u * G::RC) + r16, a_row = tw * (16u * G::TC) + r16;
@@ -171,6 +174,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     const uint32_t w_rd = w_row * 64u + swz, a_rd = G::A_OFF + a_row * 64u + swz;
     const uint32_t dw_rd = G::DW_OFF + (rw * (16u * G::RC) + 4u * kq) * 4u;
     const uint32_t dq_rd = G::DQ_OFF + a_row * 16u;
+    const uint32_t dwh_rd = G::DW_OFF + w_row * (2u * G::KB) + 2u * kq;      /* halves: this lane's of four blocks is block kq's */
     auto fetch = [&](const uint8_t *st, int p) -> Frag {
         Frag f;
 #pragma unroll
@@ -178,7 +182,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
 #pragma unroll
         for (int tc = 0; tc < TC; tc++) f.a[tc] = *reinterpret_cast<const u32x4 *>(st + (a_rd ^ (16u * ((uint32_t)p & 3u))) + (uint32_t)p * G::A_PAIR + 1024u * (uint32_t)tc);
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < (HAS_M ? 2 : 0); j++)
 #pragma unroll
             for (int rc = 0; rc < RC; rc++) {
                 const uint32_t at = ((2u * (uint32_t)p + (uint32_t)j) * G::D_PITCH + 16u * (uint32_t)rc) * 4u;
@@ -195,7 +199,24 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     auto block_of = [](const u32x4 &v, int j) -> long {
         return (long)(((unsigned long)v[2 * j + 1] << 32) | (unsigned long)v[2 * j]);
     };
-    auto compute = [&](const Frag &f, const uint8_t *st, const v4f dq[TC], const v4f qs[TC], int p) {
+    /* dw * dq of four blocks: a product of two halves is an f32 exactly, and v_mfma_f32_16x16x4_4b_f16 is four outer
+     * products side by side, block b from the operands of lanes 16 b .. 16 b + 15, the result where the integer
+     * MFMA of the block has its own */
+    auto scales = [&](const uint8_t *st, int q, v16f t[RC][TC]) {
+        v4h a[RC], b[TC];
+#pragma unroll
+        for (int rc = 0; rc < RC; rc++)
+            a[rc] = (v4h){ *reinterpret_cast<const _Float16 *>(st + dwh_rd + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)rc), (_Float16)0, (_Float16)0, (_Float16)0 };
+#pragma unroll
+        for (int tc = 0; tc < TC; tc++)
+            b[tc] = (v4h){ *reinterpret_cast<const _Float16 *>(st + dq_rd + 2u * kq + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)tc), (_Float16)0, (_Float16)0, (_Float16)0 };
+        const v16f none = {};
+#pragma unroll
+        for (int rc = 0; rc < RC; rc++)
+#pragma unroll
+            for (int tc = 0; tc < TC; tc++) t[rc][tc] = __builtin_amdgcn_mfma_f32_16x16x4f16(a[rc], b[tc], none, 0, 0, 0);
+    };
+    auto compute = [&](const Frag &f, const uint8_t *st, const v4f dq[TC], const v4f qs[TC], const v16f ts[RC][TC], int p) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int bq = 2 * (p & 1) + j;
@@ -217,7 +238,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
                 for (int tc = 0; tc < TC; tc++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const float t = f.dw[j][rc][i] * dq[tc][bq];
+                        const float t = HAS_M ? f.dw[HAS_M ? j : 0][rc][i] * dq[tc][bq] : ts[rc][tc][4 * bq + i];
                         const float up = t * (float)isum[rc][tc][i];
                         if (HAS_M) {
                             const float tm = mw[rc][i] * dq[tc][bq];
@@ -243,17 +264,19 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
         for (int q = 0; q < KP / 2; q++) {
             if (4u * (uint32_t)q < nb) {
                 v4f dq[TC], qs[TC];
+                v16f ts[RC][TC];
+                if (!HAS_M) scales(st, q, ts);
 #pragma unroll
                 for (int tc = 0; tc < TC; tc++) {
-                    dq[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
+                    if (HAS_M) dq[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
                     if (HAS_M) qs[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (G::QS_OFF - G::DQ_OFF) + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
                 }
                 const Frag nxt = fetch(st, 2 * q + 1);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(cur, st, dq, qs, 2 * q);
+                compute(cur, st, dq, qs, ts, 2 * q);
                 if (q + 1 < KP / 2) cur = fetch(st, 2 * q + 2);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(nxt, st, dq, qs, 2 * q + 1);
+                compute(nxt, st, dq, qs, ts, 2 * q + 1);
             }
             if (q == 0 && s + 1u < n_steps) {
                 store(s + 1u);

@@ -231,3 +231,30 @@ def test_segment_that_starts_two_bytes_past_a_multiple_of_four(oxh, name, qtype,
         d_x.free()
         d_o.free()
     d_w.free()
+
+
+@pytest.mark.parametrize("n_vec", [65, 100])
+@pytest.mark.parametrize("qtype", [7, 3, 4, 5, 6, 18])
+def test_prompt_scales_of_every_size(oxh, qtype, n_vec):
+    """The prompt kernel multiplies the scales as halves: subnormal, largest, infinite and NaN factors beside ordinary ones
+    have to give the f32 products' bits, and only in their own block, row and token.  Nine blocks, so that the last step
+    has one."""
+    rows, cols = 130, 288
+    rb = synth.row_bytes(qtype, cols)
+    w = np.array(synth.weights(qtype, rows, cols, seed=8)).reshape(-1, rb // 9)
+    halves = np.array([0x0001, 0x8001, 0x03FF, 0x0400, 0x7BFF, 0xFBFF, 0x0000, 0x8000, 0x2C00], np.uint16)
+    w[:, 0:2] = halves[(np.arange(len(w)) * 5) % 9].view(np.uint8).reshape(-1, 2)
+    for row, half in ((7, 0x7C00), (70, 0xFC00), (129, 0x7E00)):                    # inf, -inf, NaN
+        w[row * 9 + 8 - row % 5, 0:2] = np.array([half], np.uint16).view(np.uint8)
+    xs = np.stack([synth.normal(cols, seed=9, stream=v) * np.float32(2.0) ** (3 * (v % 9) - 20) for v in range(n_vec)]).astype(np.float32)
+    o = oxlibs.oracle()
+    got, temp = np.zeros((n_vec, rows), np.float32), np.zeros(cols, np.float32)
+    scratch = np.zeros(mv.batch_scratch_bytes(cols), np.uint8)
+    w = np.ascontiguousarray(w).reshape(-1)
+    assert mv.matvec_quantized_batch(qtype, w, rows, cols, rb, xs, cols, got, rows, n_vec, temp, scratch) == 0
+    for v in range(n_vec):
+        want = np.zeros(rows, np.float32)
+        assert o.oxo_matvec_quantized(qtype, w.ctypes.data, rows, cols, rb, xs[v].ctypes.data, want.ctypes.data, temp.ctypes.data) == 0
+        assert np.array_equal(np.isnan(got[v]), np.isnan(want)), (qtype, v)
+        fine = ~np.isnan(want)
+        assert fine.sum() >= rows - 3 and np.array_equal(got[v][fine].view(np.uint32), want[fine].view(np.uint32)), (qtype, v)
