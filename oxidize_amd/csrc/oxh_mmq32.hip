@@ -19,10 +19,12 @@
  * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues dependent
  * vector instructions 8.3 cycles apart and independent ones 4.7 to 5.4.  Steps of eight blocks, two stages in LDS, one
  * barrier per step; the next step's blocks go to LDS in the middle of a step and the ones after it are requested
- * then.  Q8_0 4096 x 4096 x 512 takes 41 us (128 x 64 tiles whose waves kept raw blocks in regions of their own, one
- * workgroup to a CU: 69; 128 x 64 on eight waves of 32 x 32: 42.5, and 162 us at 14336 rows where this takes 136).
- * At the 128 registers that four waves allow, Q4_1's narrow tile spills 12 bytes, its wide one and Q5_1's narrow one 4;
- * one reload, 8 bytes in Q4_1's narrow tile, is inside the step loop. */
+ * then.  Of the Q8_0 tile's 92 % vector issue by counter, a third was not the float step: 64-bit addresses formed anew for
+ * every block, the place within four bytes asked again, values cleared past the row's end.  With a wave's address in
+ * scalar registers and 32-bit offsets stepped along, 279 of 317 instructions are left (quantiser and
+ * matmul, us: Q8_0 4096 x 4096 x 512 48.4 -> 45.3, 14336 x 4096 x 256 81.1 -> 75.5, Q4_0 81.7 -> 74.5, Q5_0 86.0 -> 79.4,
+ * AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113; Q5_1 alone on its CUs, 900 x 8192 x 128, 69.6 -> 71.0).  128 x 64 tiles whose waves kept raw blocks in regions of their own, one
+ * workgroup to a CU, took 69 us where this took 41, eight waves of 32 x 32 42.5. */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -50,14 +52,19 @@ template <int LEG, bool WIDE> struct Mmq32Geom {
     static constexpr uint32_t QS_OFF = MW_OFF + (HAS_M ? KB * D_PITCH * 4u : 0u);
     static constexpr uint32_t STAGE_BYTES = QS_OFF + (HAS_M ? KB * TOK * 4u : 0u);
     static constexpr uint32_t LDS_BYTES = 2u * STAGE_BYTES;
-    static constexpr uint32_t W_UNITS = ROWS * KB / THREADS, A_UNITS = (TOK * KB + THREADS - 1u) / THREADS;      /* blocks a thread stages */
-    static_assert(W_UNITS * THREADS == ROWS * KB && TOK * KB % (THREADS < TOK * KB ? THREADS : TOK * KB) == 0u && KP % 2u == 0u, "staging");
+    static_assert(THREADS == ROWS * KB && TOK * KB <= THREADS && TOK * KB % 64u == 0u && KP % 2u == 0u, "staging: a thread, a block of weights");
     static_assert((WIDE ? 1u : 2u) * LDS_BYTES <= 160u * 1024u, "workgroups to a CU");
 };
 
 /* Rows lie 64 bytes apart: eight aligned rows' slots of one k fall on the eight 16-byte pieces of 128 bytes, sixteen
  * rows' on the sixteen of 256. */
 __device__ __forceinline__ uint32_t mmq32_swizzle(uint32_t row) { return ((row >> 1) & 3u) ^ ((row >> 3) & 1u); }
+
+/* a half and three zeros: an operand of one K */
+__device__ __forceinline__ v4h half_first(const uint8_t *p)
+{
+    return __builtin_bit_cast(v4h, make_uint2(*reinterpret_cast<const uint16_t *>(p), 0u));
+}
 
 template <int LEG> struct Mmq32Raw { LegRegs r; };
 template <> struct Mmq32Raw<0> { Q80Regs r; };
@@ -84,53 +91,74 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
 
     /* staging: this thread's blocks are block tid % KB of a step, rows (tokens) tid / KB and further ones */
     const uint32_t s_blk = tid % G::KB, s_row = tid / G::KB;
-    const uint8_t *w_at[G::W_UNITS], *a_at[G::A_UNITS];
-    uint32_t w_dst[G::W_UNITS], a_dst[G::A_UNITS];
-#pragma unroll
-    for (uint32_t i = 0; i < G::W_UNITS; i++) {
-        const uint32_t r = s_row + i * (G::THREADS / G::KB);
-        w_at[i] = w + (size_t)(row_first + min(r, rows_here - 1u)) * B * G::BB;
-        w_dst[i] = (s_blk >> 1) * G::W_PAIR + r * 64u + 16u * (mmq32_swizzle(r) ^ ((s_blk >> 1) & 3u)) + 8u * (s_blk & 1u);      /* ^ 16 k */
+    uint32_t w_dst, a_dst;
+    {
+        const uint32_t k = (s_blk >> 1) & 3u;
+        w_dst = (s_blk >> 1) * G::W_PAIR + s_row * 64u + 16u * (mmq32_swizzle(s_row) ^ k) + 8u * (s_blk & 1u);      /* ^ 16 k */
+        a_dst = G::A_OFF + (s_blk >> 1) * G::A_PAIR + s_row * 64u + 16u * (mmq32_swizzle(s_row) ^ k) + 8u * (s_blk & 1u);
     }
-#pragma unroll
-    for (uint32_t i = 0; i < G::A_UNITS; i++) {
-        const uint32_t t = s_row + i * (G::THREADS / G::KB);
-        a_at[i] = acts + (size_t)(tok_first + min(t, toks_here - 1u)) * B * 34u;
-        a_dst[i] = G::A_OFF + (s_blk >> 1) * G::A_PAIR + t * 64u + 16u * (mmq32_swizzle(t) ^ ((s_blk >> 1) & 3u)) + 8u * (s_blk & 1u);
-    }
-    Mmq32Raw<LEG> w_raw[G::W_UNITS];
-    Q80Regs a_raw[G::A_UNITS];
+    /* A wave stages eight rows (tokens): the first one's address is the wave's, less two bytes since an edge dword may
+     * begin there, a lane's block is a 32-bit offset from it (mmq32_launch sees to it), and so is its edge.  A thread's
+     * blocks are a step's eight apart, which is a multiple of four bytes in every format: their place within four
+     * is asked once.  Past the row's end a thread stays on its last block. */
+    static_assert(G::KB * G::BB % 4u == 0u && G::KB * 34u % 4u == 0u, "blocks of a thread");
+    const uint32_t wave_row = wave * (64u / G::KB), b_first = min(s_blk, B - 1u);
+    const uint32_t w_row0 = min(wave_row, rows_here - 1u), a_row0 = min(wave_row, toks_here - 1u);
+    const uint8_t *const w_base = w + (size_t)(row_first + w_row0) * B * G::BB - 2;
+    const uint8_t *const a_base = acts + (size_t)(tok_first + a_row0) * B * 34u - 2;
+    uint32_t w_off = 2u + ((min(s_row, rows_here - 1u) - w_row0) * B + b_first) * G::BB;
+    uint32_t a_off = 2u + ((min(s_row, toks_here - 1u) - a_row0) * B + b_first) * 34u;
+    const uint32_t w_odd = block_odd(w_base + w_off), a_odd = block_odd(a_base + a_off);
+    Mmq32Raw<LEG> w_raw;
+    Q80Regs a_raw;
+    constexpr bool W_EDGE = LEG == 0 || LegEdge<LEG ? LEG : 1>::ON;
+    uint32_t w_edge = w_off + (w_odd ? 0u - 2u : G::BB - 4u), a_edge = a_off + (a_odd ? 0u - 2u : 30u);
+    w_off += W_EDGE ? w_odd : 0u;
+    a_off += a_odd;
+    a_raw.shift = a_odd ? 0u : 16u;
+    if constexpr (LEG == 0) w_raw.r.shift = w_odd ? 0u : 16u;
+    else if (W_EDGE) w_raw.r.qh = w_odd ? 0u : 16u;
+    /* fetches step `step`, the steps in turn from 0 */
     auto load = [&](uint32_t step) {
-        const uint32_t b = min(step * G::KB + s_blk, B - 1u);
-#pragma unroll
-        for (uint32_t i = 0; i < G::W_UNITS; i++) {
-            if constexpr (LEG == 0) q80_load_at(w_raw[i].r, w_at[i] + (size_t)b * G::BB);
-            else leg_load_at<LEG>(w_raw[i].r, w_at[i] + (size_t)b * G::BB);
+        const bool on = step != 0u && step * G::KB + s_blk < B;
+        const uint32_t w_on = on ? G::KB * G::BB : 0u, a_on = on ? G::KB * 34u : 0u;
+        w_off += w_on;
+        if (W_EDGE) w_edge += w_on;
+        if constexpr (LEG == 0) {
+            w_raw.r.w0 = *reinterpret_cast<const U32x4a4g *>(w_base + w_off);
+            w_raw.r.w1 = *reinterpret_cast<const U32x4a4g *>(w_base + w_off + 16);
+            w_raw.r.edge = reinterpret_cast<const U32u2 *>(w_base + w_edge)->v;
+        } else if constexpr (W_EDGE) {
+            w_raw.r.qs = *reinterpret_cast<const U32x4a4g *>(w_base + w_off);
+            w_raw.r.hdr = reinterpret_cast<const U32u2 *>(w_base + w_edge)->v;
+        } else {
+            leg_load_at<LEG>(w_raw.r, w_base + w_off, w_odd);
         }
-#pragma unroll
-        for (uint32_t i = 0; i < G::A_UNITS; i++) q80_load_at(a_raw[i], a_at[i] + (size_t)b * 34u);
+        a_off += a_on;
+        a_edge += a_on;
+        a_raw.w0 = *reinterpret_cast<const U32x4a4g *>(a_base + a_off);
+        a_raw.w1 = *reinterpret_cast<const U32x4a4g *>(a_base + a_off + 16);
+        a_raw.edge = reinterpret_cast<const U32u2 *>(a_base + a_edge)->v;
     };
-    /* blocks past the row's end are staged as zeros with zero scales: their term is +0, which changes nothing (a
-     * sum that starts at +0 never becomes -0) */
-    auto put = [&](uint8_t *st, uint32_t dst, const uint32_t q[8], bool live) {
+    /* blocks past the row's end get zero scales (their values are another block's): their term is 0, which changes
+     * nothing (a sum that starts at +0 never becomes -0) */
+    auto put = [&](uint8_t *st, uint32_t dst, const uint32_t q[8]) {
 #pragma unroll
-        for (uint32_t k = 0; k < 4u; k++)
-            *reinterpret_cast<uint2 *>(st + (dst ^ (16u * k))) = live ? make_uint2(q[2 * k], q[2 * k + 1]) : make_uint2(0u, 0u);
+        for (uint32_t k = 0; k < 4u; k++) *reinterpret_cast<uint2 *>(st + (dst ^ (16u * k))) = make_uint2(q[2 * k], q[2 * k + 1]);
     };
     auto store = [&](uint32_t step) {
         uint8_t *st = mmq_lds + (step & 1u) * G::STAGE_BYTES;
         const bool live = step * G::KB + s_blk < B;
-#pragma unroll
-        for (uint32_t i = 0; i < G::W_UNITS; i++) {
-            const uint32_t r = s_row + i * (G::THREADS / G::KB);
+        {
+            const uint32_t r = s_row;
             uint32_t q[8], d;
             float m = 0.0f;
             if constexpr (LEG == 0) {
-                d = q80_unpack(w_raw[i].r, q);
+                d = q80_unpack(w_raw.r, q);
             } else {
                 uint32_t lo[4], hi[4];
-                d = leg_unpack<LEG>(w_raw[i].r, lo, hi);
-                if (HAS_M) m = half_to_float_hw(w_raw[i].r.hdr >> 16);
+                d = leg_unpack<LEG>(w_raw.r, lo, hi);
+                if (HAS_M) m = half_to_float_hw(w_raw.r.hdr >> 16);
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     /* code - offset as a signed byte: codes stay below 2 * offset, so no carry leaves a byte */
@@ -139,26 +167,24 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
                     q[4 + k] = HAS_M ? hi[k] : (hi[k] + UP) ^ 0x80808080u;
                 }
             }
-            put(st, w_dst[i], q, live);
-            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DW_OFF)[r * G::KB + s_blk] = live ? (uint16_t)d : (uint16_t)0u;
+            put(st, w_dst, q);
+            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DW_OFF)[tid] = live ? (uint16_t)d : (uint16_t)0u;
             if (HAS_M) reinterpret_cast<float *>(st + G::DW_OFF)[s_blk * G::D_PITCH + r] = live ? half_to_float_hw(d) : 0.0f;
             if (HAS_M) reinterpret_cast<float *>(st + G::MW_OFF)[s_blk * G::D_PITCH + r] = live ? m : 0.0f;
         }
-#pragma unroll
-        for (uint32_t i = 0; i < G::A_UNITS; i++) {
-            const uint32_t t = s_row + i * (G::THREADS / G::KB);
-            if (WIDE && wave >= G::TOK * G::KB / 64u) break;        /* more threads than token blocks */
+        if (!WIDE || wave < G::TOK * G::KB / 64u) {        /* the wide tile has more threads than token blocks */
+            const uint32_t t = s_row;
             uint32_t q[8];
-            const uint32_t d = q80_unpack(a_raw[i], q);
-            put(st, a_dst[i], q, live);
+            const uint32_t d = q80_unpack(a_raw, q);
+            put(st, a_dst, q);
             const uint32_t at = ((s_blk >> 2) * G::TOK + t) * 4u + (s_blk & 3u);
-            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DQ_OFF)[t * G::KB + s_blk] = live ? (uint16_t)d : (uint16_t)0u;
+            if (!HAS_M) reinterpret_cast<uint16_t *>(st + G::DQ_OFF)[tid] = live ? (uint16_t)d : (uint16_t)0u;
             if (HAS_M) {
                 reinterpret_cast<float *>(st + G::DQ_OFF)[at] = live ? half_to_float_hw(d) : 0.0f;
                 int qs = 0;
 #pragma unroll
                 for (int k = 0; k < 8; k++) qs = dot4(0x01010101u, q[k], qs);
-                reinterpret_cast<float *>(st + G::QS_OFF)[at] = live ? (float)qs : 0.0f;
+                reinterpret_cast<float *>(st + G::QS_OFF)[at] = (float)qs;
             }
         }
     };
@@ -195,7 +221,17 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     for (int rc = 0; rc < RC; rc++)
 #pragma unroll
         for (int tc = 0; tc < TC; tc++) acc[rc][tc] = (v4f){ 0.0f, 0.0f, 0.0f, 0.0f };
-    const v4i zero = { 0, 0, 0, 0 };
+    /* BIASED: the integer sums start at the bits of 1.5 * 2^23, as floats they are then that plus the sum, exactly (at most
+     * 2^19 here in either direction), and a subtraction makes the sum of it, where a conversion takes nearly twice a
+     * subtraction's time.  It costs four registers: AL5_XS 4096 x 4096 x 512 50.3 -> 47.9 us, Q4_0 46.0 -> 45.3, Q5_1 900 x
+     * 8192 x 128 73.4 -> 71.0; Q5_0 as before; Q8_0, which spills for it, 2048 x 2016 x 333 17.4 -> 18.3, and Q4_1
+     * 1000 x 2048 x 100 21.1 -> 21.4, so not those three. */
+    constexpr bool BIASED = LEG == 1 || LEG == 4 || LEG == 5;
+    v4i start = { 0, 0, 0, 0 };
+    if (BIASED) {
+        start = (v4i){ 0x4B400000, 0x4B400000, 0x4B400000, 0x4B400000 };
+        asm volatile("" : "+v"(start));         /* kept in registers, not made anew for every MFMA */
+    }
     auto block_of = [](const u32x4 &v, int j) -> long {
         return (long)(((unsigned long)v[2 * j + 1] << 32) | (unsigned long)v[2 * j]);
     };
@@ -206,10 +242,10 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
         v4h a[RC], b[TC];
 #pragma unroll
         for (int rc = 0; rc < RC; rc++)
-            a[rc] = (v4h){ *reinterpret_cast<const _Float16 *>(st + dwh_rd + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)rc), (_Float16)0, (_Float16)0, (_Float16)0 };
+            a[rc] = half_first(st + dwh_rd + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)rc);
 #pragma unroll
         for (int tc = 0; tc < TC; tc++)
-            b[tc] = (v4h){ *reinterpret_cast<const _Float16 *>(st + dq_rd + 2u * kq + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)tc), (_Float16)0, (_Float16)0, (_Float16)0 };
+            b[tc] = half_first(st + dq_rd + 2u * kq + 8u * (uint32_t)q + 16u * 2u * G::KB * (uint32_t)tc);
         const v16f none = {};
 #pragma unroll
         for (int rc = 0; rc < RC; rc++)
@@ -227,7 +263,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
 #pragma unroll
                 for (int tc = 0; tc < TC; tc++)
                     /* weights first: result i of a lane is row 4 kq + i against token r16 */
-                    isum[rc][tc] = __builtin_amdgcn_mfma_i32_16x16x32_i8(block_of(f.w[rc], j), block_of(f.a[tc], j), zero, 0, 0, 0);
+                    isum[rc][tc] = __builtin_amdgcn_mfma_i32_16x16x32_i8(block_of(f.w[rc], j), block_of(f.a[tc], j), start, 0, 0, 0);
                 if (HAS_M)
                     mw[rc] = *reinterpret_cast<const v4f *>(st + dw_rd + (G::MW_OFF - G::DW_OFF) +
                                                             ((2u * (uint32_t)p + (uint32_t)j) * G::D_PITCH + 16u * (uint32_t)rc) * 4u);
@@ -239,7 +275,8 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
                         const float t = HAS_M ? f.dw[HAS_M ? j : 0][rc][i] * dq[tc][bq] : ts[rc][tc][4 * bq + i];
-                        const float up = t * (float)isum[rc][tc][i];
+                        const float sum = BIASED ? __int_as_float(isum[rc][tc][i]) - 12582912.0f : (float)isum[rc][tc][i];
+                        const float up = t * sum;
                         if (HAS_M) {
                             const float tm = mw[rc][i] * dq[tc][bq];
                             const float off = tm * qs[tc][bq];
@@ -254,7 +291,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     const uint32_t n_steps = (B + G::KB - 1u) / G::KB;
     load(0u);
     store(0u);
-    load(1u < n_steps ? 1u : 0u);
+    load(1u);
     __syncthreads();
     for (uint32_t s = 0; s < n_steps; s++) {
         const uint8_t *st = mmq_lds + (s & 1u) * G::STAGE_BYTES;
@@ -280,7 +317,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
             }
             if (q == 0 && s + 1u < n_steps) {
                 store(s + 1u);
-                load(min(s + 2u, n_steps - 1u));
+                load(s + 2u);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
