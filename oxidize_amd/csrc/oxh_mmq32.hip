@@ -21,7 +21,7 @@
  * barrier per step; the next step's blocks go to LDS in the middle of a step and the ones after it are requested
  * then.  Of the Q8_0 tile's 92 % vector issue by counter, a third was not the float step: 64-bit addresses formed anew for
  * every block, the place within four bytes asked again, values cleared past the row's end.  With a wave's address in
- * scalar registers and 32-bit offsets stepped along, 279 of 317 instructions are left (quantiser and
+ * scalar registers and 32-bit offsets stepped along, 269 of 317 instructions are left (quantiser and
  * matmul, us: Q8_0 4096 x 4096 x 512 48.4 -> 45.3, 14336 x 4096 x 256 81.1 -> 75.5, Q4_0 81.7 -> 74.5, Q5_0 86.0 -> 79.4,
  * AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113; Q5_1 alone on its CUs, 900 x 8192 x 128, 69.6 -> 71.0).  128 x 64 tiles whose waves kept raw blocks in regions of their own, one
  * workgroup to a CU, took 69 us where this took 41, eight waves of 32 x 32 42.5. */
@@ -63,7 +63,9 @@ __device__ __forceinline__ uint32_t mmq32_swizzle(uint32_t row) { return ((row >
 /* a half and three zeros: an operand of one K */
 __device__ __forceinline__ v4h half_first(const uint8_t *p)
 {
-    return __builtin_bit_cast(v4h, make_uint2(*reinterpret_cast<const uint16_t *>(p), 0u));
+    uint32_t h = *reinterpret_cast<const uint16_t *>(p);
+    asm("" : "+v"(h));          /* the load has cleared the upper half; seen as halves it would be cleared once more */
+    return __builtin_bit_cast(v4h, make_uint2(h, 0u));
 }
 
 template <int LEG> struct Mmq32Raw { LegRegs r; };
