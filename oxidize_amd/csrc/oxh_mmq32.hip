@@ -23,8 +23,8 @@
  * every block, the place within four bytes asked again, values cleared past the row's end.  With a wave's address in
  * scalar registers and 32-bit offsets stepped along, 269 of 317 instructions are left (quantiser and
  * matmul, us: Q8_0 4096 x 4096 x 512 48.4 -> 45.3, 14336 x 4096 x 256 81.1 -> 75.5, Q4_0 81.7 -> 74.5, Q5_0 86.0 -> 79.4,
- * AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113; Q5_1 alone on its CUs, 900 x 8192 x 128, 69.6 -> 71.0).  128 x 64 tiles whose waves kept raw blocks in regions of their own, one
- * workgroup to a CU, took 69 us where this took 41, eight waves of 32 x 32 42.5. */
+ * AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113).  128 x 64 tiles whose waves kept raw blocks in regions of their
+ * own, one workgroup to a CU, took 69 us where this took 41, eight waves of 32 x 32 42.5. */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -226,8 +226,8 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     /* BIASED: the integer sums start at the bits of 1.5 * 2^23, as floats they are then that plus the sum, exactly (at most
      * 2^19 here in either direction), and a subtraction makes the sum of it, where a conversion takes nearly twice a
      * subtraction's time.  It costs four registers: AL5_XS 4096 x 4096 x 512 50.3 -> 47.9 us, Q4_0 46.0 -> 45.3, Q5_1 900 x
-     * 8192 x 128 73.4 -> 71.0; Q5_0 as before; Q8_0, which spills for it, 2048 x 2016 x 333 17.4 -> 18.3, and Q4_1
-     * 1000 x 2048 x 100 21.1 -> 21.4, so not those three. */
+     * 8192 x 128 73.4 -> 71.0; Q5_0 as before; Q8_0 2048 x 2016 x 333 17.4 -> 18.3 and Q4_1 1000 x 2048 x 100 21.1 -> 21.4,
+     * so not those three (all with a scheduling barrier between the pairs of a step, as it was then). */
     constexpr bool BIASED = LEG == 1 || LEG == 4 || LEG == 5;
     v4i start = { 0, 0, 0, 0 };
     if (BIASED) {
@@ -310,8 +310,10 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
                     if (HAS_M) dq[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
                     if (HAS_M) qs[tc] = *reinterpret_cast<const v4f *>(st + dq_rd + (G::QS_OFF - G::DQ_OFF) + (uint32_t)q * G::TOK * 16u + 256u * (uint32_t)tc);
                 }
+                /* (The compiler may mix this pair's reads with its sums.  Kept apart by a scheduling barrier, Q5_1 spilled three
+                 * registers and Q4_1 and Q5_1 were slower, us: 900 x 8192 x 128 71.1 / 64.6 and 70.2 / 66.2, 4096 x 4096 x 512
+                 * 62.9 / 61.2 and 65.8 / 63.3; the others within 1 %.) */
                 const Frag nxt = fetch(st, 2 * q + 1);
-                __builtin_amdgcn_sched_barrier(0);
                 compute(cur, st, dq, qs, ts, 2 * q);
                 if (q + 1 < KP / 2) cur = fetch(st, 2 * q + 2);
                 __builtin_amdgcn_sched_barrier(0);

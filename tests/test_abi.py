@@ -354,6 +354,26 @@ def test_prompts_of_the_32_value_formats_take_the_wide_tile_where_one_round_of_i
         assert mv.mmq_kernel(7, rows, 4096, n_vec) == (mv.MMQ_TILES,) + tile + (0,), (rows, n_vec)
 
 
+def test_the_prompt_tiles_of_the_32_value_formats_keep_everything_in_registers(tmp_path):
+    """No k_mmq_32 has scratch memory: what the compiler notes beside each kernel of the built library."""
+    import shutil
+    import subprocess
+    tools = "/opt/rocm/llvm/bin"
+    shutil.copy(_lib.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([tools + "/llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    scratch = {}
+    for obj in tmp_path.glob("*gfx950"):
+        name = None
+        for line in subprocess.run([tools + "/llvm-readelf", "--notes", str(obj)], check=True, capture_output=True,
+                                   text=True).stdout.splitlines():
+            if ".name:" in line and "_Z" in line:
+                name = line.split()[-1]
+            elif ".private_segment_fixed_size:" in line and name:
+                scratch[name] = int(line.split()[-1])
+    tiles = {n: v for n, v in scratch.items() if "k_mmq_32" in n}
+    assert len(tiles) == 12 and not any(tiles.values()), tiles
+
+
 def test_expert_launches_go_to_the_tile_that_measured_fastest():
     """Expert launches on 256 compute units: Q5_K and Q6_K keep the 64 x 16 tiles up to more tokens per expert than Q4_K
     while those are many, and leave them earlier where there are two or three to a unit."""
