@@ -78,6 +78,13 @@ typedef struct OxhLab {
     /* Whether the operations of a chained plan hand their results over by
      * value (1) or wait for whole operations (0). */
     int (*plan_by_value)(const OxhPlan *plan);
+    /* Prompts of the 32-value formats: the byte, counted from the start of
+     * its wave's first row, at which the thread that stages block `blk` (0..7)
+     * of row `row` (0..7) of the wave fetches step `step` of rows of `blocks`
+     * blocks, with the kernel's own 32-bit arithmetic.  The thread's block is
+     * number 8 * step + blk; past the row's end it is the one eight before,
+     * in rows of fewer than eight the last. */
+    uint64_t (*mmq32_fetched)(uint32_t block_bytes, uint32_t blocks, uint32_t row, uint32_t blk, uint32_t step);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

@@ -61,7 +61,8 @@ class OxhLab(ctypes.Structure):
                 ("experts_tile", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, ctypes.POINTER(U32 * 2))),
                 ("host_ring_chunks", ctypes.CFUNCTYPE(Z)),
                 ("experts_batch", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, Z, Z)),
-                ("plan_by_value", ctypes.CFUNCTYPE(I, V))]
+                ("plan_by_value", ctypes.CFUNCTYPE(I, V)),
+                ("mmq32_fetched", ctypes.CFUNCTYPE(ctypes.c_uint64, U32, U32, U32, U32, U32))]
 
 
 # name -> (restype, argtypes); every symbol include/oxhip.h and include/oxhip_lab.h declare

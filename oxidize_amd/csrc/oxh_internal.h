@@ -59,6 +59,7 @@ size_t oxh_internal_mmq6_tok_tiles(size_t rows, size_t n_vec, size_t cus);
 /* The 32-value formats under a batch, in tiles of 64 or 128 rows x 64 tokens (oxh_mmq32.hip); init and launch return a
  * hipError_t.  leg: 0 Q8_0, 1 Q4_0, 2 Q4_1, 3 Q5_0, 4 Q5_1, 5 AL5_XS; `fits`: whether the grid holds the launch's tiles,
  * `tile`: their rows and tokens.  Arguments checked by the caller. */
+#define OXH_MMQ32_MAX_BLOCKS 0xFFFFFFu       /* blocks of a row: 536 870 880 columns */
 int oxh_internal_mmq32_init(void);
 int oxh_internal_mmq32_fits(size_t rows, size_t n_vec);
 void oxh_internal_mmq32_tile(size_t rows, size_t n_vec, size_t cus, uint32_t tile[2]);
@@ -104,6 +105,7 @@ int oxh_debug_mmq_kernel(uint32_t qtype, size_t rows, size_t cols, size_t n_vec,
 int oxh_debug_experts_batch(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t cols, size_t top_k, size_t n_tok,
                             size_t n_cu);
 int oxh_debug_experts_tile(uint32_t qtype, size_t n_mat, size_t n_expert, size_t rows, size_t pairs, size_t n_cu, uint32_t tile[2]);
+uint64_t oxh_debug_mmq32_fetched(uint32_t block_bytes, uint32_t blocks, uint32_t row, uint32_t blk, uint32_t step);
 int oxh_debug_subblock_sums(uint32_t qtype, const void *d_w, size_t rows, size_t cols, const void *d_act,
                             int32_t *d_sums, void *stream);
 

@@ -2538,7 +2538,7 @@ static int mmq_run(uint32_t qtype, const void *d_w, size_t rows, size_t cols, co
         /* 32-value blocks against Q8_0 activations: exact f32 step only */
         if (out_stride < rows) return arg_fail("oxh_mmq: out_stride < rows");
         const size_t blocks32 = cols / OXH_QK8_0;
-        if (rows > 0x7FFFFFFFull || n_vec > 0x7FFFFFFFull || blocks32 > 0xFFFFFFull)
+        if (rows > 0x7FFFFFFFull || n_vec > 0x7FFFFFFFull || blocks32 > OXH_MMQ32_MAX_BLOCKS)
             return arg_fail("oxh_mmq: dimension too large");
         if (blocks32 * block_bytes(qtype) < 16u) {      /* a single AL5_XS block: the tiles would take it, the interface does not */
             snprintf(g_err, sizeof g_err, "oxh_mmq: rows of qtype %u with cols %zu are shorter than 16 bytes", qtype, cols);
@@ -3444,7 +3444,7 @@ extern "C" const OxhLab *oxh_lab(void)
     static const OxhLab lab = { oxh_debug_plan_stamps, oxh_debug_plan_phantom, oxh_debug_moe_workspace_parts,
                                 oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums,
                                 oxh_debug_mmq_kernel, oxh_debug_experts_tile, oxh_debug_host_ring_chunks, oxh_debug_experts_batch,
-                                oxh_debug_plan_by_value };
+                                oxh_debug_plan_by_value, oxh_debug_mmq32_fetched };
     return &lab;
 }
 

@@ -68,6 +68,36 @@ __device__ __forceinline__ v4h half_first(const uint8_t *p)
     return __builtin_bit_cast(v4h, make_uint2(h, 0u));
 }
 
+/* Where a lane's blocks lie: block `blk` of every step of eight, in row `row` of its wave's eight, as a 32-bit offset
+ * (`first`) from the wave's base, which starts `lead` bytes below the wave's first row and moves on by a step at a time.  In
+ * a last step that the row's end cuts short, lanes past the end stay on their block of the step before (`back`), in an
+ * only step on the row's last one; `lead` leaves room for that and for an edge two bytes before a block.  So an offset
+ * spans seven rows and two steps, which is below 2^32 in the longest rows oxh_mmq takes. */
+struct Mmq32Walk {
+    static constexpr uint32_t KB = 8u;
+    static __host__ __device__ constexpr uint32_t lead(uint32_t bb) { return KB * bb + 2u; }
+    static __host__ __device__ __forceinline__ uint32_t first(uint32_t row, uint32_t blk, uint32_t B, uint32_t bb)
+    {
+        return lead(bb) + (row * B + (blk < B ? blk : B - 1u)) * bb;
+    }
+    static __host__ __device__ __forceinline__ uint32_t back(uint32_t step, uint32_t blk, uint32_t B, uint32_t bb)
+    {
+        return step * KB + blk < B ? 0u : KB * bb;
+    }
+    static constexpr uint64_t reach(uint64_t B, uint32_t bb) { return lead(bb) + (7u * B + 2u * KB) * bb; }
+};
+static_assert(Mmq32Walk::reach(OXH_MMQ32_MAX_BLOCKS, 34u) <= 0xFFFFFFFFull, "a lane's offsets");
+
+/* the byte of its wave's first row at which lane (row, blk) fetches its block of step `step` */
+extern "C" uint64_t oxh_debug_mmq32_fetched(uint32_t block_bytes, uint32_t blocks, uint32_t row, uint32_t blk, uint32_t step)
+{
+    const uint32_t n_steps = (blocks + Mmq32Walk::KB - 1u) / Mmq32Walk::KB;
+    const uint64_t base = (uint64_t)step * (Mmq32Walk::KB * block_bytes) - Mmq32Walk::lead(block_bytes);
+    uint32_t off = Mmq32Walk::first(row, blk, blocks, block_bytes);
+    if (step != 0u && step + 1u == n_steps) off -= Mmq32Walk::back(step, blk, blocks, block_bytes);
+    return base + off;
+}
+
 template <int LEG> struct Mmq32Raw { LegRegs r; };
 template <> struct Mmq32Raw<0> { Q80Regs r; };
 
@@ -99,17 +129,16 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
         w_dst = (s_blk >> 1) * G::W_PAIR + s_row * 64u + 16u * (mmq32_swizzle(s_row) ^ k) + 8u * (s_blk & 1u);      /* ^ 16 k */
         a_dst = G::A_OFF + (s_blk >> 1) * G::A_PAIR + s_row * 64u + 16u * (mmq32_swizzle(s_row) ^ k) + 8u * (s_blk & 1u);
     }
-    /* A wave stages eight rows (tokens): the first one's address is the wave's, less two bytes since an edge dword may
-     * begin there, a lane's block is a 32-bit offset from it (mmq32_launch sees to it), and so is its edge.  A thread's
-     * blocks are a step's eight apart, which is a multiple of four bytes in every format: their place within four
-     * is asked once.  Past the row's end a thread stays on its last block. */
-    static_assert(G::KB * G::BB % 4u == 0u && G::KB * 34u % 4u == 0u, "blocks of a thread");
-    const uint32_t wave_row = wave * (64u / G::KB), b_first = min(s_blk, B - 1u);
+    /* A wave stages eight rows (tokens).  Its base, in scalar registers, starts at the first one's address and goes a step
+     * on at a time; a lane's block is a 32-bit offset from it, and so is its edge (Mmq32Walk).  Steps are a multiple of four
+     * bytes in every format: a block's place within four is asked once. */
+    static_assert(G::KB == Mmq32Walk::KB && G::KB * G::BB % 4u == 0u && G::KB * 34u % 4u == 0u, "blocks of a thread");
+    const uint32_t wave_row = wave * (64u / G::KB);
     const uint32_t w_row0 = min(wave_row, rows_here - 1u), a_row0 = min(wave_row, toks_here - 1u);
-    const uint8_t *const w_base = w + (size_t)(row_first + w_row0) * B * G::BB - 2;
-    const uint8_t *const a_base = acts + (size_t)(tok_first + a_row0) * B * 34u - 2;
-    uint32_t w_off = 2u + ((min(s_row, rows_here - 1u) - w_row0) * B + b_first) * G::BB;
-    uint32_t a_off = 2u + ((min(s_row, toks_here - 1u) - a_row0) * B + b_first) * 34u;
+    const uint8_t *w_base = w + (size_t)(row_first + w_row0) * B * G::BB - Mmq32Walk::lead(G::BB);
+    const uint8_t *a_base = acts + (size_t)(tok_first + a_row0) * B * 34u - Mmq32Walk::lead(34u);
+    uint32_t w_off = Mmq32Walk::first(min(s_row, rows_here - 1u) - w_row0, s_blk, B, G::BB);
+    uint32_t a_off = Mmq32Walk::first(min(s_row, toks_here - 1u) - a_row0, s_blk, B, 34u);
     const uint32_t w_odd = block_odd(w_base + w_off), a_odd = block_odd(a_base + a_off);
     Mmq32Raw<LEG> w_raw;
     Q80Regs a_raw;
@@ -120,12 +149,23 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
     a_raw.shift = a_odd ? 0u : 16u;
     if constexpr (LEG == 0) w_raw.r.shift = w_odd ? 0u : 16u;
     else if (W_EDGE) w_raw.r.qh = w_odd ? 0u : 16u;
-    /* fetches step `step`, the steps in turn from 0 */
-    auto load = [&](uint32_t step) {
-        const bool on = step != 0u && step * G::KB + s_blk < B;
-        const uint32_t w_on = on ? G::KB * G::BB : 0u, a_on = on ? G::KB * 34u : 0u;
-        w_off += w_on;
-        if (W_EDGE) w_edge += w_on;
+    /* on to step `step`, the steps in turn from 1; past the last it stays there */
+    const uint32_t n_steps = (B + G::KB - 1u) / G::KB;
+    uint32_t w_step = n_steps > 1u ? G::KB * G::BB : 0u, a_step = n_steps > 1u ? G::KB * 34u : 0u;
+    auto advance = [&](uint32_t step) {
+        w_base += w_step;
+        a_base += a_step;
+        if (__builtin_expect(step + 1u == n_steps, 0)) {
+            asm volatile("");           /* once in a launch: a branch, and not selects in every step */
+            const uint32_t w_back = Mmq32Walk::back(step, s_blk, B, G::BB), a_back = Mmq32Walk::back(step, s_blk, B, 34u);
+            w_off -= w_back;
+            w_edge -= w_back;
+            a_off -= a_back;
+            a_edge -= a_back;
+            w_step = a_step = 0u;
+        }
+    };
+    auto load = [&]() {
         if constexpr (LEG == 0) {
             w_raw.r.w0 = *reinterpret_cast<const U32x4a4g *>(w_base + w_off);
             w_raw.r.w1 = *reinterpret_cast<const U32x4a4g *>(w_base + w_off + 16);
@@ -136,8 +176,6 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
         } else {
             leg_load_at<LEG>(w_raw.r, w_base + w_off, w_odd);
         }
-        a_off += a_on;
-        a_edge += a_on;
         a_raw.w0 = *reinterpret_cast<const U32x4a4g *>(a_base + a_off);
         a_raw.w1 = *reinterpret_cast<const U32x4a4g *>(a_base + a_off + 16);
         a_raw.edge = reinterpret_cast<const U32u2 *>(a_base + a_edge)->v;
@@ -290,14 +328,15 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
         }
     };
 
-    const uint32_t n_steps = (B + G::KB - 1u) / G::KB;
-    load(0u);
+    load();
     store(0u);
-    load(1u);
+    advance(1u);
+    load();
     __syncthreads();
     for (uint32_t s = 0; s < n_steps; s++) {
         const uint8_t *st = mmq_lds + (s & 1u) * G::STAGE_BYTES;
         const uint32_t nb = min(B - s * G::KB, G::KB);
+        advance(s + 2u);
         Frag cur = fetch(st, 0);
 #pragma unroll
         for (int q = 0; q < KP / 2; q++) {
@@ -321,7 +360,7 @@ k_mmq_32(const uint8_t *__restrict__ w, uint32_t rows, uint32_t B, const uint8_t
             }
             if (q == 0 && s + 1u < n_steps) {
                 store(s + 1u);
-                load(s + 2u);
+                load();
                 __builtin_amdgcn_sched_barrier(0);
             }
         }

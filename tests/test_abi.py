@@ -374,6 +374,22 @@ def test_the_prompt_tiles_of_the_32_value_formats_keep_everything_in_registers(t
     assert len(tiles) == 12 and not any(tiles.values()), tiles
 
 
+@pytest.mark.parametrize("block_bytes", [14, 18, 20, 22, 24, 34])
+def test_prompts_of_the_32_value_formats_find_every_block_of_the_longest_rows(block_bytes):
+    """A lane's place in its wave's eight rows is a 32-bit offset: eight rows of 34-byte blocks pass 2^32 bytes from
+    15 790 321 blocks on, and oxh_mmq takes 0xFFFFFF.  Also the shortest rows and those that end within a step."""
+    at = _lib.lab().mmq32_fetched
+    for blocks in (1, 7, 8, 9, 63, 64, 15790320, 15790321, 0xFFFFF7, 0xFFFFFF):
+        last = (blocks - 1) // 8
+        for step in sorted({0, min(1, last), last // 2, max(last - 1, 0), last}):
+            for row in range(8):
+                for blk in range(8):
+                    b = 8 * step + blk
+                    if b >= blocks:
+                        b = b - 8 if step else blocks - 1
+                    assert at(block_bytes, blocks, row, blk, step) == (row * blocks + b) * block_bytes, (blocks, row, blk, step)
+
+
 def test_expert_launches_go_to_the_tile_that_measured_fastest():
     """Expert launches on 256 compute units: Q5_K and Q6_K keep the 64 x 16 tiles up to more tokens per expert than Q4_K
     while those are many, and leave them earlier where there are two or three to a unit."""

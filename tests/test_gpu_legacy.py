@@ -258,3 +258,19 @@ def test_prompt_scales_of_every_size(oxh, qtype, n_vec):
         assert np.array_equal(np.isnan(got[v]), np.isnan(want)), (qtype, v)
         fine = ~np.isnan(want)
         assert fine.sum() >= rows - 3 and np.array_equal(got[v][fine].view(np.uint32), want[fine].view(np.uint32)), (qtype, v)
+
+
+@pytest.mark.parametrize("blocks", [1, 2, 7, 8, 9, 15, 16, 17, 24, 31])
+@pytest.mark.parametrize("qtype", [7, 3, 4, 5, 6, 18])
+def test_prompt_rows_that_end_within_a_step(oxh, qtype, blocks):
+    """Steps are of eight blocks; a thread whose block lies past the row's end stays on one within it."""
+    rows, cols, n_vec = 67, 32 * blocks, 66
+    rb = synth.row_bytes(qtype, cols)
+    w = synth.weights(qtype, rows, cols, seed=blocks)
+    xs = synth.normal(n_vec * cols, seed=blocks, stream=5).reshape(n_vec, cols)
+    got, temp = np.zeros((n_vec, rows), np.float32), np.zeros(cols, np.float32)
+    scratch = np.zeros(mv.batch_scratch_bytes(cols), np.uint8)
+    assert mv.matvec_quantized_batch(qtype, w, rows, cols, rb, xs, cols, got, rows, n_vec, temp, scratch) == 0
+    for v in range(n_vec):
+        want, _ = oracle_matvec(qtype, w, rows, cols, np.ascontiguousarray(xs[v]))
+        assert np.array_equal(bits(got[v]), bits(want)), (qtype, blocks, v)
