@@ -25,7 +25,10 @@
  *     other and a fence that makes them so costs 35 us here, so there are no
  *     fences: everything one operation hands to another (outputs, residual
  *     sums) is stored and loaded with system-coherent accesses that bypass the
- *     L2s, and so are the counters.
+ *     L2s, and so are the counters.  The quantised bytes an operation stores
+ *     go past the L2s as well: a later operation may store at the same place
+ *     from another XCD, and of two dirty lines either could be written back
+ *     last.
  *   - A plan none of whose operations reads what another one writes (a decode
  *     step's matrices applied to inputs that are all there when the launch
  *     starts) runs on a second kernel, k_plan_ext: each input vector is
@@ -726,13 +729,13 @@ plan_stage_finish(const OpHead &op, const SideSlots &slots, const XStage &xs, ui
                     reinterpret_cast<int16_t *>(base + B * 256u)[(blk * 4u + j) * 2u + (l >> 3)] = (int16_t)bj;
             }
             if (dst) {
-                reinterpret_cast<uint32_t *>(dst + 4)[16u * j + l] = pk;
-                if ((l & 3u) == 0u) reinterpret_cast<int16_t *>(dst + 260)[g] = (int16_t)s16;
+                store_past<true>(reinterpret_cast<uint32_t *>(dst + 4) + 16u * j + l, pk);
+                if ((l & 3u) == 0u) store_past<true>(reinterpret_cast<int16_t *>(dst + 260) + g, (int16_t)s16);
             }
         }
         if (l == 0u) {
             reinterpret_cast<float *>(base + B * 256u + B * (Q6 ? 64u : 16u))[blk] = d;
-            if (dst) *reinterpret_cast<float *>(dst) = d;
+            if (dst) store_past<true>(reinterpret_cast<float *>(dst), d);
         }
     }
     /* the side outputs are acknowledged where the trip that follows the passes begins (k_plan), or after
@@ -808,7 +811,7 @@ plan_stage_finish_unit(const OpHead &op, const SideSlots &slots, const XUnit &xu
         if (slots.row == nullptr && pro != GEMV_PRO_NONE && storer && op.pro_out != 0u) cstore4(coh_buf(gptr<float>(op.pro_out)), at, y);
         if (slots.row != nullptr && pro != GEMV_PRO_NONE && storer) slots.store4(slots.row->reserved, slots.row->pro_out, at, y);
         const gaddr act_out = !storer ? 0u : slots.row != nullptr ? slots.row->act_out : op.act_out;
-        q8k_x_finish<KIND == 1>(y, B, wave, base, act_out ? gptr<uint8_t>(act_out) : nullptr, lane);
+        q8k_x_finish<KIND == 1, true>(y, B, wave, base, act_out ? gptr<uint8_t>(act_out) : nullptr, lane);
     }
 }
 
@@ -1024,9 +1027,9 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
         }
         plan_stamp<STAMPS>(sy, i, 1, ln, wave);
 
-        /* a prologue's side outputs: every workgroup has them, and wave w of the w-th workgroup from the end stores its
-         * part (one workgroup storing all of it was late with its rows, and everybody else late with it: 32-layer
-         * chain 1.221 against 1.210 ms, six layers of 4096 x 8192 188 against 182 us) */
+        /* The side outputs (a prologue's, and the quantised bytes): every workgroup has them, and wave w of the w-th
+         * workgroup from the end stores its part (one workgroup storing all of it was late with its rows, and everybody
+         * else late with it: 32-layer chain 1.221 against 1.210 ms, six layers of 4096 x 8192 188 against 182 us) */
         const bool storer = blockIdx.x + 1u + wave == gridDim.x || (gridDim.x <= wave && blockIdx.x == 0u);
         const SideSlots slots = { BY_VALUE ? &tab[i] : nullptr, par, sy.set_bytes };
         const uint32_t Bk = op.blocks;

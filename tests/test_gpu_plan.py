@@ -300,6 +300,46 @@ def test_an_input_made_of_two_results_waits_for_the_whole_operation(oxh):
     plan.destroy()
 
 
+def launch_one_by_one(ops):
+    for op in ops:
+        if op.get("kind"):
+            mv.gemv_segments_fused(op["qtype"], op["segs"], op["cols"], op["d_x"], op["cols"], op["kind"], op["d_b"],
+                                   op.get("eps", 0.0), op.get("d_pro_out"), op.get("d_act_out"), 1, 0, None,
+                                   d_add=op.get("d_add"), d_sum_out=op.get("d_sum_out"))
+        else:
+            mv.gemv_segments_f32(op["qtype"], op["segs"], op["cols"], op["d_x"], op["cols"], op.get("d_act_out"))
+    mv.sync()
+
+
+@pytest.mark.parametrize("apart,by_value", [(1, 0), (3, 1), (3, 0)])
+@pytest.mark.parametrize("first", [4096, 4352])
+def test_operations_that_share_the_place_of_their_quantised_bytes(oxh, monkeypatch, first, apart, by_value):
+    """A block of a vector of up to sixteen is stored by another workgroup than the same block of a longer one: the later
+    operation's bytes have to be what stays, next to each other (which by value is turned down) and a few apart."""
+    lens = [first if i % (2 * apart) < apart else 8448 - first for i in range(8)]
+    lens = [n if i % apart == 0 else 4096 for i, n in enumerate(lens)] + [4096]
+    bufs = [mv.DeviceBuffer(n * 4) for n in lens]
+    act = mv.DeviceBuffer(17 * 292)
+    ws = [mv.DeviceBuffer.from_host(synth.weights(Q4K, lens[i + 1], lens[i], seed=31, stream=i)) for i in range(8)]
+    ops = [dict(qtype=Q4K, segs=mv.make_segments([(ws[i].ptr, bufs[i + 1].ptr, lens[i + 1], 0)]), cols=lens[i], d_x=bufs[i].ptr,
+                d_act_out=act.ptr if i % apart == 0 else None) for i in range(8)]
+    if not by_value:
+        monkeypatch.setenv("OXH_PLAN_BY_VALUE", "0")
+    plan = mv.Plan(ops)
+    assert _lib.lab().plan_by_value(plan.handle) == by_value
+    for rep in range(3):
+        bufs[0].upload(synth.normal(lens[0], seed=rep, stream=90))
+        act.upload(np.zeros(17 * 292, np.uint8))
+        launch_one_by_one(ops)
+        want = act.download(np.uint8, 17 * 292), bufs[8].download(np.float32, lens[8])
+        act.upload(np.zeros(17 * 292, np.uint8))
+        plan.launch()
+        assert plan.status() == 0
+        assert np.array_equal(act.download(np.uint8, 17 * 292), want[0]), rep
+        assert np.array_equal(bits(bufs[8].download(np.float32, lens[8])), bits(want[1])), rep
+    plan.destroy()
+
+
 def test_a_wait_that_cannot_be_satisfied_gives_up(oxh):
     """The waits expect one workgroup more than exist and may poll 300 times: every workgroup must leave,
     the launch must end, the status must say so, and the plan must work again afterwards."""
