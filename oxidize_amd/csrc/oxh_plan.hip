@@ -539,11 +539,13 @@ __device__ __forceinline__ gaddr slot_at(gaddr a, uint32_t par, uint32_t set_byt
 
 /* where a prologue's side outputs are handed over by value: the operation's row of the table (NULL: they are not),
  * this launch's set of slots and the other one, which is emptied for the next launch */
-struct SideSlots {
+template <bool WORDS> struct SideSlots {
     const PlanOp *row;
     uint32_t par, set_bytes;
-    /* (addresses in vector registers, two words a store: few waves store these, and scalar registers are what every
-     * workgroup is short of) */
+    /* (addresses in vector registers: few waves store these, and scalar registers are what every workgroup is short of.
+     * Slots lie on multiples of 256 and take two words a store.  The caller's vector lies on any multiple of four: a buffer
+     * store, or in the kernel that has Q5_K, which keeps more scalars in vector lanes for its descriptor, four of a word:
+     * chains with / without Q5_K, 16 layers of 1024 x 2560, four words 335.5 / 302, a buffer store 338.2 / 298 us) */
     static __device__ __forceinline__ void two(gaddr to, uint32_t a, uint32_t b)
     {
         __hip_atomic_store(gptr<uint64_t>(to), (uint64_t)a | ((uint64_t)b << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -558,8 +560,13 @@ struct SideSlots {
             two(other + 8u, SLOT_EMPTY, SLOT_EMPTY);
         }
         if (out != 0u) {
-            two(out + byte_off, __float_as_uint(y.v0), __float_as_uint(y.v1));
-            two(out + byte_off + 8u, __float_as_uint(y.v2), __float_as_uint(y.v3));
+            if (WORDS) {
+                const float v[4] = { y.v0, y.v1, y.v2, y.v3 };
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; k++) cstore(gptr<uint32_t>(out + byte_off + 4u * k), __float_as_uint(v[k]));
+            } else {
+                cstore4(coh_buf(gptr<float>(uni(out))), byte_off, y);
+            }
         }
     }
 };
@@ -631,9 +638,9 @@ __device__ __forceinline__ int quantize_sum4(const XRegs &y, float inv, uint32_t
     return q0 + q1 + q2 + q3;
 }
 
-template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */>
+template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */, bool WORDS>
 __device__ __forceinline__ void
-plan_stage_finish(const OpHead &op, const SideSlots &slots, const XStage &xs, uint8_t *base, float *red,
+plan_stage_finish(const OpHead &op, const SideSlots<WORDS> &slots, const XStage &xs, uint8_t *base, float *red,
                   bool storer, uint32_t lane, uint32_t wave)
 {
     constexpr bool Q6 = KIND == 1;
@@ -782,9 +789,9 @@ plan_stage_issue_unit(const PlanSync &sy, const OpHead &op, XUnit &xu, uint32_t 
     return ok;
 }
 
-template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */>
+template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */, bool WORDS>
 __device__ __forceinline__ void
-plan_stage_finish_unit(const OpHead &op, const SideSlots &slots, const XUnit &xu, uint8_t *base, float *red, bool storer,
+plan_stage_finish_unit(const OpHead &op, const SideSlots<WORDS> &slots, const XUnit &xu, uint8_t *base, float *red, bool storer,
                        uint32_t lane, uint32_t wave)
 {
     const uint32_t B = op.blocks, pro = op.pro;
@@ -1031,7 +1038,7 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
          * workgroup from the end stores its part (one workgroup storing all of it was late with its rows, and everybody
          * else late with it: 32-layer chain 1.221 against 1.210 ms, six layers of 4096 x 8192 188 against 182 us) */
         const bool storer = blockIdx.x + 1u + wave == gridDim.x || (gridDim.x <= wave && blockIdx.x == 0u);
-        const SideSlots slots = { BY_VALUE ? &tab[i] : nullptr, par, sy.set_bytes };
+        const SideSlots<HAS_Q5> slots = { BY_VALUE ? &tab[i] : nullptr, par, sy.set_bytes };
         const uint32_t Bk = op.blocks;
         if (STAMPS && sy.stamps != nullptr) {         /* measurement only: when has the vector arrived? */
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1125,8 +1132,8 @@ k_plan_ext(const PlanOp *__restrict__ ins, uint32_t n_ins, const PlanOp *__restr
 #pragma unroll
         for (int u = 0; u < 4; u++) xs.x[u] = xs.t[u] = xs.b[u] = XRegs{ 0.f, 0.f, 0.f, 0.f };
         plan_stage_issue<false>(sy, op, xs, lane, wave);
-        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, SideSlots{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
-        else                      plan_stage_finish<0>(op, SideSlots{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
+        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
+        else                      plan_stage_finish<0>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
         __syncthreads();
         const uint32_t bytes = plan_image_bytes(op.kind, op.blocks);
         const CohBuf img = coh_buf(gptr<uint8_t>(uni(ins[j].xq)));

@@ -340,6 +340,66 @@ def test_operations_that_share_the_place_of_their_quantised_bytes(oxh, monkeypat
     plan.destroy()
 
 
+@pytest.mark.parametrize("by_value", [1, 0])
+@pytest.mark.parametrize("qt_up,qt_down", [(Q4K, Q6K), (Q5K, Q4K)])
+@pytest.mark.parametrize("a,b,off", [(1024, 1024, 4), (4096, 4352, 12), (4352, 4096, 4), (256, 2048, 0)])
+def test_a_chain_through_every_kind_of_hand_over(oxh, monkeypatch, a, b, off, qt_up, qt_down, by_value):
+    """What a decode chain does not have: SwiGLU over two results of an earlier operation, a prologue's output and its sum as
+    later inputs, a part of a result, stored quantised bytes, and every one of these stored at the same place by a second
+    round of the same operations; vectors on both sides of sixteen blocks, side outputs on and off multiples of eight and
+    sixteen bytes.  All of it the launches' bits, with other inputs before every launch."""
+    c = 768
+    sizes = dict(x0=c, g=a, u=a, h=a, y=a, s=a, n=a, z=b + 512, t=c, t2=c, t3=c, t4=c, o4=300, o5=40)
+    buf = {k: mv.DeviceBuffer(n * 4 + 16) for k, n in sizes.items()}
+    at = {k: v.ptr + off for k, v in buf.items()}
+    acts = [mv.DeviceBuffer(mv.act_bytes(Q4K, n)) for n in (a, b)]
+    norm = mv.DeviceBuffer.from_host((synth.normal(max(a, b), seed=4, stream=60) * np.float32(0.1) + np.float32(1)).astype(np.float32))
+    keep = []
+
+    def op(qt, x, cols, outs, part=0, **more):
+        w = mv.DeviceBuffer.from_host(synth.weights(qt, sum(sizes[o] for o in outs), cols, seed=4, stream=len(keep)))
+        keep.append(w)
+        items, row = [], 0
+        for o in outs:
+            items.append((w.ptr + row * synth.row_bytes(qt, cols), at[o], sizes[o], 0))
+            row += sizes[o]
+        return dict(qtype=qt, segs=mv.make_segments(items), cols=cols, d_x=at[x] + 4 * part, **more)
+
+    rms = dict(kind=mv.PRO_RMSNORM, d_b=norm.ptr, eps=1e-5)
+    ops = []
+    for x in ("x0", "t4"):
+        ops += [op(qt_up, x, c, ("g", "u")),
+                op(qt_down, "g", a, ("y",), kind=mv.PRO_SWIGLU, d_b=at["u"], d_pro_out=at["h"], d_act_out=acts[0].ptr),
+                op(qt_up, "h", a, ("z",), d_add=at["y"], d_sum_out=at["s"], d_pro_out=at["n"], **rms),
+                op(qt_up, "z", b, ("t",), part=131, d_act_out=acts[1].ptr),
+                op(qt_down, "s", a, ("o4",), **rms), op(qt_up, "n", a, ("o5",)),
+                op(qt_up, "t", c, ("t2",), **rms), op(qt_down, "t2", c, ("t3",)), op(qt_up, "t3", c, ("t4",), **rms)]
+    if not by_value:
+        monkeypatch.setenv("OXH_PLAN_BY_VALUE", "0")
+    plan = mv.Plan(ops)
+    assert _lib.lab().plan_by_value(plan.handle) == by_value
+
+    def state():
+        return ([buf[k].download(np.uint8, n * 4, off) for k, n in sizes.items()] +
+                [v.download(np.uint8, mv.act_bytes(Q4K, n)) for v, n in zip(acts, (a, b))])
+
+    for rep in range(4):
+        def clear():
+            for v in list(buf.values()) + acts:
+                mv.lib().oxh_memset(ctypes.c_void_p(v.ptr), 0xFF, v.nbytes, None)
+            buf["x0"].upload(synth.normal(c, seed=rep, stream=61), off)
+        clear()
+        launch_one_by_one(ops)
+        want = state()
+        clear()
+        plan.launch()
+        assert plan.status() == 0
+        for k, w_, g_ in zip(list(sizes) + ["act a", "act b"], want, state()):
+            assert np.array_equal(w_, g_), (rep, k)
+        assert np.isfinite(np.frombuffer(want[list(sizes).index("t4")].tobytes(), np.float32)).all()
+    plan.destroy()
+
+
 def test_a_wait_that_cannot_be_satisfied_gives_up(oxh):
     """The waits expect one workgroup more than exist and may poll 300 times: every workgroup must leave,
     the launch must end, the status must say so, and the plan must work again afterwards."""
