@@ -85,6 +85,19 @@ typedef struct OxhLab {
      * number 8 * step + blk; past the row's end it is the one eight before,
      * in rows of fewer than eight the last. */
     uint64_t (*mmq32_fetched)(uint32_t block_bytes, uint32_t blocks, uint32_t row, uint32_t blk, uint32_t step);
+    /* What oxh_plan_create would make of these operations on a device of n_cu
+     * compute units, without one: host arithmetic on the addresses given, which
+     * are not read.  out, 3 + 16 * n_ops words: whether results are handed over
+     * by value, the workgroups, the bytes of a set of slots; per operation by
+     * value: which inputs come out of slots (1 x, 2 the addend, 4 the prologue's
+     * other input), the workgroups that have rows, the first one of each of four
+     * segments, and, as offsets into a set of slots plus 4, or 0: x, the
+     * prologue's other input, the addend, the prologue's output, its sum, the
+     * segments' results; bit 0: the other set, bit 1: the sets change places
+     * from launch to launch.  (Inputs that come out of no slot: their address.)
+     * Else: 0, or 1 + the operation that has to be complete, and the first
+     * five of the rest. */
+    int (*plan_draft)(const OxhPlanOp *ops, size_t n_ops, uint32_t n_cu, uint64_t *out);
 } OxhLab;
 
 const OxhLab *oxh_lab(void);

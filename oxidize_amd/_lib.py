@@ -62,7 +62,8 @@ class OxhLab(ctypes.Structure):
                 ("host_ring_chunks", ctypes.CFUNCTYPE(Z)),
                 ("experts_batch", ctypes.CFUNCTYPE(I, U32, Z, Z, Z, Z, Z, Z, Z)),
                 ("plan_by_value", ctypes.CFUNCTYPE(I, V)),
-                ("mmq32_fetched", ctypes.CFUNCTYPE(ctypes.c_uint64, U32, U32, U32, U32, U32))]
+                ("mmq32_fetched", ctypes.CFUNCTYPE(ctypes.c_uint64, U32, U32, U32, U32, U32)),
+                ("plan_draft", ctypes.CFUNCTYPE(I, ctypes.POINTER(OxhPlanOp), Z, U32, ctypes.POINTER(ctypes.c_uint64)))]
 
 
 # name -> (restype, argtypes); every symbol include/oxhip.h and include/oxhip_lab.h declare

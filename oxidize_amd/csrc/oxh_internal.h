@@ -98,6 +98,7 @@ struct OxhMoe;
 int oxh_debug_plan_stamps(struct OxhPlan *plan, uint64_t *d_stamps);
 int oxh_debug_plan_phantom(struct OxhPlan *plan, int on);
 int oxh_debug_plan_by_value(const struct OxhPlan *plan);
+int oxh_debug_plan_draft(const struct OxhPlanOp *ops, size_t n_ops, uint32_t n_cu, uint64_t *out);
 int oxh_debug_moe_workspace_parts(const struct OxhMoe *m, size_t n_tok, size_t parts[12]);
 int oxh_debug_read_probe(const void *d_buf, size_t bytes, uint32_t *d_sink, void *stream);
 int oxh_debug_mfma_probe(int valu_per_mfma, int waves_per_simd, double *pops);

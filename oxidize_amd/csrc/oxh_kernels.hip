@@ -3444,7 +3444,7 @@ extern "C" const OxhLab *oxh_lab(void)
     static const OxhLab lab = { oxh_debug_plan_stamps, oxh_debug_plan_phantom, oxh_debug_moe_workspace_parts,
                                 oxh_debug_read_probe, oxh_debug_mfma_probe, oxh_debug_subblock_sums,
                                 oxh_debug_mmq_kernel, oxh_debug_experts_tile, oxh_debug_host_ring_chunks, oxh_debug_experts_batch,
-                                oxh_debug_plan_by_value, oxh_debug_mmq32_fetched };
+                                oxh_debug_plan_by_value, oxh_debug_mmq32_fetched, oxh_debug_plan_draft };
     return &lab;
 }
 

@@ -1658,29 +1658,38 @@ static int plan_create_multi(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out)
     return OXH_OK;
 }
 
-extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out)
-{
-    if (!out) return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_plan_create: NULL");
-    *out = nullptr;
-    int rc = oxh_init(oxh_internal_device() >= 0 ? oxh_internal_device() : 0);
-    if (rc) return rc;
-    if (!ops || n_ops == 0 || n_ops > 0xFFFFu)
-        return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_plan_create: 1..65535 operations");
-    if (oxh_internal_multi_which(ops[0].qtype) >= 0) return plan_create_multi(ops, n_ops, out);
-    const uint32_t n_cu = (uint32_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
-    uint32_t grid = n_cu > PLAN_MAX_WG ? PLAN_MAX_WG : n_cu;
+/* What a plan is to run, in host memory: its table, what each operation reads (four spans) and writes (eight), and the
+ * order between them.  Host arithmetic on the caller's addresses. */
+struct PlanDraft {
+    PlanOp *h;
+    Span *reads, *writes;
+    uint32_t grid, n_waits, max_act;
+    PlanLimits lim;
+    size_t img_bytes, set_bytes;
+    bool has_q5, by_value;
+};
 
-    PlanOp *h = (PlanOp *)calloc(n_ops, sizeof *h);
-    Span *reads = (Span *)calloc(n_ops * 4, sizeof *reads), *writes = (Span *)calloc(n_ops * 8, sizeof *writes);
+static void plan_draft_free(PlanDraft &p)
+{
+    free(p.h);
+    free(p.reads);
+    free(p.writes);
+    p.h = nullptr;
+    p.reads = p.writes = nullptr;
+}
+
+static int plan_draft(const OxhPlanOp *ops, size_t n_ops, uint32_t n_cu, PlanDraft &p)
+{
+    memset(&p, 0, sizeof p);
+    uint32_t grid = n_cu > PLAN_MAX_WG ? PLAN_MAX_WG : n_cu;
+    PlanOp *const h = p.h = (PlanOp *)calloc(n_ops, sizeof *h);
+    Span *const reads = p.reads = (Span *)calloc(n_ops * 4, sizeof *reads);
+    Span *const writes = p.writes = (Span *)calloc(n_ops * 8, sizeof *writes);
     if (!h || !reads || !writes) {
-        free(h); free(reads); free(writes);
+        plan_draft_free(p);
         return oxh_internal_errorf(OXH_ERR_NOMEM, "out of host memory building a plan");
     }
-    uint32_t max_act = 0, n_waits = 0;
-    PlanLimits lim = { 0, 0, 0 };
-    size_t img_bytes = 0;
-    bool has_q5 = false;
-    rc = OXH_OK;
+    int rc = OXH_OK;
     for (size_t i = 0; i < n_ops && !rc; i++) {
         const OxhPlanOp &o = ops[i];
         PlanOp &d = h[i];
@@ -1694,7 +1703,7 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         }
         if (!o.segs || o.n_segs == 0 || !o.d_x) { rc = oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: plan: operation %zu has no segments or no input", i); break; }
         d.kind = kind;
-        if (kind == PLAN_Q5_K) has_q5 = true;
+        if (kind == PLAN_Q5_K) p.has_q5 = true;
         d.blocks = (uint32_t)(o.cols / OXH_QK_K);
         d.magic = (uint32_t)((0x100000000ull + d.blocks - 1u) / d.blocks);
         d.term_stride = d.blocks + 1u;
@@ -1702,19 +1711,19 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         d.act_out = (gaddr)(uintptr_t)o.d_act_out;
         d.pro = GEMV_PRO_NONE;
         if (o.pro) {
-            const OxhPrologue &p = *o.pro;
-            if ((p.kind != OXH_PRO_RMSNORM && p.kind != OXH_PRO_SWIGLU) || !p.d_b ||
-                ((p.d_add || p.d_sum_out) && p.kind != OXH_PRO_RMSNORM) || (p.d_sum_out && !p.d_add) ||
-                (p.kind == OXH_PRO_RMSNORM && !(p.eps >= 0.0f))) {
+            const OxhPrologue &pr = *o.pro;
+            if ((pr.kind != OXH_PRO_RMSNORM && pr.kind != OXH_PRO_SWIGLU) || !pr.d_b ||
+                ((pr.d_add || pr.d_sum_out) && pr.kind != OXH_PRO_RMSNORM) || (pr.d_sum_out && !pr.d_add) ||
+                (pr.kind == OXH_PRO_RMSNORM && !(pr.eps >= 0.0f))) {
                 rc = oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: plan: operation %zu has a malformed prologue", i);
                 break;
             }
-            d.pro = p.kind == OXH_PRO_SWIGLU ? GEMV_PRO_SWIGLU : p.d_add ? GEMV_PRO_ADD_RMSNORM : GEMV_PRO_RMSNORM;
-            d.eps = p.eps;
-            d.pro_b = (gaddr)(uintptr_t)p.d_b;
-            d.pro_add = (gaddr)(uintptr_t)p.d_add;
-            d.pro_sum_out = (gaddr)(uintptr_t)p.d_sum_out;
-            d.pro_out = (gaddr)(uintptr_t)p.d_out;
+            d.pro = pr.kind == OXH_PRO_SWIGLU ? GEMV_PRO_SWIGLU : pr.d_add ? GEMV_PRO_ADD_RMSNORM : GEMV_PRO_RMSNORM;
+            d.eps = pr.eps;
+            d.pro_b = (gaddr)(uintptr_t)pr.d_b;
+            d.pro_add = (gaddr)(uintptr_t)pr.d_add;
+            d.pro_sum_out = (gaddr)(uintptr_t)pr.d_sum_out;
+            d.pro_out = (gaddr)(uintptr_t)pr.d_out;
         }
         /* segments with rows, at most four */
         size_t rows[PLAN_MAX_SEGS];
@@ -1740,12 +1749,12 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
         if (rc) break;
         if (ns == 0) { rc = oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: plan: operation %zu has no rows", i); break; }
         d.n_segs = ns;
-        const int drc = plan_deal_op(d, grid, lim);
+        const int drc = plan_deal_op(d, grid, p.lim);
         if (drc) { rc = oxh_internal_errorf(drc, "plan: operation %zu has more rows than %u workgroups can own", i, grid); break; }
         const uint32_t act = kind >= PLAN_Q6_K ? q8k6_lds_bytes(d.blocks) : q8k_lds_bytes(d.blocks);
-        if (act > max_act) max_act = act;
-        d.xq = (gaddr)img_bytes;                    /* offset for now; the base is added once it exists */
-        img_bytes += (act + 255u) & ~(size_t)255u;
+        if (act > p.max_act) p.max_act = act;
+        d.xq = (gaddr)p.img_bytes;                    /* offset for now; the base is added once it exists */
+        p.img_bytes += (act + 255u) & ~(size_t)255u;
 
         /* what the operation reads and writes, for the dependency scan */
         const size_t xb = o.cols * sizeof(float);
@@ -1780,20 +1789,42 @@ extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out
             if (hit) wait = (uint32_t)j + 1u;
         }
         d.wait = wait;
-        if (wait) { h[wait - 1].signal = 1; n_waits++; }
+        if (wait) { h[wait - 1].signal = 1; p.n_waits++; }
     }
     /* no more workgroups than some operation has rows for: the others would only wait along */
     uint32_t used = 1;
     for (size_t i = 0; !rc && i < n_ops; i++) used = h[i].n_wg > used ? h[i].n_wg : used;
-    if (n_waits != 0) grid = used;
+    p.grid = p.n_waits != 0 ? used : grid;
+    if (rc) {
+        plan_draft_free(p);
+        return rc;
+    }
     /* OXH_PLAN_BY_VALUE=0 keeps a chain on whole operations */
     const char *bv = getenv("OXH_PLAN_BY_VALUE");
-    size_t set_bytes = 0;
-    const bool by_value = !rc && n_waits != 0 && n_ops * sizeof(PlanOp) <= 160u * 1024u && !(bv && bv[0] == '0') &&
-                          plan_slots(h, n_ops, grid, reads, writes, &set_bytes);
-    free(reads);
-    free(writes);
-    if (rc) { free(h); return rc; }
+    p.by_value = p.n_waits != 0 && n_ops * sizeof(PlanOp) <= 160u * 1024u && !(bv && bv[0] == '0') &&
+                 plan_slots(h, n_ops, p.grid, reads, writes, &p.set_bytes);
+    return OXH_OK;
+}
+
+extern "C" int oxh_plan_create(const OxhPlanOp *ops, size_t n_ops, OxhPlan **out)
+{
+    if (!out) return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_plan_create: NULL");
+    *out = nullptr;
+    int rc = oxh_init(oxh_internal_device() >= 0 ? oxh_internal_device() : 0);
+    if (rc) return rc;
+    if (!ops || n_ops == 0 || n_ops > 0xFFFFu)
+        return oxh_internal_errorf(OXH_ERR_ARG, "invalid argument: oxh_plan_create: 1..65535 operations");
+    if (oxh_internal_multi_which(ops[0].qtype) >= 0) return plan_create_multi(ops, n_ops, out);
+    const uint32_t n_cu = (uint32_t)(oxh_internal_n_cu() > 0 ? oxh_internal_n_cu() : 256);
+    PlanDraft draft;
+    if ((rc = plan_draft(ops, n_ops, n_cu, draft))) return rc;
+    free(draft.reads);
+    free(draft.writes);
+    PlanOp *const h = draft.h;
+    const uint32_t grid = draft.grid, n_waits = draft.n_waits, max_act = draft.max_act;
+    const size_t img_bytes = draft.img_bytes, set_bytes = draft.set_bytes;
+    const bool has_q5 = draft.has_q5, by_value = draft.by_value;
+    PlanLimits lim = draft.lim;
 
     OxhPlan *pl = (OxhPlan *)calloc(1, sizeof *pl);
     if (!pl) { free(h); return oxh_internal_errorf(OXH_ERR_NOMEM, "out of host memory building a plan"); }
@@ -2028,6 +2059,35 @@ extern "C" int oxh_debug_plan_phantom(OxhPlan *pl, int on)
 extern "C" int oxh_debug_plan_by_value(const OxhPlan *pl)
 {
     return pl && pl->by_value ? 1 : 0;
+}
+
+/* see oxhip_lab.h */
+extern "C" int oxh_debug_plan_draft(const OxhPlanOp *ops, size_t n_ops, uint32_t n_cu, uint64_t *out)
+{
+    PlanDraft p;
+    const int rc = plan_draft(ops, n_ops, n_cu, p);
+    if (rc) return rc;
+    out[0] = p.by_value;
+    out[1] = p.grid;
+    out[2] = p.set_bytes;
+    for (size_t i = 0; i < n_ops; i++) {
+        const PlanOp &o = p.h[i];
+        uint64_t *const to = out + 3 + 16 * i;
+        memset(to, 0, 16 * sizeof *to);
+        to[0] = o.wait;
+        to[1] = o.n_wg;
+        for (uint32_t k = 0; k < o.n_segs; k++) to[2 + k] = o.s[k].wg_begin;
+        if (!p.by_value) continue;
+        to[0] >>= 16;
+        to[6] = o.x;
+        to[7] = o.pro_b;
+        to[8] = o.pro_add;
+        to[9] = o.reserved;
+        to[10] = o.xq;
+        for (uint32_t k = 0; k < o.n_segs; k++) to[11 + k] = o.s[k].rows_q;
+    }
+    plan_draft_free(p);
+    return OXH_OK;
 }
 
 extern "C" int oxh_debug_plan_stamps(OxhPlan *pl, uint64_t *d_stamps)

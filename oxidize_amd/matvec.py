@@ -323,6 +323,41 @@ def debug_subblock_sums(qtype, d_w, rows, cols, d_act, d_sums, stream=None):
                                         ctypes.c_void_p(d_act), ctypes.c_void_p(d_sums), stream))
 
 
+def _plan_ops(ops):
+    """The dicts `Plan` takes as an array of OxhPlanOp, and what has to outlive it."""
+    keep, arr = [], (_lib.OxhPlanOp * len(ops))()
+
+    def vp(a):
+        return None if a is None else ctypes.c_void_p(a)
+    for o, d in zip(arr, ops):
+        o.qtype = d["qtype"]
+        o.segs = ctypes.cast(d["segs"], ctypes.POINTER(OxhSegment))
+        o.n_segs = len(d["segs"])
+        o.cols = d["cols"]
+        o.d_x = d["d_x"]
+        if d.get("kind"):
+            pro = OxhPrologue(d["kind"], d.get("eps", 0.0), vp(d.get("d_b")), vp(d.get("d_pro_out")),
+                              vp(d.get("d_add")), vp(d.get("d_sum_out")))
+            keep.append(pro)
+            o.pro = ctypes.pointer(pro)
+        o.d_act_out = d.get("d_act_out")
+        o.out_stride = d.get("out_stride", 0)
+        keep.append(d["segs"])
+    return arr, keep
+
+
+def plan_draft(ops, n_cu=256):
+    """What oxh_plan_create would make of `ops` on a device of n_cu compute units (include/oxhip_lab.h); host arithmetic,
+    the addresses are not read."""
+    arr, _keep = _plan_ops(ops)
+    out = (ctypes.c_uint64 * (3 + 16 * len(ops)))()
+    check(_lib.lab().plan_draft(arr, len(ops), n_cu, out))
+    rows = [list(out[3 + 16 * i:19 + 16 * i]) for i in range(len(ops))]
+    keys = ("x", "b", "add", "pro_out", "sum_out")
+    return dict(by_value=bool(out[0]), grid=int(out[1]), set_bytes=int(out[2]),
+                ops=[dict(wait=r[0], n_wg=r[1], begin=r[2:6], slot=dict(zip(keys, r[6:11])), seg_slot=r[11:15]) for r in rows])
+
+
 class Plan:
     """A chain of decode matmuls compiled into one launch (oxh_plan_*).  `ops` is a list of dicts with the
     arguments of one gemv_segments_fused call each: qtype, segs (from make_segments), cols, d_x and
@@ -331,25 +366,7 @@ class Plan:
 
     def __init__(self, ops):
         n = len(ops)
-        self._keep = []
-        arr = (_lib.OxhPlanOp * n)()
-
-        def vp(a):
-            return None if a is None else ctypes.c_void_p(a)
-        for o, d in zip(arr, ops):
-            o.qtype = d["qtype"]
-            o.segs = ctypes.cast(d["segs"], ctypes.POINTER(OxhSegment))
-            o.n_segs = len(d["segs"])
-            o.cols = d["cols"]
-            o.d_x = d["d_x"]
-            if d.get("kind"):
-                pro = OxhPrologue(d["kind"], d.get("eps", 0.0), vp(d.get("d_b")), vp(d.get("d_pro_out")),
-                                  vp(d.get("d_add")), vp(d.get("d_sum_out")))
-                self._keep.append(pro)
-                o.pro = ctypes.pointer(pro)
-            o.d_act_out = d.get("d_act_out")
-            o.out_stride = d.get("out_stride", 0)
-            self._keep.append(d["segs"])
+        arr, self._keep = _plan_ops(ops)
         self.handle = ctypes.c_void_p()
         status = lib().oxh_plan_create(arr, n, ctypes.byref(self.handle))
         if status != OK:

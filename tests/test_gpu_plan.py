@@ -400,15 +400,20 @@ def test_a_chain_through_every_kind_of_hand_over(oxh, monkeypatch, a, b, off, qt
     plan.destroy()
 
 
-def test_a_wait_that_cannot_be_satisfied_gives_up(oxh):
+@pytest.mark.parametrize("by_value", [1, 0])
+def test_a_wait_that_cannot_be_satisfied_gives_up(oxh, monkeypatch, by_value):
     """The waits expect one workgroup more than exist and may poll 300 times: every workgroup must leave,
-    the launch must end, the status must say so, and the plan must work again afterwards."""
+    the launch must end, the status must say so, and the plan must work again afterwards; whether results are
+    handed over by value or whole operations are waited for."""
+    if not by_value:
+        monkeypatch.setenv("OXH_PLAN_BY_VALUE", "0")
     d = DecodeSet(hidden=1024, kv=256, ffn=2816, layers=2, seed=7)
     a, b = DecodeChain(d, seed=7), DecodeChain(d, seed=7)
     a.launch_step()
     mv.sync()
     want = chain_state(a)
     plan = mv.Plan(b.plan_ops())
+    assert _lib.lab().plan_by_value(plan.handle) == by_value
     plan.set_spin_limit(300, phantom_workgroup=True)
     plan.launch()
     assert plan.status() == _lib.ERR_TIMEOUT
