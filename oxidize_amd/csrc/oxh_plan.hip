@@ -638,7 +638,8 @@ __device__ __forceinline__ int quantize_sum4(const XRegs &y, float inv, uint32_t
     return q0 + q1 + q2 + q3;
 }
 
-template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */, bool WORDS>
+/* SHARED: another workgroup may store this operation's quantised bytes' place again in this launch (dependent operations) */
+template <int KIND /* 0 Q4_K/Q5_K layout, 1 Q6_K layout */, bool SHARED, bool WORDS>
 __device__ __forceinline__ void
 plan_stage_finish(const OpHead &op, const SideSlots<WORDS> &slots, const XStage &xs, uint8_t *base, float *red,
                   bool storer, uint32_t lane, uint32_t wave)
@@ -736,13 +737,13 @@ plan_stage_finish(const OpHead &op, const SideSlots<WORDS> &slots, const XStage 
                     reinterpret_cast<int16_t *>(base + B * 256u)[(blk * 4u + j) * 2u + (l >> 3)] = (int16_t)bj;
             }
             if (dst) {
-                store_past<true>(reinterpret_cast<uint32_t *>(dst + 4) + 16u * j + l, pk);
-                if ((l & 3u) == 0u) store_past<true>(reinterpret_cast<int16_t *>(dst + 260) + g, (int16_t)s16);
+                store_past<SHARED>(reinterpret_cast<uint32_t *>(dst + 4) + 16u * j + l, pk);
+                if ((l & 3u) == 0u) store_past<SHARED>(reinterpret_cast<int16_t *>(dst + 260) + g, (int16_t)s16);
             }
         }
         if (l == 0u) {
             reinterpret_cast<float *>(base + B * 256u + B * (Q6 ? 64u : 16u))[blk] = d;
-            if (dst) store_past<true>(reinterpret_cast<float *>(dst), d);
+            if (dst) store_past<SHARED>(reinterpret_cast<float *>(dst), d);
         }
     }
     /* the side outputs are acknowledged where the trip that follows the passes begins (k_plan), or after
@@ -1048,8 +1049,8 @@ k_plan(const PlanOp *__restrict__ ops, uint32_t n_ops, const PlanSync sy, const 
             if (op.kind >= PLAN_Q6_K) plan_stage_finish_unit<1>(op, slots, xu, act, red, storer, ln, wave);
             else                      plan_stage_finish_unit<0>(op, slots, xu, act, red, storer, ln, wave);
         } else {
-            if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, slots, xs, act, red, storer, ln, wave);
-            else                      plan_stage_finish<0>(op, slots, xs, act, red, storer, ln, wave);
+            if (op.kind >= PLAN_Q6_K) plan_stage_finish<1, true>(op, slots, xs, act, red, storer, ln, wave);
+            else                      plan_stage_finish<0, true>(op, slots, xs, act, red, storer, ln, wave);
         }
         plan_prefetch<HAS_Q5>(cur, B, 1u, ln);
         plan_stamp<STAMPS>(sy, i, 2, ln, wave);
@@ -1132,8 +1133,8 @@ k_plan_ext(const PlanOp *__restrict__ ins, uint32_t n_ins, const PlanOp *__restr
 #pragma unroll
         for (int u = 0; u < 4; u++) xs.x[u] = xs.t[u] = xs.b[u] = XRegs{ 0.f, 0.f, 0.f, 0.f };
         plan_stage_issue<false>(sy, op, xs, lane, wave);
-        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
-        else                      plan_stage_finish<0>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
+        if (op.kind >= PLAN_Q6_K) plan_stage_finish<1, false>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
+        else                      plan_stage_finish<0, false>(op, SideSlots<HAS_Q5>{ nullptr, 0u, 0u }, xs, lds, red, true, lane, wave);
         __syncthreads();
         const uint32_t bytes = plan_image_bytes(op.kind, op.blocks);
         const CohBuf img = coh_buf(gptr<uint8_t>(uni(ins[j].xq)));
