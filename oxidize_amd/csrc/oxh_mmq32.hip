@@ -12,8 +12,9 @@
  * scales; the inner loop issues MFMAs, the float step and little else but LDS reads.  The products of the scales come
  * from the matrix cores as well, four blocks to an instruction (`scales`): one of four vector instructions gone, and
  * three two-byte reads of LDS per sixteen tiles in the place of six of 16 bytes, on a pipe that was nearly as busy
- * (quantiser and matmul, us: Q8_0 4096 x 4096 x 512 50.2 -> 48.4, 14336 x 4096 x 256 85.0 -> 81.1, Q4_0 85.1 -> 81.7,
- * AL5_XS 90.7 -> 87.6).  The _1 formats have two products and no registers for both: theirs stay vector instructions.
+ * (quantiser and matmul, us, in a run of that step alone: Q8_0 4096 x 4096 x 512 50.2 -> 48.4, 14336 x 4096 x 256 85.0 -> 81.1, Q4_0
+ * 85.1 -> 81.7, AL5_XS 90.7 -> 87.6).  The _1 formats have two products and no registers for both: theirs stay vector
+ * instructions.
  *
  * Shape.  A wave computes 16 rows x 32 tokens; eight waves, 64 rows x 64 tokens, to a workgroup and two workgroups to
  * a CU, or (WIDE) sixteen waves and 128 rows; four waves per SIMD either way, since one wave alone issues dependent
@@ -21,10 +22,16 @@
  * barrier per step; the next step's blocks go to LDS in the middle of a step and the ones after it are requested
  * then.  Of the Q8_0 tile's 92 % vector issue by counter, a third was not the float step: 64-bit addresses formed anew for
  * every block, the place within four bytes asked again, values cleared past the row's end.  With a wave's address in
- * scalar registers and 32-bit offsets stepped along, 269 of 317 instructions are left (quantiser and
- * matmul, us: Q8_0 4096 x 4096 x 512 48.4 -> 45.3, 14336 x 4096 x 256 81.1 -> 75.5, Q4_0 81.7 -> 74.5, Q5_0 86.0 -> 79.4,
- * AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113).  128 x 64 tiles whose waves kept raw blocks in regions of their
- * own, one workgroup to a CU, took 69 us where this took 41, eight waves of 32 x 32 42.5. */
+ * scalar registers and 32-bit offsets, 269 of 317 instructions were left (in a run of that step: Q8_0 48.4 -> 45.3 and
+ * 81.1 -> 75.5, Q4_0 81.7 -> 74.5, Q5_0 86.0 -> 79.4, AL5_XS 87.6 -> 80.7, Q4_1 112 -> 108, Q5_1 115 -> 113), and since
+ * the wave's address moves and not the offsets, 262.  All steps of this comment and those beside the code in one run, us
+ * before the first / now:
+ *                       Q8_0       Q4_0       Q4_1        Q5_0       Q5_1        AL5_XS
+ *   4096 x 4096 x 512   43.7/39.5  44.3/39.8  58.9/54.7   47.1/42.1  60.8/57.5   48.5/41.9
+ *   900 x 8192 x 128    50.8/46.0  51.6/44.8  74.1/64.8   53.2/48.3  69.8/66.9   55.9/49.1
+ *   333 x 14336 x 700   92.4/84.8  94.4/82.9  134.7/117.8 97.3/88.3  125.3/120.7 102.0/90.2
+ * 128 x 64 tiles whose waves kept raw blocks in regions of their own, one workgroup to a CU, took 69 us where the kernel
+ * before these steps took 41, eight waves of 32 x 32 42.5. */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
