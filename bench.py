@@ -294,8 +294,8 @@ def secondary_figures(mv, synth):
         pre32[name] = {"mfma_kernel_only_us": round(us, 2), "tops": round(ops / us / 1e6, 1),
                        "frac_of_int8_peak": round(ops / us / 1e6 / INT8_PEAK_TOPS, 4)}
         d_w.free()
-    pre32["note"] = ("exact per-block float step: four vector operations per output and 32-value block beside one "
-                     "16x16x32 MFMA per 256 outputs")
+    pre32["note"] = ("exact per-block float step: three vector operations per output and 32-value block (seven where the "
+                     "format has a minimum) beside one 16x16x32 MFMA per 256 outputs")
     out["q8_0_family_prefill_4096x4096x512"] = pre32
     for b_ in (d_x, d_a, d_o):
         b_.free()
@@ -729,7 +729,7 @@ def secondary_figures(mv, synth):
     d_yt = mv.DeviceBuffer(ms.n_tok * ms.hidden * 4)
     layer.forward(d_logits.ptr, d_xt.ptr, ms.n_tok, d_yt.ptr)
     mv.sync()
-    # the six launches of oxh_moe_ffn as the call makes them, and replayed as a graph (whose replays cost about
+    # the five launches of oxh_moe_ffn (up to 128 tokens; six above) as the call makes them, and replayed as a graph (whose replays cost about
     # 10 us each to start: timed in runs of fifty); five timings each, their median
     def forward():
         layer.forward(d_logits.ptr, d_xt.ptr, ms.n_tok, d_yt.ptr)
@@ -744,10 +744,10 @@ def secondary_figures(mv, synth):
     out["moe_layer_device_routed_8x_top2_16tok_q4k"] = {
         "us": round(us, 2), "gbps": round(ms.bytes_per_step / us / 1e3, 1),
         "frac_of_hbm_peak": round(ms.bytes_per_step / us / 1e3 / HBM_PEAK_GBPS, 4),
-        "launches": 6, "weights_layout": "tile-major",
+        "launches": 5, "weights_layout": "tile-major",
         "us_fastest_and_slowest_of_five_timings": [round(runs[0], 2), round(runs[-1], 2)],
         "as_graph_us": round(graph_runs[2], 2),
-        "note": "oxh_moe_ffn, one call: route + group, gather + Q8_K, gate/up of all experts, "
+        "note": "oxh_moe_ffn, one call: route + group + Q8_K of every pair's token, gate/up of all experts, "
                 "silu(gate)*up + Q8_K, down of all experts, combine; no host step between them"}
     return out
 
